@@ -137,6 +137,8 @@ bool mlp_keeps_activations(const tfh_mlp* p, int32_t precision) {
   return p && is_std_dims(make_dims(p, bf), bf);
 }
 
+int64_t mlp_kept_floats(int64_t rows) { return kept_floats(rows); }
+
 int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rpr, float* rgb, int32_t precision, void* ws,
                      size_t ws_bytes, hipStream_t st, float* act = nullptr) {
@@ -305,7 +307,9 @@ size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
   const bool bf = precision == TFH_PREC_BF16;
   MlpDims d = make_dims(p, bf);
   GradPack gp = make_pack(d);
-  return pack_bytes(d, bf) + align_up((size_t)bwd_blocks(M) * gp.total * sizeof(float), 256);
+  const size_t tables = is_std_dims(d, bf) ? std::max(pack_bytes(d, bf), bwd_planes_table_bytes(bf))
+                                           : pack_bytes(d, bf);
+  return tables + align_up((size_t)bwd_blocks(M) * gp.total * sizeof(float), 256);
 }
 
 int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
@@ -318,6 +322,27 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   GradPack gp = make_pack(d);
   const int64_t nblk = bwd_blocks(M);
   Carve cv(ws, ws_bytes);
+  // the fused training steps: the forward kept its activations
+  if (act && is_std_dims(d, bf)) {
+    BwdPlanesArgs a{};
+    a.tables = cv.take<char>((int64_t)bwd_planes_table_bytes(bf));
+    a.nblk = (unsigned)std::min<int64_t>(ceil_div(M, bwd_planes_tile_rows(bf)), num_cus());
+    a.partials = cv.take<float>(a.nblk * gp.total);
+    if (!cv.ok)
+      return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
+                  mlp_bwd_workspace(p, M, precision));
+    a.feats = feats; a.dirs = dirs; a.cams = cams; a.grgb = grgb;
+    a.M = M; a.rpr = rpr; a.gfeat = gfeat; a.gp = gp;
+    a.act = act; a.rgb = rgb; a.gembed = g->embed; a.ncam = d.ncam;
+    {
+      ProfScope ps("mlp_bwd", st);
+      TFH_TRY(launch_bwd_planes(bf, to_w(p), a, st));
+    }
+    ProfScope ps("mlp_reduce", st);
+    hipLaunchKernelGGL(k_mlp_reduce, dim3((unsigned)ceil_div(gp.b3 + 3, 64)),
+                       dim3(64 * kRedWaves), 0, st, a.partials, (int64_t)a.nblk, gp, *g);
+    return check_launch("mlp bwd: reduce");
+  }
   MlpPack pk;
   TFH_TRY(build_pack(p, d, bf, cv, pk, st));
   float* partials = cv.take<float>(nblk * gp.total);
@@ -332,10 +357,8 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
     return v && strcmp(v, "partial") == 0;
   }();
   const bool sd = is_std_dims(d, bf) && !force_partial;
-  const bool kept_film = sd && act && d.ncam > 0;  // k_mlp_bwd_kept<BF, true>
   const size_t lds = bwd_lds_floats<kBwdTM>(d, sd ? kLdsSlots * kBwdNW : 0) * sizeof(float) +
-                     (sd && d.ncam == 0 && kBwdNW == 8 ? (bf ? kG1LdsBytes : kG1LdsBytesF) : 0) +
-                     (kept_film ? (bf ? kG1FilmBytes : kG1FilmBytesF) : 0);
+                     (sd && d.ncam == 0 && kBwdNW == 8 ? (bf ? kG1LdsBytes : kG1LdsBytesF) : 0);
   TFH_REQUIRE(lds <= 160 * 1024, "mlp bwd: tile needs %zu bytes of LDS", lds);
   {
     ProfScope ps("mlp_bwd", st);
@@ -347,13 +370,7 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
                        feats, dirs, cams, grgb, M, rpr, gfeat, partials, g->embed);          \
   } while (0)
     const bool film = d.ncam > 0;
-    if (sd && act && film)
-      launch_mlp_bwd_std_film_act(bf, (unsigned)nblk, lds, st, d, to_w(p), pk, gp, feats, dirs,
-                                  cams, grgb, M, rpr, gfeat, partials, g->embed, act, rgb);
-    else if (sd && act && !film)
-      launch_mlp_bwd_std_act(bf, (unsigned)nblk, lds, st, d, to_w(p), pk, gp, feats, dirs, grgb, M,
-                             rpr, gfeat, partials, act, rgb);
-    else if (sd && film)
+    if (sd && film)
       launch_mlp_bwd_std_film(bf, (unsigned)nblk, lds, st, d, to_w(p), pk, gp, feats, dirs, cams,
                               grgb, M, rpr, gfeat, partials, g->embed);
     else if (sd)

@@ -1,13 +1,13 @@
-// FeatureMlp kernels on gfx950 MFMA, shared by five translation units:
+// FeatureMlp kernels on gfx950 MFMA, shared by the MLP's translation units:
 // tfh_mlp.hip (forward, backward of the generic shapes), tfh_mlp_bwd_std.hip
-// (backward of the standard shape), tfh_mlp_film.hip (the same with a FiLM
-// camera embedding), tfh_mlp_bwd_act.hip and tfh_mlp_film_act.hip (the
-// backward reading the activations the forward kept, tfh_mlp_bwd_kept.h,
-// without and with the embedding). The standard backward sits at the 256-VGPR limit of two waves
-// per SIMD, and the compiler allocates its registers worse when other
-// instantiations share its translation unit (once 17/31 spilled VGPRs
-// (BF16/FP32) on its own against 26/43 next to the generic kernels and 39/67
-// next to the FiLM one).
+// (backward of the standard shape that recomputes the forward), tfh_mlp_film.hip
+// (the same with a FiLM camera embedding) and tfh_mlp_bwd_planes.hip (the
+// backward that reads the activations the forward kept,
+// tfh_mlp_bwd_planes.h). The backward kernels sit at the 256-VGPR limit of two
+// waves per SIMD, and the compiler allocates their registers worse when other
+// instantiations share their translation unit (the recomputing one once 17/31
+// spilled VGPRs (BF16/FP32) on its own against 26/43 next to the generic
+// kernels).
 //
 // FeatureMlp (networks.py:38-121).
 //
@@ -30,7 +30,7 @@
 // [in][out] (input-gradient) tables of the operand precision, L2-resident.
 // The backward recomputes the forward of its tile (only layer 0 and the
 // encoding when the forward kernel kept the hidden activations, the fused
-// training steps' case: k_mlp_bwd_kept) and accumulates the weight
+// training steps' case: k_mlp_bwd_planes) and accumulates the weight
 // gradients in registers of their owning wave (standard shape) or in a
 // per-workgroup partial buffer (other shapes, plain read-modify-write, each
 // partial tile owned by one wave), reduced across workgroups by k_mlp_reduce.
@@ -61,33 +61,38 @@ struct MlpDims {
 
 __host__ __device__ inline int round_up(int x, int m) { return (x + m - 1) / m * m; }
 
-// Kept activations (the forward's relu(z1) and layer-3 input, 256 values a
-// row, for the backward): FP32 rows, or BF16 rows with the BF16 MLP, whose
-// backward only reads them as BF16 MFMA operands and as ReLU signs (the
-// rounding keeps signs and zeros), so BF16 storage changes no result and
-// halves the traffic.
+// Kept activations: the forward's relu(z1) and relu(z2) (before any camera
+// embedding), 256 values a row, for the backward. FP32, or BF16 with the BF16
+// MLP, whose backward only reads them as BF16 MFMA operands and as ReLU signs
+// (the rounding keeps signs and zeros), so BF16 storage changes no result and
+// halves the traffic. They are stored in groups of 32 rows in the order a
+// 16x16 tile's lanes hold them: relu(z1) then relu(z2), each 8 column tiles
+// of 64 lanes x 8 values (rows 4 (lane / 16) + q of the first row tile, then
+// of the second, column lane % 16), so that the layer that computes a value
+// stores it, and the backward loads it, 16 bytes a lane from contiguous
+// kilobytes (row-major rows took a pass of their own in the forward and
+// 64-byte pieces in the backward).
+constexpr int kKeptGroup = 32;                       // rows
+constexpr int kKeptHalf = kKeptGroup * 128;          // values of relu(z1) of a group
 template <bool BF>
-constexpr int kKeptRowBytes = 256 * (BF ? 2 : 4);
-
-__device__ __forceinline__ void bf16x8_to_f32(const int4& v, float4& lo, float4& hi) {
-  // a BF16 value is the upper half of its FP32 bit pattern
-  const unsigned w[4] = {(unsigned)v.x, (unsigned)v.y, (unsigned)v.z, (unsigned)v.w};
-  lo = make_float4(__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u),
-                   __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u));
-  hi = make_float4(__uint_as_float(w[2] << 16), __uint_as_float(w[2] & 0xffff0000u),
-                   __uint_as_float(w[3] << 16), __uint_as_float(w[3] & 0xffff0000u));
+constexpr int kKeptGroupBytes = 2 * kKeptHalf * (BF ? 2 : 4);
+inline int64_t kept_floats(int64_t rows) {           // room for FP32 values
+  return (rows + kKeptGroup - 1) / kKeptGroup * 2 * kKeptHalf;
 }
 
-// Stores four kept values as FP32 or BF16 (round to nearest even).
 template <bool BF>
-__device__ __forceinline__ void store_kept4(void* row, int col, const float4& v) {
+__device__ __forceinline__ void store_kept(void* __restrict__ half, int ct, int lane,
+                                           const float (&v)[8]) {
+  const int at = (ct * 64 + lane) * 8;
   if constexpr (BF) {
-    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-    bf16x4 b;
-    b[0] = (__bf16)v.x; b[1] = (__bf16)v.y; b[2] = (__bf16)v.z; b[3] = (__bf16)v.w;
-    *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(row) + col) = b;
+    bf16x8 b;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) b[q] = (__bf16)v[q];
+    *reinterpret_cast<bf16x8*>(static_cast<__bf16*>(half) + at) = b;
   } else {
-    *reinterpret_cast<float4*>(static_cast<float*>(row) + col) = v;
+    float* f = static_cast<float*>(half) + at;
+    *reinterpret_cast<float4*>(f) = make_float4(v[0], v[1], v[2], v[3]);
+    *reinterpret_cast<float4*>(f + 4) = make_float4(v[4], v[5], v[6], v[7]);
   }
 }
 
@@ -404,13 +409,11 @@ __device__ void encode_tile(const MlpDims& d, float* X, const float* Ds,
 // FT: the feature rows' type (float, stride ldF; or __bf16 with the BF16
 // MLP, stride kFsLdB).
 template <int TM, int NW, bool BF, int RTI, bool L12 = true, class FT = float>
-// h2g (optional, rows < nvalid): relu(z2) also stored to global memory, rows
-// of 256 kept values (FP32, or BF16 with the BF16 MLP: the forward's kept
-// activations with an embedding).
+// kept (optional, TM == kKeptGroup): the tile's kept activations.
 __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<BF>& op,
                                const FT* Fs, float* X, float* H0, float* H1, float* H2p,
                                float* H2, const float* Ds, const int* Cs,
-                               void* __restrict__ h2g = nullptr, int nvalid = 0) {
+                               void* __restrict__ kept = nullptr) {
   static_assert(std::is_same<FT, float>::value || BF, "BF16 feature rows need the BF16 MLP");
   const int ldFs = std::is_same<FT, float>::value ? d.ldF : kFsLdB;
   constexpr int RG = TM / 16 / RTI;  // row groups
@@ -447,13 +450,18 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
     mma_strip<RTI, K1>(X + r0 * d.ldE, d.ldE, d.EP, op.l1(), 16 * ct, acc);
     const int col = 16 * ct + (lane & 15);
     const float bias = w.b1[col];
+    float kv[4 * RTI];
 #pragma unroll
     for (int rt = 0; rt < RTI; ++rt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = r0 + 16 * rt + 4 * (lane >> 4) + e;
-        H1[row * d.ldU + col] = fmaxf(acc[rt][e] + bias, 0.0f);
+        kv[4 * rt + e] = fmaxf(acc[rt][e] + bias, 0.0f);
+        H1[row * d.ldU + col] = kv[4 * rt + e];
       }
+    if constexpr (TM == kKeptGroup && RTI == 2) {
+      if (kept) store_kept<BF>(kept, ct, lane, kv);
+    }
   }
   __syncthreads();
   // layer 2: (TM x U) @ (U x U) + b2, relu (+ FiLM) -> H2p / H2
@@ -478,12 +486,14 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
         esh = w.embed[(size_t)tc * kU + col];
       }
     }
+    float kv[4 * RTI];
 #pragma unroll
     for (int rt = 0; rt < RTI; ++rt)
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int row = r0 + 16 * rt + 4 * (lane >> 4) + e;
         const float h = fmaxf(acc[rt][e] + bias, 0.0f);
+        kv[4 * rt + e] = h;
         float out = h;
         if (d.ncam > 0 && col >= kU / 2) {
           if (tc >= 0) {
@@ -494,14 +504,16 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
           }
         }
         if (H2p != H2) H2p[row * d.ldU + col] = h;
-        if (h2g && row < nvalid) {
-          if constexpr (BF)
-            static_cast<__bf16*>(h2g)[row * 256 + col] = (__bf16)h;
-          else
-            static_cast<float*>(h2g)[row * 256 + col] = h;
-        }
         H2[row * d.ldU + col] = out;
       }
+    if constexpr (TM == kKeptGroup && RTI == 2) {
+      if (kept) {
+        if constexpr (BF)
+          store_kept<BF>(static_cast<__bf16*>(kept) + kKeptHalf, ct, lane, kv);
+        else
+          store_kept<BF>(static_cast<float*>(kept) + kKeptHalf, ct, lane, kv);
+      }
+    }
   }
   __syncthreads();
 }
@@ -576,9 +588,7 @@ inline size_t fwd_lds_floats(const MlpDims& d, bool fs_b16 = false) {
                        4 + 4);
 }
 
-// act (optional): each row's relu(z1) and layer-3 input (relu(z2) before
-// the camera embedding when there is one), 256 values (FP32, or BF16 with
-// the BF16 MLP), kept for the backward (k_mlp_bwd_kept).
+// act (optional): the kept activations, for the backward (k_mlp_bwd_planes).
 // No tile source: the feature rows are read from feats.
 struct NoGather {};
 
@@ -634,27 +644,11 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
   __syncthreads();
   // layer 1 reads X (regB) and writes H1 over Fs (regA, dead after layer 0);
   // layer 2 reads H1 and writes H2 over X (dead after layer 1)
-  // kept activations per row: relu(z1), then relu(z2) before the embedding
-  // (the layer-3 input without one); with an embedding layer 2 stores the
-  // second half itself
-  const bool film_keep = act && d.ncam > 0;
-  char* kept = reinterpret_cast<char*>(act);
-  constexpr int kRow = kKeptRowBytes<BF>;
+  void* kept = act ? reinterpret_cast<char*>(act) + tile * kKeptGroupBytes<BF> : nullptr;
   using FT = typename std::conditional<FB16, __bf16, float>::type;
   forward_hidden<TM, NW, BF, TM / 16, true, FT>(d, w, op, reinterpret_cast<const FT*>(regA), regB,
-                                                nullptr, regA, regB, regB, Ds, Cs,
-                                      film_keep ? kept + row0 * kRow + kRow / 2 : nullptr,
-                                      (int)min((int64_t)TM, M - row0));
-  if (act) {
-    for (int e = threadIdx.x; e < TM * 64; e += blockDim.x) {
-      const int i = e >> 6, c4 = e & 63;
-      if (row0 + i < M && (c4 < 32 || !film_keep)) {
-        const float* src = c4 < 32 ? regA + i * d.ldU + 4 * c4 : regB + i * d.ldU + 4 * (c4 - 32);
-        store_kept4<BF>(kept + (row0 + i) * kRow, 4 * c4, *reinterpret_cast<const float4*>(src));
-      }
-    }
-  }
-  __syncthreads();  // H1 (region A) is read above before R3 overwrites it
+                                                nullptr, regA, regB, regB, Ds, Cs, kept);
+  // (every wave is past its reads of H1, region A, before R3 overwrites it)
   forward_out<TM, NW, BF>(d, w, op, regB, R3);
   for (int e = threadIdx.x; e < TM * 3; e += blockDim.x) {
     const int i = e / 3, c = e % 3;
@@ -868,16 +862,9 @@ constexpr size_t kG1LdsBytes = (size_t)kG1Rows * kG1Ld * 2;
 // 41 KB; 153 KB in all); the other column tiles read L2.
 constexpr int kG1RowsF = 80, kG1LdF = 132;
 constexpr size_t kG1LdsBytesF = (size_t)kG1RowsF * kG1LdF * 4;
-// With the FiLM embedding (the kept-activation backward, whose relu(z2)
-// region takes 16.5 KB of the LDS): the first 80 BF16 rows (21 KB; 158 KB
-// in all) or 48 FP32 rows (25 KB; 154 KB).
-constexpr int kG1RowsFilm = 80, kG1RowsFilmF = 48;
-constexpr size_t kG1FilmBytes = (size_t)kG1RowsFilm * kG1Ld * 2;
-constexpr size_t kG1FilmBytesF = (size_t)kG1RowsFilmF * kG1LdF * 4;
-
 // The backward that recomputes each tile's forward: callers without the
 // activations kept by the forward kernel (the training steps' backward,
-// which reads them, is k_mlp_bwd_kept in tfh_mlp_bwd_kept.h).
+// which reads them, is k_mlp_bwd_planes in tfh_mlp_bwd_planes.h).
 template <int TM, int NW, bool BF, int NT, bool STD, bool FILM>
 __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpPack pk, GradPack gp_arg,
                                                      const float* __restrict__ feats,
@@ -1242,6 +1229,24 @@ inline void allow_lds(K kernel, size_t bytes) {
   }
 }
 
+// k_mlp_bwd_planes (tfh_mlp_bwd_planes.h): operand tables, launch.
+struct BwdPlanesArgs {
+  void* tables;  // bwd_planes_table_bytes()
+  unsigned nblk;
+  const float *feats, *dirs;
+  const uint32_t* cams;
+  const float* grgb;
+  int64_t M, rpr;
+  float *gfeat, *partials;
+  GradPack gp;
+  const float *act, *rgb;  // kept by the forward
+  float* gembed;
+  int ncam;
+};
+size_t bwd_planes_table_bytes(bool bf);
+int bwd_planes_tile_rows(bool bf);
+int32_t launch_bwd_planes(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
+
 // Backward launches of the standard shape without (tfh_mlp_bwd_std.hip) and
 // with (tfh_mlp_film.hip) a camera embedding.
 void launch_mlp_bwd_std(bool bf, unsigned nblk, size_t lds, hipStream_t st, const MlpDims& d,
@@ -1249,17 +1254,6 @@ void launch_mlp_bwd_std(bool bf, unsigned nblk, size_t lds, hipStream_t st, cons
                         const float* feats, const float* dirs, const uint32_t* cams,
                         const float* grgb, int64_t M, int64_t rpr, float* gfeat,
                         float* partials, float* gembed);
-void launch_mlp_bwd_std_act(bool bf, unsigned nblk, size_t lds, hipStream_t st,
-                            const MlpDims& d, const MlpW& w, const MlpPack& pk,
-                            const GradPack& gp, const float* feats, const float* dirs,
-                            const float* grgb, int64_t M, int64_t rpr, float* gfeat,
-                            float* partials, const float* act, const float* rgb);
-void launch_mlp_bwd_std_film_act(bool bf, unsigned nblk, size_t lds, hipStream_t st,
-                                 const MlpDims& d, const MlpW& w, const MlpPack& pk,
-                                 const GradPack& gp, const float* feats, const float* dirs,
-                                 const uint32_t* cams, const float* grgb, int64_t M, int64_t rpr,
-                                 float* gfeat, float* partials, float* gembed, const float* act,
-                                 const float* rgb);
 void launch_mlp_bwd_std_film(bool bf, unsigned nblk, size_t lds, hipStream_t st,
                              const MlpDims& d, const MlpW& w, const MlpPack& pk,
                              const GradPack& gp, const float* feats, const float* dirs,

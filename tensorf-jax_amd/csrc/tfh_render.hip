@@ -22,7 +22,8 @@
 namespace tfh {
 
 int32_t check_mlp(const tfh_mlp* p, const char* who);
-// act (optional): (M, 256) activations the forward keeps for the backward,
+// act (optional): activations the forward keeps for the backward
+// (mlp_kept_floats(M) floats),
 // which then also reads the forward's rgb; only for mlp_keeps_activations().
 int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rows_per_ray, float* rgb, int32_t precision, void* ws,
@@ -37,6 +38,7 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
                      const tfh_mlp_grad* g, int32_t precision, void* ws, size_t ws_bytes,
                      hipStream_t st, const float* act = nullptr, const float* rgb = nullptr);
 bool mlp_keeps_activations(const tfh_mlp* p, int32_t precision);
+int64_t mlp_kept_floats(int64_t rows);
 // hyper (optional, device): -lr_lo * decay, -lr_hi * decay, 1 - b1^count,
 // 1 - b2^count, read by the kernel in place of the host values.
 int32_t adam_launch(float* p, float* g, float* m, float* v, int64_t n, int64_t split, float lr_lo,
@@ -523,7 +525,7 @@ struct RenderWs {
   float* dfeat;  // (M, F)
   void* mlp_ws;
   size_t mlp_ws_bytes;
-  float* act = nullptr;  // (M, 256) MLP activations kept for the backward, or null
+  float* act = nullptr;  // MLP activations kept for the backward, or null
   float* mse_part = nullptr;  // kLossSlots partial sums of the MSE
   // copies of the density / appearance line gradients for the scatters, or null
   float* dlcopy = nullptr;
@@ -589,7 +591,8 @@ static size_t carve_render(Carve& cv, const tfh_render_config* cfg, const tfh_ml
 // shaded sample past the render workspace.
 static size_t act_bytes(const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R) {
   if (!mlp_keeps_activations(mlp, cfg->mlp_precision)) return 0;
-  return align_up((size_t)R * cfg->appearance_samples_per_ray * 256 * sizeof(float), 256);
+  return align_up((size_t)mlp_kept_floats(R * cfg->appearance_samples_per_ray) * sizeof(float),
+                  256);
 }
 
 static void take_act(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R,
