@@ -58,6 +58,16 @@ static int num_cus() {
 }
 
 
+// TFH_MLP_WGRAD=partial forces the generic backward (read-modify-write
+// accumulation of the weight gradients) for every shape.
+static bool force_partial() {
+  static const bool v = [] {
+    const char* e = getenv("TFH_MLP_WGRAD");
+    return e && strcmp(e, "partial") == 0;
+  }();
+  return v;
+}
+
 int32_t check_mlp(const tfh_mlp* p, const char* who) {
   TFH_REQUIRE(p != nullptr, "%s: null tfh_mlp", who);
   TFH_REQUIRE(p->w0 && p->w1 && p->b1 && p->w2 && p->b2 && p->w3 && p->b3,
@@ -129,16 +139,44 @@ size_t mlp_fwd_workspace(const tfh_mlp* p, int32_t precision) {
   return pack_bytes(make_dims(p, bf), bf);
 }
 
-// The standard shape keeps relu(z1) and relu(z2) (before any camera
+// The shapes of k_mlp_bwd_planes keep relu(z1) and relu(z2) (before any camera
 // embedding) for the backward when the caller provides the room (the fused
 // training steps).
 bool mlp_keeps_activations(const tfh_mlp* p, int32_t precision) {
-  const bool bf = precision == TFH_PREC_BF16;
-  return p && is_std_dims(make_dims(p, bf), bf);
+  return p && bwd_kind(make_dims(p, precision == TFH_PREC_BF16)) != BwdKind::kNone &&
+         !force_partial();
 }
 
 int64_t mlp_kept_floats(int64_t rows) { return kept_floats(rows); }
 
+// The forward over feature rows with its tables built; kb: act in BF16.
+static int32_t launch_fwd(const MlpDims& d, const MlpW& w, const MlpPack& pk, bool bf, bool kb,
+                          const float* feats, const float* dirs, const uint32_t* cams, int64_t M,
+                          int64_t rpr, float* rgb, float* act, hipStream_t st) {
+  const bool sd = is_std_dims(d, bf);
+  // (the BF16 standard shape keeps its feature rows in BF16: k_mlp_fwd)
+  const size_t lds = fwd_lds_floats<kFwdTM>(d, bf && sd) * sizeof(float);
+  TFH_REQUIRE(lds <= 160 * 1024, "mlp fwd: tile needs %zu bytes of LDS", lds);
+  const int64_t blocks = ceil_div(M, kFwdTM);
+#define TFH_LAUNCH_FWD(BFV, STDV, KBV)                                                         \
+  do {                                                                                         \
+    auto kernel = k_mlp_fwd<kFwdTM, kFwdNW, BFV, STDV, NoGather, KBV>;                          \
+    allow_lds(kernel, lds);                                                                    \
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kFwdNW * 64), lds, st, d, w, pk,    \
+                       feats, dirs, cams, M, rpr, rgb, act, NoGather{});                       \
+  } while (0)
+  if (!bf) {
+    if (sd) TFH_LAUNCH_FWD(false, true, false); else TFH_LAUNCH_FWD(false, false, false);
+  } else if (kb || !act) {
+    if (sd) TFH_LAUNCH_FWD(true, true, true); else TFH_LAUNCH_FWD(true, false, true);
+  } else {
+    if (sd) TFH_LAUNCH_FWD(true, true, false); else TFH_LAUNCH_FWD(true, false, false);
+  }
+#undef TFH_LAUNCH_FWD
+  return check_launch("mlp fwd");
+}
+
+// act (optional): kept for the fused step's backward.
 int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rpr, float* rgb, int32_t precision, void* ws,
                      size_t ws_bytes, hipStream_t st, float* act = nullptr) {
@@ -147,26 +185,9 @@ int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   Carve cv(ws, ws_bytes);
   MlpPack pk;
   TFH_TRY(build_pack(p, d, bf, cv, pk, st));
-  const bool sd = is_std_dims(d, bf);
-  // (the BF16 standard shape keeps its feature rows in BF16: k_mlp_fwd)
-  const size_t lds = fwd_lds_floats<kFwdTM>(d, bf && sd) * sizeof(float);
-  TFH_REQUIRE(lds <= 160 * 1024, "mlp fwd: tile needs %zu bytes of LDS", lds);
-  const int64_t blocks = ceil_div(M, kFwdTM);
   ProfScope ps("mlp_fwd_kernel", st);
-#define TFH_LAUNCH_FWD(BFV, STDV)                                                             \
-  do {                                                                                       \
-    allow_lds(k_mlp_fwd<kFwdTM, kFwdNW, BFV, STDV>, lds);                                    \
-    hipLaunchKernelGGL((k_mlp_fwd<kFwdTM, kFwdNW, BFV, STDV>), dim3((unsigned)blocks),       \
-                       dim3(kFwdNW * 64), lds, st, d, to_w(p), pk, feats, dirs, cams, M, rpr,  \
-                       rgb, act, NoGather{});                                                     \
-  } while (0)
-  if (bf) {
-    if (sd) TFH_LAUNCH_FWD(true, true); else TFH_LAUNCH_FWD(true, false);
-  } else {
-    if (sd) TFH_LAUNCH_FWD(false, true); else TFH_LAUNCH_FWD(false, false);
-  }
-#undef TFH_LAUNCH_FWD
-  return check_launch("mlp fwd");
+  return launch_fwd(d, to_w(p), pk, bf, kept_bf16(d, bf, true), feats, dirs, cams, M, rpr, rgb,
+                    act, st);
 }
 
 // The appearance gather (TensorVM.interpolate, tensor_vm.py:42-89; the
@@ -303,15 +324,37 @@ static int64_t bwd_blocks(int64_t M) {
   return nblk < 1 ? 1 : nblk;
 }
 
+// Without kept activations k_mlp_bwd_planes's shapes run the forward again,
+// keeping them, and the backward on it in turn over this many rows (of whole
+// rays): 16 tiles of 32 rows per CU, whose activations (134 MB) the Infinity
+// Cache holds, and a workspace that does not grow with the batch past that.
+static int64_t bwd_chunk(int64_t rpr) {
+  const int64_t rows = 131072;
+  return rpr >= rows ? rpr : rows / rpr * rpr;
+}
+
 size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
   const bool bf = precision == TFH_PREC_BF16;
   MlpDims d = make_dims(p, bf);
   GradPack gp = make_pack(d);
-  const size_t tables = is_std_dims(d, bf) ? std::max(pack_bytes(d, bf), bwd_planes_table_bytes(bf))
-                                           : pack_bytes(d, bf);
-  return tables + align_up((size_t)bwd_blocks(M) * gp.total * sizeof(float), 256);
+  const size_t partials = align_up((size_t)bwd_blocks(M) * gp.total * sizeof(float), 256);
+  const BwdKind kind = bwd_kind(d);
+  if (kind == BwdKind::kNone || force_partial()) return pack_bytes(d, bf) + partials;
+  const int64_t rows = std::min<int64_t>(M, 131072);  // >= any chunk: a ray has at most 1024
+  return bwd_planes_table_bytes(kind, bf) + partials + pack_bytes(d, bf) +
+         align_up((size_t)kept_floats(rows) * sizeof(float), 256) +
+         align_up((size_t)rows * 3 * sizeof(float), 256);
 }
 
+static int32_t launch_reduce(const float* partials, int64_t nblk, const GradPack& gp,
+                             const tfh_mlp_grad& g, hipStream_t st) {
+  ProfScope ps("mlp_reduce", st);
+  hipLaunchKernelGGL(k_mlp_reduce, dim3((unsigned)ceil_div(gp.b3 + 3, 64)),
+                     dim3(64 * kRedWaves), 0, st, partials, nblk, gp, g);
+  return check_launch("mlp bwd: reduce");
+}
+
+// act, rgb: kept by the fused step's forward, or null.
 int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rpr, const float* grgb, float* gfeat,
                      const tfh_mlp_grad* g, int32_t precision, void* ws, size_t ws_bytes,
@@ -322,26 +365,52 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   GradPack gp = make_pack(d);
   const int64_t nblk = bwd_blocks(M);
   Carve cv(ws, ws_bytes);
-  // the fused training steps: the forward kept its activations
-  if (act && is_std_dims(d, bf)) {
+  const BwdKind kind = bwd_kind(d);
+  if (kind != BwdKind::kNone && !force_partial()) {
     BwdPlanesArgs a{};
-    a.tables = cv.take<char>((int64_t)bwd_planes_table_bytes(bf));
-    a.nblk = (unsigned)std::min<int64_t>(ceil_div(M, bwd_planes_tile_rows(bf)), num_cus());
-    a.partials = cv.take<float>(a.nblk * gp.total);
+    char* tables = cv.take<char>((int64_t)bwd_planes_table_bytes(kind, bf));
+    a.tables = tables;
+    a.max_blocks = num_cus();
+    a.partials = cv.take<float>(nblk * gp.total);
+    a.rpr = rpr;
+    a.gp = gp;
+    a.gembed = g->embed;
+    a.ncam = d.ncam;
+    const int64_t chunk = act ? M : std::min<int64_t>(M, bwd_chunk(rpr));
+    MlpPack pk{};
+    float *kact = nullptr, *krgb = nullptr;
+    if (!act) {
+      TFH_TRY(build_pack(p, d, bf, cv, pk, st));
+      kact = cv.take<float>(kept_floats(chunk));
+      krgb = cv.take<float>(chunk * 3);
+    }
     if (!cv.ok)
       return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
                   mlp_bwd_workspace(p, M, precision));
-    a.feats = feats; a.dirs = dirs; a.cams = cams; a.grgb = grgb;
-    a.M = M; a.rpr = rpr; a.gfeat = gfeat; a.gp = gp;
-    a.act = act; a.rgb = rgb; a.gembed = g->embed; a.ncam = d.ncam;
-    {
+    TFH_TRY(pack_bwd_planes(kind, bf, to_w(p), tables, st));
+    for (int64_t c0 = 0; c0 < M; c0 += chunk) {
+      const int64_t rows = std::min<int64_t>(chunk, M - c0);
+      a.M = rows;
+      a.feats = feats + c0 * d.F;
+      a.dirs = dirs + c0 / rpr * 3;
+      a.cams = cams ? cams + c0 / rpr : nullptr;
+      a.grgb = grgb + c0 * 3;
+      a.gfeat = gfeat ? gfeat + c0 * d.F : nullptr;
+      a.act = act ? act : kact;
+      a.rgb = act ? rgb : krgb;
       ProfScope ps("mlp_bwd", st);
-      TFH_TRY(launch_bwd_planes(bf, to_w(p), a, st));
+      if (!act)
+        TFH_TRY(launch_fwd(d, to_w(p), pk, bf, kept_bf16(d, bf, false), a.feats, a.dirs, a.cams,
+                           rows, rpr, krgb, kact, st));
+      if (kind == BwdKind::kDef)
+        TFH_TRY(launch_bwd_planes_def(bf, to_w(p), a, st));
+      else if (act)
+        TFH_TRY(launch_bwd_planes_train(bf, to_w(p), a, st));
+      else
+        TFH_TRY(launch_bwd_planes_std(bf, to_w(p), a, st));
+      TFH_TRY(launch_reduce(a.partials, bwd_planes_blocks(bf, rows, a.max_blocks), gp, *g, st));
     }
-    ProfScope ps("mlp_reduce", st);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((unsigned)ceil_div(gp.b3 + 3, 64)),
-                       dim3(64 * kRedWaves), 0, st, a.partials, (int64_t)a.nblk, gp, *g);
-    return check_launch("mlp bwd: reduce");
+    return TFH_OK;
   }
   MlpPack pk;
   TFH_TRY(build_pack(p, d, bf, cv, pk, st));
@@ -349,44 +418,24 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   if (!cv.ok)
     return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
                 mlp_bwd_workspace(p, M, precision));
-  // TFH_MLP_WGRAD=partial forces the read-modify-write accumulation of the
-  // weight gradients (the register-resident one is the default when the
-  // shape has a specialised kernel)
-  static const bool force_partial = [] {
-    const char* v = getenv("TFH_MLP_WGRAD");
-    return v && strcmp(v, "partial") == 0;
-  }();
-  const bool sd = is_std_dims(d, bf) && !force_partial;
-  const size_t lds = bwd_lds_floats<kBwdTM>(d, sd ? kLdsSlots * kBwdNW : 0) * sizeof(float) +
-                     (sd && d.ncam == 0 && kBwdNW == 8 ? (bf ? kG1LdsBytes : kG1LdsBytesF) : 0);
+  const size_t lds = bwd_lds_floats<kBwdTM>(d) * sizeof(float);
   TFH_REQUIRE(lds <= 160 * 1024, "mlp bwd: tile needs %zu bytes of LDS", lds);
   {
     ProfScope ps("mlp_bwd", st);
-#define TFH_LAUNCH_BWD(BFV, NTV, STDV, FILMV)                                                 \
-  do {                                                                                        \
-    allow_lds(k_mlp_bwd<kBwdTM, kBwdNW, BFV, NTV, STDV, FILMV>, lds);                         \
-    hipLaunchKernelGGL((k_mlp_bwd<kBwdTM, kBwdNW, BFV, NTV, STDV, FILMV>),                    \
-                       dim3((unsigned)nblk), dim3(kBwdNW * 64), lds, st, d, to_w(p), pk, gp,  \
-                       feats, dirs, cams, grgb, M, rpr, gfeat, partials, g->embed);          \
-  } while (0)
-    const bool film = d.ncam > 0;
-    if (sd && film)
-      launch_mlp_bwd_std_film(bf, (unsigned)nblk, lds, st, d, to_w(p), pk, gp, feats, dirs, cams,
-                              grgb, M, rpr, gfeat, partials, g->embed);
-    else if (sd)
-      launch_mlp_bwd_std(bf, (unsigned)nblk, lds, st, d, to_w(p), pk, gp, feats, dirs, cams, grgb,
+    if (bf) {
+      allow_lds(k_mlp_bwd<kBwdTM, kBwdNW, true>, lds);
+      hipLaunchKernelGGL((k_mlp_bwd<kBwdTM, kBwdNW, true>), dim3((unsigned)nblk),
+                         dim3(kBwdNW * 64), lds, st, d, to_w(p), pk, gp, feats, dirs, cams, grgb,
                          M, rpr, gfeat, partials, g->embed);
-    else if (bf)
-      TFH_LAUNCH_BWD(true, 0, false, true);
-    else
-      TFH_LAUNCH_BWD(false, 0, false, true);
-#undef TFH_LAUNCH_BWD
+    } else {
+      allow_lds(k_mlp_bwd<kBwdTM, kBwdNW, false>, lds);
+      hipLaunchKernelGGL((k_mlp_bwd<kBwdTM, kBwdNW, false>), dim3((unsigned)nblk),
+                         dim3(kBwdNW * 64), lds, st, d, to_w(p), pk, gp, feats, dirs, cams, grgb,
+                         M, rpr, gfeat, partials, g->embed);
+    }
   }
   TFH_TRY(check_launch("mlp bwd"));
-  ProfScope ps("mlp_reduce", st);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((unsigned)ceil_div(gp.b3 + 3, 64)),
-                     dim3(64 * kRedWaves), 0, st, partials, nblk, gp, *g);
-  return check_launch("mlp bwd: reduce");
+  return launch_reduce(partials, nblk, gp, *g, st);
 }
 
 }  // namespace tfh

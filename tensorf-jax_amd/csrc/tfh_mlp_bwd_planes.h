@@ -7,8 +7,8 @@
 //   NP = 1  the BF16 MLP: operands rounded to BF16, as everywhere in that mode.
 //   NP = 3  the FP32 MLP: v = hi + mid + lo, three BF16 values (round to nearest
 //           each; 24 significant bits, so the sum is v exactly), and a product
-//           is six MFMAs (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi) into
-//           one FP32 accumulator. The dropped terms are below 2^-25 of a
+//           is six MFMAs (hi hi, hi mid, mid hi, mid mid, hi lo, lo hi)
+//           with FP32 accumulation. The dropped terms are below 2^-25 of a
 //           product, under the rounding of an FP32 multiply-add. Six BF16
 //           products of K = 32 take 96 SIMD cycles where the eight
 //           v_mfma_f32_16x16x4_f32 they replace take 256. An operand that is
@@ -42,43 +42,57 @@
 
 #include "tfh_mlp_kernels.h"
 
+// The steps are lambdas over the kernel's registers: out of line, those would
+// live in scratch memory.
+#define TFH_INLINE __attribute__((always_inline))
+
 namespace tfh {
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 
-// Columns of X in this kernel: the Fourier features of h0 (2 nf per value:
-// nf sines, nf cosines), h0, those of the direction, the direction; each
-// block starts on an 8-byte boundary. x_orig maps a column to its row of W1.
-template <int F_, int NF_>
+// The encoded input X in this kernel: its columns in NH groups (one after the
+// other in the same LDS when a shape's X does not fit whole), each the Fourier
+// features (nf sines, nf cosines per value) of some of the values of h0, then
+// those values; the last group also those of the direction, then the
+// direction. x_orig maps a column of a group to its row of W1.
+template <int F_, int NF_, int NH_>
 struct BwdShape {
-  static constexpr int F = F_, S = 27, NF = NF_, FEW = 2 * NF_;
+  static constexpr int F = F_, S = 27, NF = NF_, FEW = 2 * NF_, NH = NH_;
   static constexpr int E = S + 3 + FEW * (S + 3);
   static constexpr int FK = (F + 31) / 32 * 32;        // K of layer 0
   static constexpr int FT = (F + 15) / 16;             // feature column tiles
-  static constexpr int XH = FEW * S;                   // first column of h0
-  static constexpr int XDF = (XH + S + 3) / 4 * 4;     // first Fourier column of the direction
-  static constexpr int XD = XDF + FEW * 3;             // first column of the direction
-  static constexpr int XT = (XD + 3 + 15) / 16;        // column tiles of X
-  static constexpr int DXT = (XH + S + 15) / 16;       // those that feed h0
-  __host__ __device__ static constexpr int x_orig(int c) {
-    return c < XH ? S + 3 + c
-                  : (c < XH + S ? c - XH
-                                : (c < XDF ? -1
-                                           : (c < XD ? S + 3 + FEW * S + (c - XDF)
-                                                     : (c < XD + 3 ? S + (c - XD) : -1))));
+  static constexpr int HF = (S + NH - 1) / NH;
+  static constexpr int first(int h) { return h * HF; }               // first value of group h
+  static constexpr int count(int h) { return h < NH - 1 ? HF : S - (NH - 1) * HF; }
+  static constexpr int values(int h) { return count(h) + (h == NH - 1 ? 3 : 0); }
+  static constexpr int XT(int h) { return (values(h) * (FEW + 1) + 15) / 16; }  // column tiles
+  static constexpr int DXT(int h) { return (count(h) * (FEW + 1) + 15) / 16; }  // that feed h0
+  static constexpr int xt0(int h) { return h == 0 ? 0 : xt0(h - 1) + XT(h - 1); }
+  static constexpr int dxt0(int h) { return h == 0 ? 0 : dxt0(h - 1) + DXT(h - 1); }
+  static constexpr int maxXT() { return NH == 1 || XT(0) > XT(NH - 1) ? XT(0) : XT(NH - 1); }
+  static constexpr int maxDXT() { return NH == 1 || DXT(0) > DXT(NH - 1) ? DXT(0) : DXT(NH - 1); }
+  __host__ __device__ static constexpr int x_orig(int h, int c) {
+    const int n = count(h), d = c - n * (FEW + 1);
+    return c < n * FEW ? S + 3 + FEW * first(h) + c
+                       : (d < 0 ? first(h) + c - n * FEW
+                                : (h < NH - 1 ? -1
+                                              : (d < 3 * FEW ? S + 3 + FEW * S + d
+                                                             : (d < 3 * FEW + 3 ? S + d - 3 * FEW
+                                                                                : -1))));
   }
 };
-using BwdStd = BwdShape<144, 2>;
+using BwdStd = BwdShape<144, 2, 1>;  // 48 channels, 2 frequencies
+using BwdDef = BwdShape<72, 6, 2>;   // 24 channels, 6 frequencies: the reference's defaults
 
 // Operand tables of the backward (B operands; B(k, j) below), zero padded:
 //   f0: W0[k][j], FK x 32    g0: W0[j][k], 32 x 16 FT    g2: W2[j][k], U x U
-//   g1: W1[j][k], U x 16 DXT (j in X's column order)     g3: W3[j][k], 32 x U
+//   g1: W1[j][k], U x 16 per dX tile (j in X's column order)     g3: W3[j][k], 32 x U
 // in the order the lanes read them: for each column tile and chunk of 32 k,
 // NP planes of 64 lanes x 8 values, so a lane's load is 16 bytes of a
 // contiguous kilobyte.
 template <class SH>
 struct BwdTables {
-  static constexpr int f0 = 32 * SH::FK, g0 = 16 * SH::FT * 32, g1 = 16 * SH::DXT * kU,
+  static constexpr int f0 = 32 * SH::FK, g0 = 16 * SH::FT * 32, g1 = 16 * SH::dxt0(SH::NH) * kU,
                        g2 = kU * kU, g3 = kU * 32;
   static constexpr int o_g0 = f0, o_g1 = o_g0 + g0, o_g2 = o_g1 + g1, o_g3 = o_g2 + g2,
                        total = o_g3 + g3;  // values; a table of NP planes starts at NP * o
@@ -107,7 +121,8 @@ __global__ void k_pack_bwd(MlpW w, __bf16* __restrict__ t) {
   } else if (base == T::o_g0) {
     if (j < SH::F && k < SH::S) v = w.w0[j * SH::S + k];
   } else if (base == T::o_g1) {
-    const int o = SH::x_orig(j);
+    const bool tail = SH::NH > 1 && j >= 16 * SH::dxt0(SH::NH - 1);
+    const int o = tail ? SH::x_orig(SH::NH - 1, j - 16 * SH::dxt0(SH::NH - 1)) : SH::x_orig(0, j);
     if (o >= 0) v = w.w1[o * kU + k];
   } else if (base == T::o_g2) {
     v = w.w2[j * kU + k];
@@ -127,18 +142,39 @@ struct Frag {
   bf16x8 p[NP];
 };
 
+// acc + low += A B. With three planes the five small products go to `low`,
+// whose values stay small: the unit aligns an MFMA's products to the largest of
+// them and C and cuts off what falls below, so small products added to a large
+// C would leave a bias towards minus infinity (-7e-9 of the result's rms at
+// K = 128, 50 times that of the separate sum, and 1e-6 in a bias gradient's
+// sum over 20,000 rows). The error of a K = 128 product against float64 is
+// 0.65e-7 of the rms, of the FP32 unit's 2.0e-7.
 template <int NP>
-__device__ __forceinline__ void mma(f32x4& acc, const Frag<NP>& a, const Frag<NP>& b) {
-  if constexpr (NP == 1) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[0], acc, 0, 0, 0);
-  } else {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[2], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[2], b.p[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[1], b.p[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[1], b.p[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[0], acc, 0, 0, 0);
+__device__ __forceinline__ void mma(f32x4& acc, f32x4& low, const Frag<NP>& a, const Frag<NP>& b) {
+  if constexpr (NP == 3) {
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[2], low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[2], b.p[0], low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[1], b.p[1], low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[1], low, 0, 0, 0);
+    low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[1], b.p[0], low, 0, 0, 0);
   }
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.p[0], b.p[0], acc, 0, 0, 0);
+}
+// acc += low, here: left alone, the adds of a whole step move to its end and
+// hold its registers.
+template <int NP>
+__device__ __forceinline__ void fold(f32x4& acc, const f32x4& low) {
+  if constexpr (NP == 3) {
+    acc += low;
+    asm volatile("" : "+v"(acc));
+  }
+}
+// The same for one product onto a running sum.
+template <int NP>
+__device__ __forceinline__ void mma_add(f32x4& acc, const Frag<NP>& a, const Frag<NP>& b) {
+  f32x4 low{0.f, 0.f, 0.f, 0.f};
+  mma<NP>(acc, low, a, b);
+  fold<NP>(acc, low);
 }
 
 // A matrix of BF16 planes in LDS: TM rows of LD values per plane.
@@ -268,48 +304,56 @@ struct TableB {
 // acc[rt] += A(rows row0 + 16 rt .., values 32 c0 ..) B(., column tile ct) over
 // the chunks [c0, c0 + KC) of 32; the first PD chunks of B are in ring, the
 // rest are requested PD chunks ahead of their use.
-template <int NP, int RT, int KC, int PD, class AP, class BT>
+template <int NP, bool AHEAD, int RT, int KC, int PD, class AP, class BT>
 __device__ __forceinline__ void strip(const AP& A, int row0, int c0, const BT& b, int ct,
                                       f32x4 (&acc)[RT], Frag<NP> (&ring)[PD]) {
   const int lane = lane_here();
   const int r = lane & 15, kq = lane >> 4;
-  Frag<NP> a[2][RT];  // the next chunk's A is read ahead of this chunk's products
+  f32x4 low[RT];
+  zero_acc(low);
+  // AHEAD: the next chunk's A is read ahead of this chunk's products
+  Frag<NP> a[AHEAD ? 2 : 1][RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) a[0][rt] = A.row8(row0 + 16 * rt + r, 32 * c0 + 8 * kq);
 #pragma unroll
   for (int c = 0; c < KC; ++c) {
-    if (c + 1 < KC) {
+    const int n = AHEAD ? c + 1 : c;
+    if (n > 0 && n < KC) {
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt)
-        a[(c + 1) & 1][rt] = A.row8(row0 + 16 * rt + r, 32 * (c0 + c + 1) + 8 * kq);
+        a[AHEAD ? n & 1 : 0][rt] = A.row8(row0 + 16 * rt + r, 32 * (c0 + n) + 8 * kq);
     }
-    __builtin_amdgcn_sched_barrier(0);
+    if (AHEAD) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int rt = 0; rt < RT; ++rt) mma<NP>(acc[rt], a[c & 1][rt], ring[c % PD]);
+    for (int rt = 0; rt < RT; ++rt) mma<NP>(acc[rt], low[rt], a[AHEAD ? c & 1 : 0][rt], ring[c % PD]);
     if (c + PD < KC) ring[c % PD] = b.load(ct, c0 + c + PD);
     __builtin_amdgcn_sched_barrier(0);
   }
+  if constexpr (NP == 3) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) acc[rt] += low[rt];
+  }
 }
 
-// Weight-gradient tiles: acc[i] += X[:, tile x0 + i xs]^T y over the 32 rows of
-// group k; tiles past xn are skipped. The next X operand is read ahead.
-template <int NP, int NX, int NY, class XP>
-__device__ __forceinline__ void wgrad(const XP& X, int x0, int xs, int xn, int k,
-                                      const Frag<NP> (&y)[NY], f32x4 (&acc)[NX][NY]) {
+// Weight-gradient tiles: acc[AT + i] += X[:, tile i]^T y over the 32 rows of
+// group k, i < NX. AHEAD: the next X operand is read ahead.
+template <int NP, bool AHEAD, int NX, int AT, int NA, class XP>
+__device__ __forceinline__ void wgrad(const XP& X, int k, const Frag<NP>& y, f32x4 (&acc)[NA]) {
   const int lane = lane_here();
-  Frag<NP> x[2];
-  x[0] = X.over_rows(16 * x0, k, lane);
+  Frag<NP> x[AHEAD ? 2 : 1];
+  f32x4 low[2];  // folded a tile later: the sum waits for no product
+  x[0] = X.over_rows(0, k, lane);
 #pragma unroll
   for (int i = 0; i < NX; ++i) {
-    if (i + 1 < NX && x0 + (i + 1) * xs < xn)
-      x[(i + 1) & 1] = X.over_rows(16 * (x0 + (i + 1) * xs), k, lane);
-    __builtin_amdgcn_sched_barrier(0);
-    if (x0 + i * xs < xn) {
-#pragma unroll
-      for (int j = 0; j < NY; ++j) mma<NP>(acc[i][j], x[i & 1], y[j]);
-    }
+    const int n = AHEAD ? i + 1 : i;
+    if (n > 0 && n < NX) x[AHEAD ? n & 1 : 0] = X.over_rows(16 * n, k, lane);
+    if (AHEAD) __builtin_amdgcn_sched_barrier(0);
+    low[i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    mma<NP>(acc[AT + i], low[i & 1], x[AHEAD ? i & 1 : 0], y);
+    if (i > 0) fold<NP>(acc[AT + i - 1], low[(i - 1) & 1]);
     __builtin_amdgcn_sched_barrier(0);
   }
+  fold<NP>(acc[AT + NX - 1], low[(NX - 1) & 1]);
 }
 
 template <int NP, int PD, class BT>
@@ -330,7 +374,7 @@ __device__ __forceinline__ int thread_here() {
 // one per SIMD) take them in the other order, so that one part's vector-ALU
 // work runs beside the other's LDS reads and MFMAs. It pays with one plane
 // (0.73 -> 0.64 ms per 1 M rows); with three, whose LDS traffic is three times
-// that, it does not (1.44 against 1.51 ms).
+// that, it does not (1.44 against 1.51 ms, both before the separate low sums).
 template <bool SWAP, class A, class B>
 __device__ __forceinline__ void either_order(bool late, A&& a, B&& b) {
   if (SWAP && late) {
@@ -342,16 +386,16 @@ __device__ __forceinline__ void either_order(bool late, A&& a, B&& b) {
   }
 }
 
-template <class SH, int NP>
+template <class SH, int NP, bool SPLIT0>
 struct BwdLds {
   static constexpr int TM = NP == 1 ? 64 : 32;
   static constexpr int ldF = SH::FK + 8, ldH = kU + 8, ldD = 40;
   using PF = Planes<NP, TM, ldF>;
-  using PX = PlanesT<NP, TM, 16 * SH::XT>;
+  using PX = PlanesT<NP, TM, 16 * SH::maxXT()>;
   using PH = Planes<NP, TM, ldH>;
   using PHT = PlanesT<NP, TM, kU>;
   using PD = Planes<NP, TM, ldD>;
-  static constexpr int ldDX = 16 * SH::DXT + 4;   // dX rows (FP32)
+  static constexpr int ldDX = 16 * SH::maxDXT() + 4;   // dX rows (FP32)
   static constexpr int ldP = 33;                  // h0 parts (FP32)
   static constexpr int max2(int a, int b) { return a > b ? a : b; }
   static constexpr int oF = 0;
@@ -361,8 +405,10 @@ struct BwdLds {
   // dX lies over dZ2 (dead after step C)
   static constexpr int oZ3p = oZ2 + max2(TM * ldDX * 4, PH::bytes);  // BF16: dZ3's operand
   static constexpr int oP = oZ3p + (NP == 1 ? PD::bytes : 0);
-  static constexpr int oD = oP;                   // dH0 over the h0 parts
-  static constexpr int oZ3 = oP + (max2(2 * TM * ldP * 4, PD::bytes) + 15) / 16 * 16;
+  static constexpr int p_bytes = ((SPLIT0 ? 2 : 1) * TM * ldP * 4 + 15) / 16 * 16;
+  // dH0 over the h0 parts, which a second group's encoding still reads
+  static constexpr int oD = oP + (SH::NH == 1 ? 0 : p_bytes);
+  static constexpr int oZ3 = max2(oP + p_bytes, oD + PD::bytes);
   static constexpr int oDs = oZ3 + TM * 12;       // dZ3 (FP32, 3 x TM), then the directions
   static constexpr int oCs = oDs + TM * 12;       // cameras
   static constexpr int oE = oCs + TM * 4;         // FiLM: running embedding gradient, 2 ids
@@ -373,18 +419,25 @@ struct BwdLds {
 // FILM: cams (per ray), gembed (ncam x U, added to) and ncam >= 1.
 // SPLIT0: layer 0 in two K parts and the doubled frequency from the first by
 // the double-angle identities (the training steps); else one K chain and a
-// sincosf per frequency (callers whose backward recomputes the forward).
-template <class SH, int NP, bool FILM, bool SPLIT0>
+// sincosf per frequency.
+// KB: the kept activations are BF16 (else FP32).
+template <class SH, int NP, bool FILM, bool SPLIT0, bool KB>
 __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     MlpW w, const __bf16* __restrict__ tables, const float* __restrict__ feats,
     const float* __restrict__ dirs, const float* __restrict__ grgb, int64_t M, int64_t rpr,
     float* __restrict__ gfeat, float* __restrict__ partials, GradPack gp,
     const float* __restrict__ act, const float* __restrict__ rgb_in,
     const uint32_t* __restrict__ cams, float* __restrict__ gembed, int ncam) {
-  using L = BwdLds<SH, NP>;
+  using L = BwdLds<SH, NP, SPLIT0>;
   using T = BwdTables<SH>;
+  static_assert(!KB || NP == 1, "BF16 activations are the BF16 MLP's");
+  static_assert(!SPLIT0 || SH::NF == 2, "the double-angle identities reach two frequencies");
   constexpr int TM = L::TM, RT = TM / 16, NT = 512, NW = 8, KR = TM / 32;
   constexpr bool BF = NP == 1;
+  // reading operands a step ahead takes registers that three planes lack and
+  // brings them nothing: the LDS is their bound (1.59 ms per 1 M rows either
+  // way, the wide shape 2.55 without and 2.78 with)
+  constexpr bool AHEAD = NP == 1;
   extern __shared__ __attribute__((aligned(16))) char smem_b[];
   const typename L::PF Fp{reinterpret_cast<__bf16*>(smem_b + L::oF)};
   const typename L::PX Xp{reinterpret_cast<__bf16*>(smem_b + L::oX)};
@@ -414,12 +467,13 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
   // row tile. Those of dW0 (feature tile ft, wave ft % 8) lie in LDS, a lane's
   // four values in 16 bytes: in registers they were the ones the compiler
   // spilled, and their reload in step F waited for the next tile's loads.
-  f32x4 a2[kU / 16][1], a1[SH::XT][1];
+  constexpr int XTN = SH::xt0(SH::NH);
+  f32x4 a2[kU / 16], a1[XTN];
   f32x4* A0 = reinterpret_cast<f32x4*>(smem_b + L::oA0);
 #pragma unroll
-  for (int i = 0; i < kU / 16; ++i) a2[i][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < kU / 16; ++i) a2[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-  for (int i = 0; i < SH::XT; ++i) a1[i][0] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < XTN; ++i) a1[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   float db1 = 0.f, db2 = 0.f, db3 = 0.f, dw3[3] = {0.f, 0.f, 0.f};
   float w3r[3] = {0.f, 0.f, 0.f};
   if constexpr (!BF) {
@@ -441,7 +495,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
   typedef int i32x4 __attribute__((ext_vector_type(4)));
   constexpr int F4 = SH::F / 4, nF = (TM * F4 + NT - 1) / NT;
   static_assert(SH::F % 4 == 0 && kKeptGroup == 32, "whole loads");
-  constexpr int nA = BF ? 1 : 2;  // 16-byte loads of the lane's 8 values of a group
+  constexpr int nA = KB ? 1 : 2;  // 16-byte loads of the lane's 8 values of a group
   i32x4 vf[nF], va[KR][nA], vb[KR][nA];
   float vs = 0.f, vg = 0.f, vd = 0.f;
   int vcam = 0;
@@ -452,7 +506,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
   const unsigned step_rem = (unsigned)(step_rows - step_rays * rpr);
   int64_t ray0 = first / rpr;
   unsigned rem0 = (unsigned)(first - ray0 * rpr);
-  auto issue = [&](int64_t row0) {
+  auto issue = [&](int64_t row0) TFH_INLINE {
     const int t = thread_here();
     const int nv = (int)max((int64_t)0, min((int64_t)TM, M - row0));
     // rays of the tile: rows [row0, row0 + nv) start rem0 rows into ray0
@@ -463,8 +517,8 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     asm volatile("" : "+s"(fbase));
     const auto rf = buffer_rsrc(fbase, nv * SH::F * 4);
     const auto ra = buffer_rsrc(
-        reinterpret_cast<const char*>(act) + row0 / kKeptGroup * kKeptGroupBytes<BF>,
-        (nv + kKeptGroup - 1) / kKeptGroup * kKeptGroupBytes<BF>);
+        reinterpret_cast<const char*>(act) + row0 / kKeptGroup * kKeptGroupBytes<KB>,
+        (nv + kKeptGroup - 1) / kKeptGroup * kKeptGroupBytes<KB>);
     const auto rs = buffer_rsrc(rgb_in + row0 * 3, nv * 12);
     const auto rg = buffer_rsrc(grgb + row0 * 3, nv * 12);
     const auto rd = buffer_rsrc(dirs + ray0 * 3, nray * 12);
@@ -478,9 +532,9 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
 #pragma unroll
       for (int h = 0; h < nA; ++h) {
         const int off = t * 16 * nA + h * 16;  // (wave, lane) in order
-        va[k][h] = __builtin_amdgcn_raw_buffer_load_b128(ra, off, k * kKeptGroupBytes<BF>, 0);
+        va[k][h] = __builtin_amdgcn_raw_buffer_load_b128(ra, off, k * kKeptGroupBytes<KB>, 0);
         vb[k][h] = __builtin_amdgcn_raw_buffer_load_b128(
-            ra, off, k * kKeptGroupBytes<BF> + kKeptGroupBytes<BF> / 2, 0);
+            ra, off, k * kKeptGroupBytes<KB> + kKeptGroupBytes<KB> / 2, 0);
       }
     const int i3 = t / 3, c3 = t - 3 * i3;
     const bool own3 = t < TM * 3;
@@ -509,11 +563,11 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
 
   // layer 0's items: (K part, column tile, row tile), the first one's B chunks
   // (ringf) requested behind the tile's own loads
-  constexpr int KC0 = SH::FK / 32, KA = SPLIT0 ? (KC0 + 1) / 2 : KC0, KB = KC0 - KA;
+  constexpr int KC0 = SH::FK / 32, KA = SPLIT0 ? (KC0 + 1) / 2 : KC0, KR0 = KC0 - KA;
   constexpr int PARTS = SPLIT0 ? 2 : 1, NI0 = 2 * RT * PARTS;
-  constexpr int PD0 = KB > 0 && KB < 2 ? 1 : 2;
+  constexpr int PD0 = NP == 3 || KR0 == 1 ? 1 : 2;
   Frag<NP> ringf[PD0];
-  auto issue_f0 = [&]() {
+  auto issue_f0 = [&]() TFH_INLINE {
     strip_pre<NP>(t_f0, (wave / PARTS) & 1, (SPLIT0 && (wave & 1)) ? KA : 0, ringf);
   };
 
@@ -540,7 +594,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
 #pragma unroll
       for (int k = 0; k < KR; ++k) {
         Frag<NP> f;
-        if constexpr (BF) {
+        if constexpr (KB) {
           f.p[0] = __builtin_bit_cast(bf16x8, va[k][0]);
 #pragma unroll
           for (int e = 0; e < 8; ++e)
@@ -548,7 +602,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float h = __uint_as_float((unsigned)va[k][BF ? 0 : e / 4][e % 4]);
+            const float h = __uint_as_float((unsigned)va[k][KB ? 0 : e / 4][e % 4]);
             set_frag<NP>(f, e, h);
             pos1 |= h > 0.0f ? 1u << (8 * k + e) : 0u;
           }
@@ -593,20 +647,20 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
       __syncthreads();
     }
     // dZ1's first B chunks
-    constexpr int PD2 = NP == 1 ? 4 : 2;
+    constexpr int PD2 = NP == 1 ? 4 : (SH::NH == 1 ? 2 : 1);
     Frag<NP> ring2[PD2];
     strip_pre<NP>(t_g2, wave, 0, ring2);
     // ---- B: layer 0 -> P0 ----
-    auto layer0 = [&]() {
+    auto layer0 = [&]() TFH_INLINE {
       for (int it = wave; it < NI0; it += NW) {
         const int kp = SPLIT0 ? it & 1 : 0, ct = (it / PARTS) & 1, rt = it / (2 * PARTS);
         f32x4 acc[1];
         zero_acc(acc);
         if (it != wave) strip_pre<NP>(t_f0, ct, kp ? KA : 0, ringf);
         if (kp == 0)
-          strip<NP, 1, KA, PD0>(Fp, 16 * rt, 0, t_f0, ct, acc, ringf);
+          strip<NP, AHEAD, 1, KA, PD0>(Fp, 16 * rt, 0, t_f0, ct, acc, ringf);
         else
-          strip<NP, 1, (KB > 0 ? KB : 1), PD0>(Fp, 16 * rt, KA, t_f0, ct, acc, ringf);
+          strip<NP, AHEAD, 1, (KR0 > 0 ? KR0 : 1), PD0>(Fp, 16 * rt, KA, t_f0, ct, acc, ringf);
         const int ln = lane_here(), r16 = ln & 15, kq4 = ln >> 4;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -614,11 +668,11 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
       }
     };
     // ---- B: dZ2 = (dZ3 W3^T) [z2 > 0] -> Z2 ; db2 ; dW3 ; dW2 += H1^T dZ2 ----
-    auto layer3 = [&]() {
-      Frag<NP> y[KR][1];
+    auto layer3 = [&]() TFH_INLINE {
+      Frag<NP> y[KR];
       f32x4 acc[RT];
       zero_acc(acc);
-      if constexpr (BF) strip<NP, RT, 1, 1>(Z3p, 0, 0, t_g3, wave, acc, ring3);
+      if constexpr (BF) strip<NP, AHEAD, RT, 1, 1>(Z3p, 0, 0, t_g3, wave, acc, ring3);
       const int lane = lane_here(), r16 = lane & 15, kq4 = lane >> 4, ucol = 16 * wave + r16;
       const bool film = FILM && 16 * wave >= kU / 2;  // wave-uniform
       int tcam = -1;
@@ -642,13 +696,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
         for (int e = 0; e < 4; ++e) {
           const int row = 16 * rt + 4 * kq4 + e;
           float g, hp;
-          if constexpr (BF) {
+          if constexpr (BF)
             g = acc[rt][e];
-            hp = (float)__builtin_bit_cast(bf16x8, vb[rt / 2][0])[4 * (rt & 1) + e];
-          } else {
+          else
             g = z[0][e] * w3r[0] + z[1][e] * w3r[1] + z[2][e] * w3r[2];
-            hp = __uint_as_float((unsigned)vb[rt / 2][BF ? 0 : rt & 1][e]);
-          }
+          if constexpr (KB)
+            hp = (float)__builtin_bit_cast(bf16x8, vb[rt / 2][0])[4 * (rt & 1) + e];
+          else
+            hp = __uint_as_float((unsigned)vb[rt / 2][KB ? 0 : rt & 1][e]);
           float hf = hp;  // the layer-3 input
           if constexpr (FILM) {
             if (film) {
@@ -677,7 +732,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
             dw3[c] += hf * (BF ? (float)(__bf16)z[c][e] : z[c][e]);
           const float dz = hp > 0.0f ? g : 0.0f;
           db2 += dz;
-          Frag<NP>& f = y[rt / 2][0];
+          Frag<NP>& f = y[rt / 2];
           const int at = 4 * (rt & 1) + e;
           set_frag<NP>(f, at, dz);
 #pragma unroll
@@ -698,52 +753,59 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
       }
 #pragma unroll
       for (int k = 0; k < KR; ++k)
-        wgrad<NP, kU / 16, 1>(H1t, 0, 1, kU / 16, k, y[k], a2);
+        wgrad<NP, AHEAD, kU / 16, 0>(H1t, k, y[k], a2);
     };
     either_order<BF>(late, layer0, layer3);
     __syncthreads();
-    // ---- C: encoding -> X ----
-    constexpr int nI = TM * 32 / NT;  // (value, row) items per thread
-    float hv[nI], sv0[nI], cv0[nI];
-    auto encode = [&]() {
+    // ---- C: encoding of a group -> X ----
+    // slots (value u, row i) of 512 threads, the same in the encoding and in
+    // step E, which finds the sines and cosines in registers (of the first
+    // frequency alone where the second is derived)
+    constexpr int nI = TM * ((SH::HF + (SH::NH == 1 ? 3 : 2) + 7) / 8 * 8) / NT;
+    constexpr int JN = nI * NT / TM, NK = SPLIT0 ? 2 : SH::FEW;
+    static_assert(JN >= SH::values(0) && JN >= SH::values(SH::NH - 1), "a slot per value");
+    float sc[nI][NK];
+    auto encode = [&](auto hc) TFH_INLINE {
+      constexpr int h = decltype(hc)::value, n = SH::count(h);
 #pragma unroll
       for (int m = 0; m < nI; ++m) {
         const int e = thread_here() + m * NT, i = e % TM, u = e / TM, pos = row_pos(i);
         float v = 0.f;
-        if (u < SH::S) {
-          v = P0[i * L::ldP + u];
-          if constexpr (SPLIT0) v += P0[(TM + i) * L::ldP + u];
-        } else if (u < SH::S + 3) {
-          v = Ds[(u - SH::S) * TM + i];
+        if (u < n) {
+          v = P0[i * L::ldP + SH::first(h) + u];
+          if constexpr (SPLIT0) v += P0[(TM + i) * L::ldP + SH::first(h) + u];
+        } else if (u < SH::values(h)) {
+          v = Ds[(u - n) * TM + i];
         }
-        hv[m] = v;
         float fe[SH::FEW];
-        sincosf(v, &sv0[m], &cv0[m]);
-        fe[0] = sv0[m];
-        fe[SH::NF] = cv0[m];
+        sincosf(v, &fe[0], &fe[SH::NF]);
+        sc[m][0] = fe[0];
+        sc[m][NK / 2] = fe[SH::NF];
 #pragma unroll
         for (int q = 1; q < SH::NF; ++q) {
-          if (SPLIT0 && q == 1) {
-            fe[1] = 2.0f * sv0[m] * cv0[m];
-            fe[SH::NF + 1] = (cv0[m] - sv0[m]) * (cv0[m] + sv0[m]);
+          if constexpr (SPLIT0) {
+            fe[1] = 2.0f * fe[0] * fe[2];
+            fe[3] = (fe[2] - fe[0]) * (fe[2] + fe[0]);
           } else {
             sincosf(v * (float)(1 << q), &fe[q], &fe[SH::NF + q]);
+            sc[m][q] = fe[q];
+            sc[m][SH::NF + q] = fe[SH::NF + q];
           }
         }
-        if (u < SH::S + 3) {
-          const int fc = u < SH::S ? SH::FEW * u : SH::XDF + SH::FEW * (u - SH::S);
+        if (u < SH::values(h)) {
+          const int fc = u < n ? SH::FEW * u : n * (SH::FEW + 1) + SH::FEW * (u - n);
 #pragma unroll
           for (int q = 0; q < SH::FEW; ++q) Xp.put(pos, fc + q, fe[q]);
-          Xp.put(pos, u < SH::S ? SH::XH + u : SH::XD + (u - SH::S), v);
+          Xp.put(pos, u < n ? n * SH::FEW + u : n * (SH::FEW + 1) + 3 * SH::FEW + (u - n), v);
         }
       }
     };
     // ---- C: dZ1 = (dZ2 W2^T) [z1 > 0] over relu(z1) ; db1 ----
-    Frag<NP> y1[KR][1];
-    auto layer2 = [&]() {
+    Frag<NP> y1[KR];
+    auto layer2 = [&]() TFH_INLINE {
       f32x4 acc[RT];
       zero_acc(acc);
-      strip<NP, RT, 4, PD2>(Z2, 0, 0, t_g2, wave, acc, ring2);
+      strip<NP, AHEAD, RT, 4, PD2>(Z2, 0, 0, t_g2, wave, acc, ring2);
       const int lane = lane_here(), kq4 = lane >> 4, ucol = 16 * wave + (lane & 15);
 #pragma unroll
       for (int q = 0; q < 4 * RT; ++q) {
@@ -751,45 +813,92 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
         const int row = 16 * rt + 4 * kq4 + e;
         const float dz = (pos1 >> q) & 1 ? acc[rt][e] : 0.0f;
         db1 += dz;
-        Frag<NP>& f = y1[rt / 2][0];
+        Frag<NP>& f = y1[rt / 2];
         const int at = 4 * (rt & 1) + e;
         set_frag<NP>(f, at, dz);
 #pragma unroll
         for (int p = 0; p < NP; ++p) Z1.m[p * L::PH::ps + row * L::ldH + ucol] = f.p[p][at];
       }
     };
-    either_order<BF>(late, encode, layer2);
-    // dX's first B chunks
+    either_order<BF>(late, [&]() TFH_INLINE { encode(std::integral_constant<int, 0>{}); }, layer2);
+    // ---- D: dW1 += X^T dZ1 ; dX = dZ1 W1^T (group h; its first B chunks in ring2) ----
+    auto layer1 = [&](auto hc) TFH_INLINE {
+      constexpr int h = decltype(hc)::value, ct0 = SH::dxt0(h);
+#pragma unroll
+      for (int k = 0; k < KR; ++k) wgrad<NP, AHEAD, SH::XT(h), SH::xt0(h)>(Xp, k, y1[k], a1);
+      // the column tiles past the last whole round go one row tile to a wave
+      constexpr int DXF = SH::DXT(h) / NW, DXR = SH::DXT(h) % NW;
+#pragma unroll 1
+      for (int i = 0; i < DXF; ++i) {
+        const int ct = wave + NW * i;
+        if (i > 0) strip_pre<NP>(t_g1, ct0 + ct, 0, ring2);
+        f32x4 acc[RT];
+        zero_acc(acc);
+        strip<NP, AHEAD, RT, 4, PD2>(Z1, 0, 0, t_g1, ct0 + ct, acc, ring2);
+        const int lane = lane_here(), r16 = lane & 15, kq4 = lane >> 4;
+#pragma unroll
+        for (int q = 0; q < 4 * RT; ++q)
+          DX[(16 * (q / 4) + 4 * kq4 + q % 4) * L::ldDX + 16 * ct + r16] = acc[q / 4][q % 4];
+      }
+#pragma unroll 1
+      for (int it = wave; it < DXR * RT; it += NW) {
+        const int ct = NW * DXF + it / RT, rt = it % RT;
+        strip_pre<NP>(t_g1, ct0 + ct, 0, ring2);
+        f32x4 acc[1];
+        zero_acc(acc);
+        strip<NP, AHEAD, 1, 4, PD2>(Z1, 16 * rt, 0, t_g1, ct0 + ct, acc, ring2);
+        const int lane = lane_here(), r16 = lane & 15, kq4 = lane >> 4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          DX[(16 * rt + 4 * kq4 + e) * L::ldDX + 16 * ct + r16] = acc[0][e];
+      }
+    };
+    // ---- E: dH0[j] = dX[h_j] + sum_q 2^q (dX[sin_q] cos(2^q h) - dX[cos_q] sin(2^q h)) ----
+    auto squash = [&](auto hc) TFH_INLINE {
+      constexpr int h = decltype(hc)::value, n = SH::count(h);
+#pragma unroll
+      for (int m = 0; m < nI; ++m) {
+        const int e = thread_here() + m * NT, i = e % TM, j = e / TM;
+        if (j < n) {
+          const float* dx = DX + i * L::ldDX;
+          float d[SH::FEW];
+#pragma unroll
+          for (int q = 0; q < SH::FEW; q += 4) {
+            const float4 v = *reinterpret_cast<const float4*>(dx + SH::FEW * j + q);
+            d[q] = v.x; d[q + 1] = v.y; d[q + 2] = v.z; d[q + 3] = v.w;
+          }
+          float g = dx[n * SH::FEW + j];
+#pragma unroll
+          for (int q = 0; q < SH::NF; ++q) {
+            float sq, cq;
+            if constexpr (SPLIT0) {
+              const float s0 = sc[m][0], c0 = sc[m][1];
+              sq = q == 0 ? s0 : 2.0f * s0 * c0;
+              cq = q == 0 ? c0 : (c0 - s0) * (c0 + s0);
+            } else {
+              sq = sc[m][q];
+              cq = sc[m][SH::NF + q];
+            }
+            const float s = (float)(1 << q);
+            g += d[q] * s * cq;
+            g -= d[SH::NF + q] * s * sq;
+          }
+          Dp.put(i, SH::first(h) + j, g);
+        } else if (h == SH::NH - 1) {  // the zero padding to 32 columns
+          for (int c = SH::S + (j - n); c < 32; c += JN - n) Dp.put(i, c, 0.0f);
+        }
+      }
+    };
     strip_pre<NP>(t_g1, wave, 0, ring2);
     __syncthreads();
-    // ---- D: dW1 += X^T dZ1 ; dX = dZ1 W1^T ----
-#pragma unroll
-    for (int k = 0; k < KR; ++k) wgrad<NP, SH::XT, 1>(Xp, 0, 1, SH::XT, k, y1[k], a1);
-    // the column tiles past the last whole round go one row tile to a wave
-    constexpr int DXF = SH::DXT / NW, DXR = SH::DXT % NW;
-#pragma unroll 1
-    for (int i = 0; i < DXF; ++i) {
-      const int ct = wave + NW * i;
-      if (i > 0) strip_pre<NP>(t_g1, ct, 0, ring2);
-      f32x4 acc[RT];
-      zero_acc(acc);
-      strip<NP, RT, 4, PD2>(Z1, 0, 0, t_g1, ct, acc, ring2);
-      const int lane = lane_here(), r16 = lane & 15, kq4 = lane >> 4;
-#pragma unroll
-      for (int q = 0; q < 4 * RT; ++q)
-        DX[(16 * (q / 4) + 4 * kq4 + q % 4) * L::ldDX + 16 * ct + r16] = acc[q / 4][q % 4];
-    }
-#pragma unroll 1
-    for (int it = wave; it < DXR * RT; it += NW) {
-      const int ct = NW * DXF + it / RT, rt = it % RT;
-      strip_pre<NP>(t_g1, ct, 0, ring2);
-      f32x4 acc[1];
-      zero_acc(acc);
-      strip<NP, 1, 4, PD2>(Z1, 16 * rt, 0, t_g1, ct, acc, ring2);
-      const int lane = lane_here(), r16 = lane & 15, kq4 = lane >> 4;
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        DX[(16 * rt + 4 * kq4 + e) * L::ldDX + 16 * ct + r16] = acc[0][e];
+    layer1(std::integral_constant<int, 0>{});
+    if constexpr (SH::NH == 2) {
+      strip_pre<NP>(t_g1, SH::dxt0(1) + wave, 0, ring2);
+      __syncthreads();
+      squash(std::integral_constant<int, 0>{});
+      encode(std::integral_constant<int, 1>{});
+      __syncthreads();
+      layer1(std::integral_constant<int, 1>{});
     }
     // dF's B chunks: column tile wave for every row tile, then one (column
     // tile, row tile) of those past the first 8, counted down from the last
@@ -801,53 +910,16 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     if (wave < SH::FT) ringg[0] = t_g0.load(wave, 0);
     if (xdf < DFX) ringg[1] = t_g0.load(NW + xdf / RT, 0);
     __syncthreads();
-    // ---- E: the next tile's loads (steps E and F wait for nothing behind them) ----
-    auto next = [&]() { issue(row0 + (int64_t)gridDim.x * TM); };
-    // ---- E: dH0[j] = dX[h_j] + sum_q 2^q (dX[sin_q] cos(2^q h) - dX[cos_q] sin(2^q h)) ----
-    auto squash = [&]() {
-#pragma unroll
-      for (int m = 0; m < nI; ++m) {
-        const int e = thread_here() + m * NT, i = e % TM, j = e / TM;
-        float g = 0.0f;
-        if (j < SH::S) {
-          const float* dx = DX + i * L::ldDX;
-          float d[SH::FEW], sc[SH::FEW];
-#pragma unroll
-          for (int q = 0; q < SH::FEW; q += 4) {
-            const float4 v = *reinterpret_cast<const float4*>(dx + SH::FEW * j + q);
-            d[q] = v.x; d[q + 1] = v.y; d[q + 2] = v.z; d[q + 3] = v.w;
-          }
-#pragma unroll
-          for (int q = 0; q < SH::NF; ++q) {
-            if (q == 0) {
-              sc[0] = sv0[m];
-              sc[SH::NF] = cv0[m];
-            } else if (SPLIT0 && q == 1) {
-              sc[1] = 2.0f * sv0[m] * cv0[m];
-              sc[SH::NF + 1] = (cv0[m] - sv0[m]) * (cv0[m] + sv0[m]);
-            } else {
-              sincosf(hv[m] * (float)(1 << q), &sc[q], &sc[SH::NF + q]);
-            }
-          }
-          g = dx[SH::XH + j];
-#pragma unroll
-          for (int q = 0; q < SH::NF; ++q) {
-            const float s = (float)(1 << q);
-            g += d[q] * s * sc[SH::NF + q];
-            g -= d[SH::NF + q] * s * sc[q];
-          }
-        }
-        Dp.put(i, j, g);
-      }
-    };
-    either_order<BF>(late, next, squash);
+    // the next tile's loads: steps E and F wait for nothing behind them
+    either_order<BF>(late, [&]() TFH_INLINE { issue(row0 + (int64_t)gridDim.x * TM); },
+                     [&]() TFH_INLINE { squash(std::integral_constant<int, SH::NH - 1>{}); });
     __syncthreads();
     // ---- F: dF = dH0 W0^T ; dW0 += F^T dH0 ----
     if (gfeat) {
       // a buffer over the tile's valid rows drops the others
       const auto rgf = buffer_rsrc(gfeat + row0 * SH::F,
                                    (int)min((int64_t)TM, M - row0) * SH::F * 4);
-      auto store = [&](const f32x4& v, int ct, int rt) {
+      auto store = [&](const f32x4& v, int ct, int rt) TFH_INLINE {
         const int ln = lane_here(), kq4 = ln >> 4, col = 16 * ct + (ln & 15);
         const int off = ((16 * rt + 4 * kq4) * SH::F + col) * 4;
         if (SH::F % 16 == 0 || col < SH::F) {
@@ -862,14 +934,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
           f32x4 acc{0.f, 0.f, 0.f, 0.f};
-          mma<NP>(acc, Dp.row8(16 * rt + (ln & 15), 8 * (ln >> 4)), ringg[0]);
+          mma_add<NP>(acc, Dp.row8(16 * rt + (ln & 15), 8 * (ln >> 4)), ringg[0]);
           store(acc, wave, rt);
         }
       }
       if (xdf < DFX) {
         const int ln = lane_here(), rt = xdf % RT;
         f32x4 acc{0.f, 0.f, 0.f, 0.f};
-        mma<NP>(acc, Dp.row8(16 * rt + (ln & 15), 8 * (ln >> 4)), ringg[1]);
+        mma_add<NP>(acc, Dp.row8(16 * rt + (ln & 15), 8 * (ln >> 4)), ringg[1]);
         store(acc, NW + xdf / RT, rt);
       }
     }
@@ -881,7 +953,7 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
       for (int k = 0; k < KR; ++k) {
         const Frag<NP> x = Fp.over_rows(16 * ft, k, ln);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) mma<NP>(acc[j], x, Dp.over_rows(16 * j, k, ln));
+        for (int j = 0; j < 2; ++j) mma_add<NP>(acc[j], x, Dp.over_rows(16 * j, k, ln));
       }
       slot[0] = acc[0];
       slot[64] = acc[1];
@@ -922,13 +994,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
   for (int i = 0; i < kU / 16; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      part[gp.w2 + (16 * i + 4 * kq4 + e) * kU + ucol] = a2[i][0][e];
+      part[gp.w2 + (16 * i + 4 * kq4 + e) * kU + ucol] = a2[i][e];
 #pragma unroll
-  for (int i = 0; i < SH::XT; ++i)
+  for (int i = 0; i < XTN; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int o = SH::x_orig(16 * i + 4 * kq4 + e);
-      if (o >= 0) part[gp.w1 + o * kU + ucol] = a1[i][0][e];
+      const int h = SH::NH > 1 && i >= SH::xt0(SH::NH - 1) ? SH::NH - 1 : 0;
+      const int o = SH::x_orig(h, 16 * (i - SH::xt0(h)) + 4 * kq4 + e);
+      if (o >= 0) part[gp.w1 + o * kU + ucol] = a1[i][e];
     }
   for (int ft = wave; ft < SH::FT; ft += NW)
 #pragma unroll
@@ -940,6 +1013,31 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
         if (f < SH::F && scol < SH::S) part[gp.w0 + f * SH::S + scol] = v[e];
       }
     }
+}
+
+template <class SH, int NP, bool FILM, bool SPLIT0, bool KB>
+int32_t run_planes(const MlpW& w, const BwdPlanesArgs& a, hipStream_t st) {
+  using L = BwdLds<SH, NP, SPLIT0>;
+  static_assert(L::bytes <= 160 * 1024, "the tile fits the LDS of a CU");
+  auto kernel = k_mlp_bwd_planes<SH, NP, FILM, SPLIT0, KB>;
+  allow_lds(kernel, L::bytes);
+  static_assert(L::TM == (NP == 1 ? kBwdRowsBf16 : kBwdRowsFp32), "bwd_planes_blocks");
+  hipLaunchKernelGGL(kernel, dim3((unsigned)bwd_planes_blocks(NP == 1, a.M, a.max_blocks)), dim3(512), L::bytes, st, w,
+                     static_cast<const __bf16*>(a.tables), a.feats, a.dirs, a.grgb, a.M, a.rpr,
+                     a.gfeat, a.partials, a.gp, a.act, a.rgb, a.cams, a.gembed, a.ncam);
+  return check_launch("mlp bwd");
+}
+
+template <class SH>
+int32_t pack_planes(bool bf, const MlpW& w, void* tables, hipStream_t st) {
+  const dim3 grid((BwdTables<SH>::total + 255) / 256);
+  if (bf)
+    hipLaunchKernelGGL((k_pack_bwd<SH, 1>), grid, dim3(256), 0, st, w,
+                       static_cast<__bf16*>(tables));
+  else
+    hipLaunchKernelGGL((k_pack_bwd<SH, 3>), grid, dim3(256), 0, st, w,
+                       static_cast<__bf16*>(tables));
+  return check_launch("mlp bwd: operand tables");
 }
 
 }  // namespace tfh

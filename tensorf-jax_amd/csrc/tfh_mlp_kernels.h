@@ -1,13 +1,6 @@
-// FeatureMlp kernels on gfx950 MFMA, shared by the MLP's translation units:
-// tfh_mlp.hip (forward, backward of the generic shapes), tfh_mlp_bwd_std.hip
-// (backward of the standard shape that recomputes the forward), tfh_mlp_film.hip
-// (the same with a FiLM camera embedding) and tfh_mlp_bwd_planes.hip (the
-// backward that reads the activations the forward kept,
-// tfh_mlp_bwd_planes.h). The backward kernels sit at the 256-VGPR limit of two
-// waves per SIMD, and the compiler allocates their registers worse when other
-// instantiations share their translation unit (the recomputing one once 17/31
-// spilled VGPRs (BF16/FP32) on its own against 26/43 next to the generic
-// kernels).
+// FeatureMlp kernels on gfx950 MFMA: the forward, the backward of the generic
+// shapes, and the declarations of the backward of the shapes with compile-time
+// dims (tfh_mlp_bwd_planes.h, in translation units of its own).
 //
 // FeatureMlp (networks.py:38-121).
 //
@@ -28,12 +21,10 @@
 //         rounded to BF16 when loaded as operands.
 // Weights are packed once per call into zero-padded [out][in] (forward) and
 // [in][out] (input-gradient) tables of the operand precision, L2-resident.
-// The backward recomputes the forward of its tile (only layer 0 and the
-// encoding when the forward kernel kept the hidden activations, the fused
-// training steps' case: k_mlp_bwd_planes) and accumulates the weight
-// gradients in registers of their owning wave (standard shape) or in a
-// per-workgroup partial buffer (other shapes, plain read-modify-write, each
-// partial tile owned by one wave), reduced across workgroups by k_mlp_reduce.
+// The generic backward recomputes the forward of its tile and accumulates the
+// weight gradients in a per-workgroup partial buffer (plain read-modify-write,
+// each partial tile owned by one wave), reduced across workgroups by
+// k_mlp_reduce.
 #pragma once
 
 #include <stdlib.h>
@@ -408,8 +399,8 @@ __device__ void encode_tile(const MlpDims& d, float* X, const float* Ds,
 // L12 == false stops after the encoding (H1 and H2 come from elsewhere).
 // FT: the feature rows' type (float, stride ldF; or __bf16 with the BF16
 // MLP, stride kFsLdB).
-template <int TM, int NW, bool BF, int RTI, bool L12 = true, class FT = float>
-// kept (optional, TM == kKeptGroup): the tile's kept activations.
+template <int TM, int NW, bool BF, int RTI, bool L12 = true, class FT = float, bool KB = BF>
+// kept (optional, TM == kKeptGroup): the tile's kept activations (KB: in BF16).
 __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<BF>& op,
                                const FT* Fs, float* X, float* H0, float* H1, float* H2p,
                                float* H2, const float* Ds, const int* Cs,
@@ -460,7 +451,7 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
         H1[row * d.ldU + col] = kv[4 * rt + e];
       }
     if constexpr (TM == kKeptGroup && RTI == 2) {
-      if (kept) store_kept<BF>(kept, ct, lane, kv);
+      if (kept) store_kept<KB>(kept, ct, lane, kv);
     }
   }
   __syncthreads();
@@ -508,10 +499,7 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
       }
     if constexpr (TM == kKeptGroup && RTI == 2) {
       if (kept) {
-        if constexpr (BF)
-          store_kept<BF>(static_cast<__bf16*>(kept) + kKeptHalf, ct, lane, kv);
-        else
-          store_kept<BF>(static_cast<float*>(kept) + kKeptHalf, ct, lane, kv);
+        store_kept<KB>(static_cast<char*>(kept) + kKeptGroupBytes<KB> / 2, ct, lane, kv);
       }
     }
   }
@@ -596,7 +584,7 @@ struct NoGather {};
 // itself (gt.load<TM, NT, CAMS, FB16>(d, row0, M, rpr, Fs, Ds, Cs, dirs,
 // cams): the appearance gather fused into the tile load, its rows also
 // written to global memory for the backward), instead of reading feats.
-template <int TM, int NW, bool BF, bool STD, class GT = NoGather>
+template <int TM, int NW, bool BF, bool STD, class GT = NoGather, bool KB = BF>
 __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpPack pk,
                                                      const float* __restrict__ feats,
                                                      const float* __restrict__ dirs,
@@ -644,9 +632,9 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
   __syncthreads();
   // layer 1 reads X (regB) and writes H1 over Fs (regA, dead after layer 0);
   // layer 2 reads H1 and writes H2 over X (dead after layer 1)
-  void* kept = act ? reinterpret_cast<char*>(act) + tile * kKeptGroupBytes<BF> : nullptr;
+  void* kept = act ? reinterpret_cast<char*>(act) + tile * kKeptGroupBytes<KB> : nullptr;
   using FT = typename std::conditional<FB16, __bf16, float>::type;
-  forward_hidden<TM, NW, BF, TM / 16, true, FT>(d, w, op, reinterpret_cast<const FT*>(regA), regB,
+  forward_hidden<TM, NW, BF, TM / 16, true, FT, KB>(d, w, op, reinterpret_cast<const FT*>(regA), regB,
                                                 nullptr, regA, regB, regB, Ds, Cs, kept);
   // (every wave is past its reads of H1, region A, before R3 overwrites it)
   forward_out<TM, NW, BF>(d, w, op, regB, R3);
@@ -740,20 +728,15 @@ __device__ __forceinline__ void add_tile(float* __restrict__ part, int64_t off, 
 }
 
 template <int TM>
-inline size_t bwd_lds_floats(const MlpDims& d, int lds_tiles) {
+inline size_t bwd_lds_floats(const MlpDims& d) {
   return (size_t)TM * (d.ldF + d.ldE + d.ldS + 2 * d.ldU + (d.ncam > 0 ? d.ldU : 0) + d.ld3 + 4 +
                        4) +
-         (d.ncam > 0 ? kU + 4 : 0) +  // FiLM: running embedding gradient + 2 camera ids
-         (size_t)lds_tiles * 256;     // weight-gradient tiles accumulated in LDS
+         (d.ncam > 0 ? kU + 4 : 0);  // FiLM: running embedding gradient + 2 camera ids
 }
 
-// Weight-gradient tiles (16x16) of the four layers, numbered
-// [dW3 | dW2 | dW1 | dW0]. With NT > 0 wave w accumulates tiles
-// w, w+NW, ..., w+(NT-1)NW in registers over all its row tiles and stores
-// them once at the end; with NT == 0 every row tile read-modify-writes the
-// workgroup partial instead (used when the tiles do not fit NT*NW).
+// Weight-gradient tiles (16x16) of the four layers.
 struct WTiles {
-  int n3, n2, n1, n0, b2, b1, b0, total;
+  int n3, n2, n1, n0;
 };
 
 __host__ __device__ inline WTiles wtiles(const MlpDims& d) {
@@ -762,111 +745,29 @@ __host__ __device__ inline WTiles wtiles(const MlpDims& d) {
   t.n2 = (kU / 16) * (kU / 16);
   t.n1 = (d.EP / 16) * (kU / 16);
   t.n0 = (d.FP / 16) * 2;
-  t.b2 = t.n3;
-  t.b1 = t.b2 + t.n2;
-  t.b0 = t.b1 + t.n1;
-  t.total = t.b0 + t.n0;
   return t;
 }
 
-// Stores a 16x16 tile (D layout) into the (rows x cols) block at `off`.
-__device__ __forceinline__ void store_tile(float* __restrict__ part, int64_t off, int rows,
-                                           int cols, int row0, int col0, const f32x4& acc) {
-  const int lane = lane_id();
-  const int col = col0 + (lane & 15);
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int row = row0 + 4 * (lane >> 4) + e;
-    if (row < rows && col < cols) part[off + (int64_t)row * cols + col] = acc[e];
-  }
-}
-
-// Weight-gradient phase of one layer: for every tile of the layer (n tiles,
-// tcols column tiles per row of tiles) add X^T Y over the TM rows of the row
-// tile. With NT > 0, wave w owns the layer's tiles w, w+NW, ..., held in the
-// register slots [SLOT0, SLOT0 + CNT); otherwise tiles read-modify-write the
-// workgroup partial.
-template <int TM, int NW, bool BF, int NT, int SLOT0, int CNT, bool IN_LDS = false>
-__device__ __forceinline__ void wgrad_phase(f32x4 (&wacc)[NT > 0 ? NT : 1], int wave, int n,
-                                            int tcols, const float* Xm, int ldx,
+// Weight-gradient phase of one layer: every tile of the layer (n tiles, tcols
+// column tiles per row of tiles), X^T Y over the TM rows of the row tile, is
+// added to the workgroup partial.
+template <int TM, int NW, bool BF>
+__device__ __forceinline__ void wgrad_phase(int wave, int n, int tcols, const float* Xm, int ldx,
                                             const float* Ym, int ldy, float* part, int64_t off,
-                                            int rows, int cols, float* Wl = nullptr) {
-  if constexpr (NT > 0 && IN_LDS) {
-    // the wave's tiles in LDS slots [SLOT0, SLOT0 + CNT): each lane keeps its
-    // own 4 accumulator values contiguous (one 16-byte read and write)
-#pragma unroll
-    for (int si = 0; si < CNT; ++si) {
-      const int t = wave + NW * si;
-      if (t < n) {
-        const int ti = t / tcols, tj = t % tcols;
-        f32x4* slot = reinterpret_cast<f32x4*>(Wl) + ((SLOT0 + si) * NW + wave) * 64 + lane_id();
-        f32x4 acc = *slot;
-        mma_wgrad_acc<BF, TM>(Xm, ldx, 16 * ti, Ym, ldy, 16 * tj, acc);
-        *slot = acc;
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else if constexpr (NT > 0) {
-    // two-stage pipeline over the wave's tiles: the LDS reads of tile si + 1
-    // are issued before the products of tile si, so their latency overlaps
-    // the MFMAs (two operand sets live at a time)
-    const int lane = lane_id();
-    float a0[TM / 4], b0[TM / 4], a1[TM / 4], b1[TM / 4];
-    if (wave < n) wgrad_load<BF, TM>(Xm, ldx, 16 * (wave / tcols), Ym, ldy, 16 * (wave % tcols),
-                                     lane, a0, b0);
-#pragma unroll
-    for (int si = 0; si < CNT; ++si) {
-      const int t = wave + NW * si, tn = t + NW;
-      if (si + 1 < CNT && tn < n) {
-        if (si & 1)
-          wgrad_load<BF, TM>(Xm, ldx, 16 * (tn / tcols), Ym, ldy, 16 * (tn % tcols), lane, a0, b0);
-        else
-          wgrad_load<BF, TM>(Xm, ldx, 16 * (tn / tcols), Ym, ldy, 16 * (tn % tcols), lane, a1, b1);
-      }
-      if (t < n) {
-        if (si & 1)
-          wgrad_mma<BF, TM>(a1, b1, wacc[SLOT0 + si]);
-        else
-          wgrad_mma<BF, TM>(a0, b0, wacc[SLOT0 + si]);
-      }
-      // keeps the reads of tile si + 2 from being hoisted above these products
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  } else {
-    for (int t = wave; t < n; t += NW) {
-      const int ti = t / tcols, tj = t % tcols;
-      add_tile(part, off, rows, cols, 16 * ti, 16 * tj,
-               mma_wgrad<BF, TM>(Xm, ldx, 16 * ti, Ym, ldy, 16 * tj));
-    }
+                                            int rows, int cols) {
+  for (int t = wave; t < n; t += NW) {
+    const int ti = t / tcols, tj = t % tcols;
+    add_tile(part, off, rows, cols, 16 * ti, 16 * tj,
+             mma_wgrad<BF, TM>(Xm, ldx, 16 * ti, Ym, ldy, 16 * tj));
   }
 }
 
-// Weight-gradient tiles per wave (kBwdNW waves) of the standard shape: dW2
-// (64 tiles) and dW1 (up to 80, encoded width <= 160) in register slots, the
-// small dW3 (8 tiles) and dW0 (up to 20, features <= 160) in LDS slots, which
-// keeps the kernel's registers within two waves per SIMD.
 constexpr int kBwdNW = 8;
-constexpr int kCnt2 = (64 + kBwdNW - 1) / kBwdNW, kSlot2 = 0;
-constexpr int kCnt1 = (80 + kBwdNW - 1) / kBwdNW, kSlot1 = kSlot2 + kCnt2;
-constexpr int kSlots = kSlot1 + kCnt1;
-constexpr int kCnt3 = (8 + kBwdNW - 1) / kBwdNW, kLSlot3 = 0;
-constexpr int kCnt0 = (20 + kBwdNW - 1) / kBwdNW, kLSlot0 = kLSlot3 + kCnt3;
-constexpr int kLdsSlots = kLSlot0 + kCnt0;
-// BF16 standard shape without an embedding: the rows of the dX strip's B
-// table (g1 rows below fe1 = 138, 9 column tiles) are copied into LDS once per
-// workgroup behind the weight-gradient slots, rows padded to 272 bytes (39 KB;
-// 154 KB in all), so that strip reads LDS instead of L2.
-constexpr int kG1Rows = 144, kG1Ld = 136;
-constexpr size_t kG1LdsBytes = (size_t)kG1Rows * kG1Ld * 2;
-// FP32: the first 80 rows (5 of the 9 column tiles, rows padded to 528 bytes,
-// 41 KB; 153 KB in all); the other column tiles read L2.
-constexpr int kG1RowsF = 80, kG1LdF = 132;
-constexpr size_t kG1LdsBytesF = (size_t)kG1RowsF * kG1LdF * 4;
-// The backward that recomputes each tile's forward: callers without the
-// activations kept by the forward kernel (the training steps' backward,
-// which reads them, is k_mlp_bwd_planes in tfh_mlp_bwd_planes.h).
-template <int TM, int NW, bool BF, int NT, bool STD, bool FILM>
-__global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpPack pk, GradPack gp_arg,
+
+// The backward of any shape, recomputing each tile's forward (the shapes with
+// compile-time dims have k_mlp_bwd_planes, tfh_mlp_bwd_planes.h).
+template <int TM, int NW, bool BF>
+__global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack pk, GradPack gp,
                                                      const float* __restrict__ feats,
                                                      const float* __restrict__ dirs,
                                                      const uint32_t* __restrict__ cams,
@@ -880,9 +781,6 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
   // loaded once per column tile) unless the workgroup has waves to spare
   constexpr int BRTI = NW >= 16 ? 1 : RT;
   constexpr int RG = RT / BRTI;
-  // the specialised shape folds the camera count to 0 without an embedding
-  const MlpDims d = STD ? (FILM ? std_dims<BF>(d_arg.ncam) : std_dims<BF>()) : d_arg;
-  const GradPack gp = STD ? make_pack(std_dims<BF>()) : gp_arg;
   extern __shared__ float smem[];
   float* Fs = smem;                         // TM x ldF
   float* X = Fs + TM * d.ldF;               // TM x ldE   (later dX)
@@ -900,24 +798,16 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
   // and at the end. Tiles with several cameras add per row directly.
   float* Eacc = reinterpret_cast<float*>(Cs + 4 * TM);
   int* Run = reinterpret_cast<int*>(Eacc + kU);  // [0] tile camera or -1, [1] camera of Eacc or -1
-  // LDS slots of the dW3 / dW0 tiles (NT > 0): after the FiLM state
-  float* Wl = reinterpret_cast<float*>(Cs + 4 * TM) + (d.ncam > 0 ? kU + 4 : 0);
   const Operands<BF> op{d, w, pk};
 
-  // masked to the block's waves (NW, a power of two): lets the compiler fold
-  // each weight-gradient slot's tile offsets into constants
-  static_assert((NW & (NW - 1)) == 0, "wave count a power of two");
-  const int wave = (threadIdx.x >> 6) & (NW - 1);
+  const int wave = threadIdx.x >> 6;
   const int lane = lane_id();
   float* part = partials + (int64_t)blockIdx.x * gp.total;
-  if (FILM && d.ncam > 0) {
+  if (d.ncam > 0) {
     for (int c = threadIdx.x; c < kU; c += blockDim.x) Eacc[c] = 0.0f;
     if (threadIdx.x == 0) Run[1] = -1;
   }
   const WTiles wt = wtiles(d);
-  f32x4 wacc[NT > 0 ? NT : 1];
-#pragma unroll
-  for (int i = 0; i < (NT > 0 ? NT : 1); ++i) wacc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   // Bias gradients, summed in registers: db1 / db2 per lane over the rows
   // 4(lane/16)+e of the row groups of column 16*(wave/RG) + lane%16 (the
   // strip phases that produce dZ1 and dZ2 give wave w the same item on every
@@ -926,29 +816,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
   static_assert((kU / 16) * (RT / (NW >= 16 ? 1 : RT)) == NW,
                 "one strip item per wave: the bias sums stay with their column");
   float db1 = 0.f, db2 = 0.f, db3 = 0.f;
-  if (NT == 0)
-    for (int64_t e = threadIdx.x; e < gp.total; e += blockDim.x) part[e] = 0.0f;
-  else
-    for (int e = threadIdx.x; e < kLdsSlots * NW * 256; e += blockDim.x) Wl[e] = 0.0f;
-  constexpr bool kG1Lds = BF && STD && !FILM && NT > 0 && NW == 8;
-  constexpr bool kG1LdsF = !BF && STD && !FILM && NT > 0 && NW == 8;
-  __bf16* G1s = reinterpret_cast<__bf16*>(Wl + kLdsSlots * NW * 256);
-  float* G1f = Wl + kLdsSlots * NW * 256;
-  if constexpr (kG1Lds) {
-    // the tile loop starts with a barrier
-    for (int e = threadIdx.x; e < kG1Rows * (kU / 8); e += blockDim.x) {
-      const int j = e / (kU / 8), c8 = e - j * (kU / 8);
-      *reinterpret_cast<uint4*>(G1s + j * kG1Ld + 8 * c8) =
-          *reinterpret_cast<const uint4*>(pk.g1 + j * kU + 8 * c8);
-    }
-  }
-  if constexpr (kG1LdsF) {
-    for (int e = threadIdx.x; e < kG1RowsF * (kU / 4); e += blockDim.x) {
-      const int j = e / (kU / 4), c4 = e - j * (kU / 4);
-      *reinterpret_cast<float4*>(G1f + j * kG1LdF + 4 * c4) =
-          *reinterpret_cast<const float4*>(pk.fg1 + j * kU + 4 * c4);
-    }
-  }
+  for (int64_t e = threadIdx.x; e < gp.total; e += blockDim.x) part[e] = 0.0f;
 
   const int64_t ntiles = (M + TM - 1) / TM;
   for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
@@ -956,7 +824,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
     __syncthreads();
     load_tile<TM>(d, feats, dirs, cams, row0, M, rpr, Fs, Ds, Cs);
     __syncthreads();
-    if (FILM && d.ncam > 0 && wave == 0) {
+    if (d.ncam > 0 && wave == 0) {
       // read before the next use: forward_hidden synchronises the workgroup
       const int nvalid = (int)min((int64_t)TM, M - row0);
       const int c0 = Cs[0];
@@ -988,8 +856,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
     }
     __syncthreads();
     // dW3 (U x 3) += H2^T dZ3 ; db3
-    wgrad_phase<TM, NW, BF, NT, kLSlot3, kCnt3, true>(wacc, wave, wt.n3, 1, H2, d.ldU, Z3, d.ld3,
-                                                      part, gp.w3, kU, 3, Wl);
+    wgrad_phase<TM, NW, BF>(wave, wt.n3, 1, H2, d.ldU, Z3, d.ld3, part, gp.w3, kU, 3);
     if (threadIdx.x < 3 * TM) db3 += Z3[(threadIdx.x / 3) * d.ld3 + threadIdx.x % 3];
     __syncthreads();
     // Strip phases below run one work item per (column tile, row group).
@@ -1000,7 +867,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
       zero_acc(acc);
       mma_strip<BRTI, 32>(Z3 + r0 * d.ld3, d.ld3, op.k3(), op.g3(), 16 * ct, acc);
       const int col = 16 * ct + (lane & 15);
-      if constexpr (FILM) {
+      {
         const bool film = d.ncam > 0 && 16 * ct >= kU / 2;  // wave-uniform
         const int tcam = d.ncam > 0 ? Run[0] : -1;
         // the tile camera's scale of this column, read once
@@ -1039,22 +906,11 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
             atomicAdd(Eacc + col, sg);
           }
         }
-      } else {
-#pragma unroll
-        for (int q = 0; q < 4 * BRTI; ++q) {
-          const int rt = q / 4, e = q % 4;
-          const int row = r0 + 16 * rt + 4 * (lane >> 4) + e;
-          const float hp = H2p[row * d.ldU + col];
-          const float dz = hp > 0.0f ? acc[rt][e] : 0.0f;
-          H2[row * d.ldU + col] = dz;
-          db2 += dz;
-        }
       }
     }
     __syncthreads();
     // dW2 (U x U) += H1^T dZ2 ; db2
-    wgrad_phase<TM, NW, BF, NT, kSlot2, kCnt2>(wacc, wave, wt.n2, kU / 16, H1, d.ldU, H2,
-                                               d.ldU, part, gp.w2, kU, kU);
+    wgrad_phase<TM, NW, BF>(wave, wt.n2, kU / 16, H1, d.ldU, H2, d.ldU, part, gp.w2, kU, kU);
     __syncthreads();
     // dH1 = dZ2 @ W2^T ; dZ1 = dH1 * (h1 > 0) written over H1 (dW2 is done)
     for (int it = wave; it < (kU / 16) * RG; it += NW) {
@@ -1075,8 +931,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
     }
     __syncthreads();
     // dW1 (E x U) += X^T dZ1 ; db1
-    wgrad_phase<TM, NW, BF, NT, kSlot1, kCnt1>(wacc, wave, wt.n1, kU / 16, X, d.ldE, H1,
-                                               d.ldU, part, gp.w1, d.E, kU);
+    wgrad_phase<TM, NW, BF>(wave, wt.n1, kU / 16, X, d.ldE, H1, d.ldU, part, gp.w1, d.E, kU);
     __syncthreads();
     // dX = dZ1 @ W1^T for the columns that feed h0: [0, S) and the FE(h0)
     // block, i.e. the column tiles below fe1 (the 3 direction columns between
@@ -1088,17 +943,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
         const int c0 = 16 * (it / RT), r0 = 16 * (it % RT);
         f32x4 acc[1];
         zero_acc(acc);
-        if constexpr (kG1Lds) {
-          mma_strip<1, kU>(H1 + r0 * d.ldU, d.ldU, kU, LdsB{G1s, kG1Ld}, c0, acc);
-        } else if constexpr (kG1LdsF) {
-          // one code path over a generic pointer: LDS rows or global rows
-          // (two strip variants in a branch cost the kernel 7 more spills)
-          const bool lds = c0 < kG1RowsF;  // wave-uniform
-          const FlatB32 b{lds ? static_cast<const float*>(G1f) : pk.fg1, lds ? kG1LdF : kU};
-          mma_strip<1, kU>(H1 + r0 * d.ldU, d.ldU, kU, b, c0, acc);
-        } else {
-          mma_strip<1, kU>(H1 + r0 * d.ldU, d.ldU, kU, op.g1(), c0, acc);
-        }
+        mma_strip<1, kU>(H1 + r0 * d.ldU, d.ldU, kU, op.g1(), c0, acc);
         const int col = c0 + (lane & 15);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -1131,8 +976,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
     }
     __syncthreads();
     // dW0 (F x S) += F^T dH0
-    wgrad_phase<TM, NW, BF, NT, kLSlot0, kCnt0, true>(wacc, wave, wt.n0, 2, Fs, d.ldF, H0, d.ldS,
-                                                      part, gp.w0, d.F, d.S, Wl);
+    wgrad_phase<TM, NW, BF>(wave, wt.n0, 2, Fs, d.ldF, H0, d.ldS, part, gp.w0, d.F, d.S);
     // dF = dH0 @ W0^T -> global
     if (gfeat) {
       for (int it = wave; it < (d.FP / 16) * RT; it += NW) {
@@ -1150,7 +994,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
       }
     }
   }
-  if (FILM && d.ncam > 0) {
+  if (d.ncam > 0) {
     __syncthreads();
     const int rc = Run[1];
     if (rc >= 0)
@@ -1176,48 +1020,15 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d_arg, MlpW w, MlpP
   if (threadIdx.x < 3 * TM) atomicAdd(bsum + 2 * kU + threadIdx.x % 3, db3);
   __syncthreads();
   // the workgroup's gradient sums -> its partial
-  if constexpr (NT > 0) {
-#pragma unroll
-    for (int si = 0; si < kSlots; ++si) {
-      if (si < kSlot1) {
-        const int t = wave + NW * (si - kSlot2);
-        if (t < wt.n2)
-          store_tile(part, gp.w2, kU, kU, 16 * (t / (kU / 16)), 16 * (t % (kU / 16)), wacc[si]);
-      } else {
-        const int t = wave + NW * (si - kSlot1);
-        if (t < wt.n1)
-          store_tile(part, gp.w1, d.E, kU, 16 * (t / (kU / 16)), 16 * (t % (kU / 16)), wacc[si]);
-      }
-    }
-    // the LDS slots are the wave's own: no barrier needed
-    const f32x4* wl = reinterpret_cast<const f32x4*>(Wl);
-    for (int si = 0; si < kLdsSlots; ++si) {
-      const f32x4 v = wl[(si * NW + wave) * 64 + lane];
-      if (si < kLSlot0) {
-        const int t = wave + NW * (si - kLSlot3);
-        if (t < wt.n3) store_tile(part, gp.w3, kU, 3, 16 * t, 0, v);
-      } else {
-        const int t = wave + NW * (si - kLSlot0);
-        if (t < wt.n0) store_tile(part, gp.w0, d.F, d.S, 16 * (t / 2), 16 * (t % 2), v);
-      }
-    }
-    if (threadIdx.x < kU) {
-      part[gp.b1 + threadIdx.x] = bsum[threadIdx.x];
-      part[gp.b2 + threadIdx.x] = bsum[kU + threadIdx.x];
-    }
-    if (threadIdx.x < 3) part[gp.b3 + threadIdx.x] = bsum[2 * kU + threadIdx.x];
-  } else {
-    if (threadIdx.x < kU) {
-      part[gp.b1 + threadIdx.x] += bsum[threadIdx.x];
-      part[gp.b2 + threadIdx.x] += bsum[kU + threadIdx.x];
-    }
-    if (threadIdx.x < 3) part[gp.b3 + threadIdx.x] += bsum[2 * kU + threadIdx.x];
+  if (threadIdx.x < kU) {
+    part[gp.b1 + threadIdx.x] += bsum[threadIdx.x];
+    part[gp.b2 + threadIdx.x] += bsum[kU + threadIdx.x];
   }
+  if (threadIdx.x < 3) part[gp.b3 + threadIdx.x] += bsum[2 * kU + threadIdx.x];
 }
 
 constexpr int kFwdTM = 32, kFwdNW = 8;
 constexpr int kBwdTM = 32;
-constexpr int kBwdNT = kSlots;  // register-resident weight-gradient tiles per wave
 
 // Dynamic LDS above 64 KB needs the per-kernel opt-in.
 template <class K>
@@ -1229,10 +1040,29 @@ inline void allow_lds(K kernel, size_t bytes) {
   }
 }
 
-// k_mlp_bwd_planes (tfh_mlp_bwd_planes.h): operand tables, launch.
+// k_mlp_bwd_planes (tfh_mlp_bwd_planes.h): the shapes it is built for, the
+// operand tables, the launches.
+enum class BwdKind { kNone, kStd, kDef };
+inline BwdKind bwd_kind(const MlpDims& d) {
+  if (d.S != 27 || d.nf != d.nv) return BwdKind::kNone;
+  if (d.F == 144 && d.nf == 2) return BwdKind::kStd;
+  if (d.F == 72 && d.nf == 6) return BwdKind::kDef;
+  return BwdKind::kNone;
+}
+// The type of the kept activations. BF16 changes no result of the BF16 MLP's
+// backward without an embedding; with one, relu(z2) also enters the
+// embedding's gradient and the layer-3 input, and only the fused steps of the
+// 48-channel shape keep it in BF16.
+inline bool kept_bf16(const MlpDims& d, bool bf, bool fused) {
+  return bf && (d.ncam == 0 || (fused && bwd_kind(d) == BwdKind::kStd));
+}
+constexpr int kBwdRowsFp32 = 32, kBwdRowsBf16 = 64;  // rows of a tile
+inline int64_t bwd_planes_blocks(bool bf, int64_t M, int64_t cus) {
+  return std::min<int64_t>(ceil_div(M, bf ? kBwdRowsBf16 : kBwdRowsFp32), cus);
+}
 struct BwdPlanesArgs {
-  void* tables;  // bwd_planes_table_bytes()
-  unsigned nblk;
+  const void* tables;
+  int64_t max_blocks;
   const float *feats, *dirs;
   const uint32_t* cams;
   const float* grgb;
@@ -1243,21 +1073,10 @@ struct BwdPlanesArgs {
   float* gembed;
   int ncam;
 };
-size_t bwd_planes_table_bytes(bool bf);
-int bwd_planes_tile_rows(bool bf);
-int32_t launch_bwd_planes(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
-
-// Backward launches of the standard shape without (tfh_mlp_bwd_std.hip) and
-// with (tfh_mlp_film.hip) a camera embedding.
-void launch_mlp_bwd_std(bool bf, unsigned nblk, size_t lds, hipStream_t st, const MlpDims& d,
-                        const MlpW& w, const MlpPack& pk, const GradPack& gp,
-                        const float* feats, const float* dirs, const uint32_t* cams,
-                        const float* grgb, int64_t M, int64_t rpr, float* gfeat,
-                        float* partials, float* gembed);
-void launch_mlp_bwd_std_film(bool bf, unsigned nblk, size_t lds, hipStream_t st,
-                             const MlpDims& d, const MlpW& w, const MlpPack& pk,
-                             const GradPack& gp, const float* feats, const float* dirs,
-                             const uint32_t* cams, const float* grgb, int64_t M, int64_t rpr,
-                             float* gfeat, float* partials, float* gembed);
+size_t bwd_planes_table_bytes(BwdKind kind, bool bf);
+int32_t pack_bwd_planes(BwdKind kind, bool bf, const MlpW& w, void* tables, hipStream_t st);
+int32_t launch_bwd_planes_train(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
+int32_t launch_bwd_planes_std(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
+int32_t launch_bwd_planes_def(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
 
 }  // namespace tfh
