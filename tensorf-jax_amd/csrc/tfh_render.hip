@@ -757,26 +757,31 @@ static int32_t render_backward(const tfh_vm* density, const tfh_vm* appearance,
   if (fuse) {
     ProfScope ps("factor_scatter", st);
     if (ws.alcopy) TFH_TRY(zero_copies(ws.alcopy, ws.anlc * aln, st));
-    const FieldOut fa{*appearance, agrad->plane, ws.alcopy ? ws.alcopy : agrad->line,
-                      ws.alcopy ? ws.anlc : 1};
-    const FieldOut fd{*density, dgrad->plane, ws.dlcopy ? ws.dlcopy : dgrad->line,
-                      ws.dlcopy ? ws.dnlc : 1};
+    const int g = (int)appearance->grid_dim;
+    const ScalarGrad dsrcg{ws.ds};
+    TFH_TRY((launch_plane_walk<16>(dsrc, g, M, ws.sort,
+                                   WalkField<RowGrad>{*appearance, gsrc, agrad->plane, 1},
+                                   WalkField<ScalarGrad>{*density, dsrcg, dgrad->plane, 1},
+                                   "factor_scatter_planes", st)));
     // the line pass in line-cell order (a second sort; adds straight into
     // the line gradients) for rays with fewer samples than the grid has
-    // cells, whose consecutive samples rarely share a line texel (proposal
-    // rays: 64 samples, 20.7 M memory-side transactions in ray order, line
-    // pass 1.07 -> 0.69 ms + 0.08 ms sort); dense rays merge well in ray order
-    // and keep it (512 samples: 1.07 ms against 1.15 + 0.11 sorted)
-    const bool sorted_lines = N < (int)appearance->grid_dim;
-    // with the scene contraction the far samples of a ray crowd into few
-    // cells, and summing a ray's runs per line cell in registers beats the
-    // four-sample merge (contracted fisheye step: lines 4.74 -> 3.78 ms); on
-    // bounded scenes the runs are short and the merge is faster (uniform-512:
-    // 1.08 against 1.19 ms)
-    const bool ray_walk = cfg->scene_contraction != 0;
-    TFH_TRY(scatter_two_fields(dsrc, M, ws.sort, gsrc, fa, ScalarGrad{ws.ds}, fd, st,
-                               sorted_lines, agrad->line, dgrad->line, ray_walk));
-    if (sorted_lines) return TFH_OK;
+    // cells, whose consecutive samples rarely share a line texel; else in ray
+    // order into the copies
+    const bool sorted_lines = N < g;
+    if (sorted_lines) {
+      TFH_TRY(sort_lines(g, dsrc, M, ws.sort, st));
+      return launch_line_walk<16>(true, dsrc, g, M, ws.sort,
+                                  WalkField<RowGrad>{*appearance, gsrc, agrad->line, 1},
+                                  WalkField<ScalarGrad>{*density, dsrcg, dgrad->line, 1},
+                                  "factor_scatter_lines", st);
+    }
+    TFH_TRY((launch_line_walk<16>(
+        false, dsrc, g, M, ws.sort,
+        WalkField<RowGrad>{*appearance, gsrc, ws.alcopy ? ws.alcopy : agrad->line,
+                           ws.alcopy ? ws.anlc : 1},
+        WalkField<ScalarGrad>{*density, dsrcg, ws.dlcopy ? ws.dlcopy : dgrad->line,
+                              ws.dlcopy ? ws.dnlc : 1},
+        "factor_scatter_lines", st)));
     if (ws.dlcopy) TFH_TRY(sum_copies(ws.dlcopy, ws.dnlc, dln, dgrad->line, st));
     if (ws.alcopy) TFH_TRY(sum_copies(ws.alcopy, ws.anlc, aln, agrad->line, st));
     return TFH_OK;

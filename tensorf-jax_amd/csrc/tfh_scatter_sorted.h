@@ -286,14 +286,431 @@ __global__ void __launch_bounds__(256) k_chunk_sort(Src src, int g, int tiles,
     if (cl[j] >= 0) order[base + hist[cl[j]] + rk[j]] = pk[j];
 }
 
+// ---- walks over pairs -----------------------------------------------------------
+// A group of LPS lanes walks `per` consecutive pairs and sums the gradients of
+// the texels of the current cell in registers; a texel is added to memory
+// when the walk leaves it. A walk that steps to a neighbouring cell keeps the
+// texels the two share. Long walks save adds, short ones fill the chip: 64
+// pairs where that leaves kWalkGroups groups, fewer (a power of two, at
+// least 8) where it does not. A training step of 256 rays with 24 of 160
+// samples shaded (16 + 48 channels, G = 128) takes 513 us with 64 pairs
+// everywhere and 264 us with this rule; one of 1024 rays with all shaded 572
+// and 505. With twice as many groups asked for, the latter takes 555 us
+// (more adds), with half as many 509.
+constexpr int kPairsPerGroup = 64;
+constexpr int64_t kWalkGroups = 32768;
+inline int walk_pairs(int64_t pairs) {
+  int per = 8;
+  while (per < kPairsPerGroup && pairs > per * kWalkGroups) per *= 2;
+  return per;
+}
+
+// The taps of one pair, computed once by the lane that loads it and handed to
+// its group lane by lane (every lane computing them for every pair is what
+// bounded these passes: 40 of 60 vector instructions a pair).
+struct PairTaps {
+  uint32_t pk;      // row * 4 + mode
+  int kl, kp;       // line0 * 2 + (line1 - line0); p00 * 4 + (row step) * 2 + (column step)
+  float wv, wa, wb; // upper weights (the lower one is 1 - w)
+};
+
+__device__ __forceinline__ PairTaps make_pair_taps(uint32_t pk, float x, float y, float z, int g) {
+  const int m = (int)(pk & 3u);
+  Tap tv, ta, tb;
+  one_mode_taps(x, y, z, g, m, tv, ta, tb);
+  PairTaps t;
+  t.pk = pk;
+  t.kl = (m * g + tv.i0) * 2 + (tv.i1 - tv.i0);
+  t.kp = ((m * g + ta.i0) * g + tb.i0) * 4 + (ta.i1 - ta.i0) * 2 + (tb.i1 - tb.i0);
+  t.wv = tv.w1;
+  t.wa = ta.w1;
+  t.wb = tb.w1;
+  return t;
+}
+
+__device__ __forceinline__ PairTaps shfl_pair(const PairTaps& t, int from) {
+  PairTaps r;
+  r.pk = __shfl(t.pk, from, 64);
+  r.kl = __shfl(t.kl, from, 64);
+  r.kp = __shfl(t.kp, from, 64);
+  r.wv = __shfl(t.wv, from, 64);
+  r.wa = __shfl(t.wa, from, 64);
+  r.wb = __shfl(t.wb, from, 64);
+  return r;
+}
+
+// Channel 16q + l of a 16-lane group whose lane j holds channels
+// 4j .. 4j+3 (v): the sums go back to one channel per lane before they are
+// added, so that each atomic instruction of a group covers 64 contiguous
+// bytes (one memory-side transaction); with the quads the lanes' adds were
+// 16 bytes apart, three transactions per instruction (the plane pass took
+// 1.54 ms instead of 0.69). All 16 lanes of the group must call it (gl0: the
+// group's first lane in the wave).
+__device__ __forceinline__ float quad_to_lane(const float (&v)[4], int q, int l, int gl0) {
+  const int from = gl0 + 4 * q + (l >> 2);
+  const float t0 = __shfl(v[0], from, 64), t1 = __shfl(v[1], from, 64);
+  const float t2 = __shfl(v[2], from, 64), t3 = __shfl(v[3], from, 64);
+  const int u = l & 3;
+  return u == 0 ? t0 : (u == 1 ? t1 : (u == 2 ? t2 : t3));
+}
+
+// One field of a walk: its factors, the upstream gradients (RowGrad or
+// ScalarGrad) and where its sums go.
+template <class GS>
+struct WalkField {
+  tfh_vm vm;
+  GS g;
+  float* out;  // the plane gradient, or nlc copies of the line gradient
+  int nlc;
+};
+struct NoField {};
+
+// A field of 16 < C <= 64 channels, C % 4 == 0, 16-byte aligned: lane l of 16
+// owns channels 4l .. 4l+3.
+template <class GS, int NT>
+struct QuadLanes {
+  const WalkField<GS>& f;
+  float* out;
+  int C, l, gl0;
+  bool on;
+  float4 acc[NT];
+  __device__ __forceinline__ QuadLanes(const WalkField<GS>& f_, float* out_, int l_, int gl0_)
+      : f(f_), out(out_), C((int)f_.vm.channels), l(l_), gl0(gl0_), on(4 * l_ < C) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __device__ __forceinline__ float4 load(const float* base, int texel) const {
+    return on ? *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) +
+                                                 (uint32_t)((texel * C + 4 * l) * 4))
+              : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __device__ __forceinline__ float4 grad(uint32_t pk) const {
+    return on ? f.g.at4((int64_t)(pk >> 2), (int)(pk & 3u), 4 * l)
+              : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __device__ __forceinline__ void add(int t, float w, const float4& v) {
+    acc[t].x += w * v.x;
+    acc[t].y += w * v.y;
+    acc[t].z += w * v.z;
+    acc[t].w += w * v.w;
+  }
+  __device__ __forceinline__ void flush(int t, int texel) {
+    const float v[4] = {acc[t].x, acc[t].y, acc[t].z, acc[t].w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (16 * q < C) {  // group-uniform
+        const float val = quad_to_lane(v, q, l, gl0);
+        const int c = 16 * q + l;
+        if (c < C && val != 0.0f) unsafeAtomicAdd(out + (size_t)texel * C + c, val);
+      }
+    }
+    acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  __device__ __forceinline__ void move(int to, int from) {
+    acc[to] = acc[from];
+    acc[from] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+};
+
+// A field of at most LPS channels: lane l owns channel l.
+template <class GS, int NT>
+struct LaneLanes {
+  const WalkField<GS>& f;
+  float* out;
+  int C, l;
+  bool on;
+  float acc[NT];
+  __device__ __forceinline__ LaneLanes(const WalkField<GS>& f_, float* out_, int l_, int)
+      : f(f_), out(out_), C((int)f_.vm.channels), l(l_), on(l_ < C) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[t] = 0.0f;
+  }
+  __device__ __forceinline__ float load(const float* base, int texel) const {
+    return on ? *reinterpret_cast<const float*>(reinterpret_cast<const char*>(base) +
+                                                (uint32_t)((texel * C + l) * 4))
+              : 0.0f;
+  }
+  __device__ __forceinline__ float grad(uint32_t pk) const {
+    return on ? f.g.at((int64_t)(pk >> 2), (int)(pk & 3u), l) : 0.0f;
+  }
+  __device__ __forceinline__ void add(int t, float w, float v) { acc[t] += w * v; }
+  __device__ __forceinline__ void flush(int t, int texel) {
+    if (on && acc[t] != 0.0f) unsafeAtomicAdd(out + (size_t)texel * C + l, acc[t]);
+    acc[t] = 0.0f;
+  }
+  __device__ __forceinline__ void move(int to, int from) {
+    acc[to] = acc[from];
+    acc[from] = 0.0f;
+  }
+};
+
+struct NoLanes {
+  template <class... T>
+  __device__ __forceinline__ explicit NoLanes(T&&...) {}
+  __device__ __forceinline__ void flush(int, int) {}
+  __device__ __forceinline__ void move(int, int) {}
+};
+
+__device__ __forceinline__ float4 mul4(const float4& a, const float4& b) {
+  return make_float4(a.x * b.x, a.y * b.y, a.z * b.z, a.w * b.w);
+}
+__device__ __forceinline__ float mul4(float a, float b) { return a * b; }
+__device__ __forceinline__ float4 mix2(float w0, const float4& a, float w1, const float4& b) {
+  return make_float4(w0 * a.x + w1 * b.x, w0 * a.y + w1 * b.y, w0 * a.z + w1 * b.z,
+                     w0 * a.w + w1 * b.w);
+}
+__device__ __forceinline__ float mix2(float w0, float a, float w1, float b) {
+  return w0 * a + w1 * b;
+}
+__device__ __forceinline__ float4 mix4(const float (&w)[4], const float4& a, const float4& b,
+                                       const float4& c, const float4& d) {
+  return make_float4(((w[0] * a.x + w[1] * b.x) + w[2] * c.x) + w[3] * d.x,
+                     ((w[0] * a.y + w[1] * b.y) + w[2] * c.y) + w[3] * d.y,
+                     ((w[0] * a.z + w[1] * b.z) + w[2] * c.z) + w[3] * d.z,
+                     ((w[0] * a.w + w[1] * b.w) + w[2] * c.w) + w[3] * d.w);
+}
+__device__ __forceinline__ float mix4(const float (&w)[4], float a, float b, float c, float d) {
+  return ((w[0] * a + w[1] * b) + w[2] * c) + w[3] * d;
+}
+
+template <class F>
+struct IsNone {
+  static constexpr bool v = false;
+};
+template <>
+struct IsNone<NoField> {
+  static constexpr bool v = true;
+};
+// The lane view of a field: quads for FA, one channel per lane for FD.
+template <class F, int NT>
+struct QuadOf;
+template <class GS, int NT>
+struct QuadOf<WalkField<GS>, NT> {
+  using T = QuadLanes<GS, NT>;
+};
+template <int NT>
+struct QuadOf<NoField, NT> {
+  using T = NoLanes;
+};
+template <class F, int NT>
+struct LaneOf;
+template <class GS, int NT>
+struct LaneOf<WalkField<GS>, NT> {
+  using T = LaneLanes<GS, NT>;
+};
+template <int NT>
+struct LaneOf<NoField, NT> {
+  using T = NoLanes;
+};
+template <class GS>
+__device__ __forceinline__ float* copy_of(const WalkField<GS>& f, int g) {
+  return f.out + (int64_t)(blockIdx.x % f.nlc) * 3 * g * f.vm.channels;
+}
+__device__ __forceinline__ float* copy_of(const NoField&, int) { return nullptr; }
+template <class GS>
+__device__ __forceinline__ float* whole_of(const WalkField<GS>& f) { return f.out; }
+__device__ __forceinline__ float* whole_of(const NoField&) { return nullptr; }
+
+// Plane gradients from pairs sorted by plane cell: dL/dplane[m][texel][c] +=
+// w_texel * line_m(c) * gout[row][m*C + c], of field FA (quad lanes, LPS = 16)
+// and field FD (a channel per lane); either may be NoField. Both fields' line
+// taps and upstream gradients are requested before the flush: one memory round
+// trip per pair.
+template <class Src, class FA, class FD, int LPS>
+__global__ void __launch_bounds__(256) k_plane_walk(Src src, int g, int64_t pairs, int per,
+                                                    const uint32_t* __restrict__ order, FA fa,
+                                                    FD fd) {
+  constexpr bool A = !IsNone<FA>::v, D = !IsNone<FD>::v;
+  static_assert(!A || LPS == 16, "quad lanes are 16 to a pair");
+  const int l = threadIdx.x % LPS;
+  const int gl0 = (threadIdx.x - l) & 63;
+  const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * per;
+  if (first >= pairs) return;  // whole group: no cross-group exchange below
+  const int64_t last = min(first + per, pairs);
+  typename QuadOf<FA, 4>::T la(fa, whole_of(fa), l, gl0);
+  typename LaneOf<FD, 4>::T ld(fd, whole_of(fd), l, gl0);
+  int cur = -1;
+  int tex[4] = {0, 0, 0, 0};
+  auto flush = [&](int t) __attribute__((always_inline)) {
+    la.flush(t, tex[t]);
+    ld.flush(t, tex[t]);
+  };
+  for (int64_t b0 = first; b0 < last; b0 += LPS) {
+    const int64_t e = b0 + l;
+    PairTaps mine{};
+    if (e < last) {
+      const uint32_t pk = order[e];
+      float x, y, z;
+      src.get((int64_t)(pk >> 2), x, y, z);
+      mine = make_pair_taps(pk, x, y, z, g);
+    }
+    const int nb = (int)min((int64_t)LPS, last - b0);
+    for (int j = 0; j < nb; ++j) {
+      const PairTaps p = shfl_pair(mine, gl0 + j);
+      const int i0 = p.kl >> 1, i1 = i0 + (p.kl & 1);
+      const float w0 = 1.0f - p.wv;
+      float4 a0, a1, ag;
+      float d0, d1, dg;
+      if constexpr (A) {
+        a0 = la.load(fa.vm.line, i0);
+        a1 = la.load(fa.vm.line, i1);
+        ag = la.grad(p.pk);
+      }
+      if constexpr (D) {
+        d0 = ld.load(fd.vm.line, i0);
+        d1 = ld.load(fd.vm.line, i1);
+        dg = ld.grad(p.pk);
+      }
+      if (p.kp != cur) {
+        int nt[4];
+        nt[0] = p.kp >> 2;
+        nt[1] = nt[0] + (p.kp & 1);
+        nt[2] = nt[0] + ((p.kp >> 1) & 1) * g;
+        nt[3] = nt[2] + (p.kp & 1);
+        if (cur >= 0) {
+          flush(0);
+          flush(2);
+          if (nt[0] == tex[1] && nt[2] == tex[3]) {  // the next cell of the row
+            la.move(0, 1);
+            la.move(2, 3);
+            ld.move(0, 1);
+            ld.move(2, 3);
+          } else {
+            flush(1);
+            flush(3);
+          }
+        }
+        cur = p.kp;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) tex[t] = nt[t];
+      }
+      const float wa0 = 1.0f - p.wa, wb0 = 1.0f - p.wb;
+      const float w[4] = {wa0 * wb0, wa0 * p.wb, p.wa * wb0, p.wa * p.wb};
+      if constexpr (A) {
+        const float4 v = mul4(ag, mix2(w0, a0, p.wv, a1));
+#pragma unroll
+        for (int t = 0; t < 4; ++t) la.add(t, w[t], v);
+      }
+      if constexpr (D) {
+        const float v = dg * mix2(w0, d0, p.wv, d1);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) ld.add(t, w[t], v);
+      }
+    }
+  }
+  if (cur >= 0) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t) flush(t);
+  }
+}
+
+// Line gradients: dL/dline[m][v][c] += w_v * plane_m(c) * gout[row][m*C + c],
+// over pairs sorted by line cell (order), or with RAY in ray order, mode by
+// mode (pair e = (row e % M, mode e / M)): a run is then a stretch of a ray
+// inside one line cell, and the adds go to copies of the line gradient (block
+// b into copy b % nlc), since every ray crosses the same few line texels.
+template <class Src, class FA, class FD, int LPS, bool RAY>
+__global__ void __launch_bounds__(256) k_line_walk(Src src, int g, int64_t pairs, int per, int64_t M,
+                                                   const uint32_t* __restrict__ order, FA fa,
+                                                   FD fd) {
+  constexpr bool A = !IsNone<FA>::v, D = !IsNone<FD>::v;
+  static_assert(!A || LPS == 16, "quad lanes are 16 to a pair");
+  const int l = threadIdx.x % LPS;
+  const int gl0 = (threadIdx.x - l) & 63;
+  const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * per;
+  if (first >= pairs) return;  // whole group: no cross-group exchange below
+  const int64_t last = min(first + per, pairs);
+  typename QuadOf<FA, 2>::T la(fa, copy_of(fa, g), l, gl0);
+  typename LaneOf<FD, 2>::T ld(fd, copy_of(fd, g), l, gl0);
+  int cur = -1, t0 = 0, t1 = 0;
+  for (int64_t b0 = first; b0 < last; b0 += LPS) {
+    const int64_t e = b0 + l;
+    PairTaps mine{};
+    if (e < last) {
+      uint32_t pk;
+      if constexpr (RAY) {
+        const int m = e >= 2 * M ? 2 : (e >= M ? 1 : 0);
+        pk = (uint32_t)(e - m * M) << 2 | (uint32_t)m;
+      } else {
+        pk = order[e];
+      }
+      float x, y, z;
+      src.get((int64_t)(pk >> 2), x, y, z);
+      mine = make_pair_taps(pk, x, y, z, g);
+    }
+    const int nb = (int)min((int64_t)LPS, last - b0);
+    for (int j = 0; j < nb; ++j) {
+      const PairTaps p = shfl_pair(mine, gl0 + j);
+      const int p00 = p.kp >> 2, p01 = p00 + (p.kp & 1);
+      const int p10 = p00 + ((p.kp >> 1) & 1) * g, p11 = p10 + (p.kp & 1);
+      float4 a[4], ag;
+      float d[4], dg;
+      if constexpr (A) {
+        a[0] = la.load(fa.vm.plane, p00);
+        a[1] = la.load(fa.vm.plane, p01);
+        a[2] = la.load(fa.vm.plane, p10);
+        a[3] = la.load(fa.vm.plane, p11);
+        ag = la.grad(p.pk);
+      }
+      if constexpr (D) {
+        d[0] = ld.load(fd.vm.plane, p00);
+        d[1] = ld.load(fd.vm.plane, p01);
+        d[2] = ld.load(fd.vm.plane, p10);
+        d[3] = ld.load(fd.vm.plane, p11);
+        dg = ld.grad(p.pk);
+      }
+      if (p.kl != cur) {
+        const int n0 = p.kl >> 1, n1 = n0 + (p.kl & 1);
+        if (cur >= 0) {
+          if (n1 == t0 && n0 != t1) {  // one texel down
+            la.flush(1, t1);
+            ld.flush(1, t1);
+            la.move(1, 0);
+            ld.move(1, 0);
+          } else {
+            la.flush(0, t0);
+            ld.flush(0, t0);
+            if (n0 == t1) {  // one texel up
+              la.move(0, 1);
+              ld.move(0, 1);
+            } else {
+              la.flush(1, t1);
+              ld.flush(1, t1);
+            }
+          }
+        }
+        cur = p.kl;
+        t0 = n0;
+        t1 = n1;
+      }
+      const float wa0 = 1.0f - p.wa, wb0 = 1.0f - p.wb, w0 = 1.0f - p.wv;
+      const float w[4] = {wa0 * wb0, wa0 * p.wb, p.wa * wb0, p.wa * p.wb};
+      if constexpr (A) {
+        const float4 v = mul4(ag, mix4(w, a[0], a[1], a[2], a[3]));
+        la.add(0, w0, v);
+        la.add(1, p.wv, v);
+      }
+      if constexpr (D) {
+        const float v = dg * mix4(w, d[0], d[1], d[2], d[3]);
+        ld.add(0, w0, v);
+        ld.add(1, p.wv, v);
+      }
+    }
+  }
+  if (cur >= 0) {
+    la.flush(0, t0);
+    la.flush(1, t1);
+    ld.flush(0, t0);
+    ld.flush(1, t1);
+  }
+}
+
 // Plane gradients from the sorted pairs: dL/dplane[m][texel][c] +=
 // w_texel * line_m(c) * gout[row][m*C + c]. Each 16-lane group owns kPairsPerGroup
 // consecutive sorted pairs; lane l owns channels l, l+16, ... . The group
 // walks its pairs in batches of 16 (one pair's index and point loaded per
 // lane, then broadcast), sums the four taps' gradients of the current bin in
 // registers and adds them when the bin changes and at the end.
-constexpr int kPairsPerGroup = 64;
-
 template <class Src, class GS>
 __global__ void __launch_bounds__(256) k_plane_scatter_sorted(tfh_vm vm, Src src, int64_t pairs,
                                                               const uint32_t* __restrict__ order,
@@ -362,109 +779,6 @@ __global__ void __launch_bounds__(256) k_plane_scatter_sorted(tfh_vm vm, Src src
           const float gl = gsrc.at(row, m, c) * lv;
 #pragma unroll
           for (int t = 0; t < 4; ++t) acc[t][q] += w[t] * gl;
-        }
-      }
-    }
-  }
-  if (cur >= 0) flush();
-}
-
-// Channel 16q + l of a 16-lane group whose lane j holds channels
-// 4j .. 4j+3 (v): the sums go back to one channel per lane before they are
-// added, so that each atomic instruction of a group covers 64 contiguous
-// bytes (one memory-side transaction) as in the scalar kernel; with the
-// quads the lanes' adds were 16 bytes apart, three transactions per
-// instruction (the plane pass took 1.54 ms instead of 0.69). All 16 lanes of
-// the group must call it (gl0: the group's first lane in the wave).
-__device__ __forceinline__ float quad_to_lane(const float (&v)[4], int q, int l, int gl0) {
-  const int from = gl0 + 4 * q + (l >> 2);
-  const float t0 = __shfl(v[0], from, 64), t1 = __shfl(v[1], from, 64);
-  const float t2 = __shfl(v[2], from, 64), t3 = __shfl(v[3], from, 64);
-  const int u = l & 3;
-  return u == 0 ? t0 : (u == 1 ? t1 : (u == 2 ? t2 : t3));
-}
-
-// k_plane_scatter_sorted with 16-byte loads: lane l of a 16-lane group of 64
-// pairs owns channels 4l .. 4l+3 (C % 4 == 0, 16 < C <= 64). The same sums
-// per channel, a third of the loads for 48 channels.
-template <class Src, class GS, int LPS>
-__global__ void __launch_bounds__(256) k_plane_scatter_sorted4(tfh_vm vm, Src src, int64_t pairs,
-                                                               const uint32_t* __restrict__ order,
-                                                               GS gsrc,
-                                                               float* __restrict__ gplane) {
-  static_assert(LPS == 16, "one channel per lane for the adds");
-  const int G = (int)vm.grid_dim, C = (int)vm.channels;
-  const int l = threadIdx.x % LPS;
-  const int gbase = threadIdx.x - l;  // first lane of the group in the block
-  const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * kPairsPerGroup;
-  if (first >= pairs) return;  // whole group: no cross-group exchange below
-  const int64_t last = min(first + (int64_t)kPairsPerGroup, pairs);
-  const int c4 = 4 * l;
-  const bool lane_on = c4 < C;
-  float4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-  int cur = -1;  // bin being summed
-  int tex[4] = {0, 0, 0, 0};
-  const int gl0 = gbase & 63;
-  auto flush = [&]() {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float v[4] = {acc[t].x, acc[t].y, acc[t].z, acc[t].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (16 * q < C) {  // group-uniform
-          const float val = quad_to_lane(v, q, l, gl0);
-          const int c = 16 * q + l;
-          if (c < C && val != 0.0f) unsafeAtomicAdd(gplane + (size_t)tex[t] * C + c, val);
-        }
-      }
-      acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    }
-  };
-  for (int64_t b0 = first; b0 < last; b0 += LPS) {
-    // lane l fetches pair b0 + l: its packed index and the row's point
-    const int64_t e = b0 + l;
-    uint32_t pk = 0xffffffffu;
-    float px = 0.f, py = 0.f, pz = 0.f;
-    if (e < last) {
-      pk = order[e];
-      src.get((int64_t)(pk >> 2), px, py, pz);
-    }
-    const int nb = (int)min((int64_t)LPS, last - b0);
-    for (int j = 0; j < nb; ++j) {
-      const uint32_t p = __shfl(pk, gbase + j, 64);
-      const float x = __shfl(px, gbase + j, 64), y = __shfl(py, gbase + j, 64),
-                  z = __shfl(pz, gbase + j, 64);
-      const int64_t row = (int64_t)(p >> 2);
-      const int m = (int)(p & 3u);
-      Tap tv, ta, tb;
-      one_mode_taps(x, y, z, G, m, tv, ta, tb);
-      const int bin = plane_bin(m, ta, tb, G);
-      if (bin != cur) {
-        if (cur >= 0) flush();
-        cur = bin;
-        const int base = m * G;
-        tex[0] = (base + ta.i0) * G + tb.i0;
-        tex[1] = (base + ta.i0) * G + tb.i1;
-        tex[2] = (base + ta.i1) * G + tb.i0;
-        tex[3] = (base + ta.i1) * G + tb.i1;
-      }
-      if (lane_on) {
-        const float w[4] = {ta.w0 * tb.w0, ta.w0 * tb.w1, ta.w1 * tb.w0, ta.w1 * tb.w1};
-        const float4 l0 = *reinterpret_cast<const float4*>(vm.line + (size_t)(m * G + tv.i0) * C + c4);
-        const float4 l1 = *reinterpret_cast<const float4*>(vm.line + (size_t)(m * G + tv.i1) * C + c4);
-        const float4 g4 = gsrc.at4(row, m, c4);
-        const float4 gl = make_float4(g4.x * (tv.w0 * l0.x + tv.w1 * l1.x),
-                                      g4.y * (tv.w0 * l0.y + tv.w1 * l1.y),
-                                      g4.z * (tv.w0 * l0.z + tv.w1 * l1.z),
-                                      g4.w * (tv.w0 * l0.w + tv.w1 * l1.w));
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          acc[t].x += w[t] * gl.x;
-          acc[t].y += w[t] * gl.y;
-          acc[t].z += w[t] * gl.z;
-          acc[t].w += w[t] * gl.w;
         }
       }
     }
@@ -546,332 +860,6 @@ __global__ void __launch_bounds__(kGatherThreads) k_line_scatter(tfh_vm vm, Src 
   }
 }
 
-// ---- both fields in one pass -------------------------------------------------
-// When every sample is shaded and the density (CD <= 16 channels, upstream
-// gradient dL/dsigma per row) and appearance (16 < CA <= 64, C % 4 == 0,
-// upstream gradient the feature row) factors share the grid, the pairs, the
-// taps and the line merge plan are the same for both: one pass computes them
-// once and scatters both fields.
-struct FieldOut {
-  tfh_vm vm;
-  float* gplane;
-  float* gline;  // nlc copies of the line gradient
-  int nlc;
-};
-
-// The plane pass of both fields: k_plane_scatter_sorted4 for the appearance
-// channels (lane l: 4l .. 4l+3) beside the scalar density channels (lane l:
-// channel l), one bin change flushing both.
-template <class Src>
-__global__ void __launch_bounds__(256) k_plane_scatter_two(Src src, int64_t pairs,
-                                                           const uint32_t* __restrict__ order,
-                                                           RowGrad ga, FieldOut fa, ScalarGrad gd,
-                                                           FieldOut fd) {
-  constexpr int LPS = 16;
-  const int G = (int)fa.vm.grid_dim, CA = (int)fa.vm.channels, CD = (int)fd.vm.channels;
-  const int l = threadIdx.x & 15;
-  const int gbase = threadIdx.x & ~15;
-  const int gl0 = gbase & 63;
-  const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * kPairsPerGroup;
-  if (first >= pairs) return;  // whole group: no cross-group exchange below
-  const int64_t last = min(first + (int64_t)kPairsPerGroup, pairs);
-  const int c4 = 4 * l;
-  const bool a_on = c4 < CA, d_on = l < CD;
-  float4 acc[4];
-  float accd[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    accd[t] = 0.0f;
-  }
-  int cur = -1;
-  int tex[4] = {0, 0, 0, 0};
-  auto flush = [&]() {
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const float v[4] = {acc[t].x, acc[t].y, acc[t].z, acc[t].w};
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        if (16 * q < CA) {  // group-uniform
-          const float val = quad_to_lane(v, q, l, gl0);
-          const int c = 16 * q + l;
-          if (c < CA && val != 0.0f) unsafeAtomicAdd(fa.gplane + (size_t)tex[t] * CA + c, val);
-        }
-      }
-      if (d_on && accd[t] != 0.0f) unsafeAtomicAdd(fd.gplane + (size_t)tex[t] * CD + l, accd[t]);
-      acc[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-      accd[t] = 0.0f;
-    }
-  };
-  for (int64_t b0 = first; b0 < last; b0 += LPS) {
-    const int64_t e = b0 + l;
-    uint32_t pk = 0xffffffffu;
-    float px = 0.f, py = 0.f, pz = 0.f;
-    if (e < last) {
-      pk = order[e];
-      src.get((int64_t)(pk >> 2), px, py, pz);
-    }
-    const int nb = (int)min((int64_t)LPS, last - b0);
-    for (int j = 0; j < nb; ++j) {
-      const uint32_t p = __shfl(pk, gbase + j, 64);
-      const float x = __shfl(px, gbase + j, 64), y = __shfl(py, gbase + j, 64),
-                  z = __shfl(pz, gbase + j, 64);
-      const int64_t row = (int64_t)(p >> 2);
-      const int m = (int)(p & 3u);
-      Tap tv, ta, tb;
-      one_mode_taps(x, y, z, G, m, tv, ta, tb);
-      // both fields' line taps and upstream gradients requested before the
-      // flush: one memory round trip per pair instead of one per field
-      float4 l0 = make_float4(0.f, 0.f, 0.f, 0.f), l1 = l0, g4 = l0;
-      float dl0 = 0.f, dl1 = 0.f, dg = 0.f;
-      if (a_on) {
-        l0 = *reinterpret_cast<const float4*>(fa.vm.line + (size_t)(m * G + tv.i0) * CA + c4);
-        l1 = *reinterpret_cast<const float4*>(fa.vm.line + (size_t)(m * G + tv.i1) * CA + c4);
-        g4 = ga.at4(row, m, c4);
-      }
-      if (d_on) {
-        dl0 = fd.vm.line[(size_t)(m * G + tv.i0) * CD + l];
-        dl1 = fd.vm.line[(size_t)(m * G + tv.i1) * CD + l];
-        dg = gd.at(row, m, l);
-      }
-      const int bin = plane_bin(m, ta, tb, G);
-      if (bin != cur) {
-        if (cur >= 0) flush();
-        cur = bin;
-        const int base = m * G;
-        tex[0] = (base + ta.i0) * G + tb.i0;
-        tex[1] = (base + ta.i0) * G + tb.i1;
-        tex[2] = (base + ta.i1) * G + tb.i0;
-        tex[3] = (base + ta.i1) * G + tb.i1;
-      }
-      const float w[4] = {ta.w0 * tb.w0, ta.w0 * tb.w1, ta.w1 * tb.w0, ta.w1 * tb.w1};
-      if (a_on) {
-        const float4 gl = make_float4(g4.x * (tv.w0 * l0.x + tv.w1 * l1.x),
-                                      g4.y * (tv.w0 * l0.y + tv.w1 * l1.y),
-                                      g4.z * (tv.w0 * l0.z + tv.w1 * l1.z),
-                                      g4.w * (tv.w0 * l0.w + tv.w1 * l1.w));
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          acc[t].x += w[t] * gl.x;
-          acc[t].y += w[t] * gl.y;
-          acc[t].z += w[t] * gl.z;
-          acc[t].w += w[t] * gl.w;
-        }
-      }
-      if (d_on) {
-        const float gl = dg * (tv.w0 * dl0 + tv.w1 * dl1);
-#pragma unroll
-        for (int t = 0; t < 4; ++t) accd[t] += w[t] * gl;
-      }
-    }
-  }
-  if (cur >= 0) flush();
-}
-
-// The line pass of both fields: k_line_scatter's groups, taps and merge plan
-// once; channel slots 0 .. NQA-1 (16 channels each) of the appearance, then
-// the density's (CD <= 16).
-template <class Src>
-__global__ void __launch_bounds__(kGatherThreads) k_line_scatter_two(Src src, int64_t M,
-                                                                     RowGrad ga, FieldOut fa,
-                                                                     ScalarGrad gd, FieldOut fd) {
-  constexpr int LPS = 16, SPB = kGatherThreads / LPS;
-  const int grp = threadIdx.x / LPS, l = threadIdx.x % LPS;
-  const int64_t s0 = (int64_t)blockIdx.x * SPB;
-  if (s0 >= M) return;
-  const int64_t s = s0 + grp;
-  const bool active = s < M;
-  const int G = (int)fa.vm.grid_dim, CA = (int)fa.vm.channels, CD = (int)fd.vm.channels;
-  float* glA = fa.gline + (int64_t)(blockIdx.x % fa.nlc) * 3 * G * CA;
-  float* glD = fd.gline + (int64_t)(blockIdx.x % fd.nlc) * 3 * G * CD;
-  float x = 0.f, y = 0.f, z = 0.f;
-  if (active) src.get(s, x, y, z);
-  ModeTaps mt[3];
-  mode_taps(x, y, z, G, mt);
-  const int wg = grp & 3;
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    TapAddr a;
-    tap_addrs(mt[m], m, G, a);
-    int k0 = active ? a.line0 : -1 - 2 * wg, k1 = active ? a.line1 : -2 - 2 * wg;
-    const bool fold = active && k1 == k0;
-    if (fold) k1 = INT_MIN + wg;
-    int src0[3], src1[3];
-    bool lead0 = active, lead1 = active && !fold;
-#pragma unroll
-    for (int oi = 0; oi < 3; ++oi) {
-      const int o = LPS * (oi + 1);
-      const bool lower = (wg ^ (oi + 1)) < wg;
-      const int p0 = __shfl_xor(k0, o, 64), p1 = __shfl_xor(k1, o, 64);
-      src0[oi] = p0 == k0 ? 0 : (p1 == k0 ? 1 : -1);
-      src1[oi] = p0 == k1 ? 0 : (p1 == k1 ? 1 : -1);
-      if (src0[oi] >= 0 && lower) lead0 = false;
-      if (src1[oi] >= 0 && lower) lead1 = false;
-    }
-    // slots 0..3 appearance (while 16 q < CA), slot 4 density
-#pragma unroll
-    for (int q = 0; q < 5; ++q) {
-      const bool dens = q == 4;
-      const int C = dens ? CD : CA;
-      if (!dens && LPS * q >= CA) continue;  // wave-uniform
-      const int c = dens ? l : l + LPS * q;
-      const bool on = active && c < C;
-      float v0 = 0.f, v1 = 0.f;
-      if (on) {
-        float lv, pv;
-        tap_values(dens ? fd.vm.plane : fa.vm.plane, dens ? fd.vm.line : fa.vm.line, C, c, a, lv,
-                   pv);
-        const float gp = (dens ? gd.at(s, m, c) : ga.at(s, m, c)) * pv;
-        v0 = a.wl0 * gp;
-        v1 = a.wl1 * gp;
-        if (fold) {
-          v0 += v1;
-          v1 = 0.f;
-        }
-      }
-      float acc0 = v0, acc1 = v1;
-#pragma unroll
-      for (int oi = 0; oi < 3; ++oi) {
-        const int o = LPS * (oi + 1);
-        const float q0 = __shfl_xor(v0, o, 64), q1 = __shfl_xor(v1, o, 64);
-        acc0 += src0[oi] == 0 ? q0 : (src0[oi] == 1 ? q1 : 0.0f);
-        acc1 += src1[oi] == 0 ? q0 : (src1[oi] == 1 ? q1 : 0.0f);
-      }
-      float* gl = dens ? glD : glA;
-      if (lead0 && acc0 != 0.0f) unsafeAtomicAdd(gl + (size_t)k0 * C + c, acc0);
-      if (lead1 && acc1 != 0.0f) unsafeAtomicAdd(gl + (size_t)k1 * C + c, acc1);
-    }
-  }
-}
-
-// The line pass of both fields over pairs ordered by line cell (sort_lines):
-// a 16-lane group walks 64 pairs, sums the two line taps' gradients of a
-// cell's run in registers (appearance: 16-byte plane taps, lane l channels
-// 4l .. 4l+3; density: lane l channel l) and adds them when the cell
-// changes. A line texel collects the adds of every sample on its plane
-// slice, so in ray order it draws one memory-side transaction per sample
-// and 16 channels wherever consecutive samples of a ray move to a new
-// texel; in cell order it draws a few per run of thousands of pairs. The
-// adds go straight to the line gradients (no copies).
-static_assert(3 * (kSortMaxGrid + 1) <= kSortMaxTiles, "line bins fit the sort's tile table");
-
-// RAY: the pairs in ray order instead, mode by mode (pair e = (row e % M,
-// mode e / M), M rows): a group walks 64 consecutive samples of one ray and
-// mode, and a run is a stretch of the ray inside one line cell; the adds go
-// to fa's / fd's line copies (block b into copy b % nlc), since every ray
-// crosses the same few line texels.
-template <class Src, bool RAY = false>
-__global__ void __launch_bounds__(256) k_line_walk_two(Src src, int64_t pairs,
-                                                       const uint32_t* __restrict__ order,
-                                                       RowGrad ga, FieldOut fa, ScalarGrad gd,
-                                                       FieldOut fd, int64_t M = 0) {
-  constexpr int LPS = 16;
-  const int G = (int)fa.vm.grid_dim, CA = (int)fa.vm.channels, CD = (int)fd.vm.channels;
-  float* glA = fa.gline + (int64_t)(blockIdx.x % fa.nlc) * 3 * G * CA;
-  float* glD = fd.gline + (int64_t)(blockIdx.x % fd.nlc) * 3 * G * CD;
-  const int l = threadIdx.x & 15;
-  const int gbase = threadIdx.x & ~15;
-  const int gl0 = gbase & 63;
-  const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * kPairsPerGroup;
-  if (first >= pairs) return;  // whole group: no cross-group exchange below
-  const int64_t last = min(first + (int64_t)kPairsPerGroup, pairs);
-  const int c4 = 4 * l;
-  const bool a_on = c4 < CA, d_on = l < CD;
-  float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), a1 = a0;
-  float d0 = 0.0f, d1 = 0.0f;
-  int cur = -1, cell0 = 0, cell1 = 0;
-  auto flush = [&]() {
-    const float v0[4] = {a0.x, a0.y, a0.z, a0.w}, v1[4] = {a1.x, a1.y, a1.z, a1.w};
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (16 * q < CA) {  // group-uniform
-        const float x0 = quad_to_lane(v0, q, l, gl0), x1 = quad_to_lane(v1, q, l, gl0);
-        const int c = 16 * q + l;
-        if (c < CA) {
-          if (x0 != 0.0f) unsafeAtomicAdd(glA + (size_t)cell0 * CA + c, x0);
-          if (x1 != 0.0f) unsafeAtomicAdd(glA + (size_t)cell1 * CA + c, x1);
-        }
-      }
-    }
-    if (d_on) {
-      if (d0 != 0.0f) unsafeAtomicAdd(glD + (size_t)cell0 * CD + l, d0);
-      if (d1 != 0.0f) unsafeAtomicAdd(glD + (size_t)cell1 * CD + l, d1);
-    }
-    a0 = a1 = make_float4(0.f, 0.f, 0.f, 0.f);
-    d0 = d1 = 0.0f;
-  };
-  for (int64_t b0 = first; b0 < last; b0 += LPS) {
-    const int64_t e = b0 + l;
-    uint32_t pk = 0xffffffffu;
-    float px = 0.f, py = 0.f, pz = 0.f;
-    if (e < last) {
-      if constexpr (RAY) {
-        const int64_t m = e / M;
-        pk = (uint32_t)(((e - m * M) << 2) | m);
-      } else {
-        pk = order[e];
-      }
-      src.get((int64_t)(pk >> 2), px, py, pz);
-    }
-    const int nb = (int)min((int64_t)LPS, last - b0);
-    for (int j = 0; j < nb; ++j) {
-      const uint32_t p = __shfl(pk, gbase + j, 64);
-      const float x = __shfl(px, gbase + j, 64), y = __shfl(py, gbase + j, 64),
-                  z = __shfl(pz, gbase + j, 64);
-      const int64_t row = (int64_t)(p >> 2);
-      const int m = (int)(p & 3u);
-      Tap tv, ta, tb;
-      one_mode_taps(x, y, z, G, m, tv, ta, tb);
-      // the four plane taps of mode m (tap_addrs' order and weights) and the
-      // upstream gradients of both fields, requested before the flush
-      const int base = m * G;
-      const int64_t p00 = (int64_t)(base + ta.i0) * G + tb.i0, p01 = (int64_t)(base + ta.i0) * G + tb.i1;
-      const int64_t p10 = (int64_t)(base + ta.i1) * G + tb.i0, p11 = (int64_t)(base + ta.i1) * G + tb.i1;
-      float4 t00 = make_float4(0.f, 0.f, 0.f, 0.f), t01 = t00, t10 = t00, t11 = t00, g4 = t00;
-      float d00 = 0.f, d01 = 0.f, d10 = 0.f, d11 = 0.f, dg = 0.f;
-      if (a_on) {
-        const float* pl = fa.vm.plane + c4;
-        t00 = *reinterpret_cast<const float4*>(pl + p00 * CA);
-        t01 = *reinterpret_cast<const float4*>(pl + p01 * CA);
-        t10 = *reinterpret_cast<const float4*>(pl + p10 * CA);
-        t11 = *reinterpret_cast<const float4*>(pl + p11 * CA);
-        g4 = ga.at4(row, m, c4);
-      }
-      if (d_on) {
-        const float* pl = fd.vm.plane + l;
-        d00 = pl[p00 * CD];
-        d01 = pl[p01 * CD];
-        d10 = pl[p10 * CD];
-        d11 = pl[p11 * CD];
-        dg = gd.at(row, m, l);
-      }
-      const int bin = m * (G + 1) + tap_code(tv, G);
-      if (bin != cur) {
-        if (cur >= 0) flush();
-        cur = bin;
-        cell0 = m * G + tv.i0;
-        cell1 = m * G + tv.i1;
-      }
-      const float w00 = ta.w0 * tb.w0, w01 = ta.w0 * tb.w1, w10 = ta.w1 * tb.w0, w11 = ta.w1 * tb.w1;
-      if (a_on) {
-        const float gx = g4.x * (((w00 * t00.x + w01 * t01.x) + w10 * t10.x) + w11 * t11.x);
-        const float gy = g4.y * (((w00 * t00.y + w01 * t01.y) + w10 * t10.y) + w11 * t11.y);
-        const float gz = g4.z * (((w00 * t00.z + w01 * t01.z) + w10 * t10.z) + w11 * t11.z);
-        const float gw = g4.w * (((w00 * t00.w + w01 * t01.w) + w10 * t10.w) + w11 * t11.w);
-        a0.x += tv.w0 * gx; a0.y += tv.w0 * gy; a0.z += tv.w0 * gz; a0.w += tv.w0 * gw;
-        a1.x += tv.w1 * gx; a1.y += tv.w1 * gy; a1.z += tv.w1 * gz; a1.w += tv.w1 * gw;
-      }
-      if (d_on) {
-        const float pv = ((w00 * d00 + w01 * d01) + w10 * d10) + w11 * d11;
-        const float gp = dg * pv;
-        d0 += tv.w0 * gp;
-        d1 += tv.w1 * gp;
-      }
-    }
-  }
-  if (cur >= 0) flush();
-}
-
 // Orders the (row, mode) pairs by line cell (3 (g+1) bins: rank, scan,
 // place; the bin is the whole key).
 template <class Src>
@@ -889,57 +877,33 @@ inline int32_t sort_lines(int g, const Src& src, int64_t M, const SortWs& s, hip
   return check_launch("vm scatter: line sort");
 }
 
-// Whether the two fields can take the one-pass scatter.
-inline bool two_field_scatter_ok(const tfh_vm& den, const tfh_vm& app, const RowGrad& ga) {
-  return den.grid_dim == app.grid_dim && den.channels >= 1 && den.channels <= 16 &&
-         app.channels > 16 && app.channels <= 64 && app.channels % 4 == 0 &&
-         (reinterpret_cast<uintptr_t>(app.plane) & 15) == 0 &&
-         (reinterpret_cast<uintptr_t>(app.line) & 15) == 0 && ga.aligned16();
+// The plane pass of field(s) fa (quad lanes) and fd (a channel per lane) over
+// the pairs sort_pairs ordered.
+template <int LPS, class Src, class FA, class FD>
+inline int32_t launch_plane_walk(const Src& src, int g, int64_t M, const SortWs& s, const FA& fa,
+                                 const FD& fd, const char* stage, hipStream_t st) {
+  ProfScope ps(stage, st);
+  const int per = walk_pairs(3 * M);
+  const int64_t blocks = ceil_div(ceil_div(3 * M, per), 256 / LPS);
+  hipLaunchKernelGGL((k_plane_walk<Src, FA, FD, LPS>), dim3((unsigned)blocks), dim3(256), 0, st,
+                     src, g, 3 * M, per, s.order, fa, fd);
+  return check_launch("vm scatter: planes");
 }
 
-// Both fields' plane and line passes over the pairs sort_pairs ordered.
-// lines_sorted: the line pass on pairs re-sorted by line cell (the sort's
-// arrays are reused after the plane pass), adding straight into lines_a /
-// lines_d (the fields' line gradients); else a ray-order pass into fa's
-// and fd's line copies: ray_walk, runs of a ray's samples in one line cell
-// summed in registers (k_line_walk_two in ray order; pays where many
-// consecutive samples share a cell), or k_line_scatter_two's merge of each
-// wave's four samples.
-template <class Src>
-inline int32_t scatter_two_fields(const Src& src, int64_t M, const SortWs& s, const RowGrad& ga,
-                                  const FieldOut& fa, const ScalarGrad& gd, const FieldOut& fd,
-                                  hipStream_t st, bool lines_sorted = false,
-                                  float* lines_a = nullptr, float* lines_d = nullptr,
-                                  bool ray_walk = false) {
-  if (M <= 0) return TFH_OK;
-  const int64_t pairs = 3 * M;
-  const int64_t groups = ceil_div(pairs, kPairsPerGroup);
-  {
-    ProfScope ps("factor_scatter_planes", st);
-    hipLaunchKernelGGL((k_plane_scatter_two<Src>), dim3((unsigned)ceil_div(groups, 16)), dim3(256),
-                       0, st, src, pairs, s.order, ga, fa, gd, fd);
-    TFH_TRY(check_launch("vm scatter: planes of both fields"));
-  }
-  if (lines_sorted) {
-    TFH_TRY(sort_lines((int)fa.vm.grid_dim, src, M, s, st));
-    ProfScope ps("factor_scatter_lines", st);
-    FieldOut la = fa, ld = fd;
-    la.gline = lines_a;
-    la.nlc = 1;
-    ld.gline = lines_d;
-    ld.nlc = 1;
-    hipLaunchKernelGGL((k_line_walk_two<Src>), dim3((unsigned)ceil_div(groups, 16)), dim3(256), 0,
-                       st, src, pairs, s.order, ga, la, gd, ld);
-    return check_launch("vm scatter: sorted lines of both fields");
-  }
-  ProfScope ps("factor_scatter_lines", st);
-  if (ray_walk)
-    hipLaunchKernelGGL((k_line_walk_two<Src, true>), dim3((unsigned)ceil_div(groups, 16)),
-                       dim3(256), 0, st, src, pairs, nullptr, ga, fa, gd, fd, M);
+// The line pass; sorted: over the pairs sort_lines ordered, else in ray order.
+template <int LPS, class Src, class FA, class FD>
+inline int32_t launch_line_walk(bool sorted, const Src& src, int g, int64_t M, const SortWs& s,
+                                const FA& fa, const FD& fd, const char* stage, hipStream_t st) {
+  ProfScope ps(stage, st);
+  const int per = walk_pairs(3 * M);
+  const int64_t blocks = ceil_div(ceil_div(3 * M, per), 256 / LPS);
+  if (sorted)
+    hipLaunchKernelGGL((k_line_walk<Src, FA, FD, LPS, false>), dim3((unsigned)blocks), dim3(256),
+                       0, st, src, g, 3 * M, per, M, s.order, fa, fd);
   else
-    hipLaunchKernelGGL((k_line_scatter_two<Src>), dim3((unsigned)ceil_div(M, kGatherThreads / 16)),
-                       dim3(kGatherThreads), 0, st, src, M, ga, fa, gd, fd);
-  return check_launch("vm scatter: lines of both fields");
+    hipLaunchKernelGGL((k_line_walk<Src, FA, FD, LPS, true>), dim3((unsigned)blocks), dim3(256), 0,
+                       st, src, g, 3 * M, per, M, nullptr, fa, fd);
+  return check_launch("vm scatter: lines");
 }
 
 // Bytes of the sort's workspace for up to M rows.
@@ -957,12 +921,25 @@ inline void take_sort_ws(Carve& cv, int64_t M, SortWs& s) {
   s.chunk_start = cv.take<int32_t>(kSortMaxTiles + 1);
 }
 
-// Whether a field takes the sorted scatter: 9..64 channels (16-lane
-// groups), a grid within the bin budget, and a row count whose packed
-// (row, mode) index fits 32 bits.
+// Whether a field takes the sorted scatter: at most 64 channels, a grid
+// within the bin budget, and a row count whose packed (row, mode) index fits
+// 32 bits.
 inline bool sorted_scatter_ok(const tfh_vm& vm, int64_t M, const SortWs& s) {
-  return s.order && vm.channels > 8 && vm.channels <= 64 && vm.grid_dim <= kSortMaxGrid &&
-         M < (1ll << 30);
+  return s.order && vm.channels <= 64 && vm.grid_dim <= kSortMaxGrid && M < (1ll << 30);
+}
+
+// Whether a field can take the walks' quad lanes.
+template <class GS>
+inline bool quad_lanes_ok(const tfh_vm& vm, const GS& g) {
+  return vm.channels > 16 && vm.channels <= 64 && vm.channels % 4 == 0 &&
+         (reinterpret_cast<uintptr_t>(vm.plane) & 15) == 0 &&
+         (reinterpret_cast<uintptr_t>(vm.line) & 15) == 0 && g.aligned16();
+}
+
+// Whether both fields can go in one walk (every sample shaded, one grid).
+inline bool two_field_scatter_ok(const tfh_vm& den, const tfh_vm& app, const RowGrad& ga) {
+  return den.grid_dim == app.grid_dim && den.channels >= 1 && den.channels <= 16 &&
+         quad_lanes_ok(app, ga);
 }
 
 // Sorts the (row, mode) pairs of M rows by plane cell of a grid of size g.
@@ -987,39 +964,39 @@ inline int32_t sort_pairs(int g, const Src& src, int64_t M, const SortWs& s, con
 }
 
 // The scatter of a field's feature gradients (gsrc) for M rows whose pairs
-// sort_pairs has ordered: planes into grad.plane, lines into grad.line (nlc
-// copies). stages: profile names of the plane and line passes.
+// sort_pairs has ordered: planes into grad.plane, lines in ray order into
+// grad.line (nlc copies). Fields of more than 16 channels that quad lanes
+// cannot take keep the general passes (four channel slots per lane). stages:
+// profile names of the plane and line passes.
 template <class Src, class GS>
 inline int32_t scatter_sorted_pairs(const tfh_vm& vm, const Src& src, int64_t M, const GS& gsrc,
                                     const tfh_vm_grad& grad, int nlc, const SortWs& s,
                                     const char* plane_stage, const char* line_stage,
                                     hipStream_t st) {
   if (M <= 0) return TFH_OK;
-  // 16-byte loads in the plane pass when the channels and every tap source
-  // allow; only for fields of more than 16 channels: a 16-channel field's
-  // 16-lane groups read a tap in one instruction either way, and narrower
-  // groups would split its adds over several transactions
-  const bool wide = vm.channels % 4 == 0 && vm.channels <= 64 &&
-                    (reinterpret_cast<uintptr_t>(vm.plane) & 15) == 0 &&
-                    (reinterpret_cast<uintptr_t>(vm.line) & 15) == 0 && gsrc.aligned16();
+  const int g = (int)vm.grid_dim;
+  const WalkField<GS> fp{vm, gsrc, grad.plane, 1}, fl{vm, gsrc, grad.line, nlc};
+  const NoField none;
+  if (quad_lanes_ok(vm, gsrc)) {
+    TFH_TRY(launch_plane_walk<16>(src, g, M, s, fp, none, plane_stage, st));
+    return launch_line_walk<16>(false, src, g, M, s, fl, none, line_stage, st);
+  }
+  if (vm.channels <= 8) {
+    TFH_TRY(launch_plane_walk<8>(src, g, M, s, none, fp, plane_stage, st));
+    return launch_line_walk<8>(false, src, g, M, s, none, fl, line_stage, st);
+  }
+  if (vm.channels <= 16) {
+    TFH_TRY(launch_plane_walk<16>(src, g, M, s, none, fp, plane_stage, st));
+    return launch_line_walk<16>(false, src, g, M, s, none, fl, line_stage, st);
+  }
   {
     ProfScope ps(plane_stage, st);
     const int64_t pairs = 3 * M;
     const int64_t groups = ceil_div(pairs, kPairsPerGroup);
-    const int C = (int)vm.channels;
-    if (wide && C > 16) {
-      hipLaunchKernelGGL((k_plane_scatter_sorted4<Src, GS, 16>),
-                         dim3((unsigned)ceil_div(groups, 16)), dim3(256), 0, st, vm, src, pairs,
-                         s.order, gsrc, grad.plane);
-    } else {
-      hipLaunchKernelGGL((k_plane_scatter_sorted<Src, GS>), dim3((unsigned)ceil_div(groups, 16)),
-                         dim3(256), 0, st, vm, src, pairs, s.order, gsrc, grad.plane);
-    }
+    hipLaunchKernelGGL((k_plane_scatter_sorted<Src, GS>), dim3((unsigned)ceil_div(groups, 16)),
+                       dim3(256), 0, st, vm, src, pairs, s.order, gsrc, grad.plane);
     TFH_TRY(check_launch("vm scatter: planes"));
   }
-  // the line pass keeps 4-byte taps: with 16-byte ones its merged adds need
-  // the sums moved back to one channel per lane, which cost more than the
-  // loads saved (0.83 -> 0.89 ms for 48 channels at 2.1 M rows)
   ProfScope ps(line_stage, st);
   hipLaunchKernelGGL((k_line_scatter<Src, GS>), dim3((unsigned)ceil_div(M, kGatherThreads / 16)),
                      dim3(kGatherThreads), 0, st, vm, src, M, gsrc, grad.line, nlc);
