@@ -135,10 +135,10 @@ struct MlpW {  // FP32 parameters (device pointers)
   const float *w0, *w1, *b1, *w2, *b2, *w3, *b3, *embed;
 };
 
-// Operand tables built per call in the workspace: forward tables [out][in]
-// and input-gradient tables [in][out], zero padded:
-//   f0 [32][FP], f1 [U][EP], f2 [U][U], f3 [16][U]
-//   g0 [FP][32], g1 [EP][U], g2 [U][U], g3 [U][32]
+// Operand tables built per call in the workspace (Table; the FP32 f3 is row-
+// major), zero padded, columns x inputs:
+//   forward f0 32 x FP, f1 U x EP, f2 U x U, f3 16 x U
+//   input gradients g0 FP x 32, g1 EP x U, g2 U x U, g3 U x 32
 struct MlpPack {
   const __bf16 *f0, *f1, *f2, *f3, *g0, *g1, *g2, *g3;      // BF16 mode
   const float *ff0, *ff1, *ff2, *ff3, *fg0, *fg1, *fg2, *fg3;  // FP32 mode
@@ -156,7 +156,6 @@ struct Operands<false> {
   __device__ PackedB32 l0() const { return PackedB32(p.ff0, d.FP, 32); }
   __device__ PackedB32 l1() const { return PackedB32(p.ff1, d.EP, kU); }
   __device__ PackedB32 l2() const { return PackedB32(p.ff2, kU, kU); }
-  __device__ PackedB32 l3() const { return PackedB32(p.ff3, kU, 16); }
   __device__ PackedB32 g3() const { return PackedB32(p.fg3, 32, kU); }
   __device__ PackedB32 g2() const { return PackedB32(p.fg2, kU, kU); }
   __device__ PackedB32 g1() const { return PackedB32(p.fg1, kU, d.EP); }
@@ -694,23 +693,29 @@ __global__ void k_pack_weights(MlpDims d, MlpW w, PackOut<T> o, PackSizes s) {
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total;
        e += (int64_t)gridDim.x * blockDim.x) {
     int64_t f = e;
-    // forward tables T[j][k] = W[k][j]
-    if (f < s.f0) { const int j = f / d.FP, k = f % d.FP; o.f0[f] = (T)wat(w.w0, d.F, d.S, k, j); continue; }
+    int k, j;  // input and column of the operand
+    // forward tables: W[k][j]
+    if (f < s.f0) { table_entry<T>(f, d.FP, k, j); o.f0[f] = (T)wat(w.w0, d.F, d.S, k, j); continue; }
     f -= s.f0;
-    if (f < s.f1) { const int j = f / d.EP, k = f % d.EP; o.f1[f] = (T)wat(w.w1, d.E, kU, k, j); continue; }
+    if (f < s.f1) { table_entry<T>(f, d.EP, k, j); o.f1[f] = (T)wat(w.w1, d.E, kU, k, j); continue; }
     f -= s.f1;
-    if (f < s.f2) { const int j = f / kU, k = f % kU; o.f2[f] = (T)wat(w.w2, kU, kU, k, j); continue; }
+    if (f < s.f2) { table_entry<T>(f, kU, k, j); o.f2[f] = (T)wat(w.w2, kU, kU, k, j); continue; }
     f -= s.f2;
-    if (f < s.f3) { const int j = f / kU, k = f % kU; o.f3[f] = (T)wat(w.w3, kU, 3, k, j); continue; }
+    if (f < s.f3) {
+      table_entry<T>(f, kU, k, j);
+      if (sizeof(T) == 4) { j = (int)f / kU; k = (int)f % kU; }  // read by column (forward_out)
+      o.f3[f] = (T)wat(w.w3, kU, 3, k, j);
+      continue;
+    }
     f -= s.f3;
-    // input-gradient tables T[j][k] = W[j][k] (j = input unit, k = output unit)
-    if (f < s.g0) { const int j = f / 32, k = f % 32; o.g0[f] = (T)wat(w.w0, d.F, d.S, j, k); continue; }
+    // input-gradient tables: W[j][k] (j = input unit, k = output unit)
+    if (f < s.g0) { table_entry<T>(f, 32, k, j); o.g0[f] = (T)wat(w.w0, d.F, d.S, j, k); continue; }
     f -= s.g0;
-    if (f < s.g1) { const int j = f / kU, k = f % kU; o.g1[f] = (T)wat(w.w1, d.E, kU, j, k); continue; }
+    if (f < s.g1) { table_entry<T>(f, kU, k, j); o.g1[f] = (T)wat(w.w1, d.E, kU, j, k); continue; }
     f -= s.g1;
-    if (f < s.g2) { const int j = f / kU, k = f % kU; o.g2[f] = (T)wat(w.w2, kU, kU, j, k); continue; }
+    if (f < s.g2) { table_entry<T>(f, kU, k, j); o.g2[f] = (T)wat(w.w2, kU, kU, j, k); continue; }
     f -= s.g2;
-    { const int j = f / 32, k = f % 32; o.g3[f] = (T)wat(w.w3, kU, 3, j, k); }
+    { table_entry<T>(f, 32, k, j); o.g3[f] = (T)wat(w.w3, kU, 3, j, k); }
   }
 }
 
