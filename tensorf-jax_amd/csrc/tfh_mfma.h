@@ -9,6 +9,9 @@
 
 #include "tfh_common.h"
 
+// for lambdas: one that is not inlined passes its captured arrays through scratch
+#define TFH_INLINE __attribute__((always_inline))
+
 namespace tfh {
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));

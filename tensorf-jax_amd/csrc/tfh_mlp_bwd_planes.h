@@ -42,10 +42,6 @@
 
 #include "tfh_mlp_kernels.h"
 
-// The steps are lambdas over the kernel's registers: out of line, those would
-// live in scratch memory.
-#define TFH_INLINE __attribute__((always_inline))
-
 namespace tfh {
 
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));

@@ -6,7 +6,7 @@
 //                    contracted schedule) -> sample t = e_i + u (e_{i+1} - e_i)
 //                    -> contracted / normalised point
 //   k_vm_gather      proposal VM features (M, 3C)
-//   prop_mlp_fwd     sigma = softplus(MLP(features)) on FP32 MFMA
+//   prop_mlp_fwd     sigma = softplus(MLP(VM features)) on FP32 MFMA
 //   k_prop_resample  one wave per ray: weights (log-space transmittance scan),
 //                    padded histogram CDF, inverse-CDF edges of the next round
 // Backward (interval loss of mip-NeRF 360 against the field's weights):
@@ -22,8 +22,8 @@
 namespace tfh {
 
 int32_t check_prop_mlp(const tfh_prop_mlp* p, const char* who);
-int32_t prop_mlp_fwd(const tfh_prop_mlp* p, const float* feats, int64_t M, float* z, float* sigma,
-                     hipStream_t st);
+int32_t prop_mlp_fwd_gather(const tfh_prop_mlp* p, const tfh_vm& field, const float* pts,
+                            int64_t M, float* feats, float* sigma, hipStream_t st);
 size_t prop_mlp_bwd_workspace(const tfh_prop_mlp* p, int64_t M);
 // idx / count (device): process only the first *count rows listed in idx
 int32_t prop_mlp_bwd(const tfh_prop_mlp* p, const float* feats, const float* dz, int64_t M,
@@ -389,12 +389,7 @@ int32_t prop_sample(const tfh_vm* field, const tfh_prop_mlp* mlp, const tfh_prop
       hipLaunchKernelGGL(k_prop_points, dim3((unsigned)blocks), dim3(256), 0, st, pp);
     }
     TFH_TRY(check_launch("proposal points"));
-    {
-      ProfScope ps("prop_gather", st);
-      RaySamples src{rd.pts, nullptr, 1, 1};
-      TFH_TRY((launch_vm_gather<RaySamples, true>(*field, src, M, rd.feats, st)));
-    }
-    TFH_TRY(prop_mlp_fwd(mlp, rd.feats, M, nullptr, rd.sigma, st));
+    TFH_TRY(prop_mlp_fwd_gather(mlp, *field, rd.pts, M, rd.feats, rd.sigma, st));
     const bool last = k + 1 == ws.rounds;
     const int n_out = last ? pc->samples_out : ws.rd[k + 1].n;
     float* next = last ? edges_out : ws.rd[k + 1].edges;

@@ -1,13 +1,14 @@
 // MLP of the proposal density field (no counterpart in the reference):
 // z = W3 relu(W2 relu(W1 f + b1) + b2) + b3, sigma = softplus(z), with
 // f the 3C <= 32 VM features of a sample, 64 hidden units, FP32 MFMA.
-// Forward: one 64-row tile per workgroup. Backward (input dL/dz): persistent
+// Forward: 32 rows per wave, in registers. Backward (input dL/dz): persistent
 // workgroups recompute the forward of each tile, keep the 28 weight-gradient
 // 16x16 tiles in registers (7 per wave) and store them once per workgroup;
 // k_prop_reduce sums the workgroups.
 #include <algorithm>
 
 #include "tfh_mfma.h"
+#include "tfh_vm_kernels.h"
 
 namespace tfh {
 
@@ -87,36 +88,184 @@ __device__ __forceinline__ void prop_hidden(const PropW& w, const float* Fs, flo
   __syncthreads();
 }
 
-// z of row tile `wave` (16 rows) into Z[row] (column 0 of the D tile).
-__device__ __forceinline__ void prop_out(const PropW& w, const float* H2, float* Z) {
-  const int wave = threadIdx.x >> 6, lane = lane_id();
-  f32x4 acc[1];
-  zero_acc(acc);
-  mma_strip<1, kPH>(H2 + 16 * wave * kPLdH, kPLdH, kPH, GlobalB(w.w3, kPH, 1), 0, acc);
-  if ((lane & 15) == 0) {
-    const float b3 = w.b3[0];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Z[16 * wave + 4 * (lane >> 4) + e] = acc[0][e] + b3;
-  }
-  __syncthreads();
+// ---- forward --------------------------------------------------------------------
+// A wave computes 32 rows in registers, the products transposed: the operand
+// with 16 rows of the result is a table of the weights, the one with 16
+// columns the wave's rows. A result tile holds, in lane (r, kq) = r + 16 kq,
+// entries 4 kq .. 4 kq + 3 of row r; with unit 16 c + 4 e + kq of tile c at
+// entry 4 kq + e (kUnit), register e of tile c is the operand that product
+// 4 c + e of the next layer (inputs 16 c + 4 e + kq) reads, and no activation
+// passes through LDS. The order of every FP32 sum is that of prop_hidden.
+//
+// Bound by the FP32 matrix rate: 24 + 64 + 16 products of 16x16x4 per 16 rows
+// (the last 16 for one output), 1.35 ms for 12.6 M rows. With activations of a
+// 64-row tile in LDS, read by single values, and the weights loaded per tile it
+// took 2885 us there after a gather of 517, 607 after 116 for the 3.1 M rows of
+// a training step; with the gather in this kernel 1770 and 414. Ten or twelve
+// waves per workgroup (5 or 6 per SIMD) took 2167 and 1812.
+constexpr int kPFwdNW = 8;            // waves per workgroup
+constexpr int kPRows = 32;            // rows per wave
+constexpr int kPLdT = 28;             // row stride of a wave's features: 16 rows x 4 inputs of a
+                                      // product are 64 different banks
+
+struct PropFwdLds {
+  float4 a1[4][2][64];  // [unit tile][four products][lane]
+  float4 a2[4][4][64];
+  float4 a3[4][64];     // the output's weights in rows 0 and 4, zero elsewhere
+  float4 b1[4][4], b2[4][4];  // [unit tile][kq]
+};
+
+__device__ __forceinline__ int prop_unit(int tile, int entry) {
+  return 16 * tile + 4 * (entry & 3) + (entry >> 2);
 }
 
-__global__ void __launch_bounds__(kPNW * 64) k_prop_mlp_fwd(PropW w, const float* __restrict__ feats,
-                                                            int64_t M, float* __restrict__ z,
-                                                            float* __restrict__ sigma) {
-  __shared__ float Fs[kPTM * kPLdF];
-  __shared__ float H1[kPTM * kPLdH];
-  __shared__ float H2[kPTM * kPLdH];
-  __shared__ float Z[kPTM];
-  const int64_t row0 = (int64_t)blockIdx.x * kPTM;
-  prop_load(feats, w.F, row0, M, Fs);
+__device__ __forceinline__ void prop_fwd_tables(const PropW& w, PropFwdLds& t) {
+  float* a1 = &t.a1[0][0][0].x;
+  for (int e = threadIdx.x; e < 4 * 2 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, k = 4 * (4 * ((e >> 8) & 1) + (e & 3)) + (lane >> 4);
+    a1[e] = k < w.F ? w.w1[k * kPH + prop_unit(e >> 9, lane & 15)] : 0.0f;
+  }
+  float* a2 = &t.a2[0][0][0].x;
+  for (int e = threadIdx.x; e < 4 * 4 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, k = 4 * (4 * ((e >> 8) & 3) + (e & 3)) + (lane >> 4);
+    a2[e] = w.w2[k * kPH + prop_unit(e >> 10, lane & 15)];
+  }
+  float* a3 = &t.a3[0][0].x;
+  for (int e = threadIdx.x; e < 4 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, k = 4 * (4 * (e >> 8) + (e & 3)) + (lane >> 4);
+    a3[e] = (lane & 11) == 0 ? w.w3[k] : 0.0f;
+  }
+  if (threadIdx.x < 64) {
+    const int u = prop_unit(threadIdx.x >> 4, threadIdx.x & 15);
+    (&t.b1[0][0].x)[threadIdx.x] = w.b1[u];
+    (&t.b2[0][0].x)[threadIdx.x] = w.b2[u];
+  }
+}
+
+// One layer's products i < N (of KI) for two sets of 16 rows and all four unit
+// tiles; in(s, i) is the operand of set s.
+template <int N, int G, class In>
+__device__ __forceinline__ void prop_layer(const float4 (&a)[4][G][64], int lane, In in,
+                                           f32x4 (&acc)[2][4]) {
+#pragma unroll
+  for (int s = 0; s < 2; ++s) zero_acc(acc[s]);
+#pragma unroll
+  for (int g = 0; 4 * g < N; ++g) {
+    float4 av[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) av[c] = a[c][g][lane];
+#pragma unroll
+    for (int e = 0; e < 4 && 4 * g + e < N; ++e)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+          acc[s][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              e == 0 ? av[c].x : (e == 1 ? av[c].y : (e == 2 ? av[c].z : av[c].w)), in(s, 4 * g + e),
+              acc[s][c], 0, 0, 0);
+  }
+}
+
+__device__ __forceinline__ void prop_relu(const float4 (&b)[4][4], int kq, f32x4 (&acc)[2][4]) {
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float4 bias = b[c][kq];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      acc[s][c][0] = fmaxf(acc[s][c][0] + bias.x, 0.0f);
+      acc[s][c][1] = fmaxf(acc[s][c][1] + bias.y, 0.0f);
+      acc[s][c][2] = fmaxf(acc[s][c][2] + bias.z, 0.0f);
+      acc[s][c][3] = fmaxf(acc[s][c][3] + bias.w, 0.0f);
+    }
+  }
+}
+
+// The features come from feats, or (GATHER: 8 channels, F = 24) from the
+// field at pts, two lanes per sample with four channels each (the arithmetic
+// of k_vm_gather4), and go to feats too. N1: first-layer products, 4 N1 >= F.
+template <int N1, bool GATHER>
+__global__ void __launch_bounds__(kPFwdNW * 64, 4)
+    k_prop_mlp_fwd(PropW w, float* __restrict__ feats, tfh_vm vm, const float* __restrict__ pts,
+                   int64_t M, float* __restrict__ z, float* __restrict__ sigma) {
+  static_assert(!GATHER || N1 == 6, "8 channels");
+  __shared__ PropFwdLds t;
+  __shared__ float4 rows[GATHER ? kPFwdNW : 1][GATHER ? kPRows * kPLdT / 4 : 1];
+  prop_fwd_tables(w, t);
   __syncthreads();
-  prop_hidden(w, Fs, H1, H2);
-  prop_out(w, H2, Z);
-  for (int i = threadIdx.x; i < kPTM; i += blockDim.x) {
-    const int64_t row = row0 + i;
-    if (row < M) {
-      const float zv = Z[i];
+  const int wave = threadIdx.x >> 6;
+  const int64_t tiles = (M + kPRows - 1) / kPRows;
+  for (int64_t tile = (int64_t)blockIdx.x * kPFwdNW + wave; tile < tiles;
+       tile += (int64_t)gridDim.x * kPFwdNW) {
+    // (computed per tile: the tables' 128 registers would be kept otherwise)
+    const int lane = lane_here(), n = lane & 15, kq = lane >> 4;
+    const int64_t row0 = tile * kPRows;
+    float f[2][N1];
+    if constexpr (GATHER) {
+      const int i = lane >> 1, c4 = 4 * (lane & 1);
+      const int64_t row = row0 + i;
+      const bool valid = row < M;
+      const int G = (int)vm.grid_dim;
+      float x = 0.f, y = 0.f, zc = 0.f;
+      if (valid) {
+        x = pts[row * 3];
+        y = pts[row * 3 + 1];
+        zc = pts[row * 3 + 2];
+      }
+      ModeTaps mt[3];
+      mode_taps(x, y, zc, G, mt);
+      float4* to = &rows[wave][i * (kPLdT / 4)];
+#pragma unroll
+      for (int m = 0; m < 3; ++m) {
+        TapAddr a;
+        tap_addrs(mt[m], m, G, a);
+        float4 lv, pv;
+        tap_values4(vm.plane, vm.line, 8, c4, a, lv, pv);
+        const float4 v = make_float4(lv.x * pv.x, lv.y * pv.y, lv.z * pv.z, lv.w * pv.w);
+        to[2 * m + (lane & 1)] = v;
+        if (valid) *reinterpret_cast<float4*>(feats + row * 24 + 8 * m + c4) = v;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      const float* from = &rows[wave][0].x;
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < N1; ++j) f[s][j] = from[(16 * s + n) * kPLdT + 4 * j + kq];
+      // (the next tile's writes follow these reads in the wave's LDS order)
+      __builtin_amdgcn_wave_barrier();
+    } else {
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int64_t row = row0 + 16 * s + n;
+#pragma unroll
+        for (int j = 0; j < N1; ++j)
+          f[s][j] = row < M && 4 * j + kq < w.F ? feats[row * w.F + 4 * j + kq] : 0.0f;
+      }
+    }
+    f32x4 h1[2][4], h2[2][4];
+    prop_layer<N1>(t.a1, lane, [&](int s, int j) TFH_INLINE { return f[s][j]; }, h1);
+    prop_relu(t.b1, kq, h1);
+    prop_layer<16>(t.a2, lane, [&](int s, int j) TFH_INLINE { return h1[s][j >> 2][j & 3]; }, h2);
+    prop_relu(t.b2, kq, h2);
+    f32x4 o[2];
+    zero_acc(o);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const float4 av = t.a3[g][lane];
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, h2[s][g][0], o[s], 0, 0, 0);
+        o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, h2[s][g][1], o[s], 0, 0, 0);
+        o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, h2[s][g][2], o[s], 0, 0, 0);
+        o[s] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, h2[s][g][3], o[s], 0, 0, 0);
+      }
+    }
+    // rows 0 and 4 of the output tile are the output: lanes 0 .. 15 take the
+    // first set's, lanes 16 .. 31 the second's
+    const float zv = (lane < 16 ? o[0][0] : o[1][0]) + w.b3[0];
+    const int64_t row = row0 + lane;
+    if (lane < kPRows && row < M) {
       if (z) z[row] = zv;
       sigma[row] = softplus(zv);
     }
@@ -324,13 +473,41 @@ static PropW to_pw(const tfh_prop_mlp* p) {
   return PropW{p->w1, p->b1, p->w2, p->b2, p->w3, p->b3, (int)p->feat_dim};
 }
 
+static unsigned prop_fwd_blocks(int64_t M) {
+  return (unsigned)std::min<int64_t>(ceil_div(M, kPFwdNW * kPRows), 2 * (int64_t)prop_num_cus());
+}
+
 int32_t prop_mlp_fwd(const tfh_prop_mlp* p, const float* feats, int64_t M, float* z, float* sigma,
                      hipStream_t st) {
   if (M == 0) return TFH_OK;
   ProfScope ps("prop_mlp_fwd", st);
-  hipLaunchKernelGGL(k_prop_mlp_fwd, dim3((unsigned)ceil_div(M, kPTM)), dim3(kPNW * 64), 0, st,
-                     to_pw(p), feats, M, z, sigma);
+  auto kernel = p->feat_dim <= 24 ? k_prop_mlp_fwd<6, false> : k_prop_mlp_fwd<8, false>;
+  hipLaunchKernelGGL(kernel, dim3(prop_fwd_blocks(M)), dim3(kPFwdNW * 64), 0, st, to_pw(p),
+                     const_cast<float*>(feats), tfh_vm{}, nullptr, M, z, sigma);
   return check_launch("proposal mlp fwd");
+}
+
+// The features of the field at pts (M, 3) to feats and the MLP on them: one
+// kernel for 8 channels behind 16-byte aligned pointers, the gather and the
+// MLP by themselves otherwise.
+int32_t prop_mlp_fwd_gather(const tfh_prop_mlp* p, const tfh_vm& field, const float* pts,
+                            int64_t M, float* feats, float* sigma, hipStream_t st) {
+  if (M == 0) return TFH_OK;
+  const uintptr_t any = reinterpret_cast<uintptr_t>(field.plane) |
+                        reinterpret_cast<uintptr_t>(field.line) |
+                        reinterpret_cast<uintptr_t>(feats);
+  if (field.channels == 8 && p->feat_dim == 24 && (any & 15) == 0) {
+    ProfScope ps("prop_mlp_fwd", st);
+    hipLaunchKernelGGL((k_prop_mlp_fwd<6, true>), dim3(prop_fwd_blocks(M)), dim3(kPFwdNW * 64), 0,
+                       st, to_pw(p), feats, field, pts, M, nullptr, sigma);
+    return check_launch("proposal mlp fwd with the gather");
+  }
+  {
+    ProfScope ps("prop_gather", st);
+    const RaySamples src{pts, nullptr, 1, 1};
+    TFH_TRY((launch_vm_gather<RaySamples, true>(field, src, M, feats, st)));
+  }
+  return prop_mlp_fwd(p, feats, M, nullptr, sigma, st);
 }
 
 size_t prop_mlp_bwd_workspace(const tfh_prop_mlp* p, int64_t M) {
