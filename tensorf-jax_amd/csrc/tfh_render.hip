@@ -90,7 +90,6 @@ __device__ float wave_topk(const uint32_t* key, const float* s_w, int n, int k,
 
 struct DensityOut {
   float* pts;    // (R*N, 3) normalised points
-  float* ts;     // (R*N) or null
   float* sigma;  // (R*N)
   float* delta;  // (R*N)
   float* w;      // (R*N)
@@ -100,14 +99,25 @@ struct DensityOut {
   float* out;    // (R) distance outputs
 };
 
-__global__ void __launch_bounds__(64) k_density_pass(tfh_vm dvm, RayIn in, DensityOut o) {
-  extern __shared__ float sm[];
+// One wave per ray, 64 samples at a time, a lane each: point, taps and (last)
+// softplus and weights; in between LPS lanes gather a sample's channels, four
+// each (WIDE; else 16 lanes and 4-byte taps), with the taps handed over from
+// the sample's lane. Its 18 16-byte taps a sample bound it: the L1 is busy for
+// 82% of the 940 us that the median distance of 65536 rays x 512 samples takes
+// (16 channels; the vector ALUs for 78%). With the point, the taps, the 64-bit
+// tap addresses and the softplus computed by every lane of a group that took
+// 1694 us (2.1 M samples of a training step: 130 us, now 89; 4.2 M: 277, 218).
+// Eight waves per SIMD spill (1191 us), seven take 1031, six 962, four 956.
+//
+// Distance modes write nothing but the distance; the median needs no sample
+// past the one where it is reached.
+template <int LPS, bool WIDE>
+__global__ void __launch_bounds__(64, 5) k_density_pass(tfh_vm dvm, RayIn in, DensityOut o) {
+  extern __shared__ float sm[];  // keys and weights of the top-k selection (k < N)
+  constexpr int SPS = 64 / LPS;  // samples per step
   const int64_t r = blockIdx.x;
   const int lane = threadIdx.x;
   const int N = in.N;
-  float* s_a = sm;       // a_i = sigma_i * delta_i  (later: top-k keys)
-  float* s_e = sm + N;   // E_i
-  float* s_w = s_e + N;  // w_i
   const float ox = in.o[3 * r], oy = in.o[3 * r + 1], oz = in.o[3 * r + 2];
   const float dx = in.d[3 * r], dy = in.d[3 * r + 1], dz = in.d[3 * r + 2];
   float t0 = 0.f, step = 0.f;
@@ -116,132 +126,143 @@ __global__ void __launch_bounds__(64) k_density_pass(tfh_vm dvm, RayIn in, Densi
   const float a0x = in.aabb[0], a0y = in.aabb[1], a0z = in.aabb[2];
   const float a1x = in.aabb[3], a1y = in.aabb[4], a1z = in.aabb[5];
   const int G = (int)dvm.grid_dim, C = (int)dvm.channels;
-  // 16-byte taps when the channels allow: lps lanes per sample (C/4 rounded
-  // up to a power of two), 64/lps samples per step; else 16 lanes and
-  // 4-byte taps
-  const bool wide = in.wide_taps;
-  const int lps = !wide ? 16 : (C <= 8 ? 2 : (C <= 16 ? 4 : (C <= 32 ? 8 : 16)));
-  const int gs = lane / lps, ls = lane % lps;
+  const int gs = lane / LPS, ls = lane % LPS;
+  const bool rgb = in.mode == TFH_MODE_RGB, select = rgb && in.k < N;
+  float carry = 0.0f;    // log of the transmittance before the chunk
+  float e_last = 0.0f;   // E_{N-1}
+  float wsum = 0.0f;     // the lane's share of the weights' sum (RGB, k == N) or mean distance
+  float depth = INFINITY;
 
-  for (int i0 = 0; i0 < N; i0 += 64 / lps) {
-    const int i = i0 + gs;
+  for (int c0 = 0; c0 < N; c0 += 64) {
+    const int i = c0 + lane;
     const bool act = i < N;
     float t = 0.f, dlt = 0.f, px = 0.f, py = 0.f, pz = 0.f;
     if (act) sample_point(in, r, i, ox, oy, oz, dx, dy, dz, t0, step, t, dlt, px, py, pz);
     const float xh = normalise(px, a0x, a1x), yh = normalise(py, a0y, a1y),
                 zh = normalise(pz, a0z, a1z);
-    ModeTaps mt[3];
-    mode_taps(xh, yh, zh, G, mt);
-    float acc = 0.0f;
+    const PackedTap tx = pack_tap(lin_tap(xh, G)), ty = pack_tap(lin_tap(yh, G)),
+                    tz = pack_tap(lin_tap(zh, G));
+    float feat = 0.0f;  // sum over the 3C channels of sample i
+    for (int u = 0; u < LPS && c0 + u * SPS < N; ++u) {
+      const int from = u * SPS + gs;
+      const PackedTap sx = shfl_tap(tx, from), sy = shfl_tap(ty, from), sz = shfl_tap(tz, from);
+      // (v, a, b) of each mode (ModeTaps)
+      const PackedTap* const tv[3] = {&sx, &sz, &sy};
+      const PackedTap* const ta[3] = {&sy, &sx, &sz};
+      const PackedTap* const tb[3] = {&sz, &sy, &sx};
+      float acc = 0.0f;
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
-      TapAddr a;
-      tap_addrs(mt[m], m, G, a);
-      if (wide) {
-        if (act && 4 * ls < C) {
-          float4 lv, pv;
-          tap_values4(dvm.plane, dvm.line, C, 4 * ls, a, lv, pv);
-          acc += lv.x * pv.x;
-          acc += lv.y * pv.y;
-          acc += lv.z * pv.z;
-          acc += lv.w * pv.w;
-        }
-      } else {
+      for (int m = 0; m < 3; ++m) {
+        if constexpr (WIDE) {
+          if (4 * ls < C) {
+            float4 lv, pv;
+            tap_values4(dvm.plane + (size_t)m * G * G * C, dvm.line + (size_t)m * G * C, G, 4 * C,
+                        16 * ls, *tv[m], *ta[m], *tb[m], lv, pv);
+            acc += lv.x * pv.x;
+            acc += lv.y * pv.y;
+            acc += lv.z * pv.z;
+            acc += lv.w * pv.w;
+          }
+        } else {
+          TapAddr a;
+          tap_addrs(ModeTaps{unpack_tap(*tv[m]), unpack_tap(*ta[m]), unpack_tap(*tb[m])}, m, G, a);
 #pragma unroll
-        for (int q = 0; q < kMaxQ; ++q) {
-          const int c = ls + 16 * q;
-          if (c < C && act) {
-            float lv, pv;
-            tap_values(dvm.plane, dvm.line, C, c, a, lv, pv);
-            acc += lv * pv;
+          for (int q = 0; q < kMaxQ; ++q) {
+            const int c = ls + 16 * q;
+            if (c < C) {
+              float lv, pv;
+              tap_values(dvm.plane, dvm.line, C, c, a, lv, pv);
+              acc += lv * pv;
+            }
           }
         }
       }
+      // sum over the sample's lanes, and to the sample's own
+#pragma unroll
+      for (int w = 1; w < LPS; w <<= 1) acc += __shfl_xor(acc, w, 64);
+      const float v = __shfl(acc, (lane % SPS) * LPS, 64);
+      if (lane / SPS == u) feat = v;
     }
-    // sum over the 3C channels: the sample's lps lanes
-    for (int o = 1; o < lps; o <<= 1) acc += __shfl_xor(acc, o, 64);
-    if (act && ls == 0) {
-      const float sig = softplus(acc + in.density_shift);  // render.py:207 (+10 there)
-      s_a[i] = sig * dlt;                          // render.py:322
-      const int64_t s = r * N + i;
-      o.sigma[s] = sig;
-      o.delta[s] = dlt;
-      if (o.ts) o.ts[s] = t;
-      o.pts[3 * s] = xh;
-      o.pts[3 * s + 1] = yh;
-      o.pts[3 * s + 2] = zh;
+    const float sig = softplus(feat + in.density_shift);  // render.py:207 (+10 there)
+    // p_exits and p_terminates as wave_segment_probs forms them
+    const float neg = act ? -(sig * dlt) : 0.0f;  // render.py:322
+    const float incl = wave_incl_scan(neg) + carry;
+    float prev = __shfl_up(incl, 1, 64);
+    if (lane == 0) prev = carry;
+    carry = __shfl(incl, 63, 64);
+    const float e = expf(incl), w = (1.0f - expf(neg)) * expf(prev);
+    e_last = __shfl(e, (N - 1) & 63, 64);  // the last chunk's is kept
+    if (rgb) {
+      if (act) {
+        const int64_t s = r * N + i;
+        o.sigma[s] = sig;
+        o.delta[s] = dlt;
+        o.pts[3 * s] = xh;
+        o.pts[3 * s + 1] = yh;
+        o.pts[3 * s + 2] = zh;
+        o.w[s] = w;
+        o.e[s] = e;
+        wsum += w;
+        if (select) {
+          // appearance sample selection (render.py:459-470)
+          reinterpret_cast<uint32_t*>(sm)[i] =
+              in.gumbel ? float_key(logf(w) + in.gumbel[i]) : float_key(w);
+          sm[N + i] = w;
+        }
+      }
+    } else if (in.mode == TFH_MODE_DIST_MEAN) {  // render.py:269-276
+      if (act) wsum += w * t;
+      if (i == N - 1) wsum += e * t;
+    } else if (in.mode == TFH_MODE_DIST_MEDIAN) {  // render.py:248-267
+      const uint64_t past = __ballot(act && (1.0f - e) > 0.5f);
+      if (past) {
+        const int first = __builtin_ctzll(past);
+        depth = c0 + first == 0 ? 0.0f : __shfl(t, first, 64);
+        break;
+      }
     }
   }
-  __syncthreads();
-  wave_segment_probs(s_a, s_e, s_w, N);
-  __syncthreads();
-  for (int i = lane; i < N; i += 64) {
-    o.w[r * N + i] = s_w[i];
-    o.e[r * N + i] = s_e[i];
-  }
-  const float e_last = s_e[N - 1];
-
-  if (in.mode == TFH_MODE_DIST_MEAN) {  // render.py:269-276
-    float acc = 0.0f;
-    for (int i = lane; i < N; i += 64) {
-      float t, dlt, px, py, pz;
-      sample_point(in, r, i, ox, oy, oz, dx, dy, dz, t0, step, t, dlt, px, py, pz);
-      acc += s_w[i] * t;
-      if (i == N - 1) acc += e_last * t;
-    }
-    acc = wave_sum(acc);
-    if (lane == 0) o.out[r] = acc;
-    return;
-  }
-  if (in.mode == TFH_MODE_DIST_MEDIAN_AS_WRITTEN) {
+  if (!rgb) {
+    if (in.mode == TFH_MODE_DIST_MEAN) depth = wave_sum(wsum);
     // render.py:250-266 as written: sum(mask * [ts, +inf]) with mask[N] =
     // (1 - E_{N-1} <= 0.5); the last column is 0 * inf = NaN or 1 * inf, and
     // the finite columns cannot undo either.
-    if (lane == 0) o.out[r] = (1.0f - e_last) > 0.5f ? NAN : INFINITY;
+    if (in.mode == TFH_MODE_DIST_MEDIAN_AS_WRITTEN)
+      depth = (1.0f - e_last) > 0.5f ? NAN : INFINITY;
+    if (lane == 0) o.out[r] = depth;
     return;
   }
-  if (in.mode == TFH_MODE_DIST_MEDIAN) {  // render.py:248-267
-    int first = N;
-    for (int c0 = 0; c0 < N && first == N; c0 += 64) {
-      const int i = c0 + lane;
-      const uint64_t m = __ballot(i < N && (1.0f - s_e[i]) > 0.5f);
-      if (m) first = c0 + __builtin_ctzll(m);
-    }
-    if (lane == 0) {
-      float depth;
-      if (first == N) {
-        depth = INFINITY;
-      } else if (first == 0) {
-        depth = 0.0f;
-      } else {
-        float t, dlt, px, py, pz;
-        sample_point(in, r, first, ox, oy, oz, dx, dy, dz, t0, step, t, dlt, px, py, pz);
-        depth = t;
-      }
-      o.out[r] = depth;
-    }
-    return;
-  }
-  // RGB: appearance sample selection (render.py:459-470) and unbiasing terms
   float ssum;
-  if (in.k < N) {
-    uint32_t* key = reinterpret_cast<uint32_t*>(s_a);
-    for (int i = lane; i < N; i += 64) {
-      const float wv = s_w[i];
-      key[i] = in.gumbel ? float_key(logf(wv) + in.gumbel[i]) : float_key(wv);
-    }
+  if (select) {
     __syncthreads();
-    ssum = wave_topk(key, s_w, N, in.k, o.idx + r * in.k);
+    ssum = wave_topk(reinterpret_cast<uint32_t*>(sm), sm + N, N, in.k, o.idx + r * in.k);
   } else {
-    float acc = 0.0f;
-    for (int i = lane; i < N; i += 64) acc += s_w[i];
-    ssum = wave_sum(acc);
+    ssum = wave_sum(wsum);
   }
   if (lane == 0) {
     o.ray[4 * r] = e_last;
     o.ray[4 * r + 1] = ssum;
     o.ray[4 * r + 2] = (1.0f - e_last + 1e-8f) / (ssum + 1e-8f);  // render.py:537-546
   }
+}
+
+// 16-byte taps with C/4 lanes (rounded up to a power of two) per sample where
+// the channels, the alignment and 32-bit offsets into a mode's plane allow.
+static int32_t launch_density_pass(const tfh_vm& vm, const RayIn& in, const DensityOut& o,
+                                   hipStream_t st) {
+  const int64_t C = vm.channels;
+  const bool wide = C % 4 == 0 && C <= 64 && (reinterpret_cast<uintptr_t>(vm.plane) & 15) == 0 &&
+                    (reinterpret_cast<uintptr_t>(vm.line) & 15) == 0 &&
+                    vm.grid_dim * vm.grid_dim * C * 4 < (1ll << 32);
+  auto kernel = !wide     ? k_density_pass<16, false>
+                : C <= 8  ? k_density_pass<2, true>
+                : C <= 16 ? k_density_pass<4, true>
+                : C <= 32 ? k_density_pass<8, true>
+                          : k_density_pass<16, true>;
+  const bool select = in.mode == TFH_MODE_RGB && in.k < in.N;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)in.R), dim3(64),
+                     select ? 2 * in.N * sizeof(float) : 0, st, vm, in, o);
+  return check_launch("render: density pass");
 }
 
 // C = U * sum_j w_{i_j} c_j + E_{N-1} (render.py:233-244). With colors != null
@@ -559,7 +580,7 @@ static size_t carve_render(Carve& cv, const tfh_render_config* cfg, const tfh_ml
   const int64_t N = cfg->density_samples_per_ray, k = cfg->appearance_samples_per_ray;
   const int64_t M = R * k;
   ws.d.pts = cv.take<float>(R * N * 3);
-  ws.d.ts = cv.take<float>(R * N);
+  cv.take<float>(R * N);  // (unused)
   ws.d.sigma = cv.take<float>(R * N);
   ws.d.delta = cv.take<float>(R * N);
   ws.d.w = cv.take<float>(R * N);
@@ -669,14 +690,8 @@ static int32_t render_forward(const tfh_vm* density, const tfh_vm* appearance, c
   dout.out = out;
   {
   ProfScope ps("density_pass", st);
-  RayIn din = in;
-  din.wide_taps = density->channels % 4 == 0 && density->channels <= 64 &&
-                  (reinterpret_cast<uintptr_t>(density->plane) & 15) == 0 &&
-                  (reinterpret_cast<uintptr_t>(density->line) & 15) == 0;
-  hipLaunchKernelGGL(k_density_pass, dim3((unsigned)R), dim3(64), 3 * N * sizeof(float), st,
-                     *density, din, dout);
+  TFH_TRY(launch_density_pass(*density, in, dout, st));
   }
-  TFH_TRY(check_launch("render: density pass"));
   if (cfg->mode != TFH_MODE_RGB) return TFH_OK;
   const int64_t M = R * k;
   RaySamples src{ws.d.pts, ws.d.idx, k, N};
@@ -850,7 +865,7 @@ static size_t carve_render_fwd(Carve& cv, const tfh_render_config* cfg, const tf
   const int64_t N = cfg->density_samples_per_ray, k = cfg->appearance_samples_per_ray;
   const int64_t M = R * k;
   ws.d.pts = cv.take<float>(R * N * 3);
-  ws.d.ts = cv.take<float>(R * N);
+  cv.take<float>(R * N);  // (unused)
   ws.d.sigma = cv.take<float>(R * N);
   ws.d.delta = cv.take<float>(R * N);
   ws.d.w = cv.take<float>(R * N);

@@ -76,6 +76,59 @@ __device__ __forceinline__ void tap_values4(const float* __restrict__ plane,
   pv.w = ((a.w00 * t00.w + a.w01 * t01.w) + a.w10 * t10.w) + a.w11 * t11.w;
 }
 
+// A coordinate's taps in two registers, to be handed from the lane that
+// computed them to others: the lower texel doubled, plus 1 when the upper one
+// is the next (0: the same, at the grid's edge), and the upper weight.
+struct PackedTap {
+  int i;
+  float w1;
+};
+
+__device__ __forceinline__ PackedTap pack_tap(const Tap& t) {
+  return PackedTap{2 * t.i0 + (t.i1 - t.i0), t.w1};
+}
+
+__device__ __forceinline__ PackedTap shfl_tap(const PackedTap& t, int lane) {
+  return PackedTap{__shfl(t.i, lane, 64), __shfl(t.w1, lane, 64)};
+}
+
+__device__ __forceinline__ Tap unpack_tap(const PackedTap& t) {
+  return Tap{t.i >> 1, (t.i >> 1) + (t.i & 1), 1.0f - t.w1, t.w1};
+}
+
+// tap_values4 from packed taps of a mode whose factors start at plane and
+// line: texels of `bytes` bytes at 32-bit offsets (the mode's plane is under
+// 4 GB), c the byte offset of the lane's four channels. The same arithmetic.
+__device__ __forceinline__ void tap_values4(const float* __restrict__ plane,
+                                            const float* __restrict__ line, unsigned g,
+                                            unsigned bytes, unsigned c, const PackedTap& v,
+                                            const PackedTap& a, const PackedTap& b, float4& lv,
+                                            float4& pv) {
+  const auto at = [](const float* base, unsigned off) __attribute__((always_inline)) {
+    return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(base) + off);
+  };
+  const unsigned o0 = (unsigned)(v.i >> 1) * bytes + c;
+  const unsigned o00 = ((unsigned)(a.i >> 1) * g + (unsigned)(b.i >> 1)) * bytes + c;
+  const unsigned db = (b.i & 1) ? bytes : 0u;
+  const unsigned o10 = o00 + ((a.i & 1) ? g * bytes : 0u);
+  const float4 l0 = at(line, o0);
+  const float4 l1 = at(line, o0 + ((v.i & 1) ? bytes : 0u));
+  const float4 t00 = at(plane, o00);
+  const float4 t01 = at(plane, o00 + db);
+  const float4 t10 = at(plane, o10);
+  const float4 t11 = at(plane, o10 + db);
+  const float vw0 = 1.0f - v.w1, aw0 = 1.0f - a.w1, bw0 = 1.0f - b.w1;
+  const float w00 = aw0 * bw0, w01 = aw0 * b.w1, w10 = a.w1 * bw0, w11 = a.w1 * b.w1;
+  lv.x = vw0 * l0.x + v.w1 * l1.x;
+  lv.y = vw0 * l0.y + v.w1 * l1.y;
+  lv.z = vw0 * l0.z + v.w1 * l1.z;
+  lv.w = vw0 * l0.w + v.w1 * l1.w;
+  pv.x = ((w00 * t00.x + w01 * t01.x) + w10 * t10.x) + w11 * t11.x;
+  pv.y = ((w00 * t00.y + w01 * t01.y) + w10 * t10.y) + w11 * t11.y;
+  pv.z = ((w00 * t00.z + w01 * t01.z) + w10 * t10.z) + w11 * t11.z;
+  pv.w = ((w00 * t00.w + w01 * t01.w) + w10 * t10.w) + w11 * t11.w;
+}
+
 // Adds `val` at dst[key*C + c] once per distinct `key` among the 64/LPS
 // groups of LPS lanes of the wave (all lanes of the wave must call it
 // together): each group sums the values of the groups with its key in the
