@@ -623,6 +623,9 @@ __global__ void __launch_bounds__(256) k_line_walk(Src src, int g, int64_t pairs
   typename QuadOf<FA, 2>::T la(fa, copy_of(fa, g), l, gl0);
   typename LaneOf<FD, 2>::T ld(fd, copy_of(fd, g), l, gl0);
   int cur = -1, t0 = 0, t1 = 0;
+  int cell = -1;  // the plane cell whose values are in a and d
+  float4 a[4];
+  float d[4];
   for (int64_t b0 = first; b0 < last; b0 += LPS) {
     const int64_t e = b0 + l;
     PairTaps mine{};
@@ -641,23 +644,26 @@ __global__ void __launch_bounds__(256) k_line_walk(Src src, int g, int64_t pairs
     const int nb = (int)min((int64_t)LPS, last - b0);
     for (int j = 0; j < nb; ++j) {
       const PairTaps p = shfl_pair(mine, gl0 + j);
-      const int p00 = p.kp >> 2, p01 = p00 + (p.kp & 1);
-      const int p10 = p00 + ((p.kp >> 1) & 1) * g, p11 = p10 + (p.kp & 1);
-      float4 a[4], ag;
-      float d[4], dg;
-      if constexpr (A) {
-        a[0] = la.load(fa.vm.plane, p00);
-        a[1] = la.load(fa.vm.plane, p01);
-        a[2] = la.load(fa.vm.plane, p10);
-        a[3] = la.load(fa.vm.plane, p11);
-        ag = la.grad(p.pk);
-      }
-      if constexpr (D) {
-        d[0] = ld.load(fd.vm.plane, p00);
-        d[1] = ld.load(fd.vm.plane, p01);
-        d[2] = ld.load(fd.vm.plane, p10);
-        d[3] = ld.load(fd.vm.plane, p11);
-        dg = ld.grad(p.pk);
+      float4 ag;
+      float dg;
+      if constexpr (A) ag = la.grad(p.pk);
+      if constexpr (D) dg = ld.grad(p.pk);
+      if (p.kp != cell) {
+        const int p00 = p.kp >> 2, p01 = p00 + (p.kp & 1);
+        const int p10 = p00 + ((p.kp >> 1) & 1) * g, p11 = p10 + (p.kp & 1);
+        if constexpr (A) {
+          a[0] = la.load(fa.vm.plane, p00);
+          a[1] = la.load(fa.vm.plane, p01);
+          a[2] = la.load(fa.vm.plane, p10);
+          a[3] = la.load(fa.vm.plane, p11);
+        }
+        if constexpr (D) {
+          d[0] = ld.load(fd.vm.plane, p00);
+          d[1] = ld.load(fd.vm.plane, p01);
+          d[2] = ld.load(fd.vm.plane, p10);
+          d[3] = ld.load(fd.vm.plane, p11);
+        }
+        cell = p.kp;
       }
       if (p.kl != cur) {
         const int n0 = p.kl >> 1, n1 = n0 + (p.kl & 1);

@@ -2,7 +2,7 @@
 densities that choose between the scatter's walks: 16 lanes of four channels,
 16 or 8 lanes of one, and the general passes (more than 16 channels, not a
 multiple of 4); both fields in one walk, or each its own (top-k); line cells in
-ray order (more samples than grid cells) or sorted. Against the float64 oracle,
+ray order or (few samples for the grid) sorted. Against the float64 oracle,
 2e-4 of the largest gradient (the order of the FP32 sums), as in the other
 gradient tests."""
 import numpy as np
@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("contraction", [False, True])
-@pytest.mark.parametrize("n,k", [(41, 41), (41, 7), (9, 9), (9, 4)])
+@pytest.mark.parametrize("n,k", [(41, 41), (41, 7), (9, 9), (9, 4), (7, 7)])
 @pytest.mark.parametrize("cd,ca", [(8, 24), (5, 20), (1, 17), (16, 48), (13, 64), (24, 8),
                                    (18, 16)])
 def test_factor_gradients(cd, ca, n, k, contraction):
