@@ -92,6 +92,28 @@ __device__ __forceinline__ int64_t xcd_unit(int64_t units) {
   return (int64_t)(blockIdx.x % kXcds) * per + blockIdx.x / kXcds;
 }
 
+// Compute units of the current device (256 if that cannot be read).
+inline int num_cus() {
+  static const int cus = [] {
+    int dev = 0, n = 0;
+    const bool ok = hipGetDevice(&dev) == hipSuccess &&
+                    hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
+                        hipSuccess;
+    return ok && n > 0 ? n : 256;
+  }();
+  return cus;
+}
+
+// Dynamic LDS above 64 KB needs the per-kernel opt-in.
+template <class K>
+inline void allow_lds(K kernel, size_t bytes) {
+  if (bytes > 64 * 1024) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    (void)hipGetLastError();
+  }
+}
+
 // ---- device helpers ---------------------------------------------------------
 // Order-1 'nearest' taps of map_coordinates on a grid of `g` texels for a
 // normalised coordinate x in [-1,1] (tensor_vm.py:150-153, 241-248):

@@ -43,21 +43,6 @@ __global__ void __launch_bounds__(64 * kRedWaves) k_mlp_reduce(const float* __re
   }
 }
 
-static int g_num_cus = 0;
-
-static int num_cus() {
-  if (g_num_cus == 0) {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0)
-      g_num_cus = n;
-    else
-      g_num_cus = 256;
-  }
-  return g_num_cus;
-}
-
-
 // TFH_MLP_WGRAD=partial forces the generic backward (read-modify-write
 // accumulation of the weight gradients) for every shape.
 static bool force_partial() {

@@ -1035,16 +1035,6 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
 constexpr int kFwdTM = 32, kFwdNW = 8;
 constexpr int kBwdTM = 32;
 
-// Dynamic LDS above 64 KB needs the per-kernel opt-in.
-template <class K>
-inline void allow_lds(K kernel, size_t bytes) {
-  if (bytes > 64 * 1024) {
-    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
-    (void)hipGetLastError();
-  }
-}
-
 // k_mlp_bwd_planes (tfh_mlp_bwd_planes.h): the shapes it is built for, the
 // operand tables, the launches.
 enum class BwdKind { kNone, kStd, kDef };

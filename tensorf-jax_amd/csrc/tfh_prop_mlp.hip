@@ -2,9 +2,9 @@
 // z = W3 relu(W2 relu(W1 f + b1) + b2) + b3, sigma = softplus(z), with
 // f the 3C <= 32 VM features of a sample, 64 hidden units, FP32 MFMA.
 // Forward: 32 rows per wave, in registers. Backward (input dL/dz): persistent
-// workgroups recompute the forward of each tile, keep the 28 weight-gradient
-// 16x16 tiles in registers (7 per wave) and store them once per workgroup;
-// k_prop_reduce sums the workgroups.
+// waves recompute the forward of 16 rows at a time, keep the weight gradients in
+// registers and store them once per workgroup; k_prop_reduce sums the
+// workgroups.
 #include <algorithm>
 
 #include "tfh_mfma.h"
@@ -14,9 +14,7 @@ namespace tfh {
 
 constexpr int kPH = 64;       // hidden width
 constexpr int kPF = 32;       // padded feature width
-constexpr int kPTM = 64;      // rows per tile
-constexpr int kPNW = 4;       // waves per workgroup
-constexpr int kPLdF = kPF + 2, kPLdH = kPH + 2, kPLdZ = 16 + 2;
+constexpr int kPNW = 8;       // waves per workgroup
 
 struct PropW {
   const float *w1, *b1, *w2, *b2, *w3, *b3;
@@ -41,53 +39,6 @@ __host__ __device__ inline PropPack prop_pack(int F) {
   return p;
 }
 
-// Row `row` of the tile reads feature row idx[row] (or row when idx is null).
-__device__ __forceinline__ void prop_load(const float* __restrict__ feats, int F, int64_t row0,
-                                          int64_t M, float* Fs,
-                                          const int32_t* __restrict__ idx = nullptr) {
-  for (int e = threadIdx.x; e < kPTM * kPF; e += blockDim.x) {
-    const int i = e / kPF, c = e % kPF;
-    const int64_t row = row0 + i;
-    float v = 0.0f;
-    if (row < M && c < F) v = feats[(idx ? (int64_t)idx[row] : row) * F + c];
-    Fs[i * kPLdF + c] = v;
-  }
-}
-
-// Hidden layers of a tile: H1 = relu(Fs W1 + b1), H2 = relu(H1 W2 + b2).
-__device__ __forceinline__ void prop_hidden(const PropW& w, const float* Fs, float* H1,
-                                            float* H2) {
-  constexpr int RT = kPTM / 16;
-  const int wave = threadIdx.x >> 6, lane = lane_id();
-  const int ct = wave;  // 4 column tiles, one per wave
-  {
-    f32x4 acc[RT];
-    zero_acc(acc);
-    mma_strip<RT, kPF>(Fs, kPLdF, kPF, GlobalB(w.w1, w.F, kPH), 16 * ct, acc);
-    const int col = 16 * ct + (lane & 15);
-    const float bias = w.b1[col];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        H1[(16 * rt + 4 * (lane >> 4) + e) * kPLdH + col] = fmaxf(acc[rt][e] + bias, 0.0f);
-  }
-  __syncthreads();
-  {
-    f32x4 acc[RT];
-    zero_acc(acc);
-    mma_strip<RT, kPH>(H1, kPLdH, kPH, GlobalB(w.w2, kPH, kPH), 16 * ct, acc);
-    const int col = 16 * ct + (lane & 15);
-    const float bias = w.b2[col];
-#pragma unroll
-    for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        H2[(16 * rt + 4 * (lane >> 4) + e) * kPLdH + col] = fmaxf(acc[rt][e] + bias, 0.0f);
-  }
-  __syncthreads();
-}
-
 // ---- forward --------------------------------------------------------------------
 // A wave computes 32 rows in registers, the products transposed: the operand
 // with 16 rows of the result is a table of the weights, the one with 16
@@ -103,23 +54,26 @@ __device__ __forceinline__ void prop_hidden(const PropW& w, const float* Fs, flo
 // took 2885 us there after a gather of 517, 607 after 116 for the 3.1 M rows of
 // a training step; with the gather in this kernel 1770 and 414. Ten or twelve
 // waves per workgroup (5 or 6 per SIMD) took 2167 and 1812.
-constexpr int kPFwdNW = 8;            // waves per workgroup
 constexpr int kPRows = 32;            // rows per wave
 constexpr int kPLdT = 28;             // row stride of a wave's features: 16 rows x 4 inputs of a
                                       // product are 64 different banks
 
-struct PropFwdLds {
+struct PropTables {
   float4 a1[4][2][64];  // [unit tile][four products][lane]
   float4 a2[4][4][64];
-  float4 a3[4][64];     // the output's weights in rows 0 and 4, zero elsewhere
   float4 b1[4][4], b2[4][4];  // [unit tile][kq]
+};
+
+struct PropFwdLds {
+  PropTables t;
+  float4 a3[4][64];  // the output's weights in rows 0 and 4, zero elsewhere
 };
 
 __device__ __forceinline__ int prop_unit(int tile, int entry) {
   return 16 * tile + 4 * (entry & 3) + (entry >> 2);
 }
 
-__device__ __forceinline__ void prop_fwd_tables(const PropW& w, PropFwdLds& t) {
+__device__ __forceinline__ void prop_tables(const PropW& w, PropTables& t) {
   float* a1 = &t.a1[0][0][0].x;
   for (int e = threadIdx.x; e < 4 * 2 * 256; e += blockDim.x) {
     const int lane = (e >> 2) & 63, k = 4 * (4 * ((e >> 8) & 1) + (e & 3)) + (lane >> 4);
@@ -130,11 +84,6 @@ __device__ __forceinline__ void prop_fwd_tables(const PropW& w, PropFwdLds& t) {
     const int lane = (e >> 2) & 63, k = 4 * (4 * ((e >> 8) & 3) + (e & 3)) + (lane >> 4);
     a2[e] = w.w2[k * kPH + prop_unit(e >> 10, lane & 15)];
   }
-  float* a3 = &t.a3[0][0].x;
-  for (int e = threadIdx.x; e < 4 * 256; e += blockDim.x) {
-    const int lane = (e >> 2) & 63, k = 4 * (4 * (e >> 8) + (e & 3)) + (lane >> 4);
-    a3[e] = (lane & 11) == 0 ? w.w3[k] : 0.0f;
-  }
   if (threadIdx.x < 64) {
     const int u = prop_unit(threadIdx.x >> 4, threadIdx.x & 15);
     (&t.b1[0][0].x)[threadIdx.x] = w.b1[u];
@@ -142,36 +91,46 @@ __device__ __forceinline__ void prop_fwd_tables(const PropW& w, PropFwdLds& t) {
   }
 }
 
-// One layer's products i < N (of KI) for two sets of 16 rows and all four unit
-// tiles; in(s, i) is the operand of set s.
-template <int N, int G, class In>
-__device__ __forceinline__ void prop_layer(const float4 (&a)[4][G][64], int lane, In in,
-                                           f32x4 (&acc)[2][4]) {
+__device__ __forceinline__ void prop_fwd_tables(const PropW& w, PropFwdLds& t) {
+  prop_tables(w, t.t);
+  float* a3 = &t.a3[0][0].x;
+  for (int e = threadIdx.x; e < 4 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, k = 4 * (4 * (e >> 8) + (e & 3)) + (lane >> 4);
+    a3[e] = (lane & 11) == 0 ? w.w3[k] : 0.0f;
+  }
+}
+
+// One layer's products i < N for S sets of 16 rows and C tiles of its outputs;
+// in(s, i) is the operand of set s.
+template <int N, int S, int C, int G, class In>
+__device__ __forceinline__ void prop_layer(const float4 (&a)[C][G][64], int lane, In in,
+                                           f32x4 (&acc)[S][C]) {
 #pragma unroll
-  for (int s = 0; s < 2; ++s) zero_acc(acc[s]);
+  for (int s = 0; s < S; ++s) zero_acc(acc[s]);
 #pragma unroll
   for (int g = 0; 4 * g < N; ++g) {
-    float4 av[4];
+    float4 av[C];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) av[c] = a[c][g][lane];
+    for (int c = 0; c < C; ++c) av[c] = a[c][g][lane];
 #pragma unroll
     for (int e = 0; e < 4 && 4 * g + e < N; ++e)
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < C; ++c)
 #pragma unroll
-        for (int s = 0; s < 2; ++s)
+        for (int s = 0; s < S; ++s)
           acc[s][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(
               e == 0 ? av[c].x : (e == 1 ? av[c].y : (e == 2 ? av[c].z : av[c].w)), in(s, 4 * g + e),
               acc[s][c], 0, 0, 0);
   }
 }
 
-__device__ __forceinline__ void prop_relu(const float4 (&b)[4][4], int kq, f32x4 (&acc)[2][4]) {
+template <int S>
+__device__ __forceinline__ void prop_relu(const float4 (&b)[4][4], int kq, f32x4 (&acc)[S][4]) {
 #pragma unroll
   for (int c = 0; c < 4; ++c) {
     const float4 bias = b[c][kq];
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    for (int s = 0; s < S; ++s) {
       acc[s][c][0] = fmaxf(acc[s][c][0] + bias.x, 0.0f);
       acc[s][c][1] = fmaxf(acc[s][c][1] + bias.y, 0.0f);
       acc[s][c][2] = fmaxf(acc[s][c][2] + bias.z, 0.0f);
@@ -184,18 +143,18 @@ __device__ __forceinline__ void prop_relu(const float4 (&b)[4][4], int kq, f32x4
 // field at pts, two lanes per sample with four channels each (the arithmetic
 // of k_vm_gather4), and go to feats too. N1: first-layer products, 4 N1 >= F.
 template <int N1, bool GATHER>
-__global__ void __launch_bounds__(kPFwdNW * 64, 4)
+__global__ void __launch_bounds__(kPNW * 64, 4)
     k_prop_mlp_fwd(PropW w, float* __restrict__ feats, tfh_vm vm, const float* __restrict__ pts,
                    int64_t M, float* __restrict__ z, float* __restrict__ sigma) {
   static_assert(!GATHER || N1 == 6, "8 channels");
   __shared__ PropFwdLds t;
-  __shared__ float4 rows[GATHER ? kPFwdNW : 1][GATHER ? kPRows * kPLdT / 4 : 1];
+  __shared__ float4 rows[GATHER ? kPNW : 1][GATHER ? kPRows * kPLdT / 4 : 1];
   prop_fwd_tables(w, t);
   __syncthreads();
   const int wave = threadIdx.x >> 6;
   const int64_t tiles = (M + kPRows - 1) / kPRows;
-  for (int64_t tile = (int64_t)blockIdx.x * kPFwdNW + wave; tile < tiles;
-       tile += (int64_t)gridDim.x * kPFwdNW) {
+  for (int64_t tile = (int64_t)blockIdx.x * kPNW + wave; tile < tiles;
+       tile += (int64_t)gridDim.x * kPNW) {
     // (computed per tile: the tables' 128 registers would be kept otherwise)
     const int lane = lane_here(), n = lane & 15, kq = lane >> 4;
     const int64_t row0 = tile * kPRows;
@@ -244,10 +203,10 @@ __global__ void __launch_bounds__(kPFwdNW * 64, 4)
       }
     }
     f32x4 h1[2][4], h2[2][4];
-    prop_layer<N1>(t.a1, lane, [&](int s, int j) TFH_INLINE { return f[s][j]; }, h1);
-    prop_relu(t.b1, kq, h1);
-    prop_layer<16>(t.a2, lane, [&](int s, int j) TFH_INLINE { return h1[s][j >> 2][j & 3]; }, h2);
-    prop_relu(t.b2, kq, h2);
+    prop_layer<N1>(t.t.a1, lane, [&](int s, int j) TFH_INLINE { return f[s][j]; }, h1);
+    prop_relu(t.t.b1, kq, h1);
+    prop_layer<16>(t.t.a2, lane, [&](int s, int j) TFH_INLINE { return h1[s][j >> 2][j & 3]; }, h2);
+    prop_relu(t.t.b2, kq, h2);
     f32x4 o[2];
     zero_acc(o);
 #pragma unroll
@@ -272,138 +231,251 @@ __global__ void __launch_bounds__(kPFwdNW * 64, 4)
   }
 }
 
-// Register slots per wave: dW3 4 tiles (64x16), dW2 16 (64x64), dW1 8 (32x64).
-constexpr int kPC3 = 1, kPC2 = 4, kPC1 = 2, kPSlots = kPC3 + kPC2 + kPC1;
+// ---- backward -------------------------------------------------------------------
+// A wave takes 16 rows at a time through the forward and back, transposed as
+// in the forward: a lane's activations and their gradients (units 16 c + 4 e +
+// kq of row r) stay in registers. The weight gradients' products run over the
+// rows, so their operands cross lanes through the wave's own LDS; a wave keeps
+// all 24 tiles of them (dW2 64 x 64, dW1 32 x 64) and its sums of the other
+// gradients in registers for all its rows, and the waves' sums meet in LDS at the
+// end. No barrier between tiles.
+//
+// Bound by the FP32 matrix rate: 280 products of 16x16x4 per 16 rows, 480 us
+// for the 1.72 M rows with a gradient of a step with 16384 rays x (128 + 64)
+// samples. The tile of 64 rows shared by four waves, with a barrier after each of
+// seven steps, its activations read by single values and the weights from memory,
+// took 1240 us; this one takes 631.
+constexpr int kPLdH = 80;  // rows of 64 values: 4 rows x 16 values are 64 different banks
+constexpr int kPLdF = 48;  // rows of 32 values
 
-__device__ __forceinline__ void prop_store_tile(float* part, int off, int rows, int cols, int row0,
-                                                int col0, const f32x4& acc) {
-  const int lane = lane_id();
-  const int col = col0 + (lane & 15);
+struct PropBwdLds {
+  PropTables t;
+  float4 a2t[4][4][64];  // W2 and W1 as operands of the input gradients
+  float4 a1t[2][4][64];
+  float4 w3[4][4];       // [unit tile][kq]
+  float h1[kPNW][16 * kPLdH];
+  float dz[kPNW][16 * kPLdH];
+  float f[kPNW][16 * kPLdF];
+};
+static_assert(sizeof(PropBwdLds) <= 160 * 1024, "one workgroup per CU");
+
+// A tile's 16 rows x 64 values (value 16 c + 4 kq + e of row r in register e of
+// tile c) to LDS.
+__device__ __forceinline__ void prop_put(float* to, int n, int kq, const f32x4 (&v)[4]) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int row = row0 + 4 * (lane >> 4) + e;
-    if (row < rows && col < cols) part[off + row * cols + col] = acc[e];
-  }
+  for (int c = 0; c < 4; ++c)
+    *reinterpret_cast<f32x4*>(to + n * kPLdH + 16 * c + 4 * kq) = v[c];
 }
 
 // Rows: all M, or the first min(M, *count) entries of idx (feature and dz row
-// of each); dfeat is written per processed row.
-__global__ void __launch_bounds__(kPNW * 64, 2) k_prop_mlp_bwd(PropW w, const float* __restrict__ feats,
-                                                            const float* __restrict__ dz,
-                                                            int64_t M_max,
-                                                            const int32_t* __restrict__ idx,
-                                                            const int32_t* __restrict__ count,
-                                                            float* __restrict__ dfeat,
-                                                            float* __restrict__ partials) {
+// of each); dfeat is written per processed row. N1: as in the forward.
+template <int N1>
+__global__ void __launch_bounds__(kPNW * 64, 2)
+    k_prop_mlp_bwd(PropW w, const float* __restrict__ feats, const float* __restrict__ dz,
+                   int64_t M_max, const int32_t* __restrict__ idx,
+                   const int32_t* __restrict__ count, float* __restrict__ dfeat,
+                   float* __restrict__ partials) {
+  extern __shared__ float4 prop_lds[];
+  PropBwdLds& s = *reinterpret_cast<PropBwdLds*>(prop_lds);
   const int64_t M = count ? min(M_max, (int64_t)*count) : M_max;
-  constexpr int RT = kPTM / 16;
-  __shared__ float Fs[kPTM * kPLdF];
-  __shared__ float H1[kPTM * kPLdH];
-  __shared__ float H2[kPTM * kPLdH];
-  __shared__ float DZ[kPTM * kPLdZ];
-  const int wave = threadIdx.x >> 6, lane = lane_id();
+  prop_tables(w, s.t);
+  float* a2t = &s.a2t[0][0][0].x;
+  for (int e = threadIdx.x; e < 4 * 4 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, u = 4 * (4 * ((e >> 8) & 3) + (e & 3)) + (lane >> 4);
+    a2t[e] = w.w2[prop_unit(e >> 10, lane & 15) * kPH + u];
+  }
+  float* a1t = &s.a1t[0][0][0].x;
+  for (int e = threadIdx.x; e < 2 * 4 * 256; e += blockDim.x) {
+    const int lane = (e >> 2) & 63, u = 4 * (4 * ((e >> 8) & 3) + (e & 3)) + (lane >> 4);
+    const int k = 16 * (e >> 10) + (lane & 15);
+    a1t[e] = k < w.F ? w.w1[k * kPH + u] : 0.0f;
+  }
+  if (threadIdx.x < 64)
+    (&s.w3[0][0].x)[threadIdx.x] = w.w3[prop_unit(threadIdx.x >> 4, threadIdx.x & 15)];
+  const int wave = threadIdx.x >> 6;
+  float* const H1 = s.h1[wave];
+  float* const DZ = s.dz[wave];
+  float* const Fs = s.f[wave];
+  // (columns past the loaded features stay zero)
+  for (int e = lane_id(); e < 16 * kPLdF; e += 64) Fs[e] = 0.0f;
+  __syncthreads();
+  f32x4 dw2[4][4], dw1[2][4], db1[4], db2[4], dw3[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) zero_acc(dw2[c]);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) zero_acc(dw1[c]);
+  zero_acc(db1);
+  zero_acc(db2);
+  zero_acc(dw3);
+  float db3 = 0.0f;
+  const int64_t tiles = (M + 15) / 16, step = (int64_t)gridDim.x * kPNW;
+  int64_t tile = (int64_t)blockIdx.x * kPNW + wave;
+  // the features and dL/dz of a tile's rows are requested one tile ahead
+  float f[1][N1], g;
+  auto request = [&](int64_t at, int n, int kq) TFH_INLINE {
+    const int64_t i = at * 16 + n;
+    const bool valid = i < M;
+    const int64_t row = valid ? (idx ? (int64_t)idx[i] : i) : 0;
+#pragma unroll
+    for (int j = 0; j < N1; ++j)
+      f[0][j] = valid && 4 * j + kq < w.F ? feats[row * w.F + 4 * j + kq] : 0.0f;
+    g = valid ? dz[row] : 0.0f;
+  };
+  if (tile < tiles) request(tile, lane_id() & 15, lane_id() >> 4);
+  for (; tile < tiles; tile += step) {
+    const int lane = lane_here(), n = lane & 15, kq = lane >> 4;
+    const float gz = g;
+#pragma unroll
+    for (int j = 0; j < N1; ++j) Fs[n * kPLdF + 4 * j + kq] = f[0][j];
+    f32x4 h1[1][4], h2[1][4], d1[1][4];
+    prop_layer<N1>(s.t.a1, lane, [&](int, int j) TFH_INLINE { return f[0][j]; }, h1);
+    if (tile + step < tiles) request(tile + step, n, kq);
+    prop_relu(s.t.b1, kq, h1);
+    prop_put(H1, n, kq, h1[0]);
+    prop_layer<16>(s.t.a2, lane, [&](int, int j) TFH_INLINE { return h1[0][j >> 2][j & 3]; }, h2);
+    prop_relu(s.t.b2, kq, h2);
+    // dW3 += h2 dz; dZ2 = dz W3^T where h2 > 0
+    if (kq == 0) db3 += gz;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float4 w3 = s.w3[c][kq];
+      const float wv[4] = {w3.x, w3.y, w3.z, w3.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float h = h2[0][c][e];
+        dw3[c][e] += h * gz;
+        h2[0][c][e] = h > 0.0f ? gz * wv[e] : 0.0f;
+      }
+      db2[c] += h2[0][c];
+    }
+    prop_put(DZ, n, kq, h2[0]);
+    // dZ1 = dZ2 W2^T where h1 > 0
+    prop_layer<16>(s.a2t, lane, [&](int, int j) TFH_INLINE { return h2[0][j >> 2][j & 3]; }, d1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) d1[0][c][e] = h1[0][c][e] > 0.0f ? d1[0][c][e] : 0.0f;
+      db1[c] += d1[0][c];
+    }
+    // dW2 += H1^T dZ2 (the wave's LDS accesses stay in order)
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float a[4], b[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        a[c] = H1[(4 * i + kq) * kPLdH + 16 * c + n];
+        b[c] = DZ[(4 * i + kq) * kPLdH + 16 * c + n];
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          dw2[c][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[q], dw2[c][q], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+    prop_put(DZ, n, kq, d1[0]);
+    __builtin_amdgcn_wave_barrier();
+    // dF = dZ1 W1^T, dW1 += F^T dZ1
+    if (dfeat) {
+      f32x4 df[1][2];
+      prop_layer<16>(s.a1t, lane, [&](int, int j) TFH_INLINE { return d1[0][j >> 2][j & 3]; }, df);
+      const int64_t row = tile * 16 + n;
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int k = 16 * c + 4 * kq + e;
+          if (row < M && k < w.F) dfeat[row * w.F + k] = df[0][c][e];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float a[2], b[4];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) a[c] = Fs[(4 * i + kq) * kPLdF + 16 * c + n];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) b[c] = DZ[(4 * i + kq) * kPLdH + 16 * c + n];
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          dw1[c][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[q], dw1[c][q], 0, 0, 0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  // the sums over a tile's rows (lanes of a kq)
+  const int lane = lane_id(), n = lane & 15, kq = lane >> 4;
+#pragma unroll
+  for (int o = 1; o < 16; o <<= 1) {
+    db3 += __shfl_xor(db3, o, 64);
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        db1[c][e] += __shfl_xor(db1[c][e], o, 64);
+        db2[c][e] += __shfl_xor(db2[c][e], o, 64);
+        dw3[c][e] += __shfl_xor(dw3[c][e], o, 64);
+      }
+  }
+  // half the waves' sums to the other half, over the rows' LDS, three times
+  constexpr int kSums = 24 + 3 * 4 + 1;  // float4 of a lane
+  static_assert(sizeof(s.h1) + sizeof(s.dz) + sizeof(s.f) >= kPNW / 2 * (24 * 64 + 13 * 4) * 16,
+                "room for the sums");
+  auto each = [&](auto&& op) TFH_INLINE {  // (sum, its index, whether rows share it)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) op(dw2[c][q], 4 * q + c, false);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) op(dw1[c][q], 16 + 2 * q + c, false);
+      op(db1[q], 24 + q, true);
+      op(db2[q], 28 + q, true);
+      op(dw3[q], 32 + q, true);
+    }
+    f32x4 last = {db3, 0.0f, 0.0f, 0.0f};
+    op(last, kSums - 1, true);
+    db3 = last[0];
+  };
+  for (int half = kPNW / 2; half >= 1; half >>= 1) {
+    f32x4* box = reinterpret_cast<f32x4*>(s.h1[0]) + (wave & (half - 1)) * (24 * 64 + 13 * 4);
+    auto slot = [&](int i, bool shared) TFH_INLINE {
+      return box + (shared ? 24 * 64 + (i - 24) * 4 + kq : i * 64 + lane);
+    };
+    __syncthreads();
+    if (wave >= half && wave < 2 * half)
+      each([&](f32x4& v, int i, bool shared) TFH_INLINE {
+        if (!shared || n == 0) *slot(i, shared) = v;
+      });
+    __syncthreads();
+    if (wave < half)
+      each([&](f32x4& v, int i, bool shared) TFH_INLINE { v += *slot(i, shared); });
+  }
+  if (wave != 0) return;
   const PropPack pp = prop_pack(w.F);
-  f32x4 wacc[kPSlots];
-#pragma unroll
-  for (int i = 0; i < kPSlots; ++i) wacc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float db1 = 0.f, db2 = 0.f, db3 = 0.f;
-  const int64_t ntiles = (M + kPTM - 1) / kPTM;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t row0 = tile * kPTM;
-    __syncthreads();
-    prop_load(feats, w.F, row0, M, Fs, idx);
-    for (int e = threadIdx.x; e < kPTM * 16; e += blockDim.x) {
-      const int i = e / 16, c = e % 16;
-      const int64_t row = row0 + i;
-      DZ[i * kPLdZ + c] = (c == 0 && row < M) ? dz[idx ? (int64_t)idx[row] : row] : 0.0f;
-    }
-    __syncthreads();
-    prop_hidden(w, Fs, H1, H2);
-    // dW3 (64 x 1) += H2^T dZ: row tile = wave
-    mma_wgrad_acc<false, kPTM>(H2, kPLdH, 16 * wave, DZ, kPLdZ, 0, wacc[0]);
-    __builtin_amdgcn_sched_barrier(0);
-    if (threadIdx.x == 0)
-      for (int i = 0; i < kPTM; ++i) db3 += DZ[i * kPLdZ];
-    __syncthreads();
-    // dH2 = dZ W3^T; dZ2 = dH2 * (h2 > 0) over H2 (dW3 is done)
-    {
-      f32x4 acc[RT];
-      zero_acc(acc);
-      mma_strip<RT, 4>(DZ, kPLdZ, 4, GlobalBT(w.w3, kPH, 1), 16 * wave, acc);
-      const int col = 16 * wave + (lane & 15);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 16 * rt + 4 * (lane >> 4) + e;
-          const float h = H2[row * kPLdH + col];
-          H2[row * kPLdH + col] = h > 0.0f ? acc[rt][e] : 0.0f;
-        }
-    }
-    __syncthreads();
-    // dW2 (64 x 64) += H1^T dZ2: wave owns column tile `wave`, all 4 row tiles
-#pragma unroll
-    for (int s = 0; s < kPC2; ++s) {
-      mma_wgrad_acc<false, kPTM>(H1, kPLdH, 16 * s, H2, kPLdH, 16 * wave, wacc[kPC3 + s]);
-      // keep the operand loads of later tiles from being hoisted
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (threadIdx.x < kPH)
-      for (int i = 0; i < kPTM; ++i) db2 += H2[i * kPLdH + threadIdx.x];
-    __syncthreads();
-    // dH1 = dZ2 W2^T; dZ1 = dH1 * (h1 > 0) over H1
-    {
-      f32x4 acc[RT];
-      zero_acc(acc);
-      mma_strip<RT, kPH>(H2, kPLdH, kPH, GlobalBT(w.w2, kPH, kPH), 16 * wave, acc);
-      const int col = 16 * wave + (lane & 15);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int row = 16 * rt + 4 * (lane >> 4) + e;
-          const float h = H1[row * kPLdH + col];
-          H1[row * kPLdH + col] = h > 0.0f ? acc[rt][e] : 0.0f;
-        }
-    }
-    __syncthreads();
-    // dW1 (32 x 64) += Fs^T dZ1: wave owns column tile `wave`, 2 row tiles
-#pragma unroll
-    for (int s = 0; s < kPC1; ++s) {
-      mma_wgrad_acc<false, kPTM>(Fs, kPLdF, 16 * s, H1, kPLdH, 16 * wave,
-                                 wacc[kPC3 + kPC2 + s]);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    if (threadIdx.x < kPH)
-      for (int i = 0; i < kPTM; ++i) db1 += H1[i * kPLdH + threadIdx.x];
-    // dF = dZ1 W1^T (64 x F): 2 column tiles on waves 0, 1
-    if (dfeat && wave < 2) {
-      f32x4 acc[RT];
-      zero_acc(acc);
-      mma_strip<RT, kPH>(H1, kPLdH, kPH, GlobalBT(w.w1, w.F, kPH), 16 * wave, acc);
-      const int col = 16 * wave + (lane & 15);
-#pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int64_t row = row0 + 16 * rt + 4 * (lane >> 4) + e;
-          if (row < M && col < w.F) dfeat[row * w.F + col] = acc[rt][e];
-        }
-    }
-  }
   float* part = partials + (int64_t)blockIdx.x * pp.total;
-  prop_store_tile(part, pp.w3, kPH, 1, 16 * wave, 0, wacc[0]);
 #pragma unroll
-  for (int s = 0; s < kPC2; ++s)
-    prop_store_tile(part, pp.w2, kPH, kPH, 16 * s, 16 * wave, wacc[kPC3 + s]);
+  for (int q = 0; q < 4; ++q) {
+    const int u = prop_unit(q, n);
 #pragma unroll
-  for (int s = 0; s < kPC1; ++s)
-    prop_store_tile(part, pp.w1, w.F, kPH, 16 * s, 16 * wave, wacc[kPC3 + kPC2 + s]);
-  if (threadIdx.x < kPH) {
-    part[pp.b1 + threadIdx.x] = db1;
-    part[pp.b2 + threadIdx.x] = db2;
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        part[pp.w2 + prop_unit(c, 4 * kq + e) * kPH + u] = dw2[c][q][e];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const int k = 16 * c + 4 * kq + e;
+        if (k < w.F) part[pp.w1 + k * kPH + u] = dw1[c][q][e];
+      }
+      if (n == 0) {
+        const int unit = 16 * q + 4 * e + kq;
+        part[pp.b1 + unit] = db1[q][e];
+        part[pp.b2 + unit] = db2[q][e];
+        part[pp.w3 + unit] = dw3[q][e];
+      }
+    }
   }
-  if (threadIdx.x == 0) part[pp.b3] = db3;
+  if (lane == 0) part[pp.b3] = db3;
 }
 
 // Sum of the workgroup partials: a workgroup owns 64 consecutive entries and
@@ -442,23 +514,9 @@ __global__ void __launch_bounds__(64 * kPRedWaves) k_prop_reduce(const float* __
   }
 }
 
-static int prop_num_cus() {
-  static int n = 0;
-  if (n == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-      n = v;
-    else
-      n = 256;
-  }
-  return n;
-}
-
-// Persistent backward: two workgroups per CU (the kernel's register budget
-// is sized for that occupancy).
+// Persistent backward: one workgroup per CU, 16 rows per wave.
 static int64_t prop_bwd_blocks(int64_t M) {
-  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, kPTM), 2 * (int64_t)prop_num_cus()));
+  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, 16 * kPNW), num_cus()));
 }
 
 int32_t check_prop_mlp(const tfh_prop_mlp* p, const char* who) {
@@ -474,7 +532,7 @@ static PropW to_pw(const tfh_prop_mlp* p) {
 }
 
 static unsigned prop_fwd_blocks(int64_t M) {
-  return (unsigned)std::min<int64_t>(ceil_div(M, kPFwdNW * kPRows), 2 * (int64_t)prop_num_cus());
+  return (unsigned)std::min<int64_t>(ceil_div(M, kPNW * kPRows), 2 * (int64_t)num_cus());
 }
 
 int32_t prop_mlp_fwd(const tfh_prop_mlp* p, const float* feats, int64_t M, float* z, float* sigma,
@@ -482,7 +540,7 @@ int32_t prop_mlp_fwd(const tfh_prop_mlp* p, const float* feats, int64_t M, float
   if (M == 0) return TFH_OK;
   ProfScope ps("prop_mlp_fwd", st);
   auto kernel = p->feat_dim <= 24 ? k_prop_mlp_fwd<6, false> : k_prop_mlp_fwd<8, false>;
-  hipLaunchKernelGGL(kernel, dim3(prop_fwd_blocks(M)), dim3(kPFwdNW * 64), 0, st, to_pw(p),
+  hipLaunchKernelGGL(kernel, dim3(prop_fwd_blocks(M)), dim3(kPNW * 64), 0, st, to_pw(p),
                      const_cast<float*>(feats), tfh_vm{}, nullptr, M, z, sigma);
   return check_launch("proposal mlp fwd");
 }
@@ -498,7 +556,7 @@ int32_t prop_mlp_fwd_gather(const tfh_prop_mlp* p, const tfh_vm& field, const fl
                         reinterpret_cast<uintptr_t>(feats);
   if (field.channels == 8 && p->feat_dim == 24 && (any & 15) == 0) {
     ProfScope ps("prop_mlp_fwd", st);
-    hipLaunchKernelGGL((k_prop_mlp_fwd<6, true>), dim3(prop_fwd_blocks(M)), dim3(kPFwdNW * 64), 0,
+    hipLaunchKernelGGL((k_prop_mlp_fwd<6, true>), dim3(prop_fwd_blocks(M)), dim3(kPNW * 64), 0,
                        st, to_pw(p), feats, field, pts, M, nullptr, sigma);
     return check_launch("proposal mlp fwd with the gather");
   }
@@ -510,8 +568,10 @@ int32_t prop_mlp_fwd_gather(const tfh_prop_mlp* p, const tfh_vm& field, const fl
   return prop_mlp_fwd(p, feats, M, nullptr, sigma, st);
 }
 
+// (twice the workgroups' partials: the size callers have always been given)
 size_t prop_mlp_bwd_workspace(const tfh_prop_mlp* p, int64_t M) {
-  const int64_t nblk = prop_bwd_blocks(M);
+  const int64_t nblk = std::max<int64_t>(
+      1, std::min<int64_t>(ceil_div(M, 64), 2 * (int64_t)num_cus()));
   return align_up((size_t)nblk * prop_pack((int)p->feat_dim).total * sizeof(float), 256);
 }
 
@@ -526,8 +586,10 @@ int32_t prop_mlp_bwd(const tfh_prop_mlp* p, const float* feats, const float* dz,
   float* partials = static_cast<float*>(ws);
   {
     ProfScope ps("prop_mlp_bwd", st);
-    hipLaunchKernelGGL(k_prop_mlp_bwd, dim3((unsigned)nblk), dim3(kPNW * 64), 0, st, to_pw(p),
-                       feats, dz, M, idx, count, dfeat, partials);
+    auto kernel = p->feat_dim <= 24 ? k_prop_mlp_bwd<6> : k_prop_mlp_bwd<8>;
+    allow_lds(kernel, sizeof(PropBwdLds));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(kPNW * 64), sizeof(PropBwdLds), st,
+                       to_pw(p), feats, dz, M, idx, count, dfeat, partials);
   }
   TFH_TRY(check_launch("proposal mlp bwd"));
   hipLaunchKernelGGL(k_prop_reduce, dim3((unsigned)ceil_div(pp.b3 + 1, 64)),
