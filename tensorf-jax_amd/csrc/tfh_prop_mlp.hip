@@ -244,7 +244,7 @@ __global__ void __launch_bounds__(kPNW * 64, 4)
 // for the 1.72 M rows with a gradient of a step with 16384 rays x (128 + 64)
 // samples. The tile of 64 rows shared by four waves, with a barrier after each of
 // seven steps, its activations read by single values and the weights from memory,
-// took 1240 us; this one takes 631.
+// took 1240 us; this one takes 573.
 constexpr int kPLdH = 80;  // rows of 64 values: 4 rows x 16 values are 64 different banks
 constexpr int kPLdF = 48;  // rows of 32 values
 
