@@ -155,6 +155,11 @@ int32_t tfh_vm_interpolate(const tfh_vm* vm, const float* ijk, int64_t num_point
 int32_t tfh_vm_interpolate_bwd(const tfh_vm* vm, const float* ijk, int64_t num_points,
                                const float* grad_out, const tfh_vm_grad* grad,
                                tfh_stream_t stream);
+/* Clears num (at most 16) arrays of counts[i] floats in one launch: the
+ * gradients a *_bwd call accumulates into. No counterpart in the reference. */
+int32_t tfh_zero_arrays(float* const* arrays, const int64_t* counts, int32_t num,
+                        tfh_stream_t stream);
+
 /* TensorVM.resize (tensor_vm.py:91-100, 183-223): align-corners linear
  * upsampling to grid_dim_out >= G. Also used for the Adam moments
  * (training.py:257-275). out_plane (3,G',G',C), out_line (3,G',C). */

@@ -78,6 +78,38 @@ __global__ void __launch_bounds__(256) k_zero_copies(float* __restrict__ p, int6
   }
 }
 
+// Several arrays in one launch: workgroup b clears kZeroChunk floats of the
+// array whose chunks it falls in (each a launch of its own took 4 us of host time
+// per array, 12 arrays for a render's gradients).
+constexpr int kZeroArrays = 16;
+constexpr int64_t kZeroChunk = 16384;
+struct ZeroList {
+  float* p[kZeroArrays];
+  int64_t n[kZeroArrays];
+};
+
+__global__ void __launch_bounds__(256) k_zero_arrays(ZeroList z) {
+  int64_t b = blockIdx.x;
+  int i = 0;
+  for (; i < kZeroArrays - 1; ++i) {
+    const int64_t chunks = (z.n[i] + kZeroChunk - 1) / kZeroChunk;
+    if (b < chunks) break;
+    b -= chunks;
+  }
+  const int64_t e0 = b * kZeroChunk, e1 = min(e0 + kZeroChunk, z.n[i]);
+  float* p = z.p[i];
+  if ((reinterpret_cast<uintptr_t>(p) & 15) == 0) {
+    for (int64_t e = e0 + threadIdx.x * 4; e < e1; e += 1024) {
+      if (e + 4 <= e1)
+        *reinterpret_cast<float4*>(p + e) = make_float4(0.f, 0.f, 0.f, 0.f);
+      else
+        for (int64_t j = e; j < e1; ++j) p[j] = 0.0f;
+    }
+  } else {
+    for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) p[e] = 0.0f;
+  }
+}
+
 // A workgroup adds up 64 consecutive entries at a time; its kSumWaves waves
 // split the copies (wave w adds copies w, w + kSumWaves, ...), so every load
 // is one coalesced 256-byte segment, and the waves' sums meet in LDS in a
@@ -153,6 +185,25 @@ int32_t tfh_vm_interpolate_bwd(const tfh_vm* vm, const float* ijk, int64_t num_p
   PlanarPoints src{ijk, num_points};
   return launch_vm_scatter<PlanarPoints, false>(*vm, src, num_points, grad_out, *grad,
                                                 as_stream(stream));
+}
+
+int32_t tfh_zero_arrays(float* const* arrays, const int64_t* counts, int32_t num,
+                        tfh_stream_t stream) {
+  TFH_REQUIRE(num >= 0 && num <= kZeroArrays, "tfh_zero_arrays: %d arrays", num);
+  TFH_REQUIRE(num == 0 || (arrays && counts), "tfh_zero_arrays: null pointer");
+  ZeroList z{};
+  int64_t blocks = 0;
+  for (int i = 0; i < num; ++i) {
+    TFH_REQUIRE(counts[i] >= 0 && (arrays[i] || counts[i] == 0), "tfh_zero_arrays: array %d", i);
+    z.p[i] = arrays[i];
+    z.n[i] = counts[i];
+    blocks += ceil_div(counts[i], kZeroChunk);
+  }
+  if (blocks == 0) return TFH_OK;
+  TFH_REQUIRE(blocks < (1ll << 31), "tfh_zero_arrays: too many values");
+  TFH_TRY(require_device());
+  hipLaunchKernelGGL(k_zero_arrays, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), z);
+  return check_launch("tfh_zero_arrays");
 }
 
 int32_t tfh_vm_resize(const tfh_vm* vm, int64_t grid_dim_out, float* out_plane, float* out_line,

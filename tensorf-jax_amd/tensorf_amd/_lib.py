@@ -98,6 +98,7 @@ _SIGS = {
     "tfh_vm_from_channel_last": (c_i32, [c_p, c_p, c_i64, c_i64, c_p, c_p, c_p]),
     "tfh_vm_interpolate": (c_i32, [P(Vm), c_p, c_i64, c_p, c_p]),
     "tfh_vm_interpolate_bwd": (c_i32, [P(Vm), c_p, c_i64, c_p, P(VmGrad), c_p]),
+    "tfh_zero_arrays": (c_i32, [P(c_p), P(c_i64), c_i32, c_p]),
     "tfh_vm_resize": (c_i32, [P(Vm), c_i64, c_p, c_p, c_p]),
     "tfh_sample_bbox": (c_i32, [c_p, c_p, c_i64, c_p, c_i64, c_p, c_p, c_p, c_p, c_p]),
     "tfh_sample_contracted": (c_i32, [c_p, c_p, c_i64, c_i64, c_p, c_p, c_p, c_p, c_p, c_p,
@@ -192,6 +193,20 @@ def ptr(t) -> Optional[int]:
 def stream() -> int:
     import torch
     return torch.cuda.current_stream().cuda_stream
+
+
+def zeros_like(tensors):
+    """[torch.zeros_like(t) for t in tensors], cleared in one launch (float32
+    tensors on the current device; others one by one)."""
+    import torch
+    out = [torch.empty_like(t) for t in tensors]
+    if len(out) > 16 or not all(t.is_cuda and t.dtype is torch.float32 and t.is_contiguous()
+                                for t in out):
+        return [t.zero_() for t in out]
+    n = len(out)
+    call("tfh_zero_arrays", (c_p * n)(*[t.data_ptr() for t in out]),
+         (c_i64 * n)(*[t.numel() for t in out]), n, stream())
+    return out
 
 
 def device_count() -> int:

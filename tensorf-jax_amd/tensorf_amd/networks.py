@@ -139,7 +139,7 @@ class _MlpFn(torch.autograd.Function):
         cams = cams if ctx.has_cams else None
         mlp, params = ctx.mlp, ctx.params
         leaves = FeatureMlp.flat_leaves(params)
-        grads = [torch.zeros_like(t) for t in leaves]
+        grads = _lib.zeros_like(leaves)
         gf = torch.empty_like(f)
         st = mlp.c_struct(params, f.shape[1])
         g = _lib.MlpGrad(*[_lib.ptr(t) for t in grads], *([None] * (8 - len(grads))))

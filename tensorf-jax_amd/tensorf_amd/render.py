@@ -264,7 +264,7 @@ class _RenderEnv:
         gout = gout.contiguous()
         self._gout = gout  # keep the buffer alive across the asynchronous call
         leaves = self.leaves()
-        grads = [torch.zeros_like(t) for t in leaves]
+        grads = _lib.zeros_like(leaves)
         dg = _lib.VmGrad(_lib.ptr(grads[0]), _lib.ptr(grads[1]))
         ag = _lib.VmGrad(_lib.ptr(grads[2]), _lib.ptr(grads[3]))
         mg = _lib.MlpGrad(*[_lib.ptr(t) for t in grads[4:]], *([None] * (12 - len(grads))))
