@@ -2,7 +2,7 @@
 // functor maps a row to its normalised sample point:
 //   PlanarPoints  : ijk (3, M), component stride M (TensorVM.interpolate API)
 //   RaySamples    : pts (R*N, 3) interleaved, row = r*k + j selects sample
-//                   idx[r*k + j] (or j when idx == NULL) of ray r.
+//                   idx[r*k + j] (or j when idx == NULL, k == N) of ray r.
 // ROW_MAJOR selects a (M, 3C) feature layout (the MLP input) instead of the
 // reference's (3C, M).
 #pragma once
@@ -26,14 +26,14 @@ struct PlanarPoints {
 
 struct RaySamples {
   const float* pts;    // (R*N, 3)
-  const int32_t* idx;  // (R, k) or null
+  const int32_t* idx;  // (R, k), or null: every sample (k == n)
   int64_t k, n;
   __device__ __forceinline__ int64_t limit(int64_t M) const { return M; }
+  __device__ __forceinline__ const float* at(int64_t row) const {
+    return pts + (idx ? row / k * n + idx[row] : row) * 3;
+  }
   __device__ __forceinline__ void get(int64_t row, float& x, float& y, float& z) const {
-    const int64_t r = row / k;
-    const int64_t j = row - r * k;
-    const int64_t i = idx ? (int64_t)idx[row] : j;
-    const float* q = pts + (r * n + i) * 3;
+    const float* q = at(row);
     x = q[0];
     y = q[1];
     z = q[2];
