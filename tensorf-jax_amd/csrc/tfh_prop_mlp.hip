@@ -2,9 +2,9 @@
 // z = W3 relu(W2 relu(W1 f + b1) + b2) + b3, sigma = softplus(z), with
 // f the 3C <= 32 VM features of a sample, 64 hidden units, FP32 MFMA.
 // Forward: 32 rows per wave, in registers. Backward (input dL/dz): persistent
-// waves recompute the forward of 16 rows at a time, keep the weight gradients in
-// registers and store them once per workgroup; k_prop_reduce sums the
-// workgroups.
+// teams of four waves recompute the forward of 64 rows at a time, keep the weight
+// gradients in registers and store them once per team; k_prop_reduce sums the
+// teams.
 #include <algorithm>
 
 #include "tfh_mfma.h"
@@ -232,49 +232,83 @@ __global__ void __launch_bounds__(kPNW * 64, 4)
 }
 
 // ---- backward -------------------------------------------------------------------
-// A wave takes 16 rows at a time through the forward and back, transposed as
-// in the forward: a lane's activations and their gradients (units 16 c + 4 e +
-// kq of row r) stay in registers. The weight gradients' products run over the
-// rows, so their operands cross lanes through the wave's own LDS; a wave keeps
-// all 24 tiles of them (dW2 64 x 64, dW1 32 x 64) and its sums of the other
-// gradients in registers for all its rows, and the waves' sums meet in LDS at the
-// end. No barrier between tiles.
+// Four waves share a tile of 64 rows, 16 each through the forward and back,
+// transposed as in the forward: a lane's activations and their gradients (units
+// 16 c + 4 e + kq of row r) stay in registers. The products of the weight
+// gradients run over the rows, so their operands cross lanes through LDS, and
+// each wave sums a quarter of the 28 tiles (dW3 64 x 1, dW2 64 x 64, dW1 32 x 64) in
+// registers for all its tiles. A workgroup holds two such teams, which share
+// the weights' LDS. A team's tiles and the order of every sum are those that
+// its number (of two per CU) and the row order give: the gradients of a batch
+// do not change from run to run.
 //
-// Bound by the FP32 matrix rate: 280 products of 16x16x4 per 16 rows, 480 us
+// Bound by the FP32 matrix rate: 296 products of 16x16x4 per 16 rows, 510 us
 // for the 1.72 M rows with a gradient of a step with 16384 rays x (128 + 64)
-// samples. The tile of 64 rows shared by four waves, with a barrier after each of
-// seven steps, its activations read by single values and the weights from memory,
-// took 1240 us; this one takes 573.
-constexpr int kPLdH = 80;  // rows of 64 values: 4 rows x 16 values are 64 different banks
-constexpr int kPLdF = 48;  // rows of 32 values
+// samples. With the activations in LDS only, read by single values, the weights
+// from memory per tile and seven barriers it took 1240 us; this one takes 714.
+constexpr int kPTM = 64;   // rows per tile
+constexpr int kPLdH = 68;  // rows of 64 values: rows 0, 4, 8, 12 x 16 values are 64 banks
+
+// A team's LDS: activations and gradients of the tile's rows, value 16 c +
+// 4 kq + e of a row for unit 16 c + 4 e + kq.
+struct PropTeam {
+  float h1[kPTM * kPLdH];  // h1, then dZ1
+  float d2[kPTM * kPLdH];  // dZ2, then the features
+  float h2[kPTM * kPLdH];
+  float g[kPTM];           // dL/dz
+};
 
 struct PropBwdLds {
   PropTables t;
   float4 a2t[4][4][64];  // W2 and W1 as operands of the input gradients
   float4 a1t[2][4][64];
   float4 w3[4][4];       // [unit tile][kq]
-  float h1[kPNW][16 * kPLdH];
-  float dz[kPNW][16 * kPLdH];
-  float f[kPNW][16 * kPLdF];
+  PropTeam team[2];
 };
-static_assert(sizeof(PropBwdLds) <= 160 * 1024, "one workgroup per CU");
+static_assert(kPNW == 8 && sizeof(PropBwdLds) <= 160 * 1024, "two teams of four, one workgroup per CU");
 
-// A tile's 16 rows x 64 values (value 16 c + 4 kq + e of row r in register e of
-// tile c) to LDS.
+// A workgroup barrier that orders LDS only: loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// 16 rows x 64 values (value 16 c + 4 kq + e of row r in register e of tile c)
+// to LDS.
 __device__ __forceinline__ void prop_put(float* to, int n, int kq, const f32x4 (&v)[4]) {
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     *reinterpret_cast<f32x4*>(to + n * kPLdH + 16 * c + 4 * kq) = v[c];
 }
 
+// acc[c] += X[:, 16 c ..]^T Y[:, col ..] over a tile's rows, 4 kq + i of each 16
+// in product i.
+template <int C>
+__device__ __forceinline__ void prop_wgrad(const float* X, const float* Y, int col, int n, int kq,
+                                           f32x4 (&acc)[C]) {
+#pragma unroll
+  for (int k0 = 0; k0 < kPTM; k0 += 16) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = (k0 + 4 * kq + i) * kPLdH;
+      const float b = Y[row + col + n];
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(X[row + 16 * c + n], b, acc[c], 0, 0, 0);
+    }
+  }
+}
+
 // Rows: all M, or the first min(M, *count) entries of idx (feature and dz row
-// of each); dfeat is written per processed row. N1: as in the forward.
+// of each); dfeat is written per processed row. teams: the partials; workgroup
+// b's teams are 2b and 2b + 1. N1: as in the forward.
 template <int N1>
 __global__ void __launch_bounds__(kPNW * 64, 2)
     k_prop_mlp_bwd(PropW w, const float* __restrict__ feats, const float* __restrict__ dz,
                    int64_t M_max, const int32_t* __restrict__ idx,
                    const int32_t* __restrict__ count, float* __restrict__ dfeat,
-                   float* __restrict__ partials) {
+                   float* __restrict__ partials, int teams) {
   extern __shared__ float4 prop_lds[];
   PropBwdLds& s = *reinterpret_cast<PropBwdLds*>(prop_lds);
   const int64_t M = count ? min(M_max, (int64_t)*count) : M_max;
@@ -292,28 +326,23 @@ __global__ void __launch_bounds__(kPNW * 64, 2)
   }
   if (threadIdx.x < 64)
     (&s.w3[0][0].x)[threadIdx.x] = w.w3[prop_unit(threadIdx.x >> 4, threadIdx.x & 15)];
-  const int wave = threadIdx.x >> 6;
-  float* const H1 = s.h1[wave];
-  float* const DZ = s.dz[wave];
-  float* const Fs = s.f[wave];
-  // (columns past the loaded features stay zero)
-  for (int e = lane_id(); e < 16 * kPLdF; e += 64) Fs[e] = 0.0f;
+  const int wave = (threadIdx.x >> 6) & 3;  // of the team
+  PropTeam& tm = s.team[threadIdx.x >> 8];
+  const int team = 2 * blockIdx.x + (threadIdx.x >> 8);
   __syncthreads();
-  f32x4 dw2[4][4], dw1[2][4], db1[4], db2[4], dw3[4];
-#pragma unroll
-  for (int c = 0; c < 4; ++c) zero_acc(dw2[c]);
-#pragma unroll
-  for (int c = 0; c < 2; ++c) zero_acc(dw1[c]);
-  zero_acc(db1);
-  zero_acc(db2);
+  f32x4 dw3[1], dw2[4], dw1[2];
   zero_acc(dw3);
-  float db3 = 0.0f;
-  const int64_t tiles = (M + 15) / 16, step = (int64_t)gridDim.x * kPNW;
-  int64_t tile = (int64_t)blockIdx.x * kPNW + wave;
+  zero_acc(dw2);
+  zero_acc(dw1);
+  float db = 0.0f;   // lane u of wave 0: db2, of wave 1: db1 of value u
+  float db3 = 0.0f;  // wave 2
+  // the same number of rounds for both teams; a team past the end has no rows
+  const int64_t tiles = (M + kPTM - 1) / kPTM;
+  int64_t tile = team < teams ? team : tiles;
   // the features and dL/dz of a tile's rows are requested one tile ahead
   float f[1][N1], g;
   auto request = [&](int64_t at, int n, int kq) TFH_INLINE {
-    const int64_t i = at * 16 + n;
+    const int64_t i = at * kPTM + 16 * wave + n;
     const bool valid = i < M;
     const int64_t row = valid ? (idx ? (int64_t)idx[i] : i) : 0;
 #pragma unroll
@@ -321,66 +350,72 @@ __global__ void __launch_bounds__(kPNW * 64, 2)
       f[0][j] = valid && 4 * j + kq < w.F ? feats[row * w.F + 4 * j + kq] : 0.0f;
     g = valid ? dz[row] : 0.0f;
   };
-  if (tile < tiles) request(tile, lane_id() & 15, lane_id() >> 4);
-  for (; tile < tiles; tile += step) {
+  request(tile, lane_id() & 15, lane_id() >> 4);
+  for (int64_t first = 2 * blockIdx.x; first < tiles; first += teams, tile += teams) {
     const int lane = lane_here(), n = lane & 15, kq = lane >> 4;
+    const int row0 = 16 * wave * kPLdH;  // the wave's rows
+    float f0[1][N1];
     const float gz = g;
-#pragma unroll
-    for (int j = 0; j < N1; ++j) Fs[n * kPLdF + 4 * j + kq] = f[0][j];
     f32x4 h1[1][4], h2[1][4], d1[1][4];
-    prop_layer<N1>(s.t.a1, lane, [&](int, int j) TFH_INLINE { return f[0][j]; }, h1);
-    if (tile + step < tiles) request(tile + step, n, kq);
+#pragma unroll
+    for (int j = 0; j < N1; ++j) f0[0][j] = f[0][j];
+    prop_layer<N1>(s.t.a1, lane, [&](int, int j) TFH_INLINE { return f0[0][j]; }, h1);
+    request(tile + teams, n, kq);
     prop_relu(s.t.b1, kq, h1);
-    prop_put(H1, n, kq, h1[0]);
+    prop_put(tm.h1 + row0, n, kq, h1[0]);
     prop_layer<16>(s.t.a2, lane, [&](int, int j) TFH_INLINE { return h1[0][j >> 2][j & 3]; }, h2);
     prop_relu(s.t.b2, kq, h2);
-    // dW3 += h2 dz; dZ2 = dz W3^T where h2 > 0
-    if (kq == 0) db3 += gz;
+    prop_put(tm.h2 + row0, n, kq, h2[0]);
+    if (kq == 0) tm.g[16 * wave + n] = gz;
+    // dZ2 = dz W3^T where h2 > 0
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       const float4 w3 = s.w3[c][kq];
       const float wv[4] = {w3.x, w3.y, w3.z, w3.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float h = h2[0][c][e];
-        dw3[c][e] += h * gz;
-        h2[0][c][e] = h > 0.0f ? gz * wv[e] : 0.0f;
-      }
-      db2[c] += h2[0][c];
+      for (int e = 0; e < 4; ++e) h2[0][c][e] = h2[0][c][e] > 0.0f ? gz * wv[e] : 0.0f;
     }
-    prop_put(DZ, n, kq, h2[0]);
+    prop_put(tm.d2 + row0, n, kq, h2[0]);
+    lds_barrier();
+    // dW3 += h2^T dz, dW2 += h1^T dZ2
+#pragma unroll
+    for (int k0 = 0; k0 < kPTM; k0 += 16)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int row = k0 + 4 * kq + i;
+        dw3[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(tm.h2[row * kPLdH + 16 * wave + n],
+                                                      n == 0 ? tm.g[row] : 0.0f, dw3[0], 0, 0, 0);
+      }
+    prop_wgrad(tm.h1, tm.d2, 16 * wave, n, kq, dw2);
+    if (wave == 0) {
+#pragma unroll 16
+      for (int i = 0; i < kPTM; ++i) db += tm.d2[i * kPLdH + lane];
+    } else if (wave == 2) {
+#pragma unroll 16
+      for (int i = 0; i < kPTM; ++i) db3 += tm.g[i];
+    }
     // dZ1 = dZ2 W2^T where h1 > 0
     prop_layer<16>(s.a2t, lane, [&](int, int j) TFH_INLINE { return h2[0][j >> 2][j & 3]; }, d1);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int e = 0; e < 4; ++e) d1[0][c][e] = h1[0][c][e] > 0.0f ? d1[0][c][e] : 0.0f;
-      db1[c] += d1[0][c];
+    lds_barrier();
+    prop_put(tm.h1 + row0, n, kq, d1[0]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      tm.d2[row0 + n * kPLdH + 4 * j + kq] = j < N1 ? f0[0][j < N1 ? j : 0] : 0.0f;
+    lds_barrier();
+    // dW1 += F^T dZ1, dF = dZ1 W1^T
+    prop_wgrad(tm.d2, tm.h1, 16 * wave, n, kq, dw1);
+    if (wave == 1) {
+#pragma unroll 16
+      for (int i = 0; i < kPTM; ++i) db += tm.h1[i * kPLdH + lane];
     }
-    // dW2 += H1^T dZ2 (the wave's LDS accesses stay in order)
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float a[4], b[4];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        a[c] = H1[(4 * i + kq) * kPLdH + 16 * c + n];
-        b[c] = DZ[(4 * i + kq) * kPLdH + 16 * c + n];
-      }
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          dw2[c][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[q], dw2[c][q], 0, 0, 0);
-    }
-    __builtin_amdgcn_wave_barrier();
-    prop_put(DZ, n, kq, d1[0]);
-    __builtin_amdgcn_wave_barrier();
-    // dF = dZ1 W1^T, dW1 += F^T dZ1
     if (dfeat) {
       f32x4 df[1][2];
       prop_layer<16>(s.a1t, lane, [&](int, int j) TFH_INLINE { return d1[0][j >> 2][j & 3]; }, df);
-      const int64_t row = tile * 16 + n;
+      const int64_t row = tile * kPTM + 16 * wave + n;
 #pragma unroll
       for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -389,93 +424,27 @@ __global__ void __launch_bounds__(kPNW * 64, 2)
           if (row < M && k < w.F) dfeat[row * w.F + k] = df[0][c][e];
         }
     }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float a[2], b[4];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) a[c] = Fs[(4 * i + kq) * kPLdF + 16 * c + n];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) b[c] = DZ[(4 * i + kq) * kPLdH + 16 * c + n];
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-          dw1[c][q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[c], b[q], dw1[c][q], 0, 0, 0);
-    }
-    __builtin_amdgcn_wave_barrier();
+    lds_barrier();
   }
-  // the sums over a tile's rows (lanes of a kq)
+  if (team >= teams) return;
   const int lane = lane_id(), n = lane & 15, kq = lane >> 4;
-#pragma unroll
-  for (int o = 1; o < 16; o <<= 1) {
-    db3 += __shfl_xor(db3, o, 64);
-#pragma unroll
-    for (int c = 0; c < 4; ++c)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        db1[c][e] += __shfl_xor(db1[c][e], o, 64);
-        db2[c][e] += __shfl_xor(db2[c][e], o, 64);
-        dw3[c][e] += __shfl_xor(dw3[c][e], o, 64);
-      }
-  }
-  // half the waves' sums to the other half, over the rows' LDS, three times
-  constexpr int kSums = 24 + 3 * 4 + 1;  // float4 of a lane
-  static_assert(sizeof(s.h1) + sizeof(s.dz) + sizeof(s.f) >= kPNW / 2 * (24 * 64 + 13 * 4) * 16,
-                "room for the sums");
-  auto each = [&](auto&& op) TFH_INLINE {  // (sum, its index, whether rows share it)
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-#pragma unroll
-      for (int c = 0; c < 4; ++c) op(dw2[c][q], 4 * q + c, false);
-#pragma unroll
-      for (int c = 0; c < 2; ++c) op(dw1[c][q], 16 + 2 * q + c, false);
-      op(db1[q], 24 + q, true);
-      op(db2[q], 28 + q, true);
-      op(dw3[q], 32 + q, true);
-    }
-    f32x4 last = {db3, 0.0f, 0.0f, 0.0f};
-    op(last, kSums - 1, true);
-    db3 = last[0];
-  };
-  for (int half = kPNW / 2; half >= 1; half >>= 1) {
-    f32x4* box = reinterpret_cast<f32x4*>(s.h1[0]) + (wave & (half - 1)) * (24 * 64 + 13 * 4);
-    auto slot = [&](int i, bool shared) TFH_INLINE {
-      return box + (shared ? 24 * 64 + (i - 24) * 4 + kq : i * 64 + lane);
-    };
-    __syncthreads();
-    if (wave >= half && wave < 2 * half)
-      each([&](f32x4& v, int i, bool shared) TFH_INLINE {
-        if (!shared || n == 0) *slot(i, shared) = v;
-      });
-    __syncthreads();
-    if (wave < half)
-      each([&](f32x4& v, int i, bool shared) TFH_INLINE { v += *slot(i, shared); });
-  }
-  if (wave != 0) return;
   const PropPack pp = prop_pack(w.F);
-  float* part = partials + (int64_t)blockIdx.x * pp.total;
+  float* part = partials + (int64_t)team * pp.total;
+  const int u = prop_unit(wave, n);
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int u = prop_unit(q, n);
+  for (int e = 0; e < 4; ++e) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int c = 0; c < 4; ++c) part[pp.w2 + prop_unit(c, 4 * kq + e) * kPH + u] = dw2[c][e];
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
-        part[pp.w2 + prop_unit(c, 4 * kq + e) * kPH + u] = dw2[c][q][e];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        const int k = 16 * c + 4 * kq + e;
-        if (k < w.F) part[pp.w1 + k * kPH + u] = dw1[c][q][e];
-      }
-      if (n == 0) {
-        const int unit = 16 * q + 4 * e + kq;
-        part[pp.b1 + unit] = db1[q][e];
-        part[pp.b2 + unit] = db2[q][e];
-        part[pp.w3 + unit] = dw3[q][e];
-      }
+    for (int c = 0; c < 2; ++c) {
+      const int k = 16 * c + 4 * kq + e;
+      if (k < w.F) part[pp.w1 + k * kPH + u] = dw1[c][e];
     }
+    if (n == 0) part[pp.w3 + prop_unit(wave, 4 * kq + e)] = dw3[0][e];
   }
-  if (lane == 0) part[pp.b3] = db3;
+  if (wave == 0) part[pp.b2 + prop_unit(lane >> 4, lane & 15)] = db;
+  if (wave == 1) part[pp.b1 + prop_unit(lane >> 4, lane & 15)] = db;
+  if (wave == 2 && lane == 0) part[pp.b3] = db3;
 }
 
 // Sum of the workgroup partials: a workgroup owns 64 consecutive entries and
@@ -514,9 +483,9 @@ __global__ void __launch_bounds__(64 * kPRedWaves) k_prop_reduce(const float* __
   }
 }
 
-// Persistent backward: one workgroup per CU, 16 rows per wave.
-static int64_t prop_bwd_blocks(int64_t M) {
-  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, 16 * kPNW), num_cus()));
+// Persistent backward: two teams per CU.
+static int64_t prop_bwd_teams(int64_t M) {
+  return std::max<int64_t>(1, std::min<int64_t>(ceil_div(M, kPTM), 2 * (int64_t)num_cus()));
 }
 
 int32_t check_prop_mlp(const tfh_prop_mlp* p, const char* who) {
@@ -568,11 +537,9 @@ int32_t prop_mlp_fwd_gather(const tfh_prop_mlp* p, const tfh_vm& field, const fl
   return prop_mlp_fwd(p, feats, M, nullptr, sigma, st);
 }
 
-// (twice the workgroups' partials: the size callers have always been given)
 size_t prop_mlp_bwd_workspace(const tfh_prop_mlp* p, int64_t M) {
-  const int64_t nblk = std::max<int64_t>(
-      1, std::min<int64_t>(ceil_div(M, 64), 2 * (int64_t)num_cus()));
-  return align_up((size_t)nblk * prop_pack((int)p->feat_dim).total * sizeof(float), 256);
+  return align_up((size_t)prop_bwd_teams(M) * prop_pack((int)p->feat_dim).total * sizeof(float),
+                  256);
 }
 
 int32_t prop_mlp_bwd(const tfh_prop_mlp* p, const float* feats, const float* dz, int64_t M,
@@ -580,7 +547,7 @@ int32_t prop_mlp_bwd(const tfh_prop_mlp* p, const float* feats, const float* dz,
                      hipStream_t st, const int32_t* idx = nullptr,
                      const int32_t* count = nullptr) {
   if (M == 0) return TFH_OK;
-  const int64_t nblk = prop_bwd_blocks(M);
+  const int64_t teams = prop_bwd_teams(M);
   const PropPack pp = prop_pack((int)p->feat_dim);
   TFH_REQUIRE(ws_bytes >= prop_mlp_bwd_workspace(p, M), "proposal mlp bwd: workspace too small");
   float* partials = static_cast<float*>(ws);
@@ -588,12 +555,13 @@ int32_t prop_mlp_bwd(const tfh_prop_mlp* p, const float* feats, const float* dz,
     ProfScope ps("prop_mlp_bwd", st);
     auto kernel = p->feat_dim <= 24 ? k_prop_mlp_bwd<6> : k_prop_mlp_bwd<8>;
     allow_lds(kernel, sizeof(PropBwdLds));
-    hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(kPNW * 64), sizeof(PropBwdLds), st,
-                       to_pw(p), feats, dz, M, idx, count, dfeat, partials);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(teams, 2)), dim3(kPNW * 64),
+                       sizeof(PropBwdLds), st, to_pw(p), feats, dz, M, idx, count, dfeat,
+                       partials, (int)teams);
   }
   TFH_TRY(check_launch("proposal mlp bwd"));
   hipLaunchKernelGGL(k_prop_reduce, dim3((unsigned)ceil_div(pp.b3 + 1, 64)),
-                     dim3(64 * kPRedWaves), 0, st, partials, nblk, pp, *g);
+                     dim3(64 * kPRedWaves), 0, st, partials, teams, pp, *g);
   return check_launch("proposal mlp reduce");
 }
 
