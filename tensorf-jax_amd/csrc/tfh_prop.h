@@ -3,7 +3,6 @@
 #pragma once
 
 #include "tfh_sampling.h"
-#include "tfh_scatter_sorted.h"
 
 namespace tfh {
 
@@ -33,10 +32,8 @@ struct PropWs {
   int32_t* nz_idx = nullptr;
   int32_t* nz_blk = nullptr;
   int64_t nz_nblk = 0;
-  SortWs sort;  // the sorted scatter (many rows)
   // npc copies of the field's plane gradient, then nlc of its line gradient:
-  // the scatter's blocks add into them round-robin, one kernel sums them (the
-  // sorted scatter adds the planes up before it adds them to the gradient)
+  // the scatter's blocks add into them round-robin, one kernel sums them
   float* gcopy = nullptr;
   int npc = 1, nlc = 1;
   float* loss_part = nullptr;  // kLossSlots partial sums of the interval loss

@@ -319,12 +319,6 @@ static int32_t check_prop_cfg(const tfh_proposal_config* pc, const char* who) {
   return TFH_OK;
 }
 
-// From this many samples on the factor gradients come from pairs sorted by
-// cell: fewer adds, seven launches more. Training steps without and with: 384
-// thousand samples 848 and 884 us, 786 thousand 1531 and 1477, 3.1 million 4338
-// and 4025 (the scatter 737 and 488).
-constexpr int64_t kPropSortRows = 5 << 17;
-
 size_t carve_prop(Carve& cv, const tfh_proposal_config* pc, const tfh_vm* field,
                   const tfh_prop_mlp* mlp, int64_t R, PropWs& ws) {
   const int64_t F = 3 * field->channels;
@@ -365,8 +359,6 @@ size_t carve_prop(Carve& cv, const tfh_proposal_config* pc, const tfh_vm* field,
   ws.npc = (int)std::max<int64_t>(1, std::min<int64_t>(32, (16 << 20) / (pn * 4)));
   ws.nlc = (int)std::max<int64_t>(1, std::min<int64_t>(256, (2 << 20) / (ln * 4)));
   ws.gcopy = cv.take<float>(ws.npc * pn + ws.nlc * ln);
-  if (field->grid_dim <= kSortMaxGrid && ws.rows >= kPropSortRows)
-    take_sort_ws(cv, ws.rows, ws.sort);
   ws.loss_part = cv.take<float>(kLossSlots);
   return cv.off;
 }
@@ -524,22 +516,13 @@ int32_t prop_loss_bwd(const tfh_vm* field, const tfh_prop_mlp* mlp,
   CompactedPoints src{ws.pts, ws.nz_idx, count};
   const int64_t pn = 3 * field->grid_dim * field->grid_dim * field->channels;
   const int64_t ln = 3 * field->grid_dim * field->channels;
-  float* lines = ws.gcopy + ws.npc * pn;
-  if (sorted_scatter_ok(*field, ws.rows, ws.sort)) {
-    TFH_TRY(zero_copies(lines, ws.nlc * ln, st));
-    TFH_TRY(sort_pairs((int)field->grid_dim, src, ws.rows, ws.sort, "prop_sort", st));
-    TFH_TRY(scatter_sorted_pairs(*field, src, ws.rows, RowGrad{ws.dfeat, (int)field->channels},
-                                 tfh_vm_grad{fgrad->plane, lines}, ws.nlc, ws.sort,
-                                 "prop_scatter_planes", "prop_scatter_lines", st));
-    return sum_copies(lines, ws.nlc, ln, fgrad->line, st);
-  }
   const int64_t ncopy = ws.npc * pn + ws.nlc * ln;
   TFH_TRY(zero_copies(ws.gcopy, ncopy, st));
-  const tfh_vm_grad priv{ws.gcopy, lines};
+  const tfh_vm_grad priv{ws.gcopy, ws.gcopy + ws.npc * pn};
   TFH_TRY((launch_vm_scatter<CompactedPoints, true>(*field, src, ws.rows, ws.dfeat, priv, st,
                                                     ws.npc, ws.nlc)));
   TFH_TRY(sum_copies(ws.gcopy, ws.npc, pn, fgrad->plane, st));
-  return sum_copies(lines, ws.nlc, ln, fgrad->line, st);
+  return sum_copies(ws.gcopy + ws.npc * pn, ws.nlc, ln, fgrad->line, st);
 }
 
 int32_t check_prop_args(const tfh_vm* field, const tfh_prop_mlp* mlp,

@@ -115,8 +115,6 @@ __global__ void __launch_bounds__(256) k_tile_rank(Src src, int64_t M, int g,
                                                    uint32_t* __restrict__ rank_of) {
   constexpr int RPT = kRowsPerRankGroup / 256;
   __shared__ int32_t cnt[kSortMaxTiles];
-  M = src.limit(M);
-  if ((int64_t)blockIdx.x * kRowsPerRankGroup >= M) return;
   const int nt = tiles_per_axis(g), tiles = LINE ? 3 * (g + 1) : 3 * nt * nt;
   for (int t = threadIdx.x; t < tiles; t += 256) cnt[t] = 0;
   __syncthreads();
@@ -165,9 +163,9 @@ __global__ void __launch_bounds__(256) k_tile_rank(Src src, int64_t M, int g,
 
 // (B) Exclusive scans of the tile counts and of the chunks per tile (one
 // workgroup; tiles <= kSortMaxTiles).
-static __global__ void __launch_bounds__(1024) k_tile_scan(const int32_t* __restrict__ tile_count,
-                                                           int tiles, int32_t* __restrict__ tile_start,
-                                                           int32_t* __restrict__ chunk_start) {
+__global__ void __launch_bounds__(1024) k_tile_scan(const int32_t* __restrict__ tile_count,
+                                                    int tiles, int32_t* __restrict__ tile_start,
+                                                    int32_t* __restrict__ chunk_start) {
   __shared__ int32_t wsum[2][16];
   __shared__ int32_t carry[2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -214,14 +212,13 @@ static __global__ void __launch_bounds__(1024) k_tile_scan(const int32_t* __rest
 }
 
 // (C) Every pair to its tile's segment.
-template <class Src>
-__global__ void __launch_bounds__(256) k_tile_place(Src src, int64_t M,
+__global__ void __launch_bounds__(256) k_tile_place(int64_t pairs,
                                                     const uint16_t* __restrict__ tile_of,
                                                     const uint32_t* __restrict__ rank_of,
                                                     const int32_t* __restrict__ tile_start,
                                                     uint32_t* __restrict__ order) {
   const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= 3 * src.limit(M)) return;
+  if (p >= pairs) return;
   const int64_t row = p / 3;
   const int m = (int)(p - 3 * row);
   order[tile_start[tile_of[p]] + rank_of[p]] = (uint32_t)row * 4u + (uint32_t)m;
@@ -520,13 +517,11 @@ __device__ __forceinline__ float* whole_of(const NoField&) { return nullptr; }
 // taps and upstream gradients are requested before the flush: one memory round
 // trip per pair.
 template <class Src, class FA, class FD, int LPS>
-__global__ void __launch_bounds__(256) k_plane_walk(Src src, int g, int64_t M, int per,
+__global__ void __launch_bounds__(256) k_plane_walk(Src src, int g, int64_t pairs, int per,
                                                     const uint32_t* __restrict__ order, FA fa,
                                                     FD fd) {
   constexpr bool A = !IsNone<FA>::v, D = !IsNone<FD>::v;
   static_assert(!A || LPS == 16, "quad lanes are 16 to a pair");
-  M = src.limit(M);
-  const int64_t pairs = 3 * M;
   const int l = threadIdx.x % LPS;
   const int gl0 = (threadIdx.x - l) & 63;
   const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * per;
@@ -615,13 +610,11 @@ __global__ void __launch_bounds__(256) k_plane_walk(Src src, int g, int64_t M, i
 // inside one line cell, and the adds go to copies of the line gradient (block
 // b into copy b % nlc), since every ray crosses the same few line texels.
 template <class Src, class FA, class FD, int LPS, bool RAY>
-__global__ void __launch_bounds__(256) k_line_walk(Src src, int g, int64_t M, int per,
+__global__ void __launch_bounds__(256) k_line_walk(Src src, int g, int64_t pairs, int per, int64_t M,
                                                    const uint32_t* __restrict__ order, FA fa,
                                                    FD fd) {
   constexpr bool A = !IsNone<FA>::v, D = !IsNone<FD>::v;
   static_assert(!A || LPS == 16, "quad lanes are 16 to a pair");
-  M = src.limit(M);
-  const int64_t pairs = 3 * M;
   const int l = threadIdx.x % LPS;
   const int gl0 = (threadIdx.x - l) & 63;
   const int64_t first = ((int64_t)blockIdx.x * (256 / LPS) + threadIdx.x / LPS) * per;
@@ -885,8 +878,8 @@ inline int32_t sort_lines(int g, const Src& src, int64_t M, const SortWs& s, hip
                      dim3(256), 0, st, src, M, g, s.tile_count, s.tile_of, s.rank_of);
   hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, st, s.tile_count, bins, s.tile_start,
                      s.chunk_start);
-  hipLaunchKernelGGL(k_tile_place<Src>, dim3((unsigned)ceil_div(pairs, 256)), dim3(256), 0, st,
-                     src, M, s.tile_of, s.rank_of, s.tile_start, s.order);
+  hipLaunchKernelGGL(k_tile_place, dim3((unsigned)ceil_div(pairs, 256)), dim3(256), 0, st, pairs,
+                     s.tile_of, s.rank_of, s.tile_start, s.order);
   return check_launch("vm scatter: line sort");
 }
 
@@ -899,7 +892,7 @@ inline int32_t launch_plane_walk(const Src& src, int g, int64_t M, const SortWs&
   const int per = walk_pairs(3 * M);
   const int64_t blocks = ceil_div(ceil_div(3 * M, per), 256 / LPS);
   hipLaunchKernelGGL((k_plane_walk<Src, FA, FD, LPS>), dim3((unsigned)blocks), dim3(256), 0, st,
-                     src, g, M, per, s.order, fa, fd);
+                     src, g, 3 * M, per, s.order, fa, fd);
   return check_launch("vm scatter: planes");
 }
 
@@ -912,10 +905,10 @@ inline int32_t launch_line_walk(bool sorted, const Src& src, int g, int64_t M, c
   const int64_t blocks = ceil_div(ceil_div(3 * M, per), 256 / LPS);
   if (sorted)
     hipLaunchKernelGGL((k_line_walk<Src, FA, FD, LPS, false>), dim3((unsigned)blocks), dim3(256),
-                       0, st, src, g, M, per, s.order, fa, fd);
+                       0, st, src, g, 3 * M, per, M, s.order, fa, fd);
   else
     hipLaunchKernelGGL((k_line_walk<Src, FA, FD, LPS, true>), dim3((unsigned)blocks), dim3(256), 0,
-                       st, src, g, M, per, nullptr, fa, fd);
+                       st, src, g, 3 * M, per, M, nullptr, fa, fd);
   return check_launch("vm scatter: lines");
 }
 
@@ -967,8 +960,8 @@ inline int32_t sort_pairs(int g, const Src& src, int64_t M, const SortWs& s, con
                      0, st, src, M, g, s.tile_count, s.tile_of, s.rank_of);
   hipLaunchKernelGGL(k_tile_scan, dim3(1), dim3(1024), 0, st, s.tile_count, tiles, s.tile_start,
                      s.chunk_start);
-  hipLaunchKernelGGL(k_tile_place<Src>, dim3((unsigned)ceil_div(pairs, 256)), dim3(256), 0, st,
-                     src, M, s.tile_of, s.rank_of, s.tile_start, s.order);
+  hipLaunchKernelGGL(k_tile_place, dim3((unsigned)ceil_div(pairs, 256)), dim3(256), 0, st, pairs,
+                     s.tile_of, s.rank_of, s.tile_start, s.order);
   // at most one partial chunk per tile beyond pairs / kSortChunk full ones
   const int64_t chunk_bound = pairs / kSortChunk + tiles;
   hipLaunchKernelGGL(k_chunk_sort<Src>, dim3((unsigned)chunk_bound), dim3(256), 0, st, src, g,

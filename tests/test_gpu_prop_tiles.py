@@ -5,7 +5,6 @@ of the other proposal tests: FP32 sums of up to 64 products, 2e-5 of the largest
 output; weights at the sampler's own intervals 1e-4."""
 import numpy as np
 import pytest
-import torch
 
 from oracle import proposal_oracle as po
 from tests.gpu_common import dev, f32, log, report
@@ -60,41 +59,3 @@ def test_sampler_gathers_the_field(channels, rays):
     for k in range(2):
         e = report(f"round {k} weights", s.round(k)[1].cpu().numpy(), rounds[k]["w"])
         assert e.max() <= 1e-4
-
-
-@pytest.mark.parametrize("fw_kind", ["half", "sparse", "none"])
-@pytest.mark.parametrize("channels", [8, 9])
-def test_sorted_scatter_matches_the_mean_of_parts(channels, fw_kind):
-    """4096 rays x 192 samples take the sorted factor scatter, 512 of them do not.
-    The loss is a mean over rays, so the whole gradient is the mean of the parts'.
-    2e-4 of the largest gradient: the order of the FP32 sums."""
-    log(f"case: {channels} channels, field weights {fw_kind}")
-    from tensorf_amd import proposal
-    rays, part = 4096, 512
-    cfg = po.ProposalConfig(samples_round0=128, samples_round1=64, samples_out=64,
-                            histogram_pad=0.02, loss_weight=0.7)
-    pp = _prop_params(c=channels, seed=6)
-    o, d = _rays(rays, 6)
-    rng = np.random.default_rng(7)
-    jit = f32(rng.uniform(size=(rays, 192)))
-    frac = {"half": 0.5, "sparse": 1.0 / 64, "none": 0.0}[fw_kind]
-    fw = f32(rng.uniform(0, 0.3, (rays, 64)) * (rng.uniform(size=(rays, 64)) < frac) / 4)
-
-    def gradients(at, n):
-        s, field, box, keep = _sample(pp, cfg, o[at:at + n], d[at:at + n], jit[at:at + n])
-        vm = field.tensor.stacked_single_vm
-        grads = proposal.ProposalField(
-            type(field.tensor)(type(vm)(torch.zeros_like(vm.plane), torch.zeros_like(vm.line))),
-            {k: torch.zeros_like(v) for k, v in field.mlp.items()})
-        s.loss_backward(s.edges, dev(fw[at:at + n]), grads)
-        torch.cuda.synchronize()
-        got = grads.tensor.stacked_single_vm
-        return [t.cpu().numpy().astype(np.float64)
-                for t in (got.plane, got.line, *grads.mlp.values())]
-
-    whole = gradients(0, rays)
-    mean = sum(np.array(g, dtype=object) for g in (gradients(at, part)
-                                                   for at in range(0, rays, part))) * part / rays
-    for name, got, want in zip(("plane", "line", *proposal.MLP_KEYS), whole, mean):
-        e = report(f"grad {name}", got, want)
-        assert e.max() <= 2e-4 * np.abs(want).max() + 1e-12, name
