@@ -163,9 +163,9 @@ __global__ void __launch_bounds__(256) k_tile_rank(Src src, int64_t M, int g,
 
 // (B) Exclusive scans of the tile counts and of the chunks per tile (one
 // workgroup; tiles <= kSortMaxTiles).
-__global__ void __launch_bounds__(1024) k_tile_scan(const int32_t* __restrict__ tile_count,
-                                                    int tiles, int32_t* __restrict__ tile_start,
-                                                    int32_t* __restrict__ chunk_start) {
+static __global__ void __launch_bounds__(1024) k_tile_scan(
+    const int32_t* __restrict__ tile_count, int tiles, int32_t* __restrict__ tile_start,
+    int32_t* __restrict__ chunk_start) {
   __shared__ int32_t wsum[2][16];
   __shared__ int32_t carry[2];
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(1024) k_tile_scan(const int32_t* __restrict__ 
 }
 
 // (C) Every pair to its tile's segment.
-__global__ void __launch_bounds__(256) k_tile_place(int64_t pairs,
+static __global__ void __launch_bounds__(256) k_tile_place(int64_t pairs,
                                                     const uint16_t* __restrict__ tile_of,
                                                     const uint32_t* __restrict__ rank_of,
                                                     const int32_t* __restrict__ tile_start,
@@ -1007,6 +1007,35 @@ inline int32_t scatter_sorted_pairs(const tfh_vm& vm, const Src& src, int64_t M,
   hipLaunchKernelGGL((k_line_scatter<Src, GS>), dim3((unsigned)ceil_div(M, kGatherThreads / 16)),
                      dim3(kGatherThreads), 0, st, vm, src, M, gsrc, grad.line, nlc);
   return check_launch("vm scatter: lines");
+}
+
+// Whether a field takes the walks by itself.
+template <class GS>
+inline bool walk_ok(const tfh_vm& vm, const GS& g) {
+  return vm.channels <= 16 || quad_lanes_ok(vm, g);
+}
+
+// The scatter of M rows in no particular order (walk_ok, sorted_scatter_ok): both
+// passes over sorted pairs.
+template <class Src, class GS>
+inline int32_t scatter_scattered_rows(const tfh_vm& vm, const Src& src, int64_t M, const GS& gsrc,
+                                      const tfh_vm_grad& grad, const SortWs& s, hipStream_t st) {
+  const int g = (int)vm.grid_dim;
+  const WalkField<GS> fp{vm, gsrc, grad.plane, 1}, fl{vm, gsrc, grad.line, 1};
+  const NoField none;
+  TFH_TRY(sort_pairs(g, src, M, s, "scatter_sort", st));
+  if (vm.channels > 16)
+    TFH_TRY(launch_plane_walk<16>(src, g, M, s, fp, none, "scatter_planes", st));
+  else if (vm.channels > 8)
+    TFH_TRY(launch_plane_walk<16>(src, g, M, s, none, fp, "scatter_planes", st));
+  else
+    TFH_TRY(launch_plane_walk<8>(src, g, M, s, none, fp, "scatter_planes", st));
+  TFH_TRY(sort_lines(g, src, M, s, st));
+  if (vm.channels > 16)
+    return launch_line_walk<16>(true, src, g, M, s, fl, none, "scatter_lines", st);
+  if (vm.channels > 8)
+    return launch_line_walk<16>(true, src, g, M, s, none, fl, "scatter_lines", st);
+  return launch_line_walk<8>(true, src, g, M, s, none, fl, "scatter_lines", st);
 }
 
 }  // namespace tfh

@@ -98,6 +98,8 @@ _SIGS = {
     "tfh_vm_from_channel_last": (c_i32, [c_p, c_p, c_i64, c_i64, c_p, c_p, c_p]),
     "tfh_vm_interpolate": (c_i32, [P(Vm), c_p, c_i64, c_p, c_p]),
     "tfh_vm_interpolate_bwd": (c_i32, [P(Vm), c_p, c_i64, c_p, P(VmGrad), c_p]),
+    "tfh_vm_interpolate_bwd_workspace_size": (c_sz, [P(Vm), c_i64]),
+    "tfh_vm_interpolate_bwd_sorted": (c_i32, [P(Vm), c_p, c_i64, c_p, P(VmGrad), c_p, c_sz, c_p]),
     "tfh_zero_arrays": (c_i32, [P(c_p), P(c_i64), c_i32, c_p]),
     "tfh_vm_resize": (c_i32, [P(Vm), c_i64, c_p, c_p, c_p]),
     "tfh_sample_bbox": (c_i32, [c_p, c_p, c_i64, c_p, c_i64, c_p, c_p, c_p, c_p, c_p]),

@@ -73,8 +73,17 @@ class _Interpolate(torch.autograd.Function):
         vm = _vm_struct(plane, line)
         gout = gout.contiguous()
         grad = _lib.VmGrad(_lib.ptr(gplane), _lib.ptr(gline))
-        _lib.call("tfh_vm_interpolate_bwd", ctypes.byref(vm), _lib.ptr(ijk), ijk.shape[1],
-                  _lib.ptr(gout), ctypes.byref(grad), _lib.stream())
+        m = ijk.shape[1]
+        # (never for so few points: not asked, the call is 4 us of a small step's 155)
+        need = 0 if m < 65536 else int(
+            _lib.lib.tfh_vm_interpolate_bwd_workspace_size(ctypes.byref(vm), m))
+        if need:
+            ws = torch.empty(need, dtype=torch.uint8, device=plane.device)
+            _lib.call("tfh_vm_interpolate_bwd_sorted", ctypes.byref(vm), _lib.ptr(ijk), m,
+                      _lib.ptr(gout), ctypes.byref(grad), _lib.ptr(ws), need, _lib.stream())
+        else:
+            _lib.call("tfh_vm_interpolate_bwd", ctypes.byref(vm), _lib.ptr(ijk), m,
+                      _lib.ptr(gout), ctypes.byref(grad), _lib.stream())
         return None, gplane, gline
 
 
