@@ -256,6 +256,14 @@ int32_t tfh_render_fwd(const tfh_vm* density, const tfh_vm* appearance, const tf
                        const float* jitter, const float* base_ts, const float* base_steps,
                        const float* gumbel, float* out, void* workspace, size_t workspace_bytes,
                        tfh_stream_t stream);
+/* tfh_render_fwd when no tfh_render_bwd follows: the same output, and the
+ * feature rows are not written where only the backward reads them. */
+int32_t tfh_render_only(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
+                        const tfh_render_config* cfg, const float* aabb, const float* origins,
+                        const float* directions, const uint32_t* camera_indices, int64_t num_rays,
+                        const float* jitter, const float* base_ts, const float* base_steps,
+                        const float* gumbel, float* out, void* workspace, size_t workspace_bytes,
+                        tfh_stream_t stream);
 /* VJP of tfh_render_fwd (RGB mode) for grad_out (R,3): accumulates the
  * density / appearance factor gradients and the MLP gradients. Must follow
  * tfh_render_fwd with the same arguments and workspace. */

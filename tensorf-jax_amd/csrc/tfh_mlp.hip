@@ -185,7 +185,7 @@ int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
 struct GatherTile {
   tfh_vm vm;         // appearance field, 48 channels, 16-byte aligned
   RaySamples src;    // the sample points of the rows
-  float* feats;      // (M, 144) out
+  float* feats;      // (M, 144) out, or null
   template <int TM, int NT, bool CAMS, bool FB16>
   __device__ void load(const MlpDims& d, int64_t row0, int64_t M, int64_t rpr, float* Fs,
                        float* Ds, int* Cs, const float* __restrict__ dirs,
@@ -256,7 +256,7 @@ struct GatherTile {
         }
       }
     }
-    if (valid && c4 < C) {
+    if (feats && valid && c4 < C) {
 #pragma unroll
       for (int m = 0; m < 3; ++m)
         *reinterpret_cast<float4*>(feats + row * 3 * C + m * C + c4) = f[m];

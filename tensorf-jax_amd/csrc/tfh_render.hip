@@ -540,6 +540,7 @@ __global__ void k_fill(float* __restrict__ p, int64_t n, float v) {
 struct RenderWs {
   DensityOut d;
   float* feats;  // (M, F)
+  bool keep = true;  // feats is written where only the backward reads it
   float* rgb;    // (M, 3)
   float* gout;   // (R, 3)
   float* dc;     // (M, 3)
@@ -700,9 +701,9 @@ static int32_t render_forward(const tfh_vm* density, const tfh_vm* appearance, c
   bool fused = false;
   {
     ProfScope ps("mlp_fwd", st);
-    TFH_TRY(mlp_fwd_rows_gather(mlp, *appearance, src, ws.feats, in.d, cams, M, k, ws.rgb,
-                                cfg->mlp_precision, ws.mlp_ws, ws.mlp_ws_bytes, st, ws.act,
-                                &fused));
+    TFH_TRY(mlp_fwd_rows_gather(mlp, *appearance, src, ws.keep ? ws.feats : nullptr, in.d, cams,
+                                M, k, ws.rgb, cfg->mlp_precision, ws.mlp_ws, ws.mlp_ws_bytes, st,
+                                ws.act, &fused));
   }
   if (!fused) {
     {
@@ -917,6 +918,7 @@ int32_t render_fwd_scratch(const tfh_vm* density, const tfh_vm* appearance, cons
   RenderWs ws;
   carve_render_fwd(cv, cfg, rgb ? mlp : nullptr, F, num_rays, ws);
   if (!cv.ok) return fail(TFH_ERR_WORKSPACE, "%s: scratch carve failed", who);
+  ws.keep = false;
   RayIn in = make_rayin(cfg, aabb, origins, directions, num_rays, jitter, base_ts, base_steps,
                         gumbel);
   return render_forward(density, appearance, mlp, cfg, in, camera_indices, out, nullptr, nullptr,
@@ -973,6 +975,34 @@ int32_t train_step_run(const tfh_vm* density, const tfh_vm* appearance, const tf
 }  // namespace tfh
 
 using namespace tfh;
+
+// keep: for a backward (tfh_render_bwd) to follow.
+static int32_t render_fwd_run(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
+                              const tfh_render_config* cfg, const float* aabb,
+                              const float* origins, const float* directions,
+                              const uint32_t* camera_indices, int64_t num_rays,
+                              const float* jitter, const float* base_ts, const float* base_steps,
+                              const float* gumbel, float* out, void* workspace,
+                              size_t workspace_bytes, tfh_stream_t stream, bool keep,
+                              const char* who) {
+  TFH_TRY(check_render_args(density, appearance, mlp, cfg, aabb, origins, directions, num_rays,
+                            jitter, base_ts, base_steps, who));
+  if (num_rays == 0) return TFH_OK;
+  TFH_REQUIRE(out != nullptr, "%s: null output", who);
+  TFH_TRY(require_device());
+  const int64_t F = cfg->mode == TFH_MODE_RGB ? 3 * appearance->channels : 0;
+  Carve cv(workspace, workspace_bytes);
+  RenderWs ws;
+  carve_render(cv, cfg, cfg->mode == TFH_MODE_RGB ? mlp : nullptr, F, num_rays, ws);
+  if (!cv.ok)
+    return fail(TFH_ERR_WORKSPACE, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes,
+                cv.off);
+  ws.keep = keep;
+  RayIn in = make_rayin(cfg, aabb, origins, directions, num_rays, jitter, base_ts, base_steps,
+                        gumbel);
+  return render_forward(density, appearance, mlp, cfg, in, camera_indices, out, nullptr, nullptr,
+                        ws, as_stream(stream));
+}
 
 extern "C" {
 
@@ -1075,22 +1105,20 @@ int32_t tfh_render_fwd(const tfh_vm* density, const tfh_vm* appearance, const tf
                        const float* jitter, const float* base_ts, const float* base_steps,
                        const float* gumbel, float* out, void* workspace, size_t workspace_bytes,
                        tfh_stream_t stream) {
-  TFH_TRY(check_render_args(density, appearance, mlp, cfg, aabb, origins, directions, num_rays,
-                            jitter, base_ts, base_steps, "tfh_render_fwd"));
-  if (num_rays == 0) return TFH_OK;
-  TFH_REQUIRE(out != nullptr, "tfh_render_fwd: null output");
-  TFH_TRY(require_device());
-  const int64_t F = cfg->mode == TFH_MODE_RGB ? 3 * appearance->channels : 0;
-  Carve cv(workspace, workspace_bytes);
-  RenderWs ws;
-  carve_render(cv, cfg, cfg->mode == TFH_MODE_RGB ? mlp : nullptr, F, num_rays, ws);
-  if (!cv.ok)
-    return fail(TFH_ERR_WORKSPACE, "tfh_render_fwd: workspace of %zu bytes, need %zu",
-                workspace_bytes, cv.off);
-  RayIn in = make_rayin(cfg, aabb, origins, directions, num_rays, jitter, base_ts, base_steps,
-                        gumbel);
-  return render_forward(density, appearance, mlp, cfg, in, camera_indices, out, nullptr, nullptr,
-                        ws, as_stream(stream));
+  return render_fwd_run(density, appearance, mlp, cfg, aabb, origins, directions, camera_indices,
+                        num_rays, jitter, base_ts, base_steps, gumbel, out, workspace,
+                        workspace_bytes, stream, true, "tfh_render_fwd");
+}
+
+int32_t tfh_render_only(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
+                        const tfh_render_config* cfg, const float* aabb, const float* origins,
+                        const float* directions, const uint32_t* camera_indices, int64_t num_rays,
+                        const float* jitter, const float* base_ts, const float* base_steps,
+                        const float* gumbel, float* out, void* workspace, size_t workspace_bytes,
+                        tfh_stream_t stream) {
+  return render_fwd_run(density, appearance, mlp, cfg, aabb, origins, directions, camera_indices,
+                        num_rays, jitter, base_ts, base_steps, gumbel, out, workspace,
+                        workspace_bytes, stream, false, "tfh_render_only");
 }
 
 int32_t tfh_render_bwd(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,

@@ -118,6 +118,8 @@ _SIGS = {
     "tfh_train_step_workspace_size": (c_sz, [P(RenderConfig), P(Mlp), c_i64, c_i64]),
     "tfh_render_fwd": (c_i32, [P(Vm), P(Vm), P(Mlp), P(RenderConfig), c_p, c_p, c_p, c_p, c_i64,
                                c_p, c_p, c_p, c_p, c_p, c_p, c_sz, c_p]),
+    "tfh_render_only": (c_i32, [P(Vm), P(Vm), P(Mlp), P(RenderConfig), c_p, c_p, c_p, c_p, c_i64,
+                               c_p, c_p, c_p, c_p, c_p, c_p, c_sz, c_p]),
     "tfh_render_bwd": (c_i32, [P(Vm), P(Vm), P(Mlp), P(RenderConfig), c_p, c_p, c_p, c_p, c_i64,
                                c_p, P(VmGrad), P(VmGrad), P(MlpGrad), c_p, c_sz, c_p]),
     "tfh_render_fwd_noalloc": (c_i32, [P(Vm), P(Vm), P(Mlp), P(RenderConfig), c_p, c_p, c_p,

@@ -244,11 +244,12 @@ class _RenderEnv:
     def _mlp_ref(self):
         return ctypes.byref(self.cmlp) if self.cmlp else None
 
-    def forward(self) -> torch.Tensor:
+    def forward(self, keep: bool = True) -> torch.Tensor:
+        """keep: write what backward() reads."""
         rgb = self.config.mode is RenderMode.RGB
         out = torch.empty((self.r, 3) if rgb else (self.r,), dtype=torch.float32,
                           device=self.device)
-        _lib.call("tfh_render_fwd", ctypes.byref(self.dvm), ctypes.byref(self.avm), self._mlp_ref(),
+        _lib.call("tfh_render_fwd" if keep else "tfh_render_only", ctypes.byref(self.dvm), ctypes.byref(self.avm), self._mlp_ref(),
                   ctypes.byref(self.cfg), _lib.ptr(self.aabb), _lib.ptr(self.o), _lib.ptr(self.d),
                   _lib.ptr(self.cams), self.r, _lib.ptr(self.jitter), _lib.ptr(self.base_ts),
                   _lib.ptr(self.base_steps), _lib.ptr(self.gumbel), _lib.ptr(out),
@@ -285,7 +286,7 @@ def render_rays(appearance_mlp: networks.FeatureMlp, learnable_params: Learnable
     if config.mode is RenderMode.RGB and torch.is_grad_enabled() and any(
             t.requires_grad for t in env.leaves()):
         return _RenderFn.apply(env, *env.leaves())
-    return env.forward()
+    return env.forward(keep=False)
 
 
 def render_rays_batched(appearance_mlp: networks.FeatureMlp, learnable_params: LearnableParams,
