@@ -176,13 +176,6 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
-// Sum over aligned groups of 16 lanes.
-__device__ __forceinline__ float group16_sum(float v) {
-#pragma unroll
-  for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 // Number of set bits of `mask` in lanes below the calling lane.
 __device__ __forceinline__ int lanes_below(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),

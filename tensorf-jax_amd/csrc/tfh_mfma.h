@@ -50,32 +50,6 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* base, 
 }
 constexpr int kOOB = 0x7ffffff0;  // a byte offset past every buffer: loads return 0
 
-// Row-major FP32 global matrix as a B operand with zero padding outside (rows, cols).
-struct GlobalB {
-  __amdgpu_buffer_rsrc_t r;
-  int rows, cols;
-  __device__ __forceinline__ GlobalB(const float* w, int rows_, int cols_)
-      : r(buffer_rsrc(w, rows_ * cols_ * 4)), rows(rows_), cols(cols_) {}
-  __device__ __forceinline__ float operator()(int k, int j) const {
-    const int off = (k < rows && j < cols) ? (k * cols + j) * 4 : kOOB;
-    // the builtin returns the raw 32 bits as an integer: reinterpret, do not convert
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-  }
-};
-
-// Transposed view of a row-major FP32 (rows x cols) matrix W as a B operand:
-// B(k, j) = W[j][k], zero outside.
-struct GlobalBT {
-  __amdgpu_buffer_rsrc_t r;
-  int rows, cols;  // of W
-  __device__ __forceinline__ GlobalBT(const float* w, int rows_, int cols_)
-      : r(buffer_rsrc(w, rows_ * cols_ * 4)), rows(rows_), cols(cols_) {}
-  __device__ __forceinline__ float operator()(int k, int j) const {
-    const int off = (j < rows && k < cols) ? (j * cols + k) * 4 : kOOB;
-    return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0));
-  }
-};
-
 // A table of B operands in the order the strips read it: one block of 1 KB per
 // column tile of 16 and chunk of KC = 16 (FP32) or 32 (BF16) inputs, in it a
 // lane's 16 bytes at 16 * lane: lane (r, kq) = r + 16 kq holds column r's
@@ -155,33 +129,6 @@ __device__ __forceinline__ void mma_strip(const float* __restrict__ A, int lda, 
   }
 }
 
-// acc[rt] += A(rows 16*rt.., K) * B(K, cols col0..col0+15), rt < NR; A from
-// LDS (row-major, lda), K <= KMAX. The whole B column strip is loaded into
-// registers first (KMAX/4 floats or KMAX/32 bf16x8 per lane) so its L2
-// latency overlaps; A is read from LDS per k-step.
-template <int NR, int KMAX, class BF32>
-__device__ __forceinline__ void mma_strip(const float* __restrict__ A, int lda, int K, BF32 b,
-                                          int col0, f32x4 (&acc)[NR]) {
-  const int lane = lane_here();
-  const int r = lane & 15, kq = lane >> 4;
-  constexpr int NS = KMAX / 4;
-  for (int kc = 0; kc < K; kc += KMAX) {  // one pass for K <= KMAX
-    float bb[NS];
-#pragma unroll
-    for (int i = 0; i < NS; ++i) bb[i] = (kc + 4 * i < K) ? b(kc + 4 * i + kq, col0 + r) : 0.0f;
-#pragma unroll
-    for (int i = 0; i < NS; ++i) {
-      if (kc + 4 * i < K) {
-#pragma unroll
-        for (int rt = 0; rt < NR; ++rt) {
-          const float a = A[(16 * rt + r) * lda + kc + 4 * i + kq];
-          acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, bb[i], acc[rt], 0, 0, 0);
-        }
-      }
-    }
-  }
-}
-
 // A lane's 8 A operands of a BF16 strip: FP32 rows rounded per use, or rows
 // kept in BF16 (one 16-byte read).
 __device__ __forceinline__ bf16x8 strip_a8(const float* ap) {
@@ -238,14 +185,11 @@ __device__ __forceinline__ void mma_strip(const __bf16* __restrict__ A, int lda,
 // floats, 4 rows are 16 mod 32 floats apart: the four groups' 16-float
 // segments fall in disjoint banks. The sum over k is unchanged; only the
 // order of the FP32 accumulation differs. Requires K % 16 == 0 (32 for BF16).
-// FRESH: the lane index from lane_here (operand addresses computed per call)
-// or the plain one (addresses loop-invariant: hoisted out of a tile loop and
-// kept in registers when the kernel has them to spare).
-template <bool BF, int K, bool FRESH = true>
-__device__ __forceinline__ void mma_wgrad_acc(const float* __restrict__ X, int ldx, int row0,
-                                              const float* __restrict__ Y, int ldy, int col0,
-                                              f32x4& acc) {
-  const int lane = FRESH ? lane_here() : lane_id();
+template <bool BF, int K>
+__device__ __forceinline__ f32x4 mma_wgrad(const float* __restrict__ X, int ldx, int row0,
+                                           const float* __restrict__ Y, int ldy, int col0) {
+  f32x4 acc{0.f, 0.f, 0.f, 0.f};
+  const int lane = lane_here();
   const int r = lane & 15, kq = lane >> 4;
   if constexpr (BF) {
     static_assert(K % 32 == 0, "BF16 weight-gradient tiles take K in steps of 32");
@@ -273,13 +217,6 @@ __device__ __forceinline__ void mma_wgrad_acc(const float* __restrict__ X, int l
       }
     }
   }
-}
-
-template <bool BF, int K>
-__device__ __forceinline__ f32x4 mma_wgrad(const float* __restrict__ X, int ldx, int row0,
-                                           const float* __restrict__ Y, int ldy, int col0) {
-  f32x4 acc{0.f, 0.f, 0.f, 0.f};
-  mma_wgrad_acc<BF, K>(X, ldx, row0, Y, ldy, col0, acc);
   return acc;
 }
 

@@ -31,7 +31,7 @@
 //
 // Measured against the FP32-MFMA / FP32-rows-in-LDS kernel this replaces
 // (32-row tiles, weight-gradient operands read a float at a time): 2.1 M rows
-// FP32 4.22 -> 2.43 ms; BF16 1.05 M rows 1.29 -> 0.63 ms; with the embedding,
+// FP32 4.22 -> 2.71 ms; BF16 1.05 M rows 1.29 -> 0.63 ms; with the embedding,
 // BF16, 4.2 M rows 5.85 -> 2.77 ms. What bounds it (counters, FP32): LDS busy
 // 52% of the cycles, MFMA 37%, vector ALU 35%, one workgroup per CU (its
 // 140-160 KB of LDS and 250 registers), so the steps' latencies show.

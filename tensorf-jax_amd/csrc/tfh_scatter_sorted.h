@@ -2,11 +2,12 @@
 // transpose of TensorVM.interpolate (tensor_vm.py:42-89, 226-250) for a
 // batch of rows, split into
 //   * planes: the (row, mode) pairs are counting-sorted by plane cell (the 2x2
-//     texel block a row's bilinear taps read); a 16-lane group walks a run of
-//     pairs of one cell and sums their four tap gradients in registers, so a
-//     cell costs one add per texel and channel instead of one per pair;
-//   * lines: rows in their own (ray) order, one 16-lane group per row, equal
-//     line texels among the four rows of a wave merged before the add.
+//     texel block a row's bilinear taps read); a group of lanes walks a run of
+//     pairs and sums the texels of the current cell in registers, so a texel
+//     costs one add per stretch of cells that share it instead of one per pair;
+//   * lines: the same walk in ray order, or over the pairs sorted by line cell.
+// Fields that the walks do not take add the lines in ray order, one 16-lane
+// group per row, equal texels among the four rows of a wave merged.
 // Float atomics to device memory are performed at the memory side on this
 // part and adds to one address serialise there; the transaction count is
 // what bounds a scatter.
