@@ -138,26 +138,28 @@ int64_t mlp_kept_floats(int64_t rows) { return kept_floats(rows); }
 static int32_t launch_fwd(const MlpDims& d, const MlpW& w, const MlpPack& pk, bool bf, bool kb,
                           const float* feats, const float* dirs, const uint32_t* cams, int64_t M,
                           int64_t rpr, float* rgb, float* act, hipStream_t st) {
-  const bool sd = is_std_dims(d, bf);
+  const Shape sh = shape_of(d);
   // (the BF16 standard shape keeps its feature rows in BF16: k_mlp_fwd)
-  const size_t lds = fwd_lds_floats<kFwdTM>(d, bf && sd) * sizeof(float);
+  const size_t lds = fwd_lds_floats<kFwdTM>(d, bf && sh == Shape::kStd) * sizeof(float);
   TFH_REQUIRE(lds <= 160 * 1024, "mlp fwd: tile needs %zu bytes of LDS", lds);
   const int64_t blocks = ceil_div(M, kFwdTM);
-#define TFH_LAUNCH_FWD(BFV, STDV, KBV)                                                         \
-  do {                                                                                         \
-    auto kernel = k_mlp_fwd<kFwdTM, kFwdNW, BFV, STDV, NoGather, KBV>;                          \
-    allow_lds(kernel, lds);                                                                    \
-    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kFwdNW * 64), lds, st, d, w, pk,    \
-                       feats, dirs, cams, M, rpr, rgb, act, NoGather{});                       \
-  } while (0)
-  if (!bf) {
-    if (sd) TFH_LAUNCH_FWD(false, true, false); else TFH_LAUNCH_FWD(false, false, false);
-  } else if (kb || !act) {
-    if (sd) TFH_LAUNCH_FWD(true, true, true); else TFH_LAUNCH_FWD(true, false, true);
-  } else {
-    if (sd) TFH_LAUNCH_FWD(true, true, false); else TFH_LAUNCH_FWD(true, false, false);
-  }
-#undef TFH_LAUNCH_FWD
+  auto launch = [&](auto any, auto std, auto def) {
+    auto kernel = sh == Shape::kStd ? std : (sh == Shape::kDef ? def : any);
+    allow_lds(kernel, lds);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(kFwdNW * 64), lds, st, d, w, pk, feats,
+                       dirs, cams, M, rpr, rgb, act, NoGather{});
+  };
+#define TFH_FWD(BFV, KBV)                                                     \
+  launch(k_mlp_fwd<kFwdTM, kFwdNW, BFV, Shape::kAny, NoGather, KBV>,          \
+         k_mlp_fwd<kFwdTM, kFwdNW, BFV, Shape::kStd, NoGather, KBV>,          \
+         k_mlp_fwd<kFwdTM, kFwdNW, BFV, Shape::kDef, NoGather, KBV>)
+  if (!bf)
+    TFH_FWD(false, false);
+  else if (kb || !act)
+    TFH_FWD(true, true);
+  else
+    TFH_FWD(true, false);
+#undef TFH_FWD
   return check_launch("mlp fwd");
 }
 
@@ -288,7 +290,7 @@ int32_t mlp_fwd_rows_gather(const tfh_mlp* p, const tfh_vm& vm, const RaySamples
   *done = false;
   const bool bf = precision == TFH_PREC_BF16;
   MlpDims d = make_dims(p, bf);
-  if (!is_std_dims(d, bf) || vm.channels != 48 || 3 * vm.channels != d.F ||
+  if (shape_of(d) != Shape::kStd || vm.channels != 48 || 3 * vm.channels != d.F ||
       (reinterpret_cast<uintptr_t>(vm.plane) & 15) || (reinterpret_cast<uintptr_t>(vm.line) & 15) ||
       (reinterpret_cast<uintptr_t>(feats) & 15) || M <= 0 ||
       vm.grid_dim * vm.grid_dim * vm.channels * 4 >= (1ll << 32))  // 32-bit offsets in a mode
@@ -302,13 +304,13 @@ int32_t mlp_fwd_rows_gather(const tfh_mlp* p, const tfh_vm& vm, const RaySamples
   const GatherTile gt{vm, src, feats};
   ProfScope ps("mlp_fwd_kernel", st);
   if (bf) {
-    allow_lds(k_mlp_fwd<kFwdTM, kFwdNW, true, true, GatherTile>, lds);
-    hipLaunchKernelGGL((k_mlp_fwd<kFwdTM, kFwdNW, true, true, GatherTile>), dim3((unsigned)blocks),
+    allow_lds(k_mlp_fwd<kFwdTM, kFwdNW, true, Shape::kStd, GatherTile>, lds);
+    hipLaunchKernelGGL((k_mlp_fwd<kFwdTM, kFwdNW, true, Shape::kStd, GatherTile>), dim3((unsigned)blocks),
                        dim3(kFwdNW * 64), lds, st, d, to_w(p), pk, nullptr, dirs, cams, M, rpr,
                        rgb, act, gt);
   } else {
-    allow_lds(k_mlp_fwd<kFwdTM, kFwdNW, false, true, GatherTile>, lds);
-    hipLaunchKernelGGL((k_mlp_fwd<kFwdTM, kFwdNW, false, true, GatherTile>),
+    allow_lds(k_mlp_fwd<kFwdTM, kFwdNW, false, Shape::kStd, GatherTile>, lds);
+    hipLaunchKernelGGL((k_mlp_fwd<kFwdTM, kFwdNW, false, Shape::kStd, GatherTile>),
                        dim3((unsigned)blocks), dim3(kFwdNW * 64), lds, st, d, to_w(p), pk,
                        nullptr, dirs, cams, M, rpr, rgb, act, gt);
   }

@@ -111,14 +111,18 @@ inline MlpDims make_dims(const tfh_mlp* p, bool bf) {
   return d;
 }
 
-// Dims of the standard appearance MLP (48 channels x 3 modes, squash 27,
-// 2+2 Fourier frequencies) as compile-time constants, so the kernels built for
-// it fold every LDS offset and tile count; the camera count stays a run-time
-// value (0 = no embedding).
-template <bool BF>
+// Dims of the two appearance MLPs of the configurations (squash 27; 48 channels x
+// 3 modes with 2 + 2 Fourier frequencies, the standard one, and 24 x 3 with 6 + 6)
+// as compile-time constants, so the kernels built for them fold every LDS
+// offset and tile count; the camera count stays a run-time value (0 = no embedding).
+// The forward of the 24-channel shape with run-time dims took 561 us for 315
+// thousand rows (FP32; its products 280), 477 with these.
+enum class Shape { kAny, kStd, kDef };
+
+template <bool BF, Shape SH = Shape::kStd>
 __host__ __device__ constexpr MlpDims std_dims(int ncam = 0) {
   const int kp = BF ? 32 : 16, pad = 4;
-  const int F = 144, S = 27, nf = 2, nv = 2;
+  const int F = SH == Shape::kDef ? 72 : 144, S = 27, nf = SH == Shape::kDef ? 6 : 2, nv = nf;
   const int E = S + 3 + 2 * nf * S + 2 * nv * 3;
   const int FP = (F + kp - 1) / kp * kp, EP = (E + kp - 1) / kp * kp;
   const int Z3W = BF ? 32 : 16;
@@ -126,9 +130,11 @@ __host__ __device__ constexpr MlpDims std_dims(int ncam = 0) {
                  Z3W + pad};
 }
 
-inline bool is_std_dims(const MlpDims& d, bool bf) {
-  const MlpDims s = bf ? std_dims<true>() : std_dims<false>();
-  return d.F == s.F && d.S == s.S && d.nf == s.nf && d.nv == s.nv;
+inline Shape shape_of(const MlpDims& d) {
+  constexpr MlpDims s = std_dims<false>(), e = std_dims<false, Shape::kDef>();
+  if (d.S != s.S || d.nf != d.nv) return Shape::kAny;
+  if (d.F == s.F && d.nf == s.nf) return Shape::kStd;
+  return d.F == e.F && d.nf == e.nf ? Shape::kDef : Shape::kAny;
 }
 
 struct MlpW {  // FP32 parameters (device pointers)
@@ -583,7 +589,7 @@ struct NoGather {};
 // itself (gt.load<TM, NT, CAMS, FB16>(d, row0, M, rpr, Fs, Ds, Cs, dirs,
 // cams): the appearance gather fused into the tile load, its rows also
 // written to global memory for the backward), instead of reading feats.
-template <int TM, int NW, bool BF, bool STD, class GT = NoGather, bool KB = BF>
+template <int TM, int NW, bool BF, Shape SH, class GT = NoGather, bool KB = BF>
 __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpPack pk,
                                                      const float* __restrict__ feats,
                                                      const float* __restrict__ dirs,
@@ -592,8 +598,9 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
                                                      float* __restrict__ rgb,
                                                      float* __restrict__ act, GT gt) {
   constexpr bool kGather = !std::is_same<GT, NoGather>::value;
-  static_assert(!kGather || STD, "the fused gather serves the standard shape");
-  const MlpDims d = STD ? std_dims<BF>(d_arg.ncam) : d_arg;
+  static_assert(!kGather || SH == Shape::kStd, "the fused gather serves the standard shape");
+  constexpr bool kFixed = SH != Shape::kAny;
+  const MlpDims d = kFixed ? std_dims<BF, SH>(d_arg.ncam) : d_arg;
   extern __shared__ float smem[];
   // regions: A = Fs, later H1, last R3 (the layer-3 output); B = X, later
   // H2; small: Ds, Cs. 40 KB per workgroup for the FP32 standard shape: four
@@ -601,7 +608,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
   // the BF16 standard shape keeps its feature rows in BF16 (layer 0 reads
   // them as BF16 operands either way): 39 KB of LDS, four workgroups per CU
   // instead of three
-  constexpr bool FB16 = BF && STD;
+  constexpr bool FB16 = BF && SH == Shape::kStd;
   float* regA = smem;
   float* regB = regA + TM * std::max(FB16 ? kFsLdB / 2 : d.ldF, d.ldU);
   float* Ds = regB + TM * std::max(d.ldE, d.ldU);
@@ -621,9 +628,9 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
       gt.template load<TM, NW * 64, false, FB16>(d, row0, M, rpr, regA, Ds, Cs, dirs, cams);
     else
       gt.template load<TM, NW * 64, true, FB16>(d, row0, M, rpr, regA, Ds, Cs, dirs, cams);
-  } else if (STD && d.ncam == 0) {
+  } else if (kFixed && d.ncam == 0) {
     load_tile_rows<TM, NW * 64, false, FB16>(d, feats, dirs, row0, M, rpr, regA, Ds);
-  } else if (STD) {
+  } else if (kFixed) {
     load_tile_rows<TM, NW * 64, true, FB16>(d, feats, dirs, row0, M, rpr, regA, Ds, cams, Cs);
   } else {
     load_tile<TM>(d, feats, dirs, cams, row0, M, rpr, regA, Ds, Cs);
@@ -1039,10 +1046,8 @@ constexpr int kBwdTM = 32;
 // operand tables, the launches.
 enum class BwdKind { kNone, kStd, kDef };
 inline BwdKind bwd_kind(const MlpDims& d) {
-  if (d.S != 27 || d.nf != d.nv) return BwdKind::kNone;
-  if (d.F == 144 && d.nf == 2) return BwdKind::kStd;
-  if (d.F == 72 && d.nf == 6) return BwdKind::kDef;
-  return BwdKind::kNone;
+  const Shape sh = shape_of(d);
+  return sh == Shape::kStd ? BwdKind::kStd : (sh == Shape::kDef ? BwdKind::kDef : BwdKind::kNone);
 }
 // The type of the kept activations. BF16 changes no result of the BF16 MLP's
 // backward without an embedding; with one, relu(z2) also enters the
