@@ -19,6 +19,9 @@ namespace tfh {
 
 // Grids up to this size use the sorted plane scatter.
 constexpr int kSortMaxGrid = 512;
+// Rows up to this many can be sorted: their pairs, three a row, are counted and
+// placed with 32-bit signed integers.
+constexpr int64_t kSortMaxRows = INT32_MAX / 3;
 
 // Code of one axis' tap pair: the lower texel when the pair is (i, i+1),
 // G-1 for the pair clamped at the low edge (0, 0), G for the high edge
@@ -929,10 +932,10 @@ inline void take_sort_ws(Carve& cv, int64_t M, SortWs& s) {
 }
 
 // Whether a field takes the sorted scatter: at most 64 channels, a grid
-// within the bin budget, and a row count whose packed (row, mode) index fits
-// 32 bits.
+// within the bin budget, and a row count whose pairs fit the sort's counters
+// (packed (row, mode) indices fit 32 bits then, too).
 inline bool sorted_scatter_ok(const tfh_vm& vm, int64_t M, const SortWs& s) {
-  return s.order && vm.channels <= 64 && vm.grid_dim <= kSortMaxGrid && M < (1ll << 30);
+  return s.order && vm.channels <= 64 && vm.grid_dim <= kSortMaxGrid && M <= kSortMaxRows;
 }
 
 // Whether a field can take the walks' quad lanes.

@@ -184,7 +184,7 @@ struct InterpWs {
 constexpr int64_t kInterpSortPoints = 5 << 14;
 
 static size_t carve_interp(Carve& cv, const tfh_vm* vm, int64_t M, InterpWs& ws) {
-  if (M < kInterpSortPoints || M >= (1ll << 30) || vm->grid_dim > kSortMaxGrid ||
+  if (M < kInterpSortPoints || M > kSortMaxRows || vm->grid_dim > kSortMaxGrid ||
       !walk_ok(*vm, RowGrad{nullptr, (int)vm->channels}))
     return 0;
   ws.rows = cv.take<float>(M * 3 * vm->channels);
