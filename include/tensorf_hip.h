@@ -249,7 +249,8 @@ size_t tfh_train_step_workspace_size(const tfh_render_config* cfg, const tfh_mlp
 /* render_rays (render.py:105-279): rays -> out (R,3) for RGB, (R) for the
  * distance modes. jitter: (N) bbox / (R,N) contraction, NULL = none.
  * base_ts/base_steps: contraction schedule (N) or NULL. gumbel: (N) or NULL.
- * The workspace keeps the residuals tfh_render_bwd consumes. */
+ * camera_indices: (R), or NULL for camera 0 (here and in every render and
+ * training call). The workspace keeps the residuals tfh_render_bwd consumes. */
 int32_t tfh_render_fwd(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
                        const tfh_render_config* cfg, const float* aabb, const float* origins,
                        const float* directions, const uint32_t* camera_indices, int64_t num_rays,

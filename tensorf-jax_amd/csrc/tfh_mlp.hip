@@ -213,7 +213,7 @@ struct GatherTile {
     if constexpr (CAMS) {
       if (t < TM) {
         const int64_t r = row0 + t;
-        if (r < M) cam = (int)cams[ray_of(r)];
+        if (cams && r < M) cam = (int)cams[ray_of(r)];
       }
     }
     // lane k < 3 of a row takes its coordinate k; the others get the taps (all

@@ -412,7 +412,7 @@ struct BwdLds {
   static constexpr int bytes = oA0 + SH::FT * 2 * 64 * 16;
 };
 
-// FILM: cams (per ray), gembed (ncam x U, added to) and ncam >= 1.
+// FILM: cams (per ray; null: camera 0), gembed (ncam x U, added to) and ncam >= 1.
 // SPLIT0: layer 0 in two K parts and the doubled frequency from the first by
 // the double-angle identities (the training steps); else one K chain and a
 // sincosf per frequency.
@@ -541,7 +541,8 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     vd = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
         rd, (own3 && i3 < nv) ? (int)(rel * 3 + c3) * 4 : kOOB, 0, 0));
     if constexpr (FILM) {
-      const auto rc = buffer_rsrc(cams + ray0, nray * 4);
+      const auto rc = buffer_rsrc(cams ? static_cast<const void*>(cams + ray0) : dirs,
+                                  cams ? nray * 4 : 0);
       const unsigned atc = rem0 + (unsigned)t;
       const unsigned relc = one ? (atc >= rp ? 1u : 0u) : atc / rp;
       vcam = (int)__builtin_amdgcn_raw_buffer_load_b32(rc, t < nv ? (int)relc * 4 : kOOB, 0, 0);

@@ -247,7 +247,7 @@ constexpr int kFsLdB = 168;
 // rows, so an offset is 32 bits and rows past M read 0 with no branch; every
 // load is issued before the first LDS store and the tile pays one memory
 // latency. With CAMS also each row's camera index (Cs, clamped to [0, ncam),
-// from the per-ray cams). FB16: the feature rows go to LDS in BF16 (Fs is
+// from the per-ray cams; null: camera 0). FB16: the feature rows go to LDS in BF16 (Fs is
 // then __bf16 with stride kFsLdB), rounded as the BF16 strips round their A
 // operands. Requires F % 4 == 0 and 0 < rpr < 2^31.
 template <int TM, int NT, bool CAMS = false, bool FB16 = false>
@@ -268,8 +268,9 @@ __device__ void load_tile_rows(const MlpDims& d, const float* __restrict__ feats
   asm volatile("" : "+s"(fbase));
   const auto rf = buffer_rsrc(fbase, nv * d.F * 4);
   const auto rd = buffer_rsrc(dirs + ray0 * 3, nray * 12);
-  const auto rc = buffer_rsrc(CAMS ? static_cast<const void*>(cams + ray0) : feats,
-                              CAMS ? nray * 4 : 0);
+  const bool given = CAMS && cams != nullptr;
+  const auto rc = buffer_rsrc(given ? static_cast<const void*>(cams + ray0) : feats,
+                              given ? nray * 4 : 0);
   const int fp4 = d.FP / 4, f4 = d.F / 4, n4 = TM * fp4;
   const int kF4 = (n4 + NT - 1) / NT;  // constant for the specialised shape
   const int t = threadIdx.x;
