@@ -96,23 +96,27 @@ static PackOut<T> carve_tables(Carve& cv, const PackSizes& s) {
   return o;
 }
 
-// Carves and fills the weight tables of the operand precision.
+// Carves and (fill) fills the weight tables of the operand precision.
 static int32_t build_pack(const tfh_mlp* p, const MlpDims& d, bool bf, Carve& cv, MlpPack& pk,
-                          hipStream_t st) {
+                          hipStream_t st, bool fill = true) {
   pk = MlpPack{};
   PackSizes s = pack_sizes(d);
   if (bf) {
     PackOut<__bf16> o = carve_tables<__bf16>(cv, s);
     if (!cv.ok) return fail(TFH_ERR_WORKSPACE, "mlp: workspace too small for the weight tables");
-    ProfScope ps("mlp_pack", st);
-    hipLaunchKernelGGL(k_pack_weights<__bf16>, dim3(128), dim3(256), 0, st, d, to_w(p), o, s);
+    if (fill) {
+      ProfScope ps("mlp_pack", st);
+      hipLaunchKernelGGL(k_pack_weights<__bf16>, dim3(128), dim3(256), 0, st, d, to_w(p), o, s);
+    }
     pk.f0 = o.f0; pk.f1 = o.f1; pk.f2 = o.f2; pk.f3 = o.f3;
     pk.g0 = o.g0; pk.g1 = o.g1; pk.g2 = o.g2; pk.g3 = o.g3;
   } else {
     PackOut<float> o = carve_tables<float>(cv, s);
     if (!cv.ok) return fail(TFH_ERR_WORKSPACE, "mlp: workspace too small for the weight tables");
-    ProfScope ps("mlp_pack", st);
-    hipLaunchKernelGGL(k_pack_weights<float>, dim3(128), dim3(256), 0, st, d, to_w(p), o, s);
+    if (fill) {
+      ProfScope ps("mlp_pack", st);
+      hipLaunchKernelGGL(k_pack_weights<float>, dim3(128), dim3(256), 0, st, d, to_w(p), o, s);
+    }
     pk.ff0 = o.f0; pk.ff1 = o.f1; pk.ff2 = o.f2; pk.ff3 = o.f3;
     pk.fg0 = o.g0; pk.fg1 = o.g1; pk.fg2 = o.g2; pk.fg3 = o.g3;
   }
@@ -340,7 +344,8 @@ size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
   const BwdKind kind = bwd_kind(d);
   if (kind == BwdKind::kNone || force_partial()) return pack_bytes(d, bf) + partials;
   const int64_t rows = std::min<int64_t>(M, 131072);  // >= any chunk: a ray has at most 1024
-  return bwd_planes_table_bytes(kind, bf) + partials + pack_bytes(d, bf) +
+  const size_t flags = align_up((bwd_planes_pack_flags(kind) + bwd_blocks(M)) * sizeof(int32_t), 256);
+  return pack_bytes(d, bf) + bwd_planes_table_bytes(kind, bf) + partials + flags +
          align_up((size_t)kept_floats(rows) * sizeof(float), 256) +
          align_up((size_t)rows * 3 * sizeof(float), 256);
 }
@@ -353,7 +358,24 @@ static int32_t launch_reduce(const float* partials, int64_t nblk, const GradPack
   return check_launch("mlp bwd: reduce");
 }
 
-// act, rgb: kept by the fused step's forward, or null.
+// k_mlp_bwd over rows with its tables built, into the partials of nblk workgroups;
+// flags: see the kernel.
+static int32_t launch_bwd_any(const MlpDims& d, const MlpW& w, const MlpPack& pk, bool bf,
+                              const GradPack& gp, const float* feats, const float* dirs,
+                              const uint32_t* cams, const float* grgb, int64_t M, int64_t rpr,
+                              float* gfeat, float* partials, int64_t nblk, float* gembed,
+                              const int32_t* flags, int nflags, hipStream_t st) {
+  const size_t lds = bwd_lds_floats<kBwdTM>(d) * sizeof(float);
+  TFH_REQUIRE(lds <= 160 * 1024, "mlp bwd: tile needs %zu bytes of LDS", lds);
+  auto kernel = bf ? k_mlp_bwd<kBwdTM, kBwdNW, true> : k_mlp_bwd<kBwdTM, kBwdNW, false>;
+  allow_lds(kernel, lds);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)nblk), dim3(kBwdNW * 64), lds, st, d, w, pk, gp, feats,
+                     dirs, cams, grgb, M, rpr, gfeat, partials, gembed, flags, nflags);
+  return check_launch("mlp bwd");
+}
+
+// act, rgb: kept by the fused step's forward, which left its weight tables at
+// the start of ws; or null.
 int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rpr, const float* grgb, float* gfeat,
                      const tfh_mlp_grad* g, int32_t precision, void* ws, size_t ws_bytes,
@@ -367,26 +389,29 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   const BwdKind kind = bwd_kind(d);
   if (kind != BwdKind::kNone && !force_partial()) {
     BwdPlanesArgs a{};
+    MlpPack pk{};
+    TFH_TRY(build_pack(p, d, bf, cv, pk, st, act == nullptr));
     char* tables = cv.take<char>((int64_t)bwd_planes_table_bytes(kind, bf));
     a.tables = tables;
     a.max_blocks = num_cus();
     a.partials = cv.take<float>(nblk * gp.total);
+    const int pack_flags = bwd_planes_pack_flags(kind);
+    int32_t* flags = cv.take<int32_t>(pack_flags + nblk);
+    a.flags = flags + pack_flags;
     a.rpr = rpr;
     a.gp = gp;
     a.gembed = g->embed;
     a.ncam = d.ncam;
     const int64_t chunk = act ? M : std::min<int64_t>(M, bwd_chunk(rpr));
-    MlpPack pk{};
     float *kact = nullptr, *krgb = nullptr;
     if (!act) {
-      TFH_TRY(build_pack(p, d, bf, cv, pk, st));
       kact = cv.take<float>(kept_floats(chunk));
       krgb = cv.take<float>(chunk * 3);
     }
     if (!cv.ok)
       return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
                   mlp_bwd_workspace(p, M, precision));
-    TFH_TRY(pack_bwd_planes(kind, bf, to_w(p), tables, st));
+    TFH_TRY(pack_bwd_planes(kind, bf, to_w(p), tables, flags, st));
     for (int64_t c0 = 0; c0 < M; c0 += chunk) {
       const int64_t rows = std::min<int64_t>(chunk, M - c0);
       a.M = rows;
@@ -407,7 +432,14 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
         TFH_TRY(launch_bwd_planes_train(bf, to_w(p), a, st));
       else
         TFH_TRY(launch_bwd_planes_std(bf, to_w(p), a, st));
-      TFH_TRY(launch_reduce(a.partials, bwd_planes_blocks(bf, rows, a.max_blocks), gp, *g, st));
+      const int64_t blocks = bwd_planes_blocks(bf, rows, a.max_blocks);
+      // values that the planes cannot hold: the rows again with FP32 products
+      // (their embedding gradient is formed without planes: it stands)
+      if (!bf)
+        TFH_TRY(launch_bwd_any(d, to_w(p), pk, false, gp, a.feats, a.dirs, a.cams, a.grgb, rows,
+                               rpr, a.gfeat, a.partials, blocks, nullptr, flags,
+                               pack_flags + (int)blocks, st));
+      TFH_TRY(launch_reduce(a.partials, blocks, gp, *g, st));
     }
     return TFH_OK;
   }
@@ -417,23 +449,11 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
   if (!cv.ok)
     return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
                 mlp_bwd_workspace(p, M, precision));
-  const size_t lds = bwd_lds_floats<kBwdTM>(d) * sizeof(float);
-  TFH_REQUIRE(lds <= 160 * 1024, "mlp bwd: tile needs %zu bytes of LDS", lds);
   {
     ProfScope ps("mlp_bwd", st);
-    if (bf) {
-      allow_lds(k_mlp_bwd<kBwdTM, kBwdNW, true>, lds);
-      hipLaunchKernelGGL((k_mlp_bwd<kBwdTM, kBwdNW, true>), dim3((unsigned)nblk),
-                         dim3(kBwdNW * 64), lds, st, d, to_w(p), pk, gp, feats, dirs, cams, grgb,
-                         M, rpr, gfeat, partials, g->embed);
-    } else {
-      allow_lds(k_mlp_bwd<kBwdTM, kBwdNW, false>, lds);
-      hipLaunchKernelGGL((k_mlp_bwd<kBwdTM, kBwdNW, false>), dim3((unsigned)nblk),
-                         dim3(kBwdNW * 64), lds, st, d, to_w(p), pk, gp, feats, dirs, cams, grgb,
-                         M, rpr, gfeat, partials, g->embed);
-    }
+    TFH_TRY(launch_bwd_any(d, to_w(p), pk, bf, gp, feats, dirs, cams, grgb, M, rpr, gfeat,
+                           partials, nblk, g->embed, nullptr, 0, st));
   }
-  TFH_TRY(check_launch("mlp bwd"));
   return launch_reduce(partials, nblk, gp, *g, st);
 }
 

@@ -12,7 +12,10 @@
 //           product, under the rounding of an FP32 multiply-add. Six BF16
 //           products of K = 32 take 96 SIMD cycles where the eight
 //           v_mfma_f32_16x16x4_f32 they replace take 256. An operand that is
-//           infinite (or above BF16's largest finite value) gives NaN.
+//           infinite (or above BF16's largest finite value) makes NaN of every
+//           sum it enters: a workgroup that finds NaN in its sums says so in
+//           its flag, and k_mlp_bwd, launched behind this kernel, then does the
+//           batch again with FP32 products.
 //
 // One workgroup of 8 waves per CU walks tiles of TM rows; every weight-gradient
 // tile stays in registers of its owning wave for the whole kernel: wave w owns
@@ -94,6 +97,9 @@ struct BwdTables {
                        total = o_g3 + g3;  // values; a table of NP planes starts at NP * o
 };
 
+constexpr int kPackThreads = 256;
+constexpr float kBf16Max = 3.38953139e38f;  // BF16's largest finite value
+
 __device__ __forceinline__ void split3(float v, __bf16& h, __bf16& m, __bf16& l) {
   h = (__bf16)v;
   const float r = v - (float)h;
@@ -101,11 +107,14 @@ __device__ __forceinline__ void split3(float v, __bf16& h, __bf16& m, __bf16& l)
   l = (__bf16)(r - (float)m);
 }
 
+// flags (three planes): one per workgroup, whether it met a weight that the planes
+// cannot hold.
 template <class SH, int NP>
-__global__ void k_pack_bwd(MlpW w, __bf16* __restrict__ t) {
+__global__ void __launch_bounds__(kPackThreads) k_pack_bwd(MlpW w, __bf16* __restrict__ t,
+                                                          int32_t* __restrict__ flags) {
   using T = BwdTables<SH>;
+  static_assert(T::total % kPackThreads == 0, "every thread has an entry");
   const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= T::total) return;
   const int base = e < T::o_g0 ? 0 : (e < T::o_g1 ? T::o_g0 : (e < T::o_g2 ? T::o_g1
                  : (e < T::o_g3 ? T::o_g2 : T::o_g3)));
   const int kc = base == 0 ? SH::FK / 32 : (base == T::o_g1 || base == T::o_g2 ? kU / 32 : 1);
@@ -126,10 +135,17 @@ __global__ void k_pack_bwd(MlpW w, __bf16* __restrict__ t) {
     v = w.w3[j * 3 + k];
   }
   __bf16* o = t + NP * base + blk * NP * 512 + (f & 511);
-  if constexpr (NP == 1)
+  if constexpr (NP == 1) {
     o[0] = (__bf16)v;
-  else
+  } else {
     split3(v, o[0], o[512], o[1024]);
+    __shared__ int bad;
+    if (threadIdx.x == 0) bad = 0;
+    __syncthreads();
+    if (!(fabsf(v) <= kBf16Max)) bad = 1;
+    __syncthreads();
+    if (threadIdx.x == 0) flags[blockIdx.x] = bad;
+  }
 }
 
 // One lane's operand of a K = 32 product: 8 values in each plane.
@@ -417,13 +433,15 @@ struct BwdLds {
 // the double-angle identities (the training steps); else one K chain and a
 // sincosf per frequency.
 // KB: the kept activations are BF16 (else FP32).
+// flags (three planes): one per workgroup, whether its sums hold NaN.
 template <class SH, int NP, bool FILM, bool SPLIT0, bool KB>
 __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     MlpW w, const __bf16* __restrict__ tables, const float* __restrict__ feats,
     const float* __restrict__ dirs, const float* __restrict__ grgb, int64_t M, int64_t rpr,
     float* __restrict__ gfeat, float* __restrict__ partials, GradPack gp,
     const float* __restrict__ act, const float* __restrict__ rgb_in,
-    const uint32_t* __restrict__ cams, float* __restrict__ gembed, int ncam) {
+    const uint32_t* __restrict__ cams, float* __restrict__ gembed, int ncam,
+    int32_t* __restrict__ flags) {
   using L = BwdLds<SH, NP, SPLIT0>;
   using T = BwdTables<SH>;
   static_assert(!KB || NP == 1, "BF16 activations are the BF16 MLP's");
@@ -981,7 +999,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
     for (int c = 0; c < 3; ++c) part[gp.w3 + ucol * 3 + c] = dw3[c];
   }
   if (t < 3 * TM) Z3[t] = db3;  // thread t: colour t % 3
+  int* Bad = Cs;
+  if (t == 0) Bad[0] = 0;
   __syncthreads();
+  bool nan = false;
+  const auto put = [&](int64_t at, float v) TFH_INLINE {
+    part[at] = v;
+    nan |= v != v;
+  };
   if (t < 3) {
     float s = 0.0f;
     for (int i = 0; i < TM; ++i) s += Z3[3 * i + t];
@@ -991,14 +1016,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
   for (int i = 0; i < kU / 16; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      part[gp.w2 + (16 * i + 4 * kq4 + e) * kU + ucol] = a2[i][e];
+      put(gp.w2 + (16 * i + 4 * kq4 + e) * kU + ucol, a2[i][e]);
 #pragma unroll
   for (int i = 0; i < XTN; ++i)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int h = SH::NH > 1 && i >= SH::xt0(SH::NH - 1) ? SH::NH - 1 : 0;
       const int o = SH::x_orig(h, 16 * (i - SH::xt0(h)) + 4 * kq4 + e);
-      if (o >= 0) part[gp.w1 + o * kU + ucol] = a1[i][e];
+      if (o >= 0) put(gp.w1 + o * kU + ucol, a1[i][e]);
     }
   for (int ft = wave; ft < SH::FT; ft += NW)
 #pragma unroll
@@ -1007,9 +1032,14 @@ __global__ void __launch_bounds__(512) k_mlp_bwd_planes(
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         const int f = 16 * ft + 4 * kq4 + e, scol = 16 * j + r16;
-        if (f < SH::F && scol < SH::S) part[gp.w0 + f * SH::S + scol] = v[e];
+        if (f < SH::F && scol < SH::S) put(gp.w0 + f * SH::S + scol, v[e]);
       }
     }
+  if constexpr (NP == 3) {
+    if (nan) Bad[0] = 1;
+    __syncthreads();
+    if (t == 0) flags[blockIdx.x] = Bad[0];
+  }
 }
 
 template <class SH, int NP, bool FILM, bool SPLIT0, bool KB>
@@ -1021,19 +1051,19 @@ int32_t run_planes(const MlpW& w, const BwdPlanesArgs& a, hipStream_t st) {
   static_assert(L::TM == (NP == 1 ? kBwdRowsBf16 : kBwdRowsFp32), "bwd_planes_blocks");
   hipLaunchKernelGGL(kernel, dim3((unsigned)bwd_planes_blocks(NP == 1, a.M, a.max_blocks)), dim3(512), L::bytes, st, w,
                      static_cast<const __bf16*>(a.tables), a.feats, a.dirs, a.grgb, a.M, a.rpr,
-                     a.gfeat, a.partials, a.gp, a.act, a.rgb, a.cams, a.gembed, a.ncam);
+                     a.gfeat, a.partials, a.gp, a.act, a.rgb, a.cams, a.gembed, a.ncam, a.flags);
   return check_launch("mlp bwd");
 }
 
 template <class SH>
-int32_t pack_planes(bool bf, const MlpW& w, void* tables, hipStream_t st) {
-  const dim3 grid((BwdTables<SH>::total + 255) / 256);
+int32_t pack_planes(bool bf, const MlpW& w, void* tables, int32_t* flags, hipStream_t st) {
+  const dim3 grid(BwdTables<SH>::total / kPackThreads);
   if (bf)
-    hipLaunchKernelGGL((k_pack_bwd<SH, 1>), grid, dim3(256), 0, st, w,
-                       static_cast<__bf16*>(tables));
+    hipLaunchKernelGGL((k_pack_bwd<SH, 1>), grid, dim3(kPackThreads), 0, st, w,
+                       static_cast<__bf16*>(tables), flags);
   else
-    hipLaunchKernelGGL((k_pack_bwd<SH, 3>), grid, dim3(256), 0, st, w,
-                       static_cast<__bf16*>(tables));
+    hipLaunchKernelGGL((k_pack_bwd<SH, 3>), grid, dim3(kPackThreads), 0, st, w,
+                       static_cast<__bf16*>(tables), flags);
   return check_launch("mlp bwd: operand tables");
 }
 

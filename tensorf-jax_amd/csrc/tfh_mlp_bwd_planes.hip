@@ -9,9 +9,15 @@ size_t bwd_planes_table_bytes(BwdKind kind, bool bf) {
   return align_up((size_t)total * 2 * (bf ? 1 : 3), 256);
 }
 
-int32_t pack_bwd_planes(BwdKind kind, bool bf, const MlpW& w, void* tables, hipStream_t st) {
-  return kind == BwdKind::kStd ? pack_planes<BwdStd>(bf, w, tables, st)
-                               : pack_planes<BwdDef>(bf, w, tables, st);
+int bwd_planes_pack_flags(BwdKind kind) {
+  return (kind == BwdKind::kStd ? BwdTables<BwdStd>::total : BwdTables<BwdDef>::total) /
+         kPackThreads;
+}
+
+int32_t pack_bwd_planes(BwdKind kind, bool bf, const MlpW& w, void* tables, int32_t* flags,
+                        hipStream_t st) {
+  return kind == BwdKind::kStd ? pack_planes<BwdStd>(bf, w, tables, flags, st)
+                               : pack_planes<BwdDef>(bf, w, tables, flags, st);
 }
 
 int32_t launch_bwd_planes_train(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st) {

@@ -778,7 +778,9 @@ __device__ __forceinline__ void wgrad_phase(int wave, int n, int tcols, const fl
 constexpr int kBwdNW = 8;
 
 // The backward of any shape, recomputing each tile's forward (the shapes with
-// compile-time dims have k_mlp_bwd_planes, tfh_mlp_bwd_planes.h).
+// compile-time dims have k_mlp_bwd_planes, tfh_mlp_bwd_planes.h). With flags
+// (nflags of them, written by the launches before) it does so only if one is
+// set. gembed null: the embedding's gradient is left out.
 template <int TM, int NW, bool BF>
 __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack pk, GradPack gp,
                                                      const float* __restrict__ feats,
@@ -787,7 +789,9 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
                                                      const float* __restrict__ grgb, int64_t M,
                                                      int64_t rpr, float* __restrict__ gfeat,
                                                      float* __restrict__ partials,
-                                                     float* __restrict__ gembed) {
+                                                     float* __restrict__ gembed,
+                                                     const int32_t* __restrict__ flags,
+                                                     int nflags) {
   constexpr int RT = TM / 16;
   static_assert(TM <= 64, "the FiLM camera check reads one tile row per lane");
   // row tiles per work item of the strip phases: all of them (the B strip is
@@ -815,6 +819,17 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
 
   const int wave = threadIdx.x >> 6;
   const int lane = lane_id();
+  if (flags) {
+    int any = 0;
+    for (int i = threadIdx.x; i < nflags; i += blockDim.x) any |= flags[i];
+    int* set = reinterpret_cast<int*>(smem);
+    if (threadIdx.x == 0) *set = 0;
+    __syncthreads();
+    if (any) *set = 1;
+    __syncthreads();
+    if (*set == 0) return;  // the whole workgroup
+    __syncthreads();
+  }
   float* part = partials + (int64_t)blockIdx.x * gp.total;
   if (d.ncam > 0) {
     for (int c = threadIdx.x; c < kU; c += blockDim.x) Eacc[c] = 0.0f;
@@ -845,7 +860,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
       const int rc = Run[1];
       if (tc >= 0 && rc >= 0 && rc != tc) {
         for (int c = lane; c < kU; c += 64) {
-          unsafeAtomicAdd(gembed + (size_t)rc * kU + c, Eacc[c]);
+          if (gembed) unsafeAtomicAdd(gembed + (size_t)rc * kU + c, Eacc[c]);
           Eacc[c] = 0.0f;
         }
       }
@@ -897,7 +912,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
               if (tcam >= 0) {
                 sh += g * hp;
                 sg += g;
-              } else {
+              } else if (gembed) {
                 float* gemb = gembed + (size_t)Cs[row] * kU;
                 unsafeAtomicAdd(gemb + col - kU / 2, g * hp);
                 unsafeAtomicAdd(gemb + col, g);
@@ -1010,7 +1025,7 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_bwd(MlpDims d, MlpW w, MlpPack 
   if (d.ncam > 0) {
     __syncthreads();
     const int rc = Run[1];
-    if (rc >= 0)
+    if (rc >= 0 && gembed)
       for (int c = threadIdx.x; c < kU; c += blockDim.x)
         unsafeAtomicAdd(gembed + (size_t)rc * kU + c, Eacc[c]);
   }
@@ -1073,9 +1088,12 @@ struct BwdPlanesArgs {
   const float *act, *rgb;  // kept by the forward
   float* gembed;
   int ncam;
+  int32_t* flags;  // (workgroups): NaN among its sums (FP32)
 };
 size_t bwd_planes_table_bytes(BwdKind kind, bool bf);
-int32_t pack_bwd_planes(BwdKind kind, bool bf, const MlpW& w, void* tables, hipStream_t st);
+int bwd_planes_pack_flags(BwdKind kind);  // flags of pack_bwd_planes (FP32)
+int32_t pack_bwd_planes(BwdKind kind, bool bf, const MlpW& w, void* tables, int32_t* flags,
+                        hipStream_t st);
 int32_t launch_bwd_planes_train(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
 int32_t launch_bwd_planes_std(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
 int32_t launch_bwd_planes_def(bool bf, const MlpW& w, const BwdPlanesArgs& a, hipStream_t st);
