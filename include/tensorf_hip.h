@@ -156,9 +156,10 @@ int32_t tfh_vm_interpolate_bwd(const tfh_vm* vm, const float* ijk, int64_t num_p
                                const float* grad_out, const tfh_vm_grad* grad,
                                tfh_stream_t stream);
 /* tfh_vm_interpolate_bwd for many points in no particular order, which it
- * sorts by cell in a workspace of tfh_vm_interpolate_bwd_workspace_size bytes
- * (0: few points, or a field it does not sort for; then it is
- * tfh_vm_interpolate_bwd). No counterpart in the reference. */
+ * sorts by cell, at most 4 Mi points at a time, in a workspace of
+ * tfh_vm_interpolate_bwd_workspace_size bytes (0: few points, or a field it does
+ * not sort for; then it is tfh_vm_interpolate_bwd). No counterpart in the
+ * reference. */
 size_t tfh_vm_interpolate_bwd_workspace_size(const tfh_vm* vm, int64_t num_points);
 int32_t tfh_vm_interpolate_bwd_sorted(const tfh_vm* vm, const float* ijk, int64_t num_points,
                                       const float* grad_out, const tfh_vm_grad* grad,

@@ -156,15 +156,17 @@ int32_t sum_copies(const float* copies, int ncopy, int64_t len, float* dst, hipS
   return check_launch("sum gradient copies");
 }
 
-// (rows, m) -> (m, rows): 64 x 64 tiles through LDS, 256 contiguous bytes each way.
+// (rows, m), rows `ld` apart, -> (m, rows): 64 x 64 tiles through LDS, 256
+// contiguous bytes each way.
 __global__ void __launch_bounds__(256) k_transpose(const float* __restrict__ in, int rows,
-                                                   int64_t m, float* __restrict__ out) {
+                                                   int64_t m, int64_t ld,
+                                                   float* __restrict__ out) {
   __shared__ float tile[64][65];
   const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
   const int64_t s0 = (int64_t)blockIdx.x * 64;
   const int c0 = blockIdx.y * 64;
   for (int c = y; c < 64 && c0 + c < rows; c += 4)
-    if (s0 + x < m) tile[c][x] = in[(int64_t)(c0 + c) * m + s0 + x];
+    if (s0 + x < m) tile[c][x] = in[(int64_t)(c0 + c) * ld + s0 + x];
   __syncthreads();
   for (int i = y; i < 64 && s0 + i < m; i += 4)
     if (c0 + x < rows) out[(s0 + i) * rows + c0 + x] = tile[x][i];
@@ -176,19 +178,24 @@ __global__ void __launch_bounds__(256) k_transpose(const float* __restrict__ in,
 // bytes a point at 48 channels), the walks by the reads of the rows and of
 // the other factor. Forward and backward at G = 300, 48 channels, direct and sorted:
 // 66 thousand points 246 and 258 us, 130 thousand 450 and 358, 250 thousand 849
-// and 571; at G = 128 a million 3224 and 1648.
+// and 571; at G = 128 a million 3224 and 1648. A point takes 12C + 30 bytes, so
+// larger batches go in equal parts of at most kInterpPart points (2.5 GB at 48
+// channels).
 struct InterpWs {
-  float* rows;  // (M, 3C)
+  int64_t part;  // points at a time
+  float* rows;   // (part, 3C)
   SortWs sort;
 };
-constexpr int64_t kInterpSortPoints = 5 << 14;
+constexpr int64_t kInterpSortPoints = 5 << 14, kInterpPart = 1 << 22;
+static_assert(kInterpPart <= kSortMaxRows, "a part can be sorted");
 
 static size_t carve_interp(Carve& cv, const tfh_vm* vm, int64_t M, InterpWs& ws) {
-  if (M < kInterpSortPoints || M > kSortMaxRows || vm->grid_dim > kSortMaxGrid ||
+  if (M < kInterpSortPoints || vm->grid_dim > kSortMaxGrid ||
       !walk_ok(*vm, RowGrad{nullptr, (int)vm->channels}))
     return 0;
-  ws.rows = cv.take<float>(M * 3 * vm->channels);
-  take_sort_ws(cv, M, ws.sort);
+  ws.part = ceil_div(M, ceil_div(M, kInterpPart));
+  ws.rows = cv.take<float>(ws.part * 3 * vm->channels);
+  take_sort_ws(cv, ws.part, ws.sort);
   return cv.off;
 }
 
@@ -248,16 +255,20 @@ int32_t tfh_vm_interpolate_bwd_sorted(const tfh_vm* vm, const float* ijk, int64_
   TFH_TRY(require_device());
   const hipStream_t st = as_stream(stream);
   const int rows = 3 * (int)vm->channels;
-  {
-    ProfScope ps("scatter_transpose", st);
-    hipLaunchKernelGGL(k_transpose,
-                       dim3((unsigned)ceil_div(num_points, 64), (unsigned)ceil_div(rows, 64)),
-                       dim3(256), 0, st, grad_out, rows, num_points, ws.rows);
-    TFH_TRY(check_launch("tfh_vm_interpolate_bwd_sorted: transpose"));
+  for (int64_t at = 0; at < num_points; at += ws.part) {
+    const int64_t n = std::min<int64_t>(ws.part, num_points - at);
+    {
+      ProfScope ps("scatter_transpose", st);
+      hipLaunchKernelGGL(k_transpose,
+                         dim3((unsigned)ceil_div(n, 64), (unsigned)ceil_div(rows, 64)), dim3(256),
+                         0, st, grad_out + at, rows, n, num_points, ws.rows);
+      TFH_TRY(check_launch("tfh_vm_interpolate_bwd_sorted: transpose"));
+    }
+    const PlanarPoints src{ijk + at, num_points};
+    TFH_TRY(scatter_scattered_rows(*vm, src, n, RowGrad{ws.rows, (int)vm->channels}, *grad,
+                                   ws.sort, st));
   }
-  const PlanarPoints src{ijk, num_points};
-  return scatter_scattered_rows(*vm, src, num_points, RowGrad{ws.rows, (int)vm->channels}, *grad,
-                                ws.sort, st);
+  return TFH_OK;
 }
 
 int32_t tfh_zero_arrays(float* const* arrays, const int64_t* counts, int32_t num,

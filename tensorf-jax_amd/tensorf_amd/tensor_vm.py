@@ -77,8 +77,13 @@ class _Interpolate(torch.autograd.Function):
         # (never for so few points: not asked, the call is 4 us of a small step's 155)
         need = 0 if m < 65536 else int(
             _lib.lib.tfh_vm_interpolate_bwd_workspace_size(ctypes.byref(vm), m))
+        ws = None
         if need:
-            ws = torch.empty(need, dtype=torch.uint8, device=plane.device)
+            try:
+                ws = torch.empty(need, dtype=torch.uint8, device=plane.device)
+            except torch.OutOfMemoryError:
+                pass  # the direct scatter needs no room
+        if ws is not None:
             _lib.call("tfh_vm_interpolate_bwd_sorted", ctypes.byref(vm), _lib.ptr(ijk), m,
                       _lib.ptr(gout), ctypes.byref(grad), _lib.ptr(ws), need, _lib.stream())
         else:
