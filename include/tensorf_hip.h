@@ -234,12 +234,16 @@ int32_t tfh_feature_mlp_bwd(const tfh_mlp* mlp, const float* features, const flo
                             tfh_stream_t stream);
 
 /* ---- render_rays -------------------------------------------------------- */
-/* Workspace of tfh_render_fwd / tfh_render_bwd / tfh_train_step for R rays. */
+/* Workspace of tfh_render_fwd / tfh_render_bwd (or tfh_train_step) for R rays. */
 size_t tfh_render_workspace_size(const tfh_render_config* cfg, const tfh_mlp* mlp,
                                  int64_t appearance_channels, int64_t num_rays);
+/* Workspace of tfh_render_only. */
+size_t tfh_render_only_workspace_size(const tfh_render_config* cfg, const tfh_mlp* mlp,
+                                      int64_t appearance_channels, int64_t num_rays);
 /* Workspace that lets tfh_train_step keep the feature MLP's hidden
- * activations (1 KB per shaded sample, standard 48-channel shape, with or
- * without a camera embedding) between its forward and backward instead of
+ * activations (1 KB per shaded sample, 512 bytes with the BF16 MLP, for the
+ * shapes of 48 channels with 2 frequencies and 24 with 6, with or without a
+ * camera embedding) between its forward and backward instead of
  * recomputing layers 1-3, plus 12 MB for copies of the factor-line gradients
  * that spread the scatters' atomics; with a tfh_render_workspace_size
  * workspace it recomputes the activations and adds straight into the
@@ -258,8 +262,8 @@ int32_t tfh_render_fwd(const tfh_vm* density, const tfh_vm* appearance, const tf
                        const float* jitter, const float* base_ts, const float* base_steps,
                        const float* gumbel, float* out, void* workspace, size_t workspace_bytes,
                        tfh_stream_t stream);
-/* tfh_render_fwd when no tfh_render_bwd follows: the same output, and the
- * feature rows are not written where only the backward reads them. */
+/* tfh_render_fwd when no tfh_render_bwd follows: the same output from a
+ * workspace without what only the backward needs. */
 int32_t tfh_render_only(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
                         const tfh_render_config* cfg, const float* aabb, const float* origins,
                         const float* directions, const uint32_t* camera_indices, int64_t num_rays,
@@ -283,8 +287,8 @@ int32_t tfh_render_bwd(const tfh_vm* density, const tfh_vm* appearance, const tf
  * inside the library, one per device, held from the first call on that device
  * until the process ends; the call allocates nothing. A call whose residuals
  * do not fit returns TFH_ERR_WORKSPACE before any device work: per ray they
- * take about 32 N + 592 k bytes in RGB mode with 48 appearance channels
- * (N=512, k=64: ~2,400 rays per call). Results equal tfh_render_fwd's. Calls
+ * take about 28 N + 592 k bytes in RGB mode with 48 appearance channels
+ * (N=512, k=64: ~2,500 rays per call). Results equal tfh_render_fwd's. Calls
  * on one device share the array: calls that overlap on one device (several
  * streams or host threads) race. The backward (tfh_render_bwd) needs the
  * workspace of tfh_render_fwd and cannot follow this call. */

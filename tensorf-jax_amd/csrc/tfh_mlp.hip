@@ -136,7 +136,12 @@ bool mlp_keeps_activations(const tfh_mlp* p, int32_t precision) {
          !force_partial();
 }
 
-int64_t mlp_kept_floats(int64_t rows) { return kept_floats(rows); }
+// Bytes that the forward of a fused step keeps of `rows` rows (0: it does not).
+size_t mlp_kept_bytes(const tfh_mlp* p, int64_t rows, int32_t precision) {
+  if (!mlp_keeps_activations(p, precision)) return 0;
+  const bool bf = precision == TFH_PREC_BF16;
+  return align_up(kept_bytes(rows, kept_bf16(make_dims(p, bf), bf, true)), 256);
+}
 
 // The forward over feature rows with its tables built; kb: act in BF16.
 static int32_t launch_fwd(const MlpDims& d, const MlpW& w, const MlpPack& pk, bool bf, bool kb,
@@ -331,11 +336,13 @@ static int64_t bwd_blocks(int64_t M) {
 // keeping them, and the backward on it in turn over this many rows (of whole
 // rays): 16 tiles of 32 rows per CU, whose activations (134 MB) the Infinity
 // Cache holds, and a workspace that does not grow with the batch past that.
+constexpr int64_t kBwdChunk = 131072;
 static int64_t bwd_chunk(int64_t rpr) {
-  const int64_t rows = 131072;
-  return rpr >= rows ? rpr : rows / rpr * rpr;
+  return rpr >= kBwdChunk ? rpr : kBwdChunk / rpr * rpr;
 }
 
+// The workspace of mlp_bwd_rows, and what it needs besides where the forward
+// kept no activations.
 size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
   const bool bf = precision == TFH_PREC_BF16;
   MlpDims d = make_dims(p, bf);
@@ -343,10 +350,15 @@ size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
   const size_t partials = align_up((size_t)bwd_blocks(M) * gp.total * sizeof(float), 256);
   const BwdKind kind = bwd_kind(d);
   if (kind == BwdKind::kNone || force_partial()) return pack_bytes(d, bf) + partials;
-  const int64_t rows = std::min<int64_t>(M, 131072);  // >= any chunk: a ray has at most 1024
   const size_t flags = align_up((bwd_planes_pack_flags(kind) + bwd_blocks(M)) * sizeof(int32_t), 256);
-  return pack_bytes(d, bf) + bwd_planes_table_bytes(kind, bf) + partials + flags +
-         align_up((size_t)kept_floats(rows) * sizeof(float), 256) +
+  return pack_bytes(d, bf) + bwd_planes_table_bytes(kind, bf) + partials + flags;
+}
+
+size_t mlp_recompute_workspace(const tfh_mlp* p, int64_t M, int32_t precision) {
+  if (!mlp_keeps_activations(p, precision)) return 0;
+  const bool bf = precision == TFH_PREC_BF16;
+  const int64_t rows = std::min<int64_t>(M, kBwdChunk);  // >= any chunk: a ray has at most 1024
+  return align_up(kept_bytes(rows, kept_bf16(make_dims(p, bf), bf, false)), 256) +
          align_up((size_t)rows * 3 * sizeof(float), 256);
 }
 
@@ -375,12 +387,12 @@ static int32_t launch_bwd_any(const MlpDims& d, const MlpW& w, const MlpPack& pk
 }
 
 // act, rgb: kept by the fused step's forward, which left its weight tables at
-// the start of ws; or null.
+// the start of ws; or null, and rws then has mlp_recompute_workspace bytes.
 int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rpr, const float* grgb, float* gfeat,
                      const tfh_mlp_grad* g, int32_t precision, void* ws, size_t ws_bytes,
-                     hipStream_t st, const float* act = nullptr,
-                     const float* rgb = nullptr) {
+                     hipStream_t st, const float* act, const float* rgb, void* rws,
+                     size_t rws_bytes) {
   const bool bf = precision == TFH_PREC_BF16;
   MlpDims d = make_dims(p, bf);
   GradPack gp = make_pack(d);
@@ -405,12 +417,16 @@ int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, co
     const int64_t chunk = act ? M : std::min<int64_t>(M, bwd_chunk(rpr));
     float *kact = nullptr, *krgb = nullptr;
     if (!act) {
-      kact = cv.take<float>(kept_floats(chunk));
-      krgb = cv.take<float>(chunk * 3);
+      Carve rcv(rws, rws_bytes);
+      kact = reinterpret_cast<float*>(
+          rcv.take<char>((int64_t)kept_bytes(chunk, kept_bf16(d, bf, false))));
+      krgb = rcv.take<float>(chunk * 3);
+      cv.ok &= rcv.ok;
     }
     if (!cv.ok)
-      return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu bytes, need %zu", ws_bytes,
-                  mlp_bwd_workspace(p, M, precision));
+      return fail(TFH_ERR_WORKSPACE, "mlp bwd: workspace of %zu + %zu bytes, need %zu + %zu",
+                  ws_bytes, rws_bytes, mlp_bwd_workspace(p, M, precision),
+                  act ? 0 : mlp_recompute_workspace(p, M, precision));
     TFH_TRY(pack_bwd_planes(kind, bf, to_w(p), tables, flags, st));
     for (int64_t c0 = 0; c0 < M; c0 += chunk) {
       const int64_t rows = std::min<int64_t>(chunk, M - c0);
@@ -488,7 +504,8 @@ int32_t tfh_feature_mlp_fwd(const tfh_mlp* mlp, const float* features, const flo
 size_t tfh_feature_mlp_bwd_workspace_size(const tfh_mlp* mlp, int64_t num_rows,
                                           int32_t precision) {
   if (check_mlp(mlp, "tfh_feature_mlp_bwd_workspace_size") != TFH_OK || num_rows < 0) return 0;
-  return mlp_bwd_workspace(mlp, num_rows, precision);
+  return mlp_bwd_workspace(mlp, num_rows, precision) +
+         mlp_recompute_workspace(mlp, num_rows, precision);
 }
 
 int32_t tfh_feature_mlp_bwd(const tfh_mlp* mlp, const float* features, const float* viewdirs,
@@ -507,9 +524,10 @@ int32_t tfh_feature_mlp_bwd(const tfh_mlp* mlp, const float* features, const flo
   TFH_REQUIRE(mlp->embed == nullptr || (camera_indices && grad->embed),
               "tfh_feature_mlp_bwd: camera_indices and grad->embed required with an embedding");
   TFH_TRY(require_device());
+  const size_t part = std::min(workspace_bytes, mlp_bwd_workspace(mlp, num_rows, precision));
   return mlp_bwd_rows(mlp, features, viewdirs, camera_indices, num_rows, 1, grad_rgb,
-                      grad_features, grad, precision, workspace, workspace_bytes,
-                      as_stream(stream));
+                      grad_features, grad, precision, workspace, part, as_stream(stream), nullptr,
+                      nullptr, static_cast<char*>(workspace) + part, workspace_bytes - part);
 }
 
 }  // extern "C"

@@ -67,8 +67,9 @@ constexpr int kKeptGroup = 32;                       // rows
 constexpr int kKeptHalf = kKeptGroup * 128;          // values of relu(z1) of a group
 template <bool BF>
 constexpr int kKeptGroupBytes = 2 * kKeptHalf * (BF ? 2 : 4);
-inline int64_t kept_floats(int64_t rows) {           // room for FP32 values
-  return (rows + kKeptGroup - 1) / kKeptGroup * 2 * kKeptHalf;
+inline size_t kept_bytes(int64_t rows, bool bf) {
+  return (size_t)((rows + kKeptGroup - 1) / kKeptGroup) *
+         (bf ? kKeptGroupBytes<true> : kKeptGroupBytes<false>);
 }
 
 template <bool BF>

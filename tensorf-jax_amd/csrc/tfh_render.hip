@@ -23,8 +23,8 @@ namespace tfh {
 
 int32_t check_mlp(const tfh_mlp* p, const char* who);
 // act (optional): activations the forward keeps for the backward
-// (mlp_kept_floats(M) floats),
-// which then also reads the forward's rgb; only for mlp_keeps_activations().
+// (mlp_kept_bytes(); 0: it does not), which then also reads the forward's rgb;
+// without them the backward forms them again in rws.
 int32_t mlp_fwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rows_per_ray, float* rgb, int32_t precision, void* ws,
                      size_t ws_bytes, hipStream_t st, float* act = nullptr);
@@ -33,12 +33,13 @@ int32_t mlp_fwd_rows_gather(const tfh_mlp* p, const tfh_vm& vm, const RaySamples
                             int64_t rpr, float* rgb, int32_t precision, void* ws,
                             size_t ws_bytes, hipStream_t st, float* act, bool* done);
 size_t mlp_bwd_workspace(const tfh_mlp* p, int64_t M, int32_t precision);
+size_t mlp_recompute_workspace(const tfh_mlp* p, int64_t M, int32_t precision);
 int32_t mlp_bwd_rows(const tfh_mlp* p, const float* feats, const float* dirs, const uint32_t* cams,
                      int64_t M, int64_t rows_per_ray, const float* grgb, float* gfeat,
                      const tfh_mlp_grad* g, int32_t precision, void* ws, size_t ws_bytes,
-                     hipStream_t st, const float* act = nullptr, const float* rgb = nullptr);
-bool mlp_keeps_activations(const tfh_mlp* p, int32_t precision);
-int64_t mlp_kept_floats(int64_t rows);
+                     hipStream_t st, const float* act, const float* rgb, void* rws,
+                     size_t rws_bytes);
+size_t mlp_kept_bytes(const tfh_mlp* p, int64_t rows, int32_t precision);
 // hyper (optional, device): -lr_lo * decay, -lr_hi * decay, 1 - b1^count,
 // 1 - b2^count, read by the kernel in place of the host values.
 int32_t adam_launch(float* p, float* g, float* m, float* v, int64_t n, int64_t split, float lr_lo,
@@ -547,6 +548,8 @@ struct RenderWs {
   float* dfeat;  // (M, F)
   void* mlp_ws;
   size_t mlp_ws_bytes;
+  void* mlp_rws = nullptr;  // where the backward forms the activations again
+  size_t mlp_rws_bytes = 0;
   float* act = nullptr;  // MLP activations kept for the backward, or null
   float* mse_part = nullptr;  // kLossSlots partial sums of the MSE
   // copies of the density / appearance line gradients for the scatters, or null
@@ -576,12 +579,13 @@ static int32_t check_cfg(const tfh_render_config* cfg, const char* who) {
   return TFH_OK;
 }
 
-static size_t carve_render(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t F,
-                           int64_t R, RenderWs& ws) {
+// The part of a layout with a backward that does not depend on where its
+// activations come from.
+static void carve_step(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t F,
+                       int64_t R, RenderWs& ws) {
   const int64_t N = cfg->density_samples_per_ray, k = cfg->appearance_samples_per_ray;
   const int64_t M = R * k;
   ws.d.pts = cv.take<float>(R * N * 3);
-  cv.take<float>(R * N);  // (unused)
   ws.d.sigma = cv.take<float>(R * N);
   ws.d.delta = cv.take<float>(R * N);
   ws.d.w = cv.take<float>(R * N);
@@ -604,25 +608,25 @@ static size_t carve_render(Carve& cv, const tfh_render_config* cfg, const tfh_ml
     ws.ds = cv.take<float>(R * N);
     take_sort_ws(cv, R * N, ws.sort);  // pairs of every sample (k <= N)
   }
+}
+
+static size_t recompute_bytes(const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R) {
+  return mlp ? mlp_recompute_workspace(mlp, R * cfg->appearance_samples_per_ray,
+                                       cfg->mlp_precision)
+             : 0;
+}
+
+static void take_recompute(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R,
+                           RenderWs& ws) {
+  ws.mlp_rws_bytes = recompute_bytes(cfg, mlp, R);
+  ws.mlp_rws = cv.take<char>((int64_t)ws.mlp_rws_bytes);
+}
+
+static size_t carve_render(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t F,
+                           int64_t R, RenderWs& ws) {
+  carve_step(cv, cfg, mlp, F, R, ws);
+  take_recompute(cv, cfg, mlp, R, ws);
   return cv.off;
-}
-
-// The fused training steps keep the MLP's hidden activations between its
-// forward and backward (the backward then recomputes only layer 0 and the
-// encoding) when the shape allows it and the workspace has the room: 1 KB per
-// shaded sample past the render workspace.
-static size_t act_bytes(const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R) {
-  if (!mlp_keeps_activations(mlp, cfg->mlp_precision)) return 0;
-  return align_up((size_t)mlp_kept_floats(R * cfg->appearance_samples_per_ray) * sizeof(float),
-                  256);
-}
-
-static void take_act(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R,
-                     RenderWs& ws) {
-  ws.act = nullptr;
-  const size_t bytes = act_bytes(cfg, mlp, R);
-  if (bytes == 0 || !cv.ok || cv.off + bytes > cv.cap) return;
-  ws.act = cv.take<float>((int64_t)(bytes / sizeof(float)));
 }
 
 // The training steps' scatters add the factor-line gradients into copies
@@ -632,6 +636,16 @@ static void take_act(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp
 // queries reserve 8 MB (appearance) + 4 MB (density) for them; up to 256
 // copies of each fit.
 constexpr size_t kALineCopyBytes = 8u << 20, kDLineCopyBytes = 4u << 20;
+
+// The fused training steps keep the MLP's hidden activations between its
+// forward and backward (the backward then recomputes only layer 0 and the
+// encoding) when the shape allows it and the workspace is of the size that the
+// queries give: 1 KB (BF16: 512 bytes) per shaded sample, in the place where a
+// smaller workspace has the room to form them again.
+static size_t train_bytes(const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R) {
+  return std::max(mlp_kept_bytes(mlp, R * cfg->appearance_samples_per_ray, cfg->mlp_precision),
+                  recompute_bytes(cfg, mlp, R));
+}
 
 static size_t line_copy_bytes() {
   return align_up(kALineCopyBytes, 256) + align_up(kDLineCopyBytes, 256);
@@ -658,6 +672,17 @@ static void take_line_copies(Carve& cv, const tfh_vm* density, const tfh_vm* app
     ws.dlcopy = cv.take<float>(df);
     ws.dnlc = dn;
   }
+}
+
+// The rest of a training step's workspace behind carve_step.
+static void take_train(Carve& cv, const tfh_render_config* cfg, const tfh_mlp* mlp, int64_t R,
+                       const tfh_vm* density, const tfh_vm* appearance, RenderWs& ws) {
+  const size_t act = mlp_kept_bytes(mlp, R * cfg->appearance_samples_per_ray, cfg->mlp_precision);
+  const bool keep =
+      act > 0 && cv.ok && cv.off + train_bytes(cfg, mlp, R) + line_copy_bytes() <= cv.cap;
+  if (!keep) take_recompute(cv, cfg, mlp, R, ws);
+  take_line_copies(cv, density, appearance, ws);
+  ws.act = keep ? reinterpret_cast<float*>(cv.take<char>((int64_t)act)) : nullptr;
 }
 
 static RayIn make_rayin(const tfh_render_config* cfg, const float* aabb, const float* o,
@@ -769,7 +794,8 @@ static int32_t render_backward(const tfh_vm* density, const tfh_vm* appearance,
     if (ws.dlcopy && !fuse) TFH_TRY(sum_copies(ws.dlcopy, ws.dnlc, dln, dgrad->line, st));
   }
   TFH_TRY(mlp_bwd_rows(mlp, ws.feats, dirs, cams, M, k, ws.dc, ws.dfeat, mgrad, cfg->mlp_precision,
-                       ws.mlp_ws, ws.mlp_ws_bytes, st, ws.act, ws.act ? ws.rgb : nullptr));
+                       ws.mlp_ws, ws.mlp_ws_bytes, st, ws.act, ws.act ? ws.rgb : nullptr,
+                       ws.mlp_rws, ws.mlp_rws_bytes));
   if (fuse) {
     ProfScope ps("factor_scatter", st);
     if (ws.alcopy) TFH_TRY(zero_copies(ws.alcopy, ws.anlc * aln, st));
@@ -867,7 +893,6 @@ static size_t carve_render_fwd(Carve& cv, const tfh_render_config* cfg, const tf
   const int64_t N = cfg->density_samples_per_ray, k = cfg->appearance_samples_per_ray;
   const int64_t M = R * k;
   ws.d.pts = cv.take<float>(R * N * 3);
-  cv.take<float>(R * N);  // (unused)
   ws.d.sigma = cv.take<float>(R * N);
   ws.d.delta = cv.take<float>(R * N);
   ws.d.w = cv.take<float>(R * N);
@@ -877,7 +902,7 @@ static size_t carve_render_fwd(Carve& cv, const tfh_render_config* cfg, const tf
   ws.d.ray = cv.take<float>(R * 4);
   ws.d.out = nullptr;
   ws.feats = cv.take<float>(M * F);
-  ws.rgb = cv.take<float>(M * 3);
+  ws.rgb = cv.take<float>(mlp ? M * 3 : 0);
   ws.gout = ws.dc = ws.dfeat = ws.mse_part = nullptr;
   ws.mlp_ws_bytes = mlp ? mlp_fwd_workspace(mlp, cfg->mlp_precision) : 0;
   ws.mlp_ws = cv.take<char>((int64_t)ws.mlp_ws_bytes);
@@ -951,12 +976,11 @@ int32_t train_step_run(const tfh_vm* density, const tfh_vm* appearance, const tf
   TFH_TRY(require_device());
   Carve cv(workspace, workspace_bytes);
   RenderWs ws;
-  carve_render(cv, cfg, mlp, 3 * appearance->channels, num_rays, ws);
+  carve_step(cv, cfg, mlp, 3 * appearance->channels, num_rays, ws);
+  take_train(cv, cfg, mlp, num_rays, density, appearance, ws);
   if (!cv.ok)
     return fail(TFH_ERR_WORKSPACE, "tfh_train_step: workspace of %zu bytes, need %zu",
                 workspace_bytes, cv.off);
-  take_act(cv, cfg, mlp, num_rays, ws);
-  take_line_copies(cv, density, appearance, ws);
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, mse_out, (int64_t)1, 0.0f);
   TFH_TRY(check_launch("train step: clear mse"));
   RayIn in = make_rayin(cfg, aabb, origins, directions, num_rays, jitter, base_ts, base_steps,
@@ -993,7 +1017,11 @@ static int32_t render_fwd_run(const tfh_vm* density, const tfh_vm* appearance, c
   const int64_t F = cfg->mode == TFH_MODE_RGB ? 3 * appearance->channels : 0;
   Carve cv(workspace, workspace_bytes);
   RenderWs ws;
-  carve_render(cv, cfg, cfg->mode == TFH_MODE_RGB ? mlp : nullptr, F, num_rays, ws);
+  const tfh_mlp* shades = cfg->mode == TFH_MODE_RGB ? mlp : nullptr;
+  if (keep)
+    carve_render(cv, cfg, shades, F, num_rays, ws);
+  else
+    carve_render_fwd(cv, cfg, shades, F, num_rays, ws);
   if (!cv.ok)
     return fail(TFH_ERR_WORKSPACE, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes,
                 cv.off);
@@ -1088,6 +1116,17 @@ size_t tfh_render_workspace_size(const tfh_render_config* cfg, const tfh_mlp* ml
   return carve_render(cv, cfg, mlp, 3 * appearance_channels, num_rays, ws);
 }
 
+size_t tfh_render_only_workspace_size(const tfh_render_config* cfg, const tfh_mlp* mlp,
+                                      int64_t appearance_channels, int64_t num_rays) {
+  if (check_cfg(cfg, "tfh_render_only_workspace_size") != TFH_OK || num_rays < 0) return 0;
+  if (mlp && check_mlp(mlp, "tfh_render_only_workspace_size") != TFH_OK) return 0;
+  const bool rgb = cfg->mode == TFH_MODE_RGB;
+  Carve cv(nullptr, 0);
+  RenderWs ws;
+  return carve_render_fwd(cv, cfg, rgb ? mlp : nullptr, rgb ? 3 * appearance_channels : 0, num_rays,
+                          ws);
+}
+
 size_t tfh_train_step_workspace_size(const tfh_render_config* cfg, const tfh_mlp* mlp,
                                      int64_t appearance_channels, int64_t num_rays) {
   if (check_cfg(cfg, "tfh_train_step_workspace_size") != TFH_OK || num_rays < 0 || !mlp ||
@@ -1095,8 +1134,8 @@ size_t tfh_train_step_workspace_size(const tfh_render_config* cfg, const tfh_mlp
     return 0;
   Carve cv(nullptr, 0);
   RenderWs ws;
-  return carve_render(cv, cfg, mlp, 3 * appearance_channels, num_rays, ws) +
-         act_bytes(cfg, mlp, num_rays) + line_copy_bytes();
+  carve_step(cv, cfg, mlp, 3 * appearance_channels, num_rays, ws);
+  return cv.off + train_bytes(cfg, mlp, num_rays) + line_copy_bytes();
 }
 
 int32_t tfh_render_fwd(const tfh_vm* density, const tfh_vm* appearance, const tfh_mlp* mlp,
@@ -1174,9 +1213,9 @@ size_t tfh_train_step_proposal_workspace_size(const tfh_render_config* cfg, cons
     return 0;
   Carve cv(nullptr, 0);
   RenderWs ws;
-  carve_render(cv, cfg, mlp, 3 * appearance_channels, num_rays, ws);
+  carve_step(cv, cfg, mlp, 3 * appearance_channels, num_rays, ws);
   cv.take<float>(num_rays * (cfg->density_samples_per_ray + 1));
-  return cv.off + prop_workspace_bytes(pc, field, num_rays) + act_bytes(cfg, mlp, num_rays) +
+  return cv.off + prop_workspace_bytes(pc, field, num_rays) + train_bytes(cfg, mlp, num_rays) +
          line_copy_bytes();
 }
 
@@ -1226,15 +1265,14 @@ int32_t tfh_train_step_proposal(const tfh_vm* density, const tfh_vm* appearance,
   const int N = cfg->density_samples_per_ray;
   Carve cv(workspace, workspace_bytes);
   RenderWs ws;
-  carve_render(cv, cfg, mlp, 3 * appearance->channels, R, ws);
+  carve_step(cv, cfg, mlp, 3 * appearance->channels, R, ws);
   float* edges = cv.take<float>(R * (N + 1));
   PropWs pws;
   carve_prop(cv, pc, field, prop_mlp, R, pws);
+  take_train(cv, cfg, mlp, R, density, appearance, ws);
   if (!cv.ok)
     return fail(TFH_ERR_WORKSPACE, "%s: workspace of %zu bytes, need %zu", who, workspace_bytes,
                 cv.off);
-  take_act(cv, cfg, mlp, R, ws);
-  take_line_copies(cv, density, appearance, ws);
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, mse_out, (int64_t)1, 0.0f);
   hipLaunchKernelGGL(k_fill, dim3(1), dim3(64), 0, st, prop_loss_out, (int64_t)1, 0.0f);
   TFH_TRY(check_launch("train step: clear losses"));

@@ -188,13 +188,20 @@ class _RenderFn(torch.autograd.Function):
         return (None, *ctx.env.backward(gout))
 
 
+def _leaves(lp: LearnableParams):
+    ds, as_ = lp.density_tensor.stacked_single_vm, lp.appearance_tensor.stacked_single_vm
+    return [ds.plane, ds.line, as_.plane, as_.line,
+            *networks.FeatureMlp.flat_leaves(lp.appearance_mlp_params)]
+
+
 class _RenderEnv:
-    """Holds the structs, noise and workspace of one render_rays call."""
+    """Holds the structs, noise and workspace of one render_rays call. keep: the
+    workspace has the room for backward(), and forward() writes what it reads."""
 
     def __init__(self, mlp: networks.FeatureMlp, lp: LearnableParams, aabb, rays, prng_key,
                  config: RenderConfig, workspace: Optional[torch.Tensor] = None,
-                 sample_proposal: bool = True, alloc_workspace: bool = True):
-        self.mlp, self.lp, self.config = mlp, lp, config
+                 sample_proposal: bool = True, alloc_workspace: bool = True, keep: bool = True):
+        self.mlp, self.lp, self.config, self.keep = mlp, lp, config, keep
         self.device = rays.origins.device
         self.aabb = aabb.to(device=self.device, dtype=torch.float32).contiguous()
         self.o = rays.origins.to(torch.float32).contiguous()
@@ -232,8 +239,10 @@ class _RenderEnv:
         self.avm = lp.appearance_tensor.c_struct()
         ca = lp.appearance_tensor.stacked_single_vm.channel_dim()
         self.cmlp = mlp.c_struct(lp.appearance_mlp_params, 3 * ca) if mlp else None
-        ws_bytes = _lib.lib.tfh_render_workspace_size(
-            ctypes.byref(self.cfg), ctypes.byref(self.cmlp) if self.cmlp else None, ca, self.r)
+        size = _lib.lib.tfh_render_workspace_size if keep else \
+            _lib.lib.tfh_render_only_workspace_size
+        ws_bytes = size(ctypes.byref(self.cfg), ctypes.byref(self.cmlp) if self.cmlp else None, ca,
+                        self.r)
         if not alloc_workspace:
             self.ws = None  # the caller runs a fused entry point with its own workspace
         elif workspace is not None and workspace.numel() >= int(ws_bytes):
@@ -244,22 +253,20 @@ class _RenderEnv:
     def _mlp_ref(self):
         return ctypes.byref(self.cmlp) if self.cmlp else None
 
-    def forward(self, keep: bool = True) -> torch.Tensor:
-        """keep: write what backward() reads."""
+    def forward(self, keep: Optional[bool] = None) -> torch.Tensor:
+        keep = self.keep if keep is None else keep
         rgb = self.config.mode is RenderMode.RGB
         out = torch.empty((self.r, 3) if rgb else (self.r,), dtype=torch.float32,
                           device=self.device)
-        _lib.call("tfh_render_fwd" if keep else "tfh_render_only", ctypes.byref(self.dvm), ctypes.byref(self.avm), self._mlp_ref(),
-                  ctypes.byref(self.cfg), _lib.ptr(self.aabb), _lib.ptr(self.o), _lib.ptr(self.d),
+        _lib.call("tfh_render_fwd" if keep else "tfh_render_only", ctypes.byref(self.dvm),
+                  ctypes.byref(self.avm), self._mlp_ref(), ctypes.byref(self.cfg), _lib.ptr(self.aabb), _lib.ptr(self.o), _lib.ptr(self.d),
                   _lib.ptr(self.cams), self.r, _lib.ptr(self.jitter), _lib.ptr(self.base_ts),
                   _lib.ptr(self.base_steps), _lib.ptr(self.gumbel), _lib.ptr(out),
                   _lib.ptr(self.ws), self.ws.numel(), _lib.stream())
         return out
 
     def leaves(self):
-        ds, as_ = self.lp.density_tensor.stacked_single_vm, self.lp.appearance_tensor.stacked_single_vm
-        return [ds.plane, ds.line, as_.plane, as_.line,
-                *networks.FeatureMlp.flat_leaves(self.lp.appearance_mlp_params)]
+        return _leaves(self.lp)
 
     def backward(self, gout):
         gout = gout.contiguous()
@@ -282,11 +289,11 @@ def render_rays(appearance_mlp: networks.FeatureMlp, learnable_params: Learnable
                 config: RenderConfig) -> torch.Tensor:
     """render.py:105-279: (R,3) RGB or (R,) distances. Differentiable w.r.t. the
     learnable parameters in RGB mode (hand-written backward in the library)."""
-    env = _RenderEnv(appearance_mlp, learnable_params, aabb, rays_wrt_world, prng_key, config)
-    if config.mode is RenderMode.RGB and torch.is_grad_enabled() and any(
-            t.requires_grad for t in env.leaves()):
-        return _RenderFn.apply(env, *env.leaves())
-    return env.forward(keep=False)
+    grad = config.mode is RenderMode.RGB and torch.is_grad_enabled() and any(
+        t.requires_grad for t in _leaves(learnable_params))
+    env = _RenderEnv(appearance_mlp, learnable_params, aabb, rays_wrt_world, prng_key, config,
+                     keep=grad)
+    return _RenderFn.apply(env, *env.leaves()) if grad else env.forward()
 
 
 def render_rays_batched(appearance_mlp: networks.FeatureMlp, learnable_params: LearnableParams,
