@@ -54,9 +54,9 @@ __host__ __device__ inline int round_up(int x, int m) { return (x + m - 1) / m *
 
 // Kept activations: the forward's relu(z1) and relu(z2) (before any camera
 // embedding), 256 values a row, for the backward. FP32, or BF16 with the BF16
-// MLP, whose backward only reads them as BF16 MFMA operands and as ReLU signs
-// (the rounding keeps signs and zeros), so BF16 storage changes no result and
-// halves the traffic. They are stored in groups of 32 rows in the order a
+// MLP, at half the traffic: without an embedding its backward only reads them as
+// BF16 MFMA operands and as ReLU signs (the rounding keeps signs and zeros), so
+// BF16 storage changes no result then (kept_bf16). They are stored in groups of 32 rows in the order a
 // 16x16 tile's lanes hold them: relu(z1) then relu(z2), each 8 column tiles
 // of 64 lanes x 8 values (rows 4 (lane / 16) + q of the first row tile, then
 // of the second, column lane % 16), so that the layer that computes a value
@@ -322,19 +322,9 @@ __device__ void load_tile_rows(const MlpDims& d, const float* __restrict__ feats
 // Fills X[:, S:EP] = [d, FE(h0, nf), FE(d, nv), 0...] from h0 = X[:, 0:S]
 // (networks.py:13-35, 68-76): FE(v, n)[j*2n + q] = sin(2^q v_j) and
 // [j*2n + n + q] = cos(2^q v_j).
-// The forward (DOUBLE = false) takes one sincosf per (row, value, frequency).
-// The backward's recompute (DOUBLE = true) takes one per (row, value): q = 0
-// by sincosf, q = 1 from it by sin 2a = 2 sin a cos a and
-// cos 2a = (cos a - sin a)(cos a + sin a), q >= 2 by sincosf again; its
-// values feed only the weight gradient of layer 1 and the encoding's own
-// backward, where the identities' ~2 ulp stay below the gradient tolerance
-// (taken in the forward, their bias shifted the outputs a whole-batch
-// gradient sums over a million rows). With XB (stride ldB), h0 is first
-// formed as X[:, 0:S] + XB[:, 0:S] and written back to X (a layer 0
-// computed in two K parts).
-template <int TM, bool DOUBLE = false>
-__device__ void encode_tile(const MlpDims& d, float* X, const float* Ds,
-                            const float* XB = nullptr, int ldB = 0) {
+// One sincosf per (row, value, frequency).
+template <int TM>
+__device__ void encode_tile(const MlpDims& d, float* X, const float* Ds) {
   const int fe0 = d.S + 3;
   const int fe1 = fe0 + 2 * d.nf * d.S;
   const int fe2 = fe1 + 2 * d.nv * 3;
@@ -345,55 +335,19 @@ __device__ void encode_tile(const MlpDims& d, float* X, const float* Ds,
     const int c = t < 3 ? d.S + t : fe2 + (t - 3);
     X[i * d.ldE + c] = t < 3 ? Ds[i * 3 + t] : 0.0f;
   }
-  if constexpr (!DOUBLE) {
-    const int nfe = d.S * d.nf + 3 * d.nv;  // (value, frequency) pairs per row
-    for (int e = threadIdx.x; e < TM * nfe; e += blockDim.x) {
-      const int i = e / nfe, t = e % nfe;
-      const bool feat = t < d.S * d.nf;
-      const int u = feat ? t : t - d.S * d.nf;
-      const int n = feat ? d.nf : d.nv;
-      const int j = u / n, q = u % n;
-      const float src = feat ? X[i * d.ldE + j] : Ds[i * 3 + j];
-      float sv, cv;
-      sincosf(src * (float)(1 << q), &sv, &cv);
-      const int c = (feat ? fe0 : fe1) + j * 2 * n + q;
-      X[i * d.ldE + c] = sv;
-      X[i * d.ldE + c + n] = cv;
-    }
-    return;
-  }
-  const int nval = d.S + 3;  // values per row: h0, then the direction
-  for (int e = threadIdx.x; e < TM * nval; e += blockDim.x) {
-    const int i = e / nval, u = e % nval;
-    const bool feat = u < d.S;
-    const int j = feat ? u : u - d.S;
+  const int nfe = d.S * d.nf + 3 * d.nv;  // (value, frequency) pairs per row
+  for (int e = threadIdx.x; e < TM * nfe; e += blockDim.x) {
+    const int i = e / nfe, t = e % nfe;
+    const bool feat = t < d.S * d.nf;
+    const int u = feat ? t : t - d.S * d.nf;
     const int n = feat ? d.nf : d.nv;
-    float v;
-    if (feat) {
-      v = X[i * d.ldE + j];
-      if (XB) {
-        v += XB[i * ldB + j];
-        X[i * d.ldE + j] = v;
-      }
-    } else {
-      v = Ds[i * 3 + j];
-    }
-    if (n == 0) continue;
-    float* fe = X + i * d.ldE + (feat ? fe0 : fe1) + j * 2 * n;
+    const int j = u / n, q = u % n;
+    const float src = feat ? X[i * d.ldE + j] : Ds[i * 3 + j];
     float sv, cv;
-    sincosf(v, &sv, &cv);
-    fe[0] = sv;
-    fe[n] = cv;
-    if (n > 1) {
-      fe[1] = 2.0f * sv * cv;
-      fe[n + 1] = (cv - sv) * (cv + sv);
-    }
-    for (int q = 2; q < n; ++q) {
-      float s2, c2;
-      sincosf(v * (float)(1 << q), &s2, &c2);
-      fe[q] = s2;
-      fe[n + q] = c2;
-    }
+    sincosf(src * (float)(1 << q), &sv, &cv);
+    const int c = (feat ? fe0 : fe1) + j * 2 * n + q;
+    X[i * d.ldE + c] = sv;
+    X[i * d.ldE + c + n] = cv;
   }
 }
 
@@ -403,10 +357,9 @@ __device__ void encode_tile(const MlpDims& d, float* X, const float* Ds,
 // Work items are (column tile, group of RTI row tiles): RTI = TM/16 keeps a
 // column strip's B operands for all rows of the tile (few waves), RTI = 1
 // spreads a layer over more waves.
-// L12 == false stops after the encoding (H1 and H2 come from elsewhere).
 // FT: the feature rows' type (float, stride ldF; or __bf16 with the BF16
 // MLP, stride kFsLdB).
-template <int TM, int NW, bool BF, int RTI, bool L12 = true, class FT = float, bool KB = BF>
+template <int TM, int NW, bool BF, int RTI, class FT = float, bool KB = BF>
 // kept (optional, TM == kKeptGroup): the tile's kept activations (KB: in BF16).
 __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<BF>& op,
                                const FT* Fs, float* X, float* H0, float* H1, float* H2p,
@@ -439,7 +392,6 @@ __device__ void forward_hidden(const MlpDims& d, const MlpW& w, const Operands<B
   __syncthreads();
   encode_tile<TM>(d, X, Ds);
   __syncthreads();
-  if constexpr (!L12) return;
   // layer 1: (TM x EP) @ (EP x U) + b1, relu -> H1
   for (int it = wave; it < (kU / 16) * RG; it += NW) {
     const int ct = it / RG, r0 = 16 * RTI * (it % RG);
@@ -642,8 +594,8 @@ __global__ void __launch_bounds__(NW * 64) k_mlp_fwd(MlpDims d_arg, MlpW w, MlpP
   // layer 2 reads H1 and writes H2 over X (dead after layer 1)
   void* kept = act ? reinterpret_cast<char*>(act) + tile * kKeptGroupBytes<KB> : nullptr;
   using FT = typename std::conditional<FB16, __bf16, float>::type;
-  forward_hidden<TM, NW, BF, TM / 16, true, FT, KB>(d, w, op, reinterpret_cast<const FT*>(regA), regB,
-                                                nullptr, regA, regB, regB, Ds, Cs, kept);
+  forward_hidden<TM, NW, BF, TM / 16, FT, KB>(d, w, op, reinterpret_cast<const FT*>(regA), regB,
+                                              nullptr, regA, regB, regB, Ds, Cs, kept);
   // (every wave is past its reads of H1, region A, before R3 overwrites it)
   forward_out<TM, NW, BF>(d, w, op, regB, R3);
   for (int e = threadIdx.x; e < TM * 3; e += blockDim.x) {

@@ -46,7 +46,8 @@ __host__ __device__ inline PropPack prop_pack(int F) {
 // entries 4 kq .. 4 kq + 3 of row r; with unit 16 c + 4 e + kq of tile c at
 // entry 4 kq + e (kUnit), register e of tile c is the operand that product
 // 4 c + e of the next layer (inputs 16 c + 4 e + kq) reads, and no activation
-// passes through LDS. The order of every FP32 sum is that of prop_hidden.
+// passes through LDS. Every FP32 sum runs over the inputs in ascending order,
+// four to a product.
 //
 // Bound by the FP32 matrix rate: 24 + 64 + 16 products of 16x16x4 per 16 rows
 // (the last 16 for one output), 1.35 ms for 12.6 M rows. With activations of a
