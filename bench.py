@@ -41,7 +41,9 @@ def stage_model(stage, R, N, k, cd, ca, precision, n_params, prop=None):
     (nf=nv=2) and 11,392 per proposal-MLP row (2 (24*64 + 64*64 + 64)). The
     training step keeps the MLP's hidden activations, so its backward does
     the input and weight gradients of every layer (2 x 79,712 per row) plus
-    the recompute of layer 0 (2 x 144 x 27).
+    the recompute of layer 0 (2 x 144 x 27). The FP32 backward forms a product
+    from six BF16 ones (three planes per operand), so its peak is a sixth of
+    the BF16 matrix peak.
     prop: (samples per ray over the proposal rounds, proposal channels)."""
     M = R * k
     mlp_row = 2 * (144 * 27 + 150 * 128 + 128 * 128 + 128 * 3)
@@ -53,7 +55,8 @@ def stage_model(stage, R, N, k, cd, ca, precision, n_params, prop=None):
     if stage == "mlp_fwd_kernel":
         return "mfma", M * mlp_row, "TFLOP/s", mfma_peak
     if stage == "mlp_bwd":
-        return "mfma", M * (2 * mlp_row + 2 * 144 * 27), "TFLOP/s", mfma_peak
+        peak = PEAK_TFLOPS["bf16"] / 6 if precision == "fp32" else mfma_peak
+        return "mfma", M * (2 * mlp_row + 2 * 144 * 27), "TFLOP/s", round(peak, 1)
     if stage == "composite_bwd_density_scatter":
         return "hbm", R * N * (2 * 72 * cd + 36), "GB/s", PEAK_HBM_GBS
     if stage == "appearance_scatter":

@@ -43,3 +43,14 @@ def test_compositing_compulsory_bytes():
     assert bench.compulsory_bytes("composite_rgb", R, N, K, CD, CA, G, 1) == M * 16 + R * 44
     topk = bench.compulsory_bytes("composite_rgb", R, N, 64, CD, CA, G, 1)
     assert topk == R * 64 * 20 + R * 44
+
+
+def test_backward_peak_is_that_of_its_products():
+    """The FP32 MLP backward runs on the BF16 units, six products for one; the
+    BF16 one takes one, and the FP32 forward the FP32 units."""
+    def peak(stage, precision):
+        return bench.stage_model(stage, R, N, K, CD, CA, precision, 1)[3]
+
+    assert peak("mlp_bwd", "fp32") == round(2500.0 / 6, 1)
+    assert peak("mlp_bwd", "bf16") == 2500.0
+    assert peak("mlp_fwd_kernel", "fp32") == 157.3
