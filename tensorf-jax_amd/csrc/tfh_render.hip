@@ -762,12 +762,13 @@ static int32_t render_backward(const tfh_vm* density, const tfh_vm* appearance,
   const int64_t aln = 3 * appearance->grid_dim * appearance->channels;
   // every density sample, row r*N + i
   const RaySamples dsrc{ws.d.pts, nullptr, N, N};
-  const bool dsorted = ws.ds && sorted_scatter_ok(*density, R * N, ws.sort);
+  const bool dsort = ws.ds && sorted_scatter_ok(*density, R * N, ws.sort);
   // every sample shaded, one grid: one sort and one pass per scatter serve
   // both fields, after the MLP backward (dL/dsigma waits in the workspace)
   const RowGrad gsrc{ws.dfeat, (int)appearance->channels};
-  const bool fuse = dsorted && ws.d.idx == nullptr && sorted_scatter_ok(*appearance, M, ws.sort) &&
+  const bool fuse = dsort && ws.d.idx == nullptr && sorted_scatter_ok(*appearance, M, ws.sort) &&
                     two_field_scatter_ok(*density, *appearance, gsrc);
+  const bool dsorted = fuse || (dsort && sorted_scatter_pays(*density, R * N));
   {
     ProfScope ps(fuse ? "composite_bwd" : "composite_bwd_density_scatter", st);
     tfh_vm_grad dg = *dgrad;
@@ -831,7 +832,8 @@ static int32_t render_backward(const tfh_vm* density, const tfh_vm* appearance,
   }
   RaySamples src{ws.d.pts, ws.d.idx, k, N};
   ProfScope ps("appearance_scatter", st);
-  const bool sorted = sorted_scatter_ok(*appearance, M, ws.sort);
+  const bool sorted =
+      sorted_scatter_ok(*appearance, M, ws.sort) && sorted_scatter_pays(*appearance, M);
   if (sorted) {
     // with every sample shaded the rows are the density scatter's, and on the
     // same grid its sorted pairs serve again

@@ -938,6 +938,18 @@ inline bool sorted_scatter_ok(const tfh_vm& vm, int64_t M, const SortWs& s) {
   return s.order && vm.channels <= 64 && vm.grid_dim <= kSortMaxGrid && M <= kSortMaxRows;
 }
 
+// Whether the sort pays for a field by itself. Up to 8 channels the direct scatter
+// adds 32 bytes a tap from 8 lanes a row, and for few rows it is done before the
+// sort's four launches are: 8 channels, compositing backward and scatter, direct and
+// sorted, us: 2 thousand rows 24 and 73, 33 thousand 54 and 79, 102 thousand 95 and
+// 102 (G = 128; 127 and 105 at G = 24), 226 thousand 167 and 131; the appearance
+// scatter of 34 thousand 36 and 77. Wider fields take the sort from the first row
+// (16 and 48 channels, 256 rows: 334 and 115).
+constexpr int64_t kSortNarrowRows = 3 << 15;
+inline bool sorted_scatter_pays(const tfh_vm& vm, int64_t M) {
+  return vm.channels > 8 || M >= kSortNarrowRows;
+}
+
 // Whether a field can take the walks' quad lanes.
 template <class GS>
 inline bool quad_lanes_ok(const tfh_vm& vm, const GS& g) {
